@@ -15,7 +15,7 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "lib
 
 FSP_F32 = 0
 FSP_F64 = 1
-ABI_VERSION = 17
+ABI_VERSION = 18
 
 _lib = None
 
@@ -50,6 +50,12 @@ SIGNATURES = {
     "fsp_plan_row_blocks": (_i32, [_p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _p]),
     "fsp_spmv_csr": (_i32, [_i32, _i32, _p, _p, _p, _i32, _i64, _i64, _p, _p, _p, _i64, _p, _p,
                             _i64, _i64, _p, _p, _p, _p, _i64, _i32, _p]),
+    "fsp_spmv_slices": (_i64, [_i64, _i64]),
+    "fsp_spmv_slice_keep": (_i64, []),
+    "fsp_spmv_sliced": (_i32, [_i32, _i32, _p, _p, _p, _i32, _i64, _i64, _p, _p, _p, _p, _i32,
+                               _p]),
+    "fsp_csr_check_partial_len": (_i64, []),
+    "fsp_csr_check": (_i32, [_p, _i32, _i64, _p, _i32, _i64, _p, _p, _i32, _p, _p, _p]),
     "fsp_spmv_scratch_slots": (_i64, []),
     "fsp_spmv_csr_static": (_i32, [_i32, _i32, _p, _p, _p, _i32, _i64, _i64, _p, _p, _p, _i64, _p,
                                    _p, _i64, _i64, _i64, _p, _p, _p, _i64, _i32, _p]),

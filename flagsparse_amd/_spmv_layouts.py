@@ -227,6 +227,48 @@ class RowBlockLayout:
         return y
 
 
+class SliceLayout:
+    """CSR arrays (16-byte aligned) cut into slices of equal work inside the call itself
+    (csrc/slices.hip): nothing is planned, so it is what a matrix used once runs on."""
+
+    kind = "slices"
+
+    def __init__(self, data, cols, rowptr, max_row_nnz=None):
+        self.data = _aligned(data)
+        self.cols = _aligned(cols)
+        self.nnz = int(data.numel())
+        self.rowptr_bits = 32 if self.nnz <= _common.ROWPTR32_MAX_NNZ else 64
+        self.rowptr = rowptr.to(torch.int32 if self.rowptr_bits == 32
+                                else torch.int64).contiguous()
+        self.n_rows = int(rowptr.numel()) - 1
+        L = _abi.lib()
+        # an unknown longest row may be cut
+        self.cut_rows = max_row_nnz is None or max_row_nnz > L.fsp_spmv_slice_keep()
+        n = int(L.fsp_spmv_slices(self.n_rows, self.nnz))
+        self._scratch = torch.empty(2 * (n + 1) + 2 * n, dtype=torch.int64,
+                                    device=self.data.device)
+        self._sums = self._scratch.data_ptr() + 16 * (n + 1)
+        self._order = StreamOrder(self.data.device)
+
+    def kernel_name(self):
+        return "spmv_slices_kernel"
+
+    def describe(self):
+        return {"layout": self.kind, "cut_rows": self.cut_rows}
+
+    def launch(self, x, y, acc_f64):
+        stream = self._order.stream(y.device, (self._scratch, self.data, self.cols, self.rowptr))
+        _abi.check(
+            _abi.lib().fsp_spmv_sliced(_abi.dtype_code(self.data.dtype), int(acc_f64),
+                                       self.data.data_ptr(), self.cols.data_ptr(),
+                                       self.rowptr.data_ptr(), self.rowptr_bits, self.n_rows,
+                                       self.nnz, x.data_ptr(), y.data_ptr(),
+                                       self._scratch.data_ptr(), self._sums, int(self.cut_rows),
+                                       stream),
+            "fsp_spmv_sliced")
+        return y
+
+
 def band_block_offset(cols, rowptr, n_desc):
     """The dominant distance, in row blocks, between a row and the far diagonals it reads, for
     banded / stencil matrices (a 2-D 5-point stencil on a W-wide grid reads rows +-W): the most
@@ -1368,15 +1410,16 @@ def xcs_layout(data, cols, rowptr, n_cols, panels_per_xcd=None):
     return XcsLayout(data, cols, rowptr, n_cols, panels_per_xcd, item_format=0)
 
 
-def build_layout(data, cols, rowptr, n_cols, one_shot=False):
+def build_layout(data, cols, rowptr, n_cols, one_shot=False, max_row_nnz=None):
     """The layout for one CSR (or COO row-run) matrix: XCS when it pays, else row blocks.
-    one_shot: the layout serves a single call (no prepared object), so the row-block layout,
-    which builds in about a millisecond, is taken; the XCS layouts take tens of milliseconds to
-    build (cfg3: 46 ms for a 0.32 ms product, against 3.3 ms for the row-block product)."""
+    one_shot: the layout serves a single call (no prepared object) and is asked for no run to
+    row map, so the slices, which need no plan, are taken; the row blocks' plan alone takes 0.6
+    ms for a million rows and the staged-x layout tens of milliseconds (a power law of 8.4M rows:
+    28 ms for a 0.2 ms product).  max_row_nnz: the longest row, where the caller knows it."""
     mode = FORCE
     nnz = int(data.numel())
     if mode is None and one_shot:
-        mode = "rowblock"
+        return SliceLayout(data, cols, rowptr, max_row_nnz)
     if mode is None:
         mode = ("xstage" if STAGED else "xcs") \
             if prefers_xcs(cols, rowptr, n_cols, data.element_size()) else "rowblock"
@@ -1408,7 +1451,7 @@ def build_layout(data, cols, rowptr, n_cols, one_shot=False):
     return RowBlockLayout(data, cols, rowptr)
 
 
-__all__ = ["RowBlockLayout", "XcsLayout", "PanelLayout", "XcsHybridLayout", "XstageLayout",
+__all__ = ["RowBlockLayout", "SliceLayout", "XcsLayout", "PanelLayout", "XcsHybridLayout", "XstageLayout",
            "build_layout",
            "xcs_layout",
            "prefers_xcs", "sample_indices", "FORCE"]

@@ -19,6 +19,11 @@ constexpr int64_t kSpmvChunkCap = kSpmvChunkUnitsPerThread * 4 * 256 - 3;
 constexpr int64_t kSpmmSlots = 2048;                     // LDS (col, val) slots per SpMM block
 constexpr int64_t kSpmmNnzCap = kSpmmSlots - 3;
 constexpr int64_t kIndexStatsBlocks = 1024;             // first-pass workgroups of fsp_index_stats
+constexpr int64_t kCsrCheckBlocks = 2048;               // first-pass workgroups of fsp_csr_check
+// Sliced SpMV: positions (rows + entries) per slice, and the longest row that no boundary cuts.
+constexpr int64_t kSpmvSliceSlots = 1024;               // LDS product slots per slice
+constexpr int64_t kSpmvSliceItems = 760;
+constexpr int64_t kSpmvSliceKeep = 256;
 constexpr int64_t kXcsItemCap = 2048;                    // entries of one XCS item
 constexpr int64_t kXcsRowsCap = 8192;                    // rows of one XCS tile
 constexpr int64_t kXcsWinSlotsCap = 4096;                // partial slots of one combine window
@@ -43,6 +48,12 @@ template <> inline int fill_zero<float>(float* y, int64_t n, hipStream_t st) {
 template <> inline int fill_zero<double>(double* y, int64_t n, hipStream_t st) {
   return fill_zero_f64(y, n, st);
 }
+
+// Slices of W positions (slices.hip): their number, and the table of their n + 1 boundaries
+// {row, entry} as int64 pairs; rows of at most T entries are not cut.
+int64_t slice_count(int64_t n_rows, int64_t nnz, int64_t W);
+int launch_slice_table(const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t nnz,
+                       int64_t W, int64_t T, int64_t* table, hipStream_t st);
 
 int set_error(int code, const std::string& msg);
 int check_hip(hipError_t e, const char* what);

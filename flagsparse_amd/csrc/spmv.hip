@@ -32,43 +32,6 @@ constexpr int kStreamUPT = kStreamSlots / (4 * kBlock);  // quads per thread in 
 constexpr int kChunkUPT = (int)kSpmvChunkUnitsPerThread;
 static_assert(kStreamUPT * 4 * kBlock == kStreamSlots, "stream slots must be whole quads per thread");
 
-// x[c] for the entries a thread holds (c >= 0), 0 for the empty positions (c < 0), with all
-// of a thread's gathers in flight together.  When the value is widened to the accumulator
-// type (fp32 x summed in fp64), a load under a per-lane condition became an exec-masked region
-// with the conversion inside, and the compiler waited for each gather before issuing the next;
-// those gathers are therefore issued for every position - an empty one reads x[0], which
-// exists whenever the descriptor has an entry (any), the only case in which it runs - and the
-// value dropped afterwards.  Without a conversion the conditional form keeps its loads
-// together and needs fewer registers (fp64 row blocks: 72 against 84 VGPRs, 7 against 5 waves
-// per SIMD).
-template <int U, typename A, typename T>
-__device__ __forceinline__ void gather_x(const T* __restrict__ x, const int (&c)[U][4], bool any,
-                                         T (&xv)[U][4]) {
-  if constexpr (sizeof(A) == sizeof(T)) {
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) xv[u][j] = c[u][j] >= 0 ? x[c[u][j]] : T(0);
-  } else {
-    if (!any) {  // uniform per workgroup
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) xv[u][j] = T(0);
-      return;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) xv[u][j] = x[c[u][j] >= 0 ? c[u][j] : 0];
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (c[u][j] < 0) xv[u][j] = T(0);
-  }
-}
-
 template <typename T, typename A, typename P, bool NT>
 __global__ __launch_bounds__(kBlock) void spmv_rowblock_kernel(
     const T* __restrict__ vals, const int* __restrict__ cols, const P* __restrict__ rowptr,

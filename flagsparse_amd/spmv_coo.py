@@ -15,9 +15,9 @@ import time
 
 import torch
 
-from . import _abi
+from . import _abi, _spmv_layouts
 from ._common import _INDEX_LIMIT_INT32
-from ._spmv_layouts import build_layout
+from ._spmv_layouts import RowBlockLayout, build_layout
 
 
 class PreparedCoo:
@@ -61,8 +61,10 @@ class PreparedCoo:
         """Kernel layout over the row runs (flagsparse_amd/_spmv_layouts.py) and the
         run -> row map, omitted when it is the identity."""
         if self._layout is None:
-            self._layout = build_layout(self.data, self.col, self.seg_starts, self.n_cols,
-                                        one_shot=self._one_shot)
+            if self._one_shot and _spmv_layouts.FORCE is None:
+                self._layout = RowBlockLayout(self.data, self.col, self.seg_starts)
+            else:
+                self._layout = build_layout(self.data, self.col, self.seg_starts, self.n_cols)
             if self.n_segs == self.n_rows:
                 self._run_rows = None  # sorted and every row present: run k is row k
             else:

@@ -25,6 +25,7 @@ from ._common import (
     _INDEX_LIMIT_INT32,
     _require_kernel_dtype,
 )
+from ._csr_check import csr_check
 from ._plan import truncate_rows
 from ._spmv_layouts import build_layout
 
@@ -80,7 +81,7 @@ class PreparedCsrSpmv:
         "max_row_nnz",
         "supports_opt",
         "_user_max_segments",
-        "_row_lengths",
+        "_lengths",
         "_opt_buckets",
         "_kernels",
         "_baseline_compute_dtype",
@@ -89,7 +90,7 @@ class PreparedCsrSpmv:
     )
 
     def __init__(self, data, kernel_indices, kernel_indptr, shape, n_rows, n_cols, block_nnz,
-                 max_segments, max_row_nnz, row_lengths, user_max_segments):
+                 max_segments, max_row_nnz, user_max_segments):
         self.data = data
         self.kernel_indices = kernel_indices
         self.kernel_indptr = kernel_indptr
@@ -109,9 +110,15 @@ class PreparedCsrSpmv:
             self._baseline_compute_dtype = data.dtype
         self._baseline_data = None
         self._user_max_segments = user_max_segments
-        self._row_lengths = row_lengths
+        self._lengths = None
         self._opt_buckets = None
         self._kernels = {}
+
+    @property
+    def _row_lengths(self):
+        if self._lengths is None:
+            self._lengths = self.kernel_indptr[1:] - self.kernel_indptr[:-1]
+        return self._lengths
 
     @property
     def opt_buckets(self):
@@ -151,14 +158,14 @@ class PreparedCsrSpmv:
 
     def _row_caps(self, opt):
         """Entries of each row the reference visits, or None when every row is complete."""
-        lengths = self._row_lengths.to(torch.int64)
         if not opt:
             limit = max(0, int(self.max_segments)) * int(self.block_nnz)
             if self.max_row_nnz <= limit:
                 return None
-            return torch.clamp(lengths, max=limit)
+            return torch.clamp(self._row_lengths.to(torch.int64), max=limit)
         if self._user_max_segments is None:
             return None
+        lengths = self._row_lengths.to(torch.int64)
         bs = _opt_bucket_block_sizes(lengths, self.data.dtype == torch.float64)
         caps = torch.minimum(lengths, bs * max(0, int(self._user_max_segments)))
         if bool(torch.equal(caps, lengths)):
@@ -176,7 +183,8 @@ class PreparedCsrSpmv:
             kc = self._kernels.get("full")
             if kc is None:
                 kc = build_layout(self.data, self.kernel_indices, self.kernel_indptr,
-                                  self.n_cols, one_shot=self._one_shot)
+                                  self.n_cols, one_shot=self._one_shot,
+                                  max_row_nnz=self.max_row_nnz)
                 self._kernels["full"] = kc
         else:
             d, c, ip = truncate_rows(self.data, self.kernel_indices, self.kernel_indptr, caps)
@@ -186,8 +194,7 @@ class PreparedCsrSpmv:
 
 
 def _prepare_spmv_csr_matrix(data, indices, indptr, shape):
-    """Validation and narrowing - spmv_csr.py:379-436 (same checks, order and exceptions;
-    the device-side checks are gathered into one host synchronisation)."""
+    """Validation and narrowing - spmv_csr.py:379-436 (same checks, order and exceptions)."""
     if not all(torch.is_tensor(t) for t in (data, indices, indptr)):
         raise TypeError("data, indices, indptr must all be torch.Tensor")
     if data.ndim != 1 or indices.ndim != 1 or indptr.ndim != 1:
@@ -210,38 +217,24 @@ def _prepare_spmv_csr_matrix(data, indices, indptr, shape):
     indices = indices.contiguous()
     indptr = indptr.contiguous()
     nnz = data.numel()
-
-    probes = []
-    if indptr.numel() > 0:
-        probes += [indptr[0].to(torch.int64), indptr[-1].to(torch.int64)]
-        if indptr.numel() > 1:
-            probes.append(torch.any(indptr[1:] < indptr[:-1]).to(torch.int64))
-    if nnz > 0:
-        probes += [indices.min().to(torch.int64), indices.max().to(torch.int64)]
-    vals = torch.stack(probes).tolist() if probes else []
-    pos = 0
-    if indptr.numel() > 0:
-        first, last = vals[0], vals[1]
-        pos = 2
+    # one pass over the index arrays, one host synchronisation
+    ptr_bits = 32 if nnz <= _INDEX_LIMIT_INT32 else 64
+    no_rows = indptr.numel() == 0  # n_rows of -1: nothing to check in the row pointers
+    (first, last, decreases, max_row_nnz, min_index, max_index), kernel_indices, kernel_indptr = \
+        csr_check(indices, indptr.new_zeros(1) if no_rows else indptr, ptr_bits)
+    if not no_rows:
         if first != 0:
             raise ValueError("indptr must start at zero")
         if last != nnz:
             raise ValueError("indptr[-1] must equal nnz")
-        if indptr.numel() > 1:
-            if vals[2]:
-                raise ValueError("indptr must be non-decreasing")
-            pos = 3
+        if decreases:
+            raise ValueError("indptr must be non-decreasing")
     if nnz > 0:
-        min_index, max_index = vals[pos], vals[pos + 1]
         if min_index < 0 or max_index >= n_cols:
             raise IndexError("indices out of range for n_cols")
         if max_index > _INDEX_LIMIT_INT32:
             raise ValueError(f"int64 column index {max_index} exceeds Triton int32 kernel range")
-    kernel_indices = indices.to(torch.int32) if indices.dtype == torch.int64 else indices
-    kernel_indptr = indptr.to(torch.int32) if nnz <= _INDEX_LIMIT_INT32 else indptr.to(torch.int64)
-    row_lengths = kernel_indptr[1:] - kernel_indptr[:-1]
-    max_row_nnz = int(row_lengths.max().item()) if n_rows > 0 else 0
-    return data, kernel_indices, kernel_indptr, n_rows, n_cols, row_lengths, max_row_nnz
+    return data, kernel_indices, kernel_indptr, n_rows, n_cols, max_row_nnz
 
 
 def _validate_spmv_x(x, prepared):
@@ -269,7 +262,7 @@ def prepare_spmv_csr(data, indices, indptr, shape, block_nnz=256, max_segments=N
 def _prepare_spmv_csr(data, indices, indptr, shape, block_nnz, max_segments, one_shot):
     """prepare_spmv_csr; one_shot marks a prepared object made for a single call (the layout
     that builds fastest)."""
-    (data, kernel_indices, kernel_indptr, n_rows, n_cols, row_lengths,
+    (data, kernel_indices, kernel_indptr, n_rows, n_cols,
      max_row_nnz) = _prepare_spmv_csr_matrix(data, indices, indptr, shape)
     block_nnz_use = block_nnz
     if max_segments is None:
@@ -280,10 +273,9 @@ def _prepare_spmv_csr(data, indices, indptr, shape, block_nnz, max_segments, one
     else:
         max_segments_use = max_segments
     prepared = PreparedCsrSpmv(data, kernel_indices, kernel_indptr, shape, n_rows, n_cols,
-                               block_nnz_use, max_segments_use, max_row_nnz, row_lengths,
-                               max_segments)
+                               block_nnz_use, max_segments_use, max_row_nnz, max_segments)
     prepared._one_shot = bool(one_shot)
-    if prepared.supports_opt and n_rows > 0:
+    if prepared.supports_opt and n_rows > 0 and not one_shot:
         prepared._kernel(False)  # build the descriptor table now, outside the timed calls
     return prepared
 

@@ -139,6 +139,24 @@ int fsp_plan_panel_chunks_device(const int64_t* panel_runs, int64_t n_panels,
                                  int64_t* run_pos, int64_t* panel_len, void* stream);
 
 /*
+ * The checks a CSR matrix needs before a kernel may use it, in one pass over its index arrays
+ * (spmv_csr.py:379-436, spmm_csr.py:197-255, sddmm_csr.py:46-79), with their narrowing.
+ *   indices, idx_bits  nnz columns, int32 or int64
+ *   indptr, ptr_bits   n_rows + 1 row pointers, int32 or int64
+ *   idx32              NULL, or nnz int32 (16-byte aligned): the columns, narrowed
+ *   ptr_out            NULL, or n_rows + 1 row pointers of ptr_out_bits (32 / 64)
+ *   partial            device scratch, fsp_csr_check_partial_len() int64
+ *   out                6 int64 (device, or host memory the device can write): indptr[0],
+ *                      indptr[n_rows], the number of decreases, the longest row, the smallest
+ *                      and the largest column (INT64_MAX and INT64_MIN when nnz is 0)
+ * The narrowed copies hold meaningless values where the checks fail.
+ */
+int64_t fsp_csr_check_partial_len(void);
+int fsp_csr_check(const void* indices, int idx_bits, int64_t nnz, const void* indptr,
+                  int ptr_bits, int64_t n_rows, int32_t* idx32, void* ptr_out, int ptr_out_bits,
+                  int64_t* partial, int64_t* out, void* stream);
+
+/*
  * The same plan built on the device in two passes (no host copy of rowptr, no host loop):
  * the rows are cut into windows of window_rows rows and each window is planned with the rules
  * of fsp_plan_row_blocks, except that no block crosses a window boundary.  Replaces the host
@@ -196,6 +214,24 @@ int fsp_spmv_csr(int dtype, int acc_f64, const void* vals, const int32_t* cols,
                  const int32_t* desc, const int64_t* ranges, int64_t n_desc, int64_t chunk,
                  void* partials, const int32_t* groups, const int64_t* group_base,
                  const int32_t* split_rows, int64_t n_groups, int xcd_remap, void* stream);
+
+/*
+ * y = A @ x for CSR A without a plan, for a matrix used once: the matrix is cut into
+ * fsp_spmv_slices(n_rows, nnz) slices of about equal rows + entries, found by binary search in
+ * the row pointers; rows of more than fsp_spmv_slice_keep() entries may be cut, their pieces
+ * added in order by a second pass.  Replaces the same launches as fsp_spmv_csr.
+ *   vals, cols, rowptr, x, y, dtype, acc_f64   as fsp_spmv_csr (no row_map); n_rows < 2^31
+ *   table      device scratch, 2 * (slices + 1) int64: the slices' boundaries {row, entry}
+ *   sums       device scratch, 2 * slices doubles: the pieces of cut rows
+ *   cut_rows   0: no row is longer than fsp_spmv_slice_keep() (the second pass is left out)
+ * table and sums need no initial value; calls sharing them must not overlap.
+ */
+int64_t fsp_spmv_slices(int64_t n_rows, int64_t nnz);
+int64_t fsp_spmv_slice_keep(void);
+int fsp_spmv_sliced(int dtype, int acc_f64, const void* vals, const int32_t* cols,
+                    const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t nnz,
+                    const void* x, void* y, int64_t* table, void* sums, int cut_rows,
+                    void* stream);
 
 /*
  * fsp_spmv_csr without a caller workspace, for callers that cannot allocate device memory
