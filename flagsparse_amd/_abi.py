@@ -71,6 +71,10 @@ SIGNATURES = {
     "fsp_spmv_coo_atomic": (_i32, [_i32, _p, _p, _p, _i64, _p, _p, _i64, _i64, _p]),
     "fsp_spmm_csr": (_i32, [_i32, _i32, _p, _p, _p, _i32, _i64, _i64, _p, _i64, _i64, _p, _i64, _p,
                             _i64, _i64, _i32, _i32, _p, _p, _p, _p, _i64, _i32, _p]),
+    "fsp_slice_count": (_i64, [_i64, _i64, _i64]),
+    "fsp_slice_table": (_i32, [_p, _i32, _i64, _i64, _i64, _i64, _p, _p]),
+    "fsp_spmm_sliced": (_i32, [_i32, _i32, _p, _p, _p, _i32, _i64, _i64, _p, _i64, _i64, _p, _i64,
+                               _p, _i64, _i64, _p, _i32, _i32, _i32, _i32, _p]),
     "fsp_index_stats": (_i32, [_p, _i32, _p, _i32, _i64, _p, _p, _p]),
     "fsp_index_stats_partial_len": (_i64, []),
     "fsp_spmm_coo_atomic": (_i32, [_i32, _i32, _p, _p, _p, _i64, _p, _i64, _i64, _p, _i64, _i64,

@@ -21,7 +21,8 @@ LIB_NAME = "libflagsparse_hip.so"
 LIB_PATH = os.path.join(LIB_DIR, LIB_NAME)
 
 SOURCES = ("abi.cpp", "mtx.cpp", "plan.hip", "spmv.hip", "spmv_xcs.hip", "spmm.hip", "sddmm.hip",
-           "index_stats.hip", "check.hip", "slices.hip", "probe.hip")
+           "index_stats.hip", "check.hip", "slices.hip",
+           "spmm_slices.hip", "probe.hip")
 ARCH = "gfx950"
 
 # Packed-FP32 instructions (v_pk_*_f32) are disabled for all device code.

@@ -26,7 +26,7 @@ from ._common import (
     _require_kernel_dtype,
     _tolerance_for_dtype,
 )
-from ._index_stats import index_stats_device
+from ._csr_check import csr_check
 from ._plan import StreamOrder, build_row_block_plan_device
 from .synthetic import build_random_csr, build_random_dense
 
@@ -35,12 +35,9 @@ SUPPORTED_SPMM_VALUE_DTYPES = SUPPORTED_VALUE_DTYPES
 XCD_REMAP = 1
 # The row-block plan is built in windows of SPMM_PLAN_WINDOW_BLOCKS x the block row cap (each
 # window's last block may be short).  Windows of one block's rows cut a block after every
-# row-cap rows even when the entry cap ended the one before, adding a tiny block per window;
-# wider windows make the planner (one thread per window) slower, which the paths that plan
-# on every call pay each time.  Measured on MI355X, cfg5's matrix, fp32 N=16, per call
-# (prepared / COO / base): 380 / 813 / 633 us with windows of 1 block, 329 / 840 / 657 with 4,
-# 327 / 1124 / 957 with 16; N=64: 663 / 1087 / 924, 663 / 1099 / 930, 662 / 1174 / 1006.  So
-# prepared matrices plan with 4 and the per-call paths with 1.
+# row-cap rows even when the entry cap ended the one before.  Measured on MI355X, cfg5's matrix
+# prepared: fp32 N=16 380 / 329 / 327 us with windows of 1 / 4 / 16 blocks, N=64 663 / 663 / 662
+# (the planner takes longer on wide windows: one thread each).
 SPMM_PLAN_WINDOW_BLOCKS = 4
 # Rows longer than this go to the part path (several lane groups per row).
 _SPMM_ROW_SPLIT_THRESHOLD = 128
@@ -133,9 +130,9 @@ def _spmm_opt_reference_error(candidate, reference, value_dtype):
 # ------------------------------------------------------------------------------------------
 
 
-def _prepare_spmm_csr_matrix(data, indices, indptr, shape):
-    """spmm_csr.py:197-255 (same checks, order and exceptions; the device-side checks are
-    gathered into one host synchronisation)."""
+def _check_spmm_csr_matrix(data, indices, indptr, shape, ptr_bits):
+    """The checks of spmm_csr.py:197-255 (same order and exceptions): (data, int32 columns, row
+    pointers of ``ptr_bits``, n_rows, n_cols, longest row)."""
     if len(shape) != 2:
         raise ValueError("shape must be a 2-tuple: (n_rows, n_cols)")
     if data.ndim != 1 or indices.ndim != 1 or indptr.ndim != 1:
@@ -161,48 +158,41 @@ def _prepare_spmm_csr_matrix(data, indices, indptr, shape):
         raise TypeError("indptr dtype must be torch.int32 or torch.int64")
 
     nnz = data.numel()
-    probes = [indptr[0].to(torch.int64), indptr[-1].to(torch.int64)]
-    if indptr.numel() > 1:
-        probes.append(torch.any(indptr[1:] < indptr[:-1]).to(torch.int64))
-        probes.append(torch.max(indptr[1:] - indptr[:-1]).to(torch.int64))
-    if nnz > 0:
-        probes += list(index_stats_device(indices.contiguous(), indices.contiguous())[:2])
-    vals = torch.stack(probes).tolist()
-    if vals[0] != 0:
+    data, indices, indptr = data.contiguous(), indices.contiguous(), indptr.contiguous()
+    # one pass over the index arrays, one host synchronisation
+    (first, last, decreases, max_row_nnz, min_col, max_col), kernel_indices, kernel_ptr = \
+        csr_check(indices, indptr, ptr_bits)
+    if first != 0:
         raise ValueError("indptr[0] must be 0")
-    if vals[1] != nnz:
-        raise ValueError(f"indptr[-1] must equal nnz={nnz}, got {vals[1]}")
-    pos = 2
-    max_row_nnz = 0
-    if indptr.numel() > 1:
-        if vals[2]:
-            raise ValueError("indptr must be nondecreasing")
-        max_row_nnz = vals[3]
-        pos = 4
+    if last != nnz:
+        raise ValueError(f"indptr[-1] must equal nnz={nnz}, got {last}")
+    if decreases:
+        raise ValueError("indptr must be nondecreasing")
     if nnz > 0:
-        min_col, max_col = vals[pos], vals[pos + 1]
         if min_col < 0 or max_col >= n_cols:
             raise IndexError("indices out of range for n_cols")
         if max_col > _INDEX_LIMIT_INT32:
             raise ValueError(
                 "column indices exceed the int32 range supported by the Triton kernel")
+    return data, kernel_indices, kernel_ptr, n_rows, n_cols, int(max_row_nnz)
 
-    data = data.contiguous()
-    indices = indices.contiguous()
-    indptr = indptr.contiguous()
-    kernel_indices = indices.to(torch.int32) if indices.dtype == torch.int64 else indices
-    kernel_indptr = indptr.to(torch.int64)
+
+def _prepare_spmm_csr_matrix(data, indices, indptr, shape):
+    """spmm_csr.py:197-255 (same checks, order and exceptions), row pointers as int64."""
+    data, kernel_indices, kernel_indptr, n_rows, n_cols, max_row_nnz = \
+        _check_spmm_csr_matrix(data, indices, indptr, shape, 64)
     row_lengths = (kernel_indptr[1:] - kernel_indptr[:-1] if n_rows > 0
                    else kernel_indptr.new_empty((0,)))
-    return data, kernel_indices, kernel_indptr, n_rows, n_cols, row_lengths, int(max_row_nnz)
+    return data, kernel_indices, kernel_indptr, n_rows, n_cols, row_lengths, max_row_nnz
 
 
 def _prepare_spmm_csr_inputs(data, indices, indptr, B, shape):
-    """spmm_csr.py:258-281."""
+    """spmm_csr.py:258-281, row pointers at the width the kernels read."""
     if B.ndim != 2:
         raise ValueError("B must be a 2D dense tensor")
-    (data, kernel_indices, kernel_indptr, n_rows, n_cols, _row_lengths,
-     max_row_nnz) = _prepare_spmm_csr_matrix(data, indices, indptr, shape)
+    data, kernel_indices, kernel_indptr, n_rows, n_cols, max_row_nnz = \
+        _check_spmm_csr_matrix(data, indices, indptr, shape,
+                               32 if data.numel() <= _common.ROWPTR32_MAX_NNZ else 64)
     if B.shape[0] != n_cols:
         raise ValueError(f"B.shape[0] must be n_cols={n_cols}, got {B.shape[0]}")
     if not B.is_cuda:
@@ -287,24 +277,50 @@ def _spmm_lane_shape(n_dense_cols, dtype, B, C, tile_cols=None):
     return lanes, vec
 
 
+def _spmm_slice_lanes(n_dense_cols, dtype, tile_cols=None):
+    """(lanes per B row G, elements per lane vec) for the sliced kernel: 16-byte loads for every
+    N that holds one (any alignment), single elements for N = 3 (measured on MI355X, fp32, 15M
+    entries: 75.6 us against 76.4 with pairs)."""
+    vec = 4 if dtype == torch.float32 else 2
+    if n_dense_cols < vec:
+        vec = 2 if n_dense_cols == 2 else 1
+    width = n_dense_cols if tile_cols is None else max(1, min(n_dense_cols, int(tile_cols)))
+    return min(64, _next_pow2(-(-width // vec))), vec
+
+
+def _spmm_slice_shape(lanes, positions):
+    """(rows + entries per slice, longest row never cut).  A slice should give each of a
+    workgroup's 256 / lanes groups several entries, and the matrix enough slices to fill the
+    256 CUs.  Measured on MI355X with 128 / 256 / 512 / 1024 positions: 16 lanes (fp32 N=64, 33.5M
+    entries) 781 / 670 / 661 / 701 us; 64 lanes (N=256, 4M) 557 / 564 / - / -; 8 lanes (N=32,
+    1.2M) 29.8 / 22.0 / 19.7 / 19.2; the same with 80k entries 5.2 / 5.3 / 6.3 / 6.9, hence the
+    limit by size."""
+    items = {64: 128, 32: 256, 16: 512, 8: 1024}.get(lanes, 1536)
+    while items > 64 and positions < 1024 * items:
+        items >>= 1
+    return items, 256 if items >= 128 else 128
+
+
 class _SpmmKernelCsr:
-    """Kernel-facing CSR arrays (aligned, int32 offsets when they fit) and plans per G."""
+    """Kernel-facing CSR arrays (aligned, int32 offsets when they fit), their row-block plans per
+    G and their slices.  max_row_nnz: the longest row, where known; one_shot: the object serves
+    one call, so nothing is planned."""
 
     __slots__ = ("data", "cols", "rowptr", "rowptr_bits", "nnz", "n_rows", "_plans", "_args",
-                 "_keep", "window_blocks", "_order")
+                 "_keep", "_order", "max_row_nnz", "one_shot", "_tables")
 
-    def __init__(self, data, cols, indptr64, window_blocks=None):
-        # window_blocks: plan window in blocks' rows (SPMM_PLAN_WINDOW_BLOCKS when None); the
-        # paths that plan on every call use 1, which plans fastest
-        self.window_blocks = window_blocks
+    def __init__(self, data, cols, indptr, max_row_nnz=None, one_shot=False):
+        self.max_row_nnz = max_row_nnz
+        self.one_shot = one_shot
         self.data = _aligned(data)
         self.cols = _aligned(cols)
         self.nnz = int(data.numel())
-        self.n_rows = int(indptr64.numel()) - 1
+        self.n_rows = int(indptr.numel()) - 1
         if self.nnz <= _common.ROWPTR32_MAX_NNZ:
-            self.rowptr, self.rowptr_bits = indptr64.to(torch.int32), 32
+            self.rowptr, self.rowptr_bits = indptr.to(torch.int32), 32
         else:
-            self.rowptr, self.rowptr_bits = indptr64.to(torch.int64).contiguous(), 64
+            self.rowptr, self.rowptr_bits = indptr.to(torch.int64).contiguous(), 64
+        self._tables = {}
         self._plans = {}
         self._args = {}
         self._keep = [self.data, self.cols, self.rowptr]  # what a launch reads or writes
@@ -316,7 +332,35 @@ class _SpmmKernelCsr:
     def describe(self):
         return {"layout": "rowblock", "plans": {g: {"descriptors": p.n_desc,
                                                     "split_rows": p.n_split_rows}
-                                                for g, p in self._plans.items()}}
+                                                for g, p in self._plans.items()},
+                "slices": {items: int(t.numel()) // 2 - 1
+                           for (items, _), t in self._tables.items()}}
+
+    def sliced(self):
+        """Whether products run on slices whatever their N.  Row blocks are kept where they are
+        the faster: prepared, every row one group's work (and, in _run_spmm, N, B and C whole
+        vectors).  Measured on MI355X, row blocks / slices: fp32 N=16, 100k rows of 0 to 32
+        entries 18.4 / 20.8 us; N=33, 3M entries 80.6 / 53.0; a power law, N=128 457 / 316, N=47
+        326 / 214.  A matrix used once has no plan to use."""
+        if self.one_shot or self.max_row_nnz is None:
+            return True
+        return self.max_row_nnz > _SPMM_ROW_SPLIT_THRESHOLD
+
+    def table(self, items, keep):
+        """The slices' boundaries (built on the current stream, once)."""
+        t = self._tables.get((items, keep))
+        if t is None:
+            if torch.cuda.is_current_stream_capturing():
+                raise RuntimeError("an SpMM must run once before it is captured into a graph "
+                                   "(the first call with this N builds its slices)")
+            L = _abi.lib()
+            n = L.fsp_slice_count(self.n_rows, self.nnz, items)
+            t = torch.empty(2 * (n + 1), dtype=torch.int64, device=self.data.device)
+            _abi.check(L.fsp_slice_table(self.rowptr.data_ptr(), self.rowptr_bits, self.n_rows,
+                                         self.nnz, items, keep, t.data_ptr(),
+                                         _abi.raw_stream(t.device)), "fsp_slice_table")
+            self._tables[(items, keep)] = t
+        return t
 
     def plan(self, lanes):
         p = self._plans.get(lanes)
@@ -326,8 +370,7 @@ class _SpmmKernelCsr:
             threshold = min(_SPMM_ROW_SPLIT_THRESHOLD, cap)
             chunk = min(cap, max(threshold, 16 * ngrp))
             p = build_row_block_plan_device(self.rowptr, cap, ngrp, threshold, chunk,
-                                            window_rows=(self.window_blocks
-                                                         or SPMM_PLAN_WINDOW_BLOCKS) * ngrp)
+                                            window_rows=SPMM_PLAN_WINDOW_BLOCKS * ngrp)
             self._plans[lanes] = p
         return p
 
@@ -353,16 +396,47 @@ def _auto_tile_cols(B):
     return t if t < n else None
 
 
+def _run_spmm_sliced(kc, B, C, acc_f64, lanes, vec):
+    n_dense_cols = int(B.shape[1])
+    key = ("slices", lanes, vec, n_dense_cols, bool(acc_f64), B.dtype)
+    stream = kc._order.stream(C.device, kc._keep)
+    args = kc._args.get(key)
+    if args is None:  # the arguments that do not change between calls, converted once
+        items, keep = _spmm_slice_shape(lanes, kc.n_rows + kc.nnz)
+        table = kc.table(items, keep)
+        cut = kc.max_row_nnz is None or kc.max_row_nnz > keep
+        sums = None
+        if cut:  # the pieces of cut rows: a carry and a head per slice
+            n = int(table.numel()) // 2 - 1
+            sums = torch.empty(2 * n * n_dense_cols, device=C.device,
+                               dtype=torch.float64 if acc_f64 else B.dtype)
+        args = [_abi.dtype_code(B.dtype), 1 if acc_f64 else 0, kc.data.data_ptr(),
+                kc.cols.data_ptr(), kc.rowptr.data_ptr(), kc.rowptr_bits, kc.n_rows, kc.nnz,
+                None, 0, n_dense_cols, None, 0, table.data_ptr(), items, keep,
+                None if sums is None else sums.data_ptr(), int(cut), lanes, vec, XCD_REMAP, None]
+        kc._args[key] = args
+        kc._keep.extend((table, sums))
+    a = list(args)
+    a[8], a[9], a[11], a[12] = B.data_ptr(), B.stride(0), C.data_ptr(), C.stride(0)
+    a[21] = stream
+    _abi.check(_abi.lib().fsp_spmm_sliced(*a), "fsp_spmm_sliced")
+    return C
+
+
 def _run_spmm(kc, B, C, acc_f64, tile_cols=None):
-    """Launch fsp_spmm_csr: C[n_rows, N] = A @ B (B, C contiguous row-major).  Without an
-    explicit tile (the reference's block_n), a B over SPMM_B_TILE_BYTES is tiled by columns."""
+    """C[n_rows, N] = A @ B (B, C contiguous row-major) on slices or row blocks (kc.sliced).
+    Without an explicit tile (the reference's block_n), a B over SPMM_B_TILE_BYTES is tiled by
+    columns."""
     n_dense_cols = int(B.shape[1])
     if kc.n_rows == 0 or n_dense_cols == 0:
         return C
     if tile_cols is None:
         tile_cols = _auto_tile_cols(B)
     dtype = B.dtype
+    slice_lanes, slice_vec = _spmm_slice_lanes(n_dense_cols, dtype, tile_cols)
     lanes, vec = _spmm_lane_shape(n_dense_cols, dtype, B, C, tile_cols)
+    if kc.sliced() or vec < slice_vec:  # the row-block kernel's loads need aligned vectors
+        return _run_spmm_sliced(kc, B, C, acc_f64, slice_lanes, slice_vec)
     key = (lanes, vec, n_dense_cols, bool(acc_f64), dtype)
     args = kc._args.get(key)
     if args is None:  # the arguments that do not change between calls, converted once
@@ -444,7 +518,8 @@ class PreparedCsrSpmmOpt:
 
     def _kernel_csr(self):
         if self._kernel is None:
-            self._kernel = _SpmmKernelCsr(self.data, self.kernel_indices, self.kernel_indptr)
+            self._kernel = _SpmmKernelCsr(self.data, self.kernel_indices, self.kernel_indptr,
+                                          self.max_row_nnz)
         return self._kernel
 
     def _reference_metadata(self):
@@ -638,7 +713,7 @@ def flagsparse_spmm_csr(data, indices, indptr, B, shape, block_n=None, block_nnz
         direct = False
     else:
         _require_kernel_dtype(dtype, "flagsparse_spmm_csr")
-        kc = _SpmmKernelCsr(data, kernel_indices, kernel_indptr, window_blocks=1)
+        kc = _SpmmKernelCsr(data, kernel_indices, kernel_indptr, max_row_nnz, one_shot=True)
         direct = _out_ok_direct(out, (B, data))
         C = out if direct else torch.empty((n_rows, n_dense_cols), dtype=dtype,
                                            device=data.device)

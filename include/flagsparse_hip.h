@@ -425,6 +425,36 @@ int fsp_spmm_csr(int dtype, int acc_f64, const void* vals, const int32_t* cols,
                  const int32_t* split_rows, int64_t n_groups, int xcd_remap, void* stream);
 
 /*
+ * Slices of equal work, for products without a row-block plan: rows and entries on one line, row
+ * r at positions rowptr[r] + r .. rowptr[r+1] + r, slice k starting at position k * items; a
+ * boundary inside a row of at most keep entries moves to that row's start.
+ *   fsp_slice_count  the number of slices, ceil((n_rows + nnz) / items)
+ *   fsp_slice_table  writes their boundaries, slices + 1 int64 pairs {row, entry}
+ */
+int64_t fsp_slice_count(int64_t n_rows, int64_t nnz, int64_t items);
+int fsp_slice_table(const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t nnz,
+                    int64_t items, int64_t keep, int64_t* table, void* stream);
+
+/*
+ * C[n_rows, N] = A @ B over the slices of fsp_slice_table, otherwise as fsp_spmm_csr.
+ *   table, items, keep  the slices' boundaries and what they were built with; items + keep <=
+ *                  2042
+ *   sums           2 * slices * N slots of the accumulation type, 16-byte aligned: the pieces
+ *                  of cut rows.  Calls sharing sums must not overlap.
+ *   cut_rows       0: no row is longer than keep (sums may be NULL, and the second pass that
+ *                  adds the pieces is left out)
+ *   lanes_per_row  G in {1,2,4,...,64}: lanes sharing one B row; a workgroup covers G * vec
+ *                  columns
+ *   vec            elements per lane per load: 1, 2 or 4 (fp32) / 1 or 2 (fp64), at most N;
+ *                  needs no alignment of B, C, ldb or ldc beyond the element's own
+ */
+int fsp_spmm_sliced(int dtype, int acc_f64, const void* vals, const int32_t* cols,
+                    const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t nnz,
+                    const void* B, int64_t ldb, int64_t N, void* C, int64_t ldc,
+                    const int64_t* table, int64_t items, int64_t keep, void* sums, int cut_rows,
+                    int lanes_per_row, int vec, int xcd_remap, void* stream);
+
+/*
  * COO SpMM with atomics: C_acc[rows[e], n] += vals[e] * B[cols[e], n] for every entry e and
  * n < N.  Replaces the reference's atomic route, spmm_coo.py:244-271 (_spmm_coo_atomic_real_
  * kernel) and :464-523 (_triton_spmm_coo_atomic_impl).  C_acc[0 .. n_rows*ldc) is zeroed first;

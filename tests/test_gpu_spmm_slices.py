@@ -1,0 +1,121 @@
+"""SpMM over slices (csrc/spmm_slices.hip) against the fp64 oracle where it can go wrong: widths
+that are no whole number of vectors, column tiles, unaligned B and C, rows at the longest uncut
+length and beyond, rows crossing many slices, one row for a whole slice, runs of empty rows,
+64-bit row pointers, infinities outside a row's columns; and the rule that picks it."""
+
+import numpy as np
+import pytest
+import torch
+
+import flagsparse_amd as fs
+from flagsparse_amd import _common, spmm_csr, synthetic
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = {
+    "empty": [0] * 700,
+    "one_row": [9000],
+    "short": [1, 0, 2, 5, 33, 3] * 200,
+    "at_keep": [255, 256, 257, 0, 127, 128, 129] * 12,
+    "crossing": [5, 4000, 0, 0, 1, 61, 7, 64, 65] + [0] * 1500 + [3000] * 3 + [2] * 90,
+    "uniform60": [60] * 300,
+}
+
+
+def _case(name, n_cols, N, dtype, dev, seed=3):
+    lengths = LENGTHS[name]
+    ip = torch.zeros(len(lengths) + 1, dtype=torch.int64)
+    ip[1:] = torch.cumsum(torch.as_tensor(lengths), 0)
+    nnz = int(ip[-1])
+    cols = synthetic.randint(seed, 1, nnz, n_cols, "cpu")
+    vals = synthetic.uniform_values(seed, 2, nnz, dtype, "cpu")
+    B = synthetic.dense_uniform(n_cols, N, dtype, seed=seed, device="cpu")
+    return vals, cols, ip, B, (len(lengths), n_cols)
+
+
+def _run(vals, cols, ip, B, shape, dev, acc_f64, tile=None, one_shot=True):
+    lengths = ip[1:] - ip[:-1]
+    kc = spmm_csr._SpmmKernelCsr(vals.to(dev), cols.to(torch.int32).to(dev), ip.to(dev),
+                                 int(lengths.max()), one_shot=one_shot)
+    C = torch.full((shape[0], B.shape[1]), float("nan"), dtype=B.dtype, device=dev)
+    spmm_csr._run_spmm(kc, B.to(dev), C, acc_f64, tile)
+    return C, kc
+
+
+@pytest.mark.parametrize("name", sorted(LENGTHS))
+@pytest.mark.parametrize("N", [1, 2, 3, 4, 5, 7, 16, 33, 47, 64, 130, 257])
+@pytest.mark.parametrize("dtype,acc", [(torch.float32, False), (torch.float32, True),
+                                       (torch.float64, True)])
+def test_sliced_spmm(dev, name, N, dtype, acc):
+    vals, cols, ip, B, shape = _case(name, 901, N, dtype, dev)
+    print(f"sliced spmm {name} N={N} {dtype} acc64={acc}", flush=True)
+    C, kc = _run(vals, cols, ip, B, shape, dev, acc)
+    assert kc._tables and not kc._plans
+    ref = oracle.spmm_csr(ip, cols, vals, B)
+    assert oracle.rel_l2(C, ref) <= oracle.REL_L2_BOUND[str(dtype)[6:]]
+    if dtype == torch.float32 and acc:  # one rounding of an fp64 sum
+        np.testing.assert_allclose(C.cpu().numpy(), ref, rtol=1.2e-7, atol=1e-12)
+    again = torch.empty_like(C)
+    spmm_csr._run_spmm(kc, B.to(dev), again, acc)
+    assert torch.equal(C, again)
+
+
+@pytest.mark.parametrize("N,tile", [(130, 32), (33, 8), (257, 64), (70, 1)])
+def test_sliced_spmm_tiles_and_alignment(dev, N, tile):
+    vals, cols, ip, B, shape = _case("crossing", 901, N, torch.float32, dev)
+    C, _ = _run(vals, cols, ip, B, shape, dev, False)
+    Ct, _ = _run(vals, cols, ip, B, shape, dev, False, tile)
+    ref = oracle.spmm_csr(ip, cols, vals, B)
+    assert oracle.rel_l2(Ct, ref) <= 1e-5 and oracle.rel_l2(C, ref) <= 1e-5
+    # B one element past a 16-byte boundary: same sums
+    flat = torch.empty(B.numel() + 1, device=dev)
+    Bu = flat[1:].view(B.shape)
+    Bu.copy_(B)
+    p = fs.prepare_spmm_csr_opt(vals.to(dev), cols.to(dev), ip.to(dev), shape)
+    assert torch.equal(fs.flagsparse_spmm_csr_opt(B=Bu, prepared=p), C)
+
+
+def test_sliced_spmm_rowptr64(dev, monkeypatch):
+    vals, cols, ip, B, shape = _case("crossing", 901, 20, torch.float64, dev)
+    C, _ = _run(vals, cols, ip, B, shape, dev, True)
+    monkeypatch.setattr(_common, "ROWPTR32_MAX_NNZ", 0)
+    C64, kc = _run(vals, cols, ip, B, shape, dev, True)
+    assert kc.rowptr_bits == 64 and torch.equal(C, C64)
+
+
+def test_sliced_spmm_nonfinite(dev):
+    # the masked loads of a row's last entries read B's first row; nothing of it may show
+    vals, cols, ip, B, shape = _case("short", 901, 47, torch.float32, dev)
+    B[0], B[5, 3] = float("inf"), float("nan")
+    C, _ = _run(vals, cols, ip, B, shape, dev, False)
+    ref = oracle.spmm_csr(ip, cols, vals, B)
+    np.testing.assert_array_equal(np.isnan(C.cpu().numpy()), np.isnan(ref))
+    np.testing.assert_array_equal(np.isfinite(C.cpu().numpy()), np.isfinite(ref))
+
+
+def test_spmm_route(dev):
+    # row blocks: prepared, short rows, whole aligned vectors; else slices
+    for name, N, blocks in (("short", 16, True), ("short", 15, False), ("at_keep", 16, False)):
+        vals, cols, ip, B, shape = _case(name, 901, N, torch.float32, dev)
+        p = fs.prepare_spmm_csr_opt(vals.to(dev), cols.to(dev), ip.to(dev), shape)
+        C = fs.flagsparse_spmm_csr_opt(B=B.to(dev), prepared=p)
+        kc = p._kernel_csr()
+        assert bool(kc._plans) == blocks and bool(kc._tables) == (not blocks)
+        Cs, _ = _run(vals, cols, ip, B, shape, dev, False)  # the other route
+        ref = oracle.spmm_csr(ip, cols, vals, B)
+        assert oracle.rel_l2(C, ref) <= 1e-5 and oracle.rel_l2(Cs, ref) <= 1e-5
+
+
+def test_spmm_capture_needs_a_first_call(dev):
+    vals, cols, ip, B, shape = _case("at_keep", 901, 8, torch.float32, dev)
+    p = fs.prepare_spmm_csr_opt(vals.to(dev), cols.to(dev), ip.to(dev), shape)
+    Bd = B.to(dev)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with pytest.raises(RuntimeError, match="once before"):
+        with torch.cuda.graph(g):
+            fs.flagsparse_spmm_csr_opt(B=Bd, prepared=p)
+    torch.cuda.synchronize()
+    ref = oracle.spmm_csr(ip, cols, vals, B)
+    assert oracle.rel_l2(fs.flagsparse_spmm_csr_opt(B=Bd, prepared=p), ref) <= 1e-5
