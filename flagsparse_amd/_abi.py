@@ -75,6 +75,10 @@ SIGNATURES = {
     "fsp_slice_table": (_i32, [_p, _i32, _i64, _i64, _i64, _i64, _p, _p]),
     "fsp_spmm_sliced": (_i32, [_i32, _i32, _p, _p, _p, _i32, _i64, _i64, _p, _i64, _i64, _p, _i64,
                                _p, _i64, _i64, _p, _i32, _i32, _i32, _i32, _p]),
+    "fsp_coo_sort_max_nnz": (_i64, []),
+    "fsp_coo_sort_scratch": (_i64, [_i32, _i64, _i64]),
+    "fsp_coo_sort_rows": (_i32, [_i32, _p, _i32, _p, _i32, _p, _i64, _i64, _p, _p, _p, _p, _p]),
+    "fsp_coo_rowptr": (_i32, [_p, _i32, _i64, _i64, _p, _i32, _p]),
     "fsp_index_stats": (_i32, [_p, _i32, _p, _i32, _i64, _p, _p, _p]),
     "fsp_index_stats_partial_len": (_i64, []),
     "fsp_spmm_coo_atomic": (_i32, [_i32, _i32, _p, _p, _p, _i64, _p, _i64, _i64, _p, _i64, _i64,

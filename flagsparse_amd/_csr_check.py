@@ -8,7 +8,8 @@ from . import _abi
 
 def csr_check(indices, indptr, ptr_bits=None):
     """((first, last, decreases, longest row, min column, max column) as Python ints, the columns
-    as int32, the row pointers at ``ptr_bits``) of contiguous 1-D int32 / int64 device arrays.
+    as int32, the row pointers at ``ptr_bits``) of contiguous 1-D device arrays (columns int32 or
+    int64; row pointers of another type are converted first).
 
     The two arrays are the arguments themselves where they already have that width (or where
     ``ptr_bits`` is None); the column bounds are meaningless without entries.  Copies are made
@@ -16,6 +17,11 @@ def csr_check(indices, indptr, ptr_bits=None):
     """
     L = _abi.lib()
     dev = indices.device
+    if indptr.device != dev:
+        raise RuntimeError(f"indices and indptr are on different devices: {dev} and "
+                           f"{indptr.device}")
+    if indptr.dtype not in (torch.int32, torch.int64):
+        indptr = indptr.to(torch.int64)
     nnz, n_rows = int(indices.numel()), int(indptr.numel()) - 1
     idx_bits = 32 if indices.dtype == torch.int32 else 64
     have_bits = 32 if indptr.dtype == torch.int32 else 64

@@ -256,7 +256,8 @@ class SliceLayout:
     def describe(self):
         return {"layout": self.kind, "cut_rows": self.cut_rows}
 
-    def launch(self, x, y, acc_f64):
+    def launch(self, x, y, acc_f64, row_map=None, n_out=0):
+        assert row_map is None, "slices write every row"
         stream = self._order.stream(y.device, (self._scratch, self.data, self.cols, self.rowptr))
         _abi.check(
             _abi.lib().fsp_spmv_sliced(_abi.dtype_code(self.data.dtype), int(acc_f64),

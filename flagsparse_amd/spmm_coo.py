@@ -7,10 +7,10 @@ Public API and error behaviour mirror ``src/flagsparse/sparse_operations/spmm_co
 
 The reference coalesces duplicate (row, col) entries, sorts them lexicographically and runs one
 program per row run (:136-180, :394-461), in float64 for float32 inputs (:11-18).  Here the
-entries are brought into row order (no sort when they already are), a row pointer found by
-binary search turns them into CSR - a row run is a CSR row, and a row without entries is an empty row that
-the kernel writes as 0 - and ``spmm_rowblock_kernel`` computes C with float64 accumulation for
-float32 (duplicates are summed by the accumulation itself).  The reference's "atomic" route
+entries are brought into row order (no sort when they already are; _coo_order.py), a row pointer
+found by binary search turns them into CSR - a row run is a CSR row, and a row without entries is
+an empty row that the kernel writes as 0 - and ``spmm_slices_kernel`` computes C with float64
+accumulation for float32 (duplicates are summed by the accumulation itself).  The reference's "atomic" route
 (:244-271, :464-523), reachable through the benchmark case, runs ``spmm_coo_atomic_kernel``.
 """
 
@@ -19,6 +19,7 @@ import time
 import torch
 
 from . import _abi
+from ._coo_order import row_pointers, rows_in_order
 from ._index_stats import index_stats
 from ._common import (
     SUPPORTED_INDEX_DTYPES,
@@ -39,9 +40,10 @@ from .spmm_csr import (
 from .synthetic import build_random_coo, build_random_dense
 
 
-def _prepare_spmm_coo_inputs_checked(data, row, col, B, shape):
-    """Validation and narrowing of spmm_coo.py:312-371 (same checks, messages and types), plus
-    whether the rows are already in order (from the same pass over the indices)."""
+def _check_spmm_coo_inputs(data, row, col, B, shape):
+    """The checks of spmm_coo.py:312-371 (same order, messages and types): (data, row, col, B) as
+    contiguous arrays, the sizes, and whether the rows are already in order (from the same pass
+    over the indices)."""
     if len(shape) != 2:
         raise ValueError("shape must be a 2-tuple: (n_rows, n_cols)")
     if data.ndim != 1 or row.ndim != 1 or col.ndim != 1:
@@ -87,18 +89,17 @@ def _prepare_spmm_coo_inputs_checked(data, row, col, B, shape):
         if max_col > _INDEX_LIMIT_INT32:
             raise ValueError(
                 "column indices exceed the int32 range supported by the Triton kernel")
-    data = data.contiguous()
-    kernel_row = row.contiguous().to(torch.int32)
-    kernel_col = col.contiguous().to(torch.int32)
-    B = B.contiguous()
-    return data, kernel_row, kernel_col, B, n_rows, n_cols, int(B.shape[1]), row_sorted
+    return (data.contiguous(), row, col, B.contiguous(), n_rows, n_cols, int(B.shape[1]),
+            row_sorted)
 
 
 def _prepare_spmm_coo_inputs(data, row, col, B, shape):
     """spmm_coo.py:312-371: the validated, narrowed inputs (data, row int32, col int32, B,
     n_rows, n_cols, n_dense_cols) - the seven values the reference's scripts unpack
     (tests/test_spmm_coo.py:290)."""
-    return _prepare_spmm_coo_inputs_checked(data, row, col, B, shape)[:7]
+    data, row, col, B, n_rows, n_cols, n_dense_cols, _ = _check_spmm_coo_inputs(data, row, col,
+                                                                                B, shape)
+    return (data, row.to(torch.int32), col.to(torch.int32), B, n_rows, n_cols, n_dense_cols)
 
 
 def _resolve_spmm_coo_launch_config(n_dense_cols, nnz, block_n=None, block_nnz=256):
@@ -127,32 +128,27 @@ def _normalize_spmm_coo_route(route):
 
 
 class _CooRowOrder:
-    """Row-ordered COO (int32 rows and columns) plus its CSR view for the SpMM kernel."""
+    """Row-ordered COO plus its CSR view for the SpMM kernel.  Rows must lie in [0, n_rows)."""
 
     __slots__ = ("data", "row", "col", "n_rows", "n_cols", "_kc")
 
     def __init__(self, data, row, col, n_rows, n_cols, row_sorted=None):
         nnz = int(data.numel())
+        data, row, col = data.contiguous(), row.contiguous(), col.contiguous()
         if row_sorted is None:
             row_sorted = nnz <= 1 or bool((row[1:] >= row[:-1]).all().item())
         if not row_sorted:
-            # (row, col) order, stable, so equal keys keep their input order
-            key = row.to(torch.int64) * max(1, n_cols) + col.to(torch.int64)
-            order = torch.sort(key, stable=True).indices
-            data, row, col = data[order], row[order], col[order]
-        self.data = data.contiguous()
-        self.row = row.contiguous()
-        self.col = col.contiguous()
+            data, row, col = rows_in_order(data, row, col, n_rows - 1)
+        self.data = data
+        self.row = row
+        self.col = col.to(torch.int32)
         self.n_rows, self.n_cols = n_rows, n_cols
         self._kc = None
 
     def kernel_csr(self):
         if self._kc is None:
-            # rows are in order, so row r's entries start at the first position whose row
-            # is >= r: one binary search per row (no atomics, unlike a bincount)
-            bounds = torch.arange(self.n_rows + 1, dtype=self.row.dtype, device=self.row.device)
-            indptr = torch.searchsorted(self.row, bounds).to(torch.int64)
-            self._kc = _SpmmKernelCsr(self.data, self.col, indptr, one_shot=True)
+            self._kc = _SpmmKernelCsr(self.data, self.col, row_pointers(self.row, self.n_rows),
+                                      one_shot=True)
         return self._kc
 
 
@@ -166,6 +162,7 @@ def _spmm_coo_atomic(data, row, col, n_rows, B, n_dense_cols):
     """The atomic route, entries in any order: an fp64 accumulation buffer (fp32 inputs are
     computed in fp64, as in the reference), rounded to the input dtype at the end."""
     dtype = data.dtype
+    row, col = row.to(torch.int32), col.to(torch.int32)
     C_acc = torch.empty((n_rows, n_dense_cols), dtype=torch.float64, device=B.device)
     L = _abi.lib()
     _abi.check(
@@ -186,7 +183,7 @@ def _run_spmm_coo_route(data, row, col, B, shape, block_n=None, block_nnz=256, o
     if block_nnz is not None and block_nnz <= 0:
         raise ValueError("block_nnz must be positive when provided")
     data, row, col, B, n_rows, n_cols, n_dense_cols, row_sorted = \
-        _prepare_spmm_coo_inputs_checked(data, row, col, B, shape)
+        _check_spmm_coo_inputs(data, row, col, B, shape)
     launch = _resolve_spmm_coo_launch_config(n_dense_cols, data.numel(), block_n=block_n,
                                              block_nnz=block_nnz)
     dtype = data.dtype

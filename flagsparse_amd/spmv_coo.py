@@ -17,7 +17,9 @@ import torch
 
 from . import _abi, _spmv_layouts
 from ._common import _INDEX_LIMIT_INT32
-from ._spmv_layouts import RowBlockLayout, build_layout
+from ._coo_order import row_pointers, rows_in_order
+from ._index_stats import index_stats
+from ._spmv_layouts import RowBlockLayout, SliceLayout, build_layout
 
 
 class PreparedCoo:
@@ -61,7 +63,7 @@ class PreparedCoo:
         """Kernel layout over the row runs (flagsparse_amd/_spmv_layouts.py) and the
         run -> row map, omitted when it is the identity."""
         if self._layout is None:
-            if self._one_shot and _spmv_layouts.FORCE is None:
+            if self._one_shot and _spmv_layouts.FORCE is None:  # the layout that builds fastest
                 self._layout = RowBlockLayout(self.data, self.col, self.seg_starts)
             else:
                 self._layout = build_layout(self.data, self.col, self.seg_starts, self.n_cols)
@@ -111,8 +113,8 @@ def _seg_starts_from_sorted_rows(row_sorted, nnz, device):
     ])
 
 
-def _prepare_coo_tensors(data, row, col, shape, sort_by_row):
-    """spmv_coo.py:182-217 (same checks, order and exceptions)."""
+def _check_coo_tensors(data, row, col, shape):
+    """The host checks of spmv_coo.py:182-217 (same order and exceptions): (n_rows, n_cols)."""
     if not all(torch.is_tensor(t) for t in (data, row, col)):
         raise TypeError("data, row, col must all be torch.Tensor")
     if data.ndim != 1 or row.ndim != 1 or col.ndim != 1:
@@ -126,6 +128,21 @@ def _prepare_coo_tensors(data, row, col, shape, sort_by_row):
         raise TypeError(
             "this COO SpMV path supports float32/float64 only (use CSR for other dtypes)"
         )
+    return n_rows, n_cols
+
+
+def _check_coo_bounds(rmin, rmax, cmin, cmax, n_rows, n_cols):
+    if rmin < 0 or rmax >= n_rows:
+        raise IndexError("row indices out of range")
+    if cmin < 0 or cmax >= n_cols:
+        raise IndexError("col indices out of range")
+    if rmax > _INDEX_LIMIT_INT32 or cmax > _INDEX_LIMIT_INT32:
+        raise ValueError("indices exceed int32 Triton kernel range")
+
+
+def _prepare_coo_tensors(data, row, col, shape, sort_by_row):
+    """spmv_coo.py:182-217 (same checks, order and exceptions)."""
+    n_rows, n_cols = _check_coo_tensors(data, row, col, shape)
     if sort_by_row:
         data, row64, col64 = _sort_coo_lex_inplace(data, row, col, n_cols)
         seg = _seg_starts_from_sorted_rows(row64, data.numel(), data.device)
@@ -137,12 +154,7 @@ def _prepare_coo_tensors(data, row, col, shape, sort_by_row):
     if data.numel() > 0:
         rmin, rmax, cmin, cmax = torch.stack(
             [row64.min(), row64.max(), col64.min(), col64.max()]).tolist()
-        if rmin < 0 or rmax >= n_rows:
-            raise IndexError("row indices out of range")
-        if cmin < 0 or cmax >= n_cols:
-            raise IndexError("col indices out of range")
-        if rmax > _INDEX_LIMIT_INT32 or cmax > _INDEX_LIMIT_INT32:
-            raise ValueError("indices exceed int32 Triton kernel range")
+        _check_coo_bounds(rmin, rmax, cmin, cmax, n_rows, n_cols)
     return data, row64.to(torch.int32), col64.to(torch.int32), seg
 
 
@@ -152,12 +164,37 @@ def prepare_spmv_coo(data, row, col, shape, sort_by_row=True):
 
 
 def _prepare_spmv_coo(data, row, col, shape, sort_by_row, one_shot):
-    """prepare_spmv_coo; one_shot: for a single call (the layout that builds fastest)."""
     d, kr, kc, seg = _prepare_coo_tensors(data, row, col, shape, sort_by_row)
     prepared = PreparedCoo(d, kr, kc, shape, seg_starts=seg)
     prepared._one_shot = bool(one_shot)
     if prepared.use_seg_kernel:
         prepared._run_layout()
+    return prepared
+
+
+def _prepare_one_call(data, row, col, shape, sort_by_row):
+    """prepare_spmv_coo for a single call.  Only the sums are asked for, so the entries are put in
+    row order rather than (row, column) order, by a sort that carries them, and run as CSR slices:
+    nothing is planned, and a row without entries is an empty row.  The prepared way is left for
+    what that does not take: index types other than int32 / int64, no entries, and so many more
+    rows than entries (beyond 64M rows) that row pointers would be most of the memory."""
+    if not (sort_by_row and _spmv_layouts.FORCE is None
+            and all(torch.is_tensor(t) and t.dtype in (torch.int32, torch.int64)
+                    for t in (row, col))):
+        return _prepare_spmv_coo(data, row, col, shape, sort_by_row, True)
+    n_rows, n_cols = _check_coo_tensors(data, row, col, shape)
+    nnz = data.numel()
+    if nnz == 0 or n_rows > max(1 << 26, 4 * nnz) or not data.device == row.device == col.device:
+        return _prepare_spmv_coo(data, row, col, shape, sort_by_row, True)
+    data, row, col = data.contiguous(), row.contiguous(), col.contiguous()
+    # one pass over both index arrays and one host synchronisation: bounds and row order
+    rmin, rmax, cmin, cmax, descents = index_stats(row, col)
+    _check_coo_bounds(rmin, rmax, cmin, cmax, n_rows, n_cols)
+    if descents:
+        data, row, col = rows_in_order(data, row, col, rmax)
+    prepared = PreparedCoo(data, row, col.to(torch.int32), shape)
+    prepared.use_seg_kernel = True
+    prepared._layout = SliceLayout(data, prepared.col, row_pointers(row, n_rows))
     return prepared
 
 
@@ -220,7 +257,7 @@ def flagsparse_spmv_coo(
     if prepared is None:
         if any(a is None for a in (data, row, col, x, shape)):
             raise ValueError("data, row, col, x, shape required when prepared is None")
-        prepared = _prepare_spmv_coo(data, row, col, shape, sort_by_row, True)
+        prepared = _prepare_one_call(data, row, col, shape, sort_by_row)
     else:
         if x is None:
             raise TypeError("x is required when prepared is set")

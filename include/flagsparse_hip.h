@@ -455,6 +455,25 @@ int fsp_spmm_sliced(int dtype, int acc_f64, const void* vals, const int32_t* col
                     int lanes_per_row, int vec, int xcd_remap, void* stream);
 
 /*
+ * COO entries into row order (stable), in place of the lexicographic sorts of
+ * spmv_coo.py:153-164 and spmm_coo.py:136-180: a radix sort by row that carries the columns and
+ * values and narrows the indices to int32.
+ *   rows, cols     nnz indices, int32 or int64 each, rows in [0, max_row], max_row < 2^31
+ *   nnz            at most fsp_coo_sort_max_nnz()
+ *   out_rows, out_cols, out_vals   the ordered entries; may not overlap the inputs
+ *   scratch        fsp_coo_sort_scratch(dtype, nnz, max_row) bytes, 16-byte aligned
+ * fsp_coo_rowptr: ptr[r], r = 0 .. n_rows, = the number of entries of row-ordered rows whose row
+ * is below r (the CSR row pointers when all rows are in [0, n_rows)).
+ */
+int64_t fsp_coo_sort_max_nnz(void);
+int64_t fsp_coo_sort_scratch(int dtype, int64_t nnz, int64_t max_row);
+int fsp_coo_sort_rows(int dtype, const void* rows, int row_bits, const void* cols, int col_bits,
+                      const void* vals, int64_t nnz, int64_t max_row, int32_t* out_rows,
+                      int32_t* out_cols, void* out_vals, void* scratch, void* stream);
+int fsp_coo_rowptr(const void* rows, int row_bits, int64_t nnz, int64_t n_rows, void* ptr,
+                   int ptr_bits, void* stream);
+
+/*
  * COO SpMM with atomics: C_acc[rows[e], n] += vals[e] * B[cols[e], n] for every entry e and
  * n < N.  Replaces the reference's atomic route, spmm_coo.py:244-271 (_spmm_coo_atomic_real_
  * kernel) and :464-523 (_triton_spmm_coo_atomic_impl).  C_acc[0 .. n_rows*ldc) is zeroed first;
