@@ -22,7 +22,7 @@ LIB_PATH = os.path.join(LIB_DIR, LIB_NAME)
 
 SOURCES = ("abi.cpp", "mtx.cpp", "plan.hip", "spmv.hip", "spmv_xcs.hip", "spmm.hip", "sddmm.hip",
            "index_stats.hip", "check.hip", "slices.hip",
-           "spmm_slices.hip", "coo_sort.hip", "probe.hip")
+           "spmm_slices.hip", "sddmm_slices.hip", "coo_sort.hip", "probe.hip")
 ARCH = "gfx950"
 
 # Packed-FP32 instructions (v_pk_*_f32) are disabled for all device code.

@@ -126,6 +126,46 @@ __device__ __forceinline__ void gather_x(const T* __restrict__ x, const int (&c)
   }
 }
 
+// A vector of VW elements at any element's address.
+template <typename T, int VW> struct AnyVec { typedef T type; };
+template <> struct AnyVec<float, 4> {
+  typedef float type __attribute__((ext_vector_type(4), aligned(4)));
+};
+template <> struct AnyVec<float, 2> {
+  typedef float type __attribute__((ext_vector_type(2), aligned(4)));
+};
+template <> struct AnyVec<double, 2> {
+  typedef double type __attribute__((ext_vector_type(2), aligned(8)));
+};
+template <> struct AnyVec<double, 4> {  // sums of float32 vectors taken in float64
+  typedef double type __attribute__((ext_vector_type(4), aligned(8)));
+};
+
+template <typename T, int VW>
+__device__ __forceinline__ void load_any(const T* p, T (&o)[VW]) {
+  typedef typename AnyVec<T, VW>::type V;
+  const V v = *reinterpret_cast<const V*>(p);
+  if constexpr (VW == 1) {
+    o[0] = v;
+  } else {
+#pragma unroll
+    for (int j = 0; j < VW; ++j) o[j] = v[j];
+  }
+}
+
+template <typename T, typename A, int VW>
+__device__ __forceinline__ void store_any(T* p, const A (&a)[VW]) {
+  typedef typename AnyVec<T, VW>::type V;
+  V v;
+  if constexpr (VW == 1) {
+    v = T(a[0]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < VW; ++j) v[j] = T(a[j]);
+  }
+  *reinterpret_cast<V*>(p) = v;
+}
+
 // Lane permutes through DPP (a VALU modifier, no LDS round trip).  dpp_add<CTRL>(v) adds the
 // value of the lane that the DPP control word CTRL selects; all sources used here lie inside
 // the lane's 16-lane row, so every lane reads a valid source.

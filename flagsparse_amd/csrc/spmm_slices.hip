@@ -32,46 +32,6 @@ namespace {
 
 constexpr int kInFlight = 4;  // B rows requested together per lane
 
-// A vector of VW elements at any element's address.
-template <typename T, int VW> struct AnyVec { typedef T type; };
-template <> struct AnyVec<float, 4> {
-  typedef float type __attribute__((ext_vector_type(4), aligned(4)));
-};
-template <> struct AnyVec<float, 2> {
-  typedef float type __attribute__((ext_vector_type(2), aligned(4)));
-};
-template <> struct AnyVec<double, 2> {
-  typedef double type __attribute__((ext_vector_type(2), aligned(8)));
-};
-template <> struct AnyVec<double, 4> {  // sums of float32 vectors taken in float64
-  typedef double type __attribute__((ext_vector_type(4), aligned(8)));
-};
-
-template <typename T, int VW>
-__device__ __forceinline__ void load_any(const T* p, T (&o)[VW]) {
-  typedef typename AnyVec<T, VW>::type V;
-  const V v = *reinterpret_cast<const V*>(p);
-  if constexpr (VW == 1) {
-    o[0] = v;
-  } else {
-#pragma unroll
-    for (int j = 0; j < VW; ++j) o[j] = v[j];
-  }
-}
-
-template <typename T, typename A, int VW>
-__device__ __forceinline__ void store_any(T* p, const A (&a)[VW]) {
-  typedef typename AnyVec<T, VW>::type V;
-  V v;
-  if constexpr (VW == 1) {
-    v = T(a[0]);
-  } else {
-#pragma unroll
-    for (int j = 0; j < VW; ++j) v[j] = T(a[j]);
-  }
-  *reinterpret_cast<V*>(p) = v;
-}
-
 // acc += the products of entries a, a + step, ... < e of the staged slice.
 template <typename T, typename A, int VW>
 __device__ __forceinline__ void add_entries(const int* s_col, const T* s_val, int a, int e,

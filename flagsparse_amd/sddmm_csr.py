@@ -7,10 +7,9 @@ diagnostic variants of ``_run_sddmm_prepared`` (:243-347) and ``benchmark_sddmm_
 (:472-572).
 
 out[p] = alpha * dot(x[row(p)], y[col(p)]) + beta * data[p] for every stored entry p, computed
-by flagsparse_amd/csrc/sddmm.hip in the input precision (float64 for the "acc64" variants) with
-a fixed reduction order: ``sddmm_rowblock_kernel`` over a row-block plan built on the device
-(one lane group per row, the row of x held in registers) when K <= 4 * 64 lanes * vector
-width, ``sddmm_flat_kernel`` (one lane group per entry) otherwise.
+in the input precision (float64 for the "acc64" variants) with a fixed reduction order:
+``sddmm_slices_kernel`` (csrc/sddmm_slices.hip; slices of equal work, no plan) when K <= 4 * 64
+lanes * vector width, ``sddmm_flat_kernel`` (csrc/sddmm.hip; one lane group per entry) otherwise.
 """
 
 import time
@@ -26,27 +25,20 @@ from ._common import (  # noqa: F401  (cp and the converters: the reference scri
     _torch_from_cupy,
     cp,
 )
-from ._plan import build_row_block_plan_device
+from ._csr_check import csr_check
 from .synthetic import build_random_csr, build_random_dense
 
 SUPPORTED_SDDMM_VALUE_DTYPES = (torch.float32, torch.float64)
 SUPPORTED_SDDMM_DIAGNOSTIC_VARIANTS = ("baseline", "acc64", "acc64_out64", "altreduce")
 
-_BLOCK_THREADS = 256
-# Rows longer than this are cut into chunks that all lane groups of a workgroup share.
-_SDDMM_ROW_SPLIT_THRESHOLD = 128
-# The row-block plan is built in windows of this many blocks' rows (windows of one block's
-# rows add a tiny block whenever the entry cap ends a block before the row cap does; wider
-# windows plan more slowly), as for SpMM.
-SDDMM_PLAN_WINDOW_BLOCKS = 4
-
 
 class SDDMMPrepared:
     """Prepared CSR pattern for SDDMM (sddmm_csr.py:9-33): int32 columns, int64 row pointers,
-    one int32 row id per entry, and the reference's launch attributes (block_k, num_warps)."""
+    one int32 row id per entry (made when first asked for), and the reference's launch attributes
+    (block_k, num_warps)."""
 
-    __slots__ = ("indices", "indptr", "shape", "n_rows", "n_cols", "nnz", "row_ids", "block_k",
-                 "num_warps", "_plans", "_kernel_ptr", "_window_blocks")
+    __slots__ = ("indices", "indptr", "shape", "n_rows", "n_cols", "nnz", "_row_ids", "block_k",
+                 "num_warps", "_tables", "_kernel_ptr", "_one_call")
 
     def __init__(self, indices, indptr, shape, row_ids, block_k, num_warps):
         self.indices = indices
@@ -55,29 +47,41 @@ class SDDMMPrepared:
         self.n_rows = self.shape[0]
         self.n_cols = self.shape[1]
         self.nnz = int(indices.numel())
-        self.row_ids = row_ids
+        self._row_ids = row_ids
         self.block_k = int(block_k)
         self.num_warps = int(num_warps)
-        self._plans = {}
+        self._tables = {}
         self._kernel_ptr = None
-        self._window_blocks = SDDMM_PLAN_WINDOW_BLOCKS  # 1 for a prepared object of one call
+        self._one_call = False  # made by and for a single call
 
-    def _row_plan(self, lanes):
-        """Row-block plan for ``lanes`` lanes per entry (built on the device, cached)."""
-        plan = self._plans.get(lanes)
-        if plan is None:
+    @property
+    def row_ids(self):
+        if self._row_ids is None:
+            self._row_ids = _build_row_ids(self.indptr)
+        return self._row_ids
+
+    def _slices(self, items):
+        """The boundaries of slices of ``items`` rows + entries (built once per size)."""
+        table = self._tables.get(items)
+        if table is None:
+            if torch.cuda.is_current_stream_capturing():
+                raise RuntimeError("an SDDMM must run once before it is captured into a graph "
+                                   "(the first call with this K builds its slices)")
+            L = _abi.lib()
+            dev = self.indices.device
             if self._kernel_ptr is None:
-                self._kernel_ptr = (self.indptr.to(torch.int32)
-                                    if self.nnz <= _common.ROWPTR32_MAX_NNZ
-                                    else self.indptr.to(torch.int64))
-            cap = _abi.caps()["spmm_block_nnz"]
-            rows_cap = _BLOCK_THREADS // lanes
-            plan = build_row_block_plan_device(self._kernel_ptr, cap, rows_cap,
-                                               min(_SDDMM_ROW_SPLIT_THRESHOLD, cap), cap,
-                                               window_rows=self._window_blocks * rows_cap)
-            self._plans[lanes] = plan
-        return plan
-
+                self._kernel_ptr = self.indptr.to(
+                    torch.int32 if self.nnz <= _common.ROWPTR32_MAX_NNZ else torch.int64)
+            rp = self._kernel_ptr
+            n = L.fsp_slice_count(self.n_rows, self.nnz, items)
+            table = torch.empty(2 * (n + 1), dtype=torch.int64, device=dev)
+            _abi.check(L.fsp_slice_table(rp.data_ptr(), 32 if rp.dtype == torch.int32 else 64,
+                                         self.n_rows, self.nnz, items, 0, table.data_ptr(),
+                                         _abi.raw_stream(dev)), "fsp_slice_table")
+            if not self._one_call:  # later calls may come from other streams
+                torch.cuda.current_stream(dev).synchronize()
+            self._tables[items] = table
+        return table
 
 
 def _resolve_sddmm_launch_config(k):
@@ -91,8 +95,9 @@ def _resolve_sddmm_launch_config(k):
     return 128, 8
 
 
-def _prepare_sddmm_csr_pattern(indices, indptr, shape):
-    """Validation of sddmm_csr.py:46-79 (same checks, order, messages and types)."""
+def _prepare_sddmm_csr_pattern(indices, indptr, shape, ptr_bits=64):
+    """Validation of sddmm_csr.py:46-79 (same checks, order, messages and types); the row pointers
+    come back at ``ptr_bits``."""
     if len(shape) != 2:
         raise ValueError("shape must be a 2-tuple")
     if indices.ndim != 1 or indptr.ndim != 1:
@@ -108,25 +113,20 @@ def _prepare_sddmm_csr_pattern(indices, indptr, shape):
         raise TypeError("indices dtype must be torch.int32")
     if indptr.dtype not in (torch.int32, torch.int64):
         raise TypeError("indptr dtype must be torch.int32 or torch.int64")
-    indptr64 = indptr.to(torch.int64).contiguous()
     indices = _aligned(indices.contiguous())  # 16-byte loads of the columns
     nnz = int(indices.numel())
-    # one host sync for the structural checks: first, last, monotone
-    first, last, bad = torch.stack([
-        indptr64[0], indptr64[-1],
-        (indptr64[1:] < indptr64[:-1]).any().to(torch.int64) if n_rows > 0
-        else torch.zeros((), dtype=torch.int64, device=indptr64.device)]).tolist()
+    # one pass over both arrays, one host synchronisation
+    (first, last, decreases, _, min_col, max_col), indices, indptr = csr_check(
+        indices, indptr.contiguous(), ptr_bits)
     if first != 0:
         raise ValueError("indptr[0] must be 0")
     if last != nnz:
         raise ValueError(f"indptr[-1] must equal nnz={nnz}")
-    if bad:
+    if decreases:
         raise ValueError("indptr must be nondecreasing")
-    if nnz > 0:
-        min_col, max_col = torch.stack([indices.min(), indices.max()]).tolist()
-        if min_col < 0 or max_col >= n_cols:
-            raise IndexError("indices out of range for shape[1]")
-    return indices, indptr64, (n_rows, n_cols)
+    if nnz > 0 and (min_col < 0 or max_col >= n_cols):
+        raise IndexError("indices out of range for shape[1]")
+    return indices, indptr, (n_rows, n_cols)
 
 
 def _build_row_ids(indptr):
@@ -138,12 +138,23 @@ def _build_row_ids(indptr):
 
 
 def prepare_sddmm_csr(indices, indptr, shape, k_hint=64):
-    """Validate a CSR pattern and build its per-entry row ids (sddmm_csr.py:93-104)."""
-    indices, indptr, shape = _prepare_sddmm_csr_pattern(indices, indptr, shape)
-    row_ids = _build_row_ids(indptr)
+    """Validate a CSR pattern (sddmm_csr.py:93-104)."""
+    return _prepare_sddmm(indices, indptr, shape, k_hint, False)
+
+
+def _prepare_sddmm(indices, indptr, shape, k_hint, one_call):
+    """prepare_sddmm_csr; one_call: row pointers only at the width the kernel reads."""
+    narrow = one_call and torch.is_tensor(indices) and \
+        indices.numel() <= _common.ROWPTR32_MAX_NNZ
+    indices, indptr, shape = _prepare_sddmm_csr_pattern(indices, indptr, shape,
+                                                        32 if narrow else 64)
     block_k, num_warps = _resolve_sddmm_launch_config(int(k_hint))
-    return SDDMMPrepared(indices=indices, indptr=indptr, shape=shape, row_ids=row_ids,
-                         block_k=block_k, num_warps=num_warps)
+    prepared = SDDMMPrepared(indices=indices, indptr=indptr, shape=shape, row_ids=None,
+                             block_k=block_k, num_warps=num_warps)
+    if one_call:
+        prepared._one_call = True
+        prepared._kernel_ptr = indptr
+    return prepared
 
 
 def _validate_sddmm_dense_inputs(data, prepared, x, y):
@@ -225,28 +236,65 @@ def _sddmm_lane_shape(K, x, y):
     return lanes, vec
 
 
+def _sddmm_slice_lanes(K, dtype):
+    """(lanes per entry G, elements per lane vec) for the sliced kernel: 16-byte loads for every K
+    that holds one.  Half the lanes that would cover K in one step, at most 16 while four steps
+    hold K: a group's sum over its lanes costs more than its second load.  Measured on MI355X,
+    fp32 K=64, 33.5M entries (16 / 8 / 4 lanes, best slice size) 676 / 674 / 700 us; K=33, 1.6M
+    52.3 / 48.9 / 51.7; fp64 K=50, 1M, a power law (32 / 16 / 8) 70.4 / 67.6 / 68.2; up to 4
+    lanes the full number is the faster (fp32 K=16, 4.8M: 4 / 2 / 1 lanes 41.7 / 43.2 / 57.9)."""
+    vec = 4 if dtype == torch.float32 else 2
+    if K < vec:
+        vec = 2 if K >= 2 else 1
+    lanes = 1
+    while lanes * vec < K and lanes < 64:
+        lanes <<= 1
+    if lanes > 4:
+        lanes = min(16, lanes // 2)
+    while lanes < 64 and K > 4 * lanes * vec:
+        lanes <<= 1
+    return lanes, vec
+
+
+def _sddmm_slice_items(lanes, positions):
+    """Rows + entries per slice: small, so that many workgroups are in flight and one XCD's lie
+    close together, but not so small that launching workgroups is the bound (fp32 K=64, 34.6M
+    positions, 8 lanes: 674 / 689 / 739 us with 256 / 512 / 1024; 16 lanes: 818 / 676 / 704 with
+    128 / 256 / 512), and fewer where the slices would not fill the 256 CUs."""
+    items = {1: 1024, 2: 1024, 4: 512, 8: 256}.get(lanes, 128)
+    while positions > 150000 * items and items < 4096:
+        items <<= 1
+    while items > 64 and positions < 256 * items:
+        items >>= 1
+    return items
+
+
 def _launch_sddmm(prepared, x, y, data, alpha, beta, out, acc_f64):
-    """fsp_sddmm_csr with the row-block schedule when K fits four steps of the lane group
-    (x rows kept in registers), else one lane group per entry."""
+    """The sliced kernel when K fits four steps of a lane group, else one lane group per entry."""
     K = int(x.shape[1])
-    lanes, vec = _sddmm_lane_shape(K, x, y)
     L = _abi.lib()
+    code = _abi.dtype_code(x.dtype)
+    out_f64 = int(out.dtype == torch.float64 and x.dtype == torch.float32)
     cols = prepared.indices
-    if K <= 4 * lanes * vec and cols.data_ptr() % 16 == 0:
-        plan = prepared._row_plan(lanes)
+    lanes, vec = _sddmm_slice_lanes(K, x.dtype)
+    if 1 <= K <= 4 * lanes * vec and cols.data_ptr() % 16 == 0:
+        items = _sddmm_slice_items(lanes, prepared.n_rows + prepared.nnz)
+        table = prepared._slices(items)
         rp = prepared._kernel_ptr
-        sched = (_abi.ptr(rp), 32 if rp.dtype == torch.int32 else 64, _abi.ptr(plan.desc),
-                 _abi.ptr(plan.ranges), plan.n_desc)
-    else:
-        sched = (None, 32, None, None, 0)
-    rowptr, bits, desc, ranges, n_desc = sched
+        _abi.check(
+            L.fsp_sddmm_sliced(code, int(acc_f64), out_f64, cols.data_ptr(), rp.data_ptr(),
+                               32 if rp.dtype == torch.int32 else 64, prepared.n_rows,
+                               prepared.nnz, x.data_ptr(), x.stride(0), y.data_ptr(),
+                               y.stride(0), K, None if data is None else data.data_ptr(),
+                               float(alpha), float(beta), out.data_ptr(), table.data_ptr(), items,
+                               lanes, vec, _abi.raw_stream(x.device)), "fsp_sddmm_sliced")
+        return
+    lanes, vec = _sddmm_lane_shape(K, x, y)
     _abi.check(
-        L.fsp_sddmm_csr(_abi.dtype_code(x.dtype), int(acc_f64),
-                        int(out.dtype == torch.float64 and x.dtype == torch.float32),
-                        _abi.ptr(cols), _abi.ptr(prepared.row_ids), rowptr, bits, prepared.nnz,
-                        _abi.ptr(x), x.stride(0), _abi.ptr(y), y.stride(0), K, _abi.ptr(data),
-                        float(alpha), float(beta), _abi.ptr(out), desc, ranges, n_desc, lanes,
-                        vec, _abi.stream_handle(x.device)),
+        L.fsp_sddmm_csr(code, int(acc_f64), out_f64, _abi.ptr(cols), _abi.ptr(prepared.row_ids),
+                        None, 32, prepared.nnz, _abi.ptr(x), x.stride(0), _abi.ptr(y),
+                        y.stride(0), K, _abi.ptr(data), float(alpha), float(beta), _abi.ptr(out),
+                        None, None, 0, lanes, vec, _abi.stream_handle(x.device)),
         "fsp_sddmm_csr")
 
 
@@ -302,17 +350,19 @@ def flagsparse_sddmm_csr(data=None, indices=None, indptr=None, x=None, y=None, s
                          return_meta=False, allow_fallback=False):
     """CSR SDDMM: out[p] = alpha * dot(x[row(p)], y[col(p)]) + beta * data[p]
     (sddmm_csr.py:350-422; returns out, optionally with the elapsed ms and/or metadata)."""
+    timed = return_time or return_meta  # the only calls that wait for the device
     prepare_ms = 0.0
     if prepared is None:
         if any(v is None for v in (indices, indptr, shape)):
             raise ValueError(
                 "indices, indptr, and shape are required when prepared is not provided")
-        torch.cuda.synchronize()
+        if timed:
+            torch.cuda.synchronize()
         t0 = time.perf_counter()
         k_hint = int(x.shape[1]) if (x is not None and x.ndim == 2) else 64
-        prepared = prepare_sddmm_csr(indices, indptr, shape, k_hint=k_hint)
-        prepared._window_blocks = 1  # planned for this call only: the fastest plan to build
-        torch.cuda.synchronize()
+        prepared = _prepare_sddmm(indices, indptr, shape, k_hint, True)
+        if timed:
+            torch.cuda.synchronize()
         prepare_ms = (time.perf_counter() - t0) * 1000.0
     elif not isinstance(prepared, SDDMMPrepared):
         raise TypeError("prepared must be a SDDMMPrepared instance")
@@ -336,13 +386,15 @@ def flagsparse_sddmm_csr(data=None, indices=None, indptr=None, x=None, y=None, s
         if return_meta:
             return out, meta
         return out
-    torch.cuda.synchronize()
+    if timed:
+        torch.cuda.synchronize()
     t0 = time.perf_counter()
     out_tensor, launch_meta = _run_sddmm_prepared(
         prepared, x.contiguous(), y.contiguous(),
         data.contiguous() if data is not None else None, alpha, beta, out,
         allow_fallback=allow_fallback)
-    torch.cuda.synchronize()
+    if timed:
+        torch.cuda.synchronize()
     elapsed_ms = (time.perf_counter() - t0) * 1000.0
     meta = {"prepare_ms": prepare_ms, **launch_meta}
     if return_time and return_meta:

@@ -523,6 +523,21 @@ int fsp_sddmm_csr(int dtype, int acc_f64, int out_f64, const int32_t* cols,
                   int lanes_per_entry, int vec, void* stream);
 
 /*
+ * The same over the slices of fsp_slice_table(rowptr, .., items, 0, table): no plan, row by row,
+ * for vec <= K <= 4 * lanes_per_entry * vec, K >= 1.
+ *   items          rows + entries per slice, at most 4096
+ *   vec            elements per lane per load: 1, 2 or 4 (fp32) / 1 or 2 (fp64); needs no
+ *                  alignment of x, y, ldx or ldy beyond the element's own
+ *   cols           16-byte aligned; the other arguments as fsp_sddmm_csr
+ */
+int fsp_sddmm_sliced(int dtype, int acc_f64, int out_f64, const int32_t* cols,
+                     const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t nnz,
+                     const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t K,
+                     const void* data_in, double alpha, double beta, void* out,
+                     const int64_t* table, int64_t items, int lanes_per_entry, int vec,
+                     void* stream);
+
+/*
  * Matrix Market coordinate file reader (host only, no GPU): the format of the reference's
  * SuiteSparse test drivers (tests/test_spmv.py:29-103, tests/test_spmm_coo.py:156-249,
  * tests/test_spmv_coo.py:257-305).  info[0..7) receives n_rows, n_cols, the header nnz, the
