@@ -52,8 +52,9 @@ SIGNATURES = {
                             _i64, _i64, _p, _p, _p, _p, _i64, _i32, _p]),
     "fsp_spmv_slices": (_i64, [_i64, _i64]),
     "fsp_spmv_slice_keep": (_i64, []),
-    "fsp_spmv_sliced": (_i32, [_i32, _i32, _p, _p, _p, _i32, _i64, _i64, _p, _p, _p, _p, _i32,
-                               _p]),
+    "fsp_spmv_slice_items": (_i64, []),
+    "fsp_spmv_sliced": (_i32, [_i32, _i32, _p, _p, _p, _i32, _i64, _i64, _p, _p, _p, _i32, _p,
+                               _i32, _p]),
     "fsp_csr_check_partial_len": (_i64, []),
     "fsp_csr_check": (_i32, [_p, _i32, _i64, _p, _i32, _i64, _p, _p, _i32, _p, _p, _p]),
     "fsp_spmv_scratch_slots": (_i64, []),
@@ -73,8 +74,10 @@ SIGNATURES = {
                             _i64, _i64, _i32, _i32, _p, _p, _p, _p, _i64, _i32, _p]),
     "fsp_slice_count": (_i64, [_i64, _i64, _i64]),
     "fsp_slice_table": (_i32, [_p, _i32, _i64, _i64, _i64, _i64, _p, _p]),
+    "fsp_slice_order_scratch": (_i64, [_i64]),
+    "fsp_slice_order": (_i32, [_p, _i64, _p, _i64, _p, _p, _p]),
     "fsp_spmm_sliced": (_i32, [_i32, _i32, _p, _p, _p, _i32, _i64, _i64, _p, _i64, _i64, _p, _i64,
-                               _p, _i64, _i64, _p, _i32, _i32, _i32, _i32, _p]),
+                               _p, _p, _i64, _i64, _p, _i32, _i32, _i32, _i32, _p]),
     "fsp_coo_sort_max_nnz": (_i64, []),
     "fsp_coo_sort_scratch": (_i64, [_i32, _i64, _i64]),
     "fsp_coo_sort_rows": (_i32, [_i32, _p, _i32, _p, _i32, _p, _i64, _i64, _p, _p, _p, _p, _p]),
@@ -90,7 +93,7 @@ SIGNATURES = {
     "fsp_sddmm_csr": (_i32, [_i32, _i32, _i32, _p, _p, _p, _i32, _i64, _p, _i64, _p, _i64, _i64,
                              _p, _f64, _f64, _p, _p, _p, _i64, _i32, _i32, _p]),
     "fsp_sddmm_sliced": (_i32, [_i32, _i32, _i32, _p, _p, _i32, _i64, _i64, _p, _i64, _p, _i64, _i64,
-                                _p, _f64, _f64, _p, _p, _i64, _i32, _i32, _p]),
+                                _p, _f64, _f64, _p, _p, _p, _i64, _i32, _i32, _p]),
     "fsp_probe_gather_blocks": (_i64, [_i64]),
     "fsp_probe_gather": (_i32, [_p, _i64, _p, _i64, _p, _p]),
     "fsp_probe_rows_blocks": (_i64, [_i64]),

@@ -228,12 +228,12 @@ class RowBlockLayout:
 
 
 class SliceLayout:
-    """CSR arrays (16-byte aligned) cut into slices of equal work inside the call itself
-    (csrc/slices.hip): nothing is planned, so it is what a matrix used once runs on."""
+    """CSR arrays (16-byte aligned) cut into slices of equal work (csrc/slices.hip).  one_shot: the
+    call itself builds the slices' table; else it is built here."""
 
     kind = "slices"
 
-    def __init__(self, data, cols, rowptr, max_row_nnz=None):
+    def __init__(self, data, cols, rowptr, max_row_nnz=None, one_shot=False):
         self.data = _aligned(data)
         self.cols = _aligned(cols)
         self.nnz = int(data.numel())
@@ -243,30 +243,40 @@ class SliceLayout:
         self.n_rows = int(rowptr.numel()) - 1
         L = _abi.lib()
         # an unknown longest row may be cut
-        self.cut_rows = max_row_nnz is None or max_row_nnz > L.fsp_spmv_slice_keep()
+        cut_rows = max_row_nnz is None or max_row_nnz > L.fsp_spmv_slice_keep()
         n = int(L.fsp_spmv_slices(self.n_rows, self.nnz))
-        self._scratch = torch.empty(2 * (n + 1) + 2 * n, dtype=torch.int64,
-                                    device=self.data.device)
-        self._sums = self._scratch.data_ptr() + 16 * (n + 1)
+        scratch = torch.empty(2 * (n + 1) + 2 * n, dtype=torch.int64, device=self.data.device)
+        if not one_shot:
+            _abi.check(L.fsp_slice_table(self.rowptr.data_ptr(), self.rowptr_bits, self.n_rows,
+                                         self.nnz, L.fsp_spmv_slice_items(),
+                                         L.fsp_spmv_slice_keep(), scratch.data_ptr(),
+                                         _abi.raw_stream(scratch.device)), "fsp_slice_table")
+        self.cut_rows = cut_rows
+        self._keep = (scratch, self.data, self.cols, self.rowptr)
+        self._args = [_abi.dtype_code(self.data.dtype), None, self.data.data_ptr(),
+                      self.cols.data_ptr(), self.rowptr.data_ptr(), self.rowptr_bits,
+                      self.n_rows, self.nnz, None, None, scratch.data_ptr(), int(not one_shot),
+                      scratch.data_ptr() + 16 * (n + 1), int(cut_rows), None]
         self._order = StreamOrder(self.data.device)
 
     def kernel_name(self):
         return "spmv_slices_kernel"
+
+    def held_bytes(self, caller=()):
+        """Device bytes this layout holds beyond the caller's arrays ``caller``."""
+        theirs = {t.untyped_storage().data_ptr() for t in caller if isinstance(t, torch.Tensor)}
+        return tensor_bytes(*[t for t in self._keep
+                              if t.untyped_storage().data_ptr() not in theirs])
 
     def describe(self):
         return {"layout": self.kind, "cut_rows": self.cut_rows}
 
     def launch(self, x, y, acc_f64, row_map=None, n_out=0):
         assert row_map is None, "slices write every row"
-        stream = self._order.stream(y.device, (self._scratch, self.data, self.cols, self.rowptr))
-        _abi.check(
-            _abi.lib().fsp_spmv_sliced(_abi.dtype_code(self.data.dtype), int(acc_f64),
-                                       self.data.data_ptr(), self.cols.data_ptr(),
-                                       self.rowptr.data_ptr(), self.rowptr_bits, self.n_rows,
-                                       self.nnz, x.data_ptr(), y.data_ptr(),
-                                       self._scratch.data_ptr(), self._sums, int(self.cut_rows),
-                                       stream),
-            "fsp_spmv_sliced")
+        a = list(self._args)
+        a[1], a[8], a[9] = int(acc_f64), x.data_ptr(), y.data_ptr()
+        a[14] = self._order.stream(y.device, self._keep)
+        _abi.check(_abi.lib().fsp_spmv_sliced(*a), "fsp_spmv_sliced")
         return y
 
 
@@ -1420,7 +1430,7 @@ def build_layout(data, cols, rowptr, n_cols, one_shot=False, max_row_nnz=None):
     mode = FORCE
     nnz = int(data.numel())
     if mode is None and one_shot:
-        return SliceLayout(data, cols, rowptr, max_row_nnz)
+        return SliceLayout(data, cols, rowptr, max_row_nnz, one_shot=True)
     if mode is None:
         mode = ("xstage" if STAGED else "xcs") \
             if prefers_xcs(cols, rowptr, n_cols, data.element_size()) else "rowblock"

@@ -39,8 +39,8 @@ __global__ __launch_bounds__(kBlock) void sddmm_slices_kernel(
     const int* __restrict__ cols, const void* __restrict__ rowptr, int rowptr_bits,
     int64_t nnz_total, const T* __restrict__ x, int64_t ldx, const T* __restrict__ y,
     uint32_t ldy, int K, const T* __restrict__ in, double alpha, double beta,
-    O* __restrict__ out, const int64_t* __restrict__ table, int n_slices, int cap, int rows_cap,
-    int lg) {
+    O* __restrict__ out, const int64_t* __restrict__ table, const int* __restrict__ order,
+    int n_slices, int cap, int rows_cap, int lg) {
   extern __shared__ __attribute__((aligned(16))) unsigned char s_raw[];
   // s_out [cap] (a 4-byte result takes its column's slot) | s_col [cap] | s_ptr [rows_cap + 2]
   constexpr bool kShared = sizeof(O) == sizeof(int);
@@ -50,7 +50,7 @@ __global__ __launch_bounds__(kBlock) void sddmm_slices_kernel(
   const int G = 1 << lg, ngrp = kBlock >> lg;
 
   const int tid = threadIdx.x;
-  const int64_t k = xcd_logical_block(blockIdx.x, n_slices);
+  const int64_t k = order ? order[blockIdx.x] : xcd_logical_block(blockIdx.x, n_slices);
   const int grp = tid >> lg, lane = tid & (G - 1);
   const int64_t i0 = table[2 * k], p0 = table[2 * k + 1];
   const int64_t i1 = table[2 * k + 2], p1 = table[2 * k + 3];
@@ -200,6 +200,7 @@ struct SdArgs {
   double alpha, beta;
   void* out;
   const int64_t* table;
+  const int32_t* order;
   int64_t items;
   int lg;
   hipStream_t st;
@@ -216,7 +217,7 @@ int launch_sd(const SdArgs& a) {
                      dim3(kBlock), lds, a.st, a.cols, a.rowptr, a.rowptr_bits, a.nnz,
                      static_cast<const T*>(a.x), a.ldx, static_cast<const T*>(a.y),
                      (uint32_t)a.ldy, (int)a.K, static_cast<const T*>(a.in), a.alpha, a.beta,
-                     static_cast<O*>(a.out), a.table, (int)n, cap, rows_cap, a.lg);
+                     static_cast<O*>(a.out), a.table, a.order, (int)n, cap, rows_cap, a.lg);
   return check_hip(hipGetLastError(), "sddmm_slices_kernel launch");
 }
 
@@ -256,8 +257,8 @@ extern "C" int fsp_sddmm_sliced(int dtype, int acc_f64, int out_f64, const int32
                                 const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t nnz,
                                 const void* x, int64_t ldx, const void* y, int64_t ldy,
                                 int64_t K, const void* data_in, double alpha, double beta,
-                                void* out, const int64_t* table, int64_t items,
-                                int lanes_per_entry, int vec, void* stream) {
+                                void* out, const int64_t* table, const int32_t* order,
+                                int64_t items, int lanes_per_entry, int vec, void* stream) {
   if (dtype != FSP_F32 && dtype != FSP_F64)
     return set_error(FSP_ENOTSUP, "fsp_sddmm_sliced: dtype");
   if (nnz < 0 || n_rows < 0 || K < 1)
@@ -290,7 +291,7 @@ extern "C" int fsp_sddmm_sliced(int dtype, int acc_f64, int out_f64, const int32
   if (reinterpret_cast<uintptr_t>(cols) % 16)
     return set_error(FSP_EINVAL, "fsp_sddmm_sliced: cols must be 16-byte aligned");
   const SdArgs a{cols, rowptr, rowptr_bits, n_rows, nnz,   x,    ldx,  y,     ldy,
-                 K,    data_in, alpha,      beta,   out,   table, items, lg,
+                 K,    data_in, alpha,      beta,   out,   table, order, items, lg,
                  static_cast<hipStream_t>(stream)};
   if (dtype == FSP_F64) return launch_vec<double, double, double>(a, vec);
   if (out_f64) return launch_vec<float, double, double>(a, vec);

@@ -75,8 +75,8 @@ template <typename T, typename A, typename P, int VW, int UPT>
 __global__ __launch_bounds__(kBlock, 8) void spmm_slices_kernel(
     const T* __restrict__ vals, const int* __restrict__ cols, const P* __restrict__ rowptr,
     P nnz_total, const T* __restrict__ B, uint32_t ldb, int N, T* __restrict__ C, int64_t ldc,
-    const int64_t* __restrict__ table, int n_slices, int cap, int rows_cap, int lg,
-    A* __restrict__ carry, A* __restrict__ head, int xcd_remap) {
+    const int64_t* __restrict__ table, const int* __restrict__ order, int n_slices, int cap,
+    int rows_cap, int lg, A* __restrict__ carry, A* __restrict__ head, int xcd_remap) {
   extern __shared__ __attribute__((aligned(16))) unsigned char s_raw[];
   // s_red [4 waves][G * VW] | s_val [cap] | s_col [cap] | s_ptr [rows_cap + 2] | s_list | s_n
   const int G = 1 << lg, ngrp = kBlock >> lg, W = G * VW;
@@ -89,7 +89,8 @@ __global__ __launch_bounds__(kBlock, 8) void spmm_slices_kernel(
 
   const int tid = threadIdx.x;
   int k = blockIdx.x;
-  if (xcd_remap) k = xcd_logical_block(k, n_slices);
+  if (order) k = order[k];
+  else if (xcd_remap) k = xcd_logical_block(k, n_slices);
   const int tile = blockIdx.y;
   const int grp = tid >> lg, lane = tid & (G - 1);
   const int64_t i0 = table[2 * (int64_t)k], i1 = table[2 * (int64_t)k + 2];
@@ -271,6 +272,7 @@ struct SliceArgs {
   void* C;
   int64_t ldc;
   const int64_t* table;
+  const int32_t* order;
   void* sums;
   int64_t items, keep;
   int cut_rows, lg, xcd_remap;
@@ -291,8 +293,8 @@ int launch_upt(const SliceArgs& a) {
   hipLaunchKernelGGL((spmm_slices_kernel<T, A, P, VW, UPT>), dim3((unsigned)n, (unsigned)tiles),
                      dim3(kBlock), lds, a.st, static_cast<const T*>(a.vals), a.cols,
                      static_cast<const P*>(a.rowptr), (P)a.nnz, static_cast<const T*>(a.B),
-                     (uint32_t)a.ldb, (int)a.N, static_cast<T*>(a.C), a.ldc, a.table, (int)n, cap, rows_cap,
-                     a.lg, carry, head, a.xcd_remap);
+                     (uint32_t)a.ldb, (int)a.N, static_cast<T*>(a.C), a.ldc, a.table, a.order, (int)n, cap,
+                     rows_cap, a.lg, carry, head, a.xcd_remap);
   int rc = check_hip(hipGetLastError(), "spmm_slices_kernel launch");
   if (rc || !a.cut_rows) return rc;
   int cw = 1;
@@ -346,8 +348,8 @@ extern "C" int fsp_slice_table(const void* rowptr, int rowptr_bits, int64_t n_ro
 extern "C" int fsp_spmm_sliced(int dtype, int acc_f64, const void* vals, const int32_t* cols,
                                const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t nnz,
                                const void* B, int64_t ldb, int64_t N, void* C, int64_t ldc,
-                               const int64_t* table, int64_t items, int64_t keep, void* sums,
-                               int cut_rows, int lanes_per_row, int vec, int xcd_remap,
+                               const int64_t* table, const int32_t* order, int64_t items,
+                               int64_t keep, void* sums, int cut_rows, int lanes_per_row, int vec, int xcd_remap,
                                void* stream) {
   if (dtype != FSP_F32 && dtype != FSP_F64)
     return set_error(FSP_ENOTSUP, "fsp_spmm_sliced: dtype");
@@ -383,7 +385,7 @@ extern "C" int fsp_spmm_sliced(int dtype, int acc_f64, const void* vals, const i
   if (slice_count(n_rows, nnz, items) > 0x7fffffffLL)
     return set_error(FSP_EINVAL, "fsp_spmm_sliced: more than 2^31-1 slices");
   const SliceArgs a{vals, cols, rowptr, n_rows, nnz,   B,    ldb,      N,  C,
-                    ldc,  table, sums,  items,  keep,  cut_rows, lg, xcd_remap,
+                    ldc,  table, order, sums,  items,  keep,  cut_rows, lg, xcd_remap,
                     static_cast<hipStream_t>(stream)};
   const bool p32 = rowptr_bits == 32;
   if (dtype == FSP_F64)

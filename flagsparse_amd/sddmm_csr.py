@@ -16,7 +16,7 @@ import time
 
 import torch
 
-from . import _abi, _common
+from . import _abi, _common, _slices
 from ._common import (  # noqa: F401  (cp and the converters: the reference scripts' names)
     _aligned,
     _benchmark_cuda_op,
@@ -38,7 +38,7 @@ class SDDMMPrepared:
     (block_k, num_warps)."""
 
     __slots__ = ("indices", "indptr", "shape", "n_rows", "n_cols", "nnz", "_row_ids", "block_k",
-                 "num_warps", "_tables", "_kernel_ptr", "_one_call")
+                 "num_warps", "_tables", "_kernel_ptr", "_one_call", "_max_row_nnz")
 
     def __init__(self, indices, indptr, shape, row_ids, block_k, num_warps):
         self.indices = indices
@@ -53,6 +53,7 @@ class SDDMMPrepared:
         self._tables = {}
         self._kernel_ptr = None
         self._one_call = False  # made by and for a single call
+        self._max_row_nnz = None  # where known
 
     @property
     def row_ids(self):
@@ -60,28 +61,20 @@ class SDDMMPrepared:
             self._row_ids = _build_row_ids(self.indptr)
         return self._row_ids
 
-    def _slices(self, items):
-        """The boundaries of slices of ``items`` rows + entries (built once per size)."""
-        table = self._tables.get(items)
-        if table is None:
-            if torch.cuda.is_current_stream_capturing():
-                raise RuntimeError("an SDDMM must run once before it is captured into a graph "
-                                   "(the first call with this K builds its slices)")
-            L = _abi.lib()
-            dev = self.indices.device
+    def slices(self, items, by_column):
+        """The boundaries of slices of ``items`` rows + entries and their launch order (built once
+        per size)."""
+        t = self._tables.get((items, by_column))
+        if t is None:
             if self._kernel_ptr is None:
                 self._kernel_ptr = self.indptr.to(
                     torch.int32 if self.nnz <= _common.ROWPTR32_MAX_NNZ else torch.int64)
-            rp = self._kernel_ptr
-            n = L.fsp_slice_count(self.n_rows, self.nnz, items)
-            table = torch.empty(2 * (n + 1), dtype=torch.int64, device=dev)
-            _abi.check(L.fsp_slice_table(rp.data_ptr(), 32 if rp.dtype == torch.int32 else 64,
-                                         self.n_rows, self.nnz, items, 0, table.data_ptr(),
-                                         _abi.raw_stream(dev)), "fsp_slice_table")
+            t = _slices.build(self._kernel_ptr, self.n_rows, self.nnz, items, 0, "SDDMM",
+                              self.indices if by_column else None, self.n_cols)
             if not self._one_call:  # later calls may come from other streams
-                torch.cuda.current_stream(dev).synchronize()
-            self._tables[items] = table
-        return table
+                torch.cuda.current_stream(self.indices.device).synchronize()
+            self._tables[(items, by_column)] = t
+        return t
 
 
 def _resolve_sddmm_launch_config(k):
@@ -96,8 +89,8 @@ def _resolve_sddmm_launch_config(k):
 
 
 def _prepare_sddmm_csr_pattern(indices, indptr, shape, ptr_bits=64):
-    """Validation of sddmm_csr.py:46-79 (same checks, order, messages and types); the row pointers
-    come back at ``ptr_bits``."""
+    """Validation of sddmm_csr.py:46-79 (same checks, order, messages and types): (columns, row
+    pointers of ``ptr_bits``, shape, longest row)."""
     if len(shape) != 2:
         raise ValueError("shape must be a 2-tuple")
     if indices.ndim != 1 or indptr.ndim != 1:
@@ -116,7 +109,7 @@ def _prepare_sddmm_csr_pattern(indices, indptr, shape, ptr_bits=64):
     indices = _aligned(indices.contiguous())  # 16-byte loads of the columns
     nnz = int(indices.numel())
     # one pass over both arrays, one host synchronisation
-    (first, last, decreases, _, min_col, max_col), indices, indptr = csr_check(
+    (first, last, decreases, longest, min_col, max_col), indices, indptr = csr_check(
         indices, indptr.contiguous(), ptr_bits)
     if first != 0:
         raise ValueError("indptr[0] must be 0")
@@ -126,7 +119,7 @@ def _prepare_sddmm_csr_pattern(indices, indptr, shape, ptr_bits=64):
         raise ValueError("indptr must be nondecreasing")
     if nnz > 0 and (min_col < 0 or max_col >= n_cols):
         raise IndexError("indices out of range for shape[1]")
-    return indices, indptr, (n_rows, n_cols)
+    return indices, indptr, (n_rows, n_cols), longest
 
 
 def _build_row_ids(indptr):
@@ -146,11 +139,12 @@ def _prepare_sddmm(indices, indptr, shape, k_hint, one_call):
     """prepare_sddmm_csr; one_call: row pointers only at the width the kernel reads."""
     narrow = one_call and torch.is_tensor(indices) and \
         indices.numel() <= _common.ROWPTR32_MAX_NNZ
-    indices, indptr, shape = _prepare_sddmm_csr_pattern(indices, indptr, shape,
-                                                        32 if narrow else 64)
+    indices, indptr, shape, longest = _prepare_sddmm_csr_pattern(indices, indptr, shape,
+                                                                 32 if narrow else 64)
     block_k, num_warps = _resolve_sddmm_launch_config(int(k_hint))
     prepared = SDDMMPrepared(indices=indices, indptr=indptr, shape=shape, row_ids=None,
                              block_k=block_k, num_warps=num_warps)
+    prepared._max_row_nnz = longest
     if one_call:
         prepared._one_call = True
         prepared._kernel_ptr = indptr
@@ -279,15 +273,18 @@ def _launch_sddmm(prepared, x, y, data, alpha, beta, out, acc_f64):
     lanes, vec = _sddmm_slice_lanes(K, x.dtype)
     if 1 <= K <= 4 * lanes * vec and cols.data_ptr() % 16 == 0:
         items = _sddmm_slice_items(lanes, prepared.n_rows + prepared.nnz)
-        table = prepared._slices(items)
+        row_bytes = K * x.element_size()
+        by_column = _slices.ordered(prepared._max_row_nnz, items, prepared.n_cols * row_bytes,
+                                    prepared.nnz * row_bytes, prepared._one_call)
+        table, order = prepared.slices(items, by_column)
         rp = prepared._kernel_ptr
         _abi.check(
             L.fsp_sddmm_sliced(code, int(acc_f64), out_f64, cols.data_ptr(), rp.data_ptr(),
                                32 if rp.dtype == torch.int32 else 64, prepared.n_rows,
                                prepared.nnz, x.data_ptr(), x.stride(0), y.data_ptr(),
                                y.stride(0), K, None if data is None else data.data_ptr(),
-                               float(alpha), float(beta), out.data_ptr(), table.data_ptr(), items,
-                               lanes, vec, _abi.raw_stream(x.device)), "fsp_sddmm_sliced")
+                               float(alpha), float(beta), out.data_ptr(), table.data_ptr(),
+                               None if order is None else order.data_ptr(), items, lanes, vec, _abi.raw_stream(x.device)), "fsp_sddmm_sliced")
         return
     lanes, vec = _sddmm_lane_shape(K, x, y)
     _abi.check(

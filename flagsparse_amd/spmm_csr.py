@@ -15,7 +15,7 @@ import time
 
 import torch
 
-from . import _abi, _common
+from . import _abi, _common, _slices
 from ._common import (
     SUPPORTED_INDEX_DTYPES,
     SUPPORTED_VALUE_DTYPES,
@@ -288,16 +288,21 @@ def _spmm_slice_lanes(n_dense_cols, dtype, tile_cols=None):
     return min(64, _next_pow2(-(-width // vec))), vec
 
 
-def _spmm_slice_shape(lanes, positions):
+def _spmm_slice_shape(lanes, positions, by_column=False):
     """(rows + entries per slice, longest row never cut).  A slice should give each of a
     workgroup's 256 / lanes groups several entries, and the matrix enough slices to fill the
     256 CUs.  Measured on MI355X with 128 / 256 / 512 / 1024 positions: 16 lanes (fp32 N=64, 33.5M
     entries) 781 / 670 / 661 / 701 us; 64 lanes (N=256, 4M) 557 / 564 / - / -; 8 lanes (N=32,
     1.2M) 29.8 / 22.0 / 19.7 / 19.2; the same with 80k entries 5.2 / 5.3 / 6.3 / 6.9, hence the
-    limit by size."""
-    items = {64: 128, 32: 256, 16: 512, 8: 1024}.get(lanes, 1536)
+    limit by size.  Slices that run by column are shorter, so that more rows hold several (a power
+    law, 128 / 256 / 512 positions: N=128, 32 lanes 190 / 200 / - us; N=47, 16 lanes 151 / 125 /
+    127; 4 lanes, N=16, 512 / 1024 / 1536: 120 / 123 / 131)."""
+    if by_column:
+        items = {64: 128, 32: 128, 16: 256}.get(lanes, 512)
+    else:
+        items = {64: 128, 32: 256, 16: 512, 8: 1024}.get(lanes, 1536)
     while items > 64 and positions < 1024 * items:
-        items >>= 1
+        items = max(64, items >> 1)
     return items, 256 if items >= 128 else 128
 
 
@@ -333,8 +338,7 @@ class _SpmmKernelCsr:
         return {"layout": "rowblock", "plans": {g: {"descriptors": p.n_desc,
                                                     "split_rows": p.n_split_rows}
                                                 for g, p in self._plans.items()},
-                "slices": {items: int(t.numel()) // 2 - 1
-                           for (items, _), t in self._tables.items()}}
+                "slices": {k[0]: int(t[0].numel()) // 2 - 1 for k, t in self._tables.items()}}
 
     def sliced(self):
         """Whether products run on slices whatever their N.  Row blocks are kept where they are
@@ -346,20 +350,14 @@ class _SpmmKernelCsr:
             return True
         return self.max_row_nnz > _SPMM_ROW_SPLIT_THRESHOLD
 
-    def table(self, items, keep):
-        """The slices' boundaries (built on the current stream, once)."""
-        t = self._tables.get((items, keep))
+    def slices(self, items, keep, n_cols, by_column):
+        """The slices' boundaries and launch order (built on the current stream, once)."""
+        key = (items, keep, by_column)
+        t = self._tables.get(key)
         if t is None:
-            if torch.cuda.is_current_stream_capturing():
-                raise RuntimeError("an SpMM must run once before it is captured into a graph "
-                                   "(the first call with this N builds its slices)")
-            L = _abi.lib()
-            n = L.fsp_slice_count(self.n_rows, self.nnz, items)
-            t = torch.empty(2 * (n + 1), dtype=torch.int64, device=self.data.device)
-            _abi.check(L.fsp_slice_table(self.rowptr.data_ptr(), self.rowptr_bits, self.n_rows,
-                                         self.nnz, items, keep, t.data_ptr(),
-                                         _abi.raw_stream(t.device)), "fsp_slice_table")
-            self._tables[(items, keep)] = t
+            t = _slices.build(self.rowptr, self.n_rows, self.nnz, items, keep, "SpMM",
+                              self.cols if by_column else None, n_cols)
+            self._tables[key] = t
         return t
 
     def plan(self, lanes):
@@ -402,8 +400,14 @@ def _run_spmm_sliced(kc, B, C, acc_f64, lanes, vec):
     stream = kc._order.stream(C.device, kc._keep)
     args = kc._args.get(key)
     if args is None:  # the arguments that do not change between calls, converted once
-        items, keep = _spmm_slice_shape(lanes, kc.n_rows + kc.nnz)
-        table = kc.table(items, keep)
+        n_cols, positions = int(B.shape[0]), kc.n_rows + kc.nnz
+        row_bytes = min(n_dense_cols, lanes * vec) * B.element_size()  # of one column tile
+        items, keep = _spmm_slice_shape(lanes, positions, True)
+        by_column = _slices.ordered(kc.max_row_nnz, items, n_cols * row_bytes,
+                                    kc.nnz * row_bytes, kc.one_shot)
+        if not by_column:
+            items, keep = _spmm_slice_shape(lanes, positions)
+        table, order = kc.slices(items, keep, n_cols, by_column)
         cut = kc.max_row_nnz is None or kc.max_row_nnz > keep
         sums = None
         if cut:  # the pieces of cut rows: a carry and a head per slice
@@ -412,13 +416,14 @@ def _run_spmm_sliced(kc, B, C, acc_f64, lanes, vec):
                                dtype=torch.float64 if acc_f64 else B.dtype)
         args = [_abi.dtype_code(B.dtype), 1 if acc_f64 else 0, kc.data.data_ptr(),
                 kc.cols.data_ptr(), kc.rowptr.data_ptr(), kc.rowptr_bits, kc.n_rows, kc.nnz,
-                None, 0, n_dense_cols, None, 0, table.data_ptr(), items, keep,
+                None, 0, n_dense_cols, None, 0, table.data_ptr(),
+                None if order is None else order.data_ptr(), items, keep,
                 None if sums is None else sums.data_ptr(), int(cut), lanes, vec, XCD_REMAP, None]
         kc._args[key] = args
-        kc._keep.extend((table, sums))
+        kc._keep.extend((table, order, sums))
     a = list(args)
     a[8], a[9], a[11], a[12] = B.data_ptr(), B.stride(0), C.data_ptr(), C.stride(0)
-    a[21] = stream
+    a[22] = stream
     _abi.check(_abi.lib().fsp_spmm_sliced(*a), "fsp_spmm_sliced")
     return C
 

@@ -194,7 +194,7 @@ def _prepare_one_call(data, row, col, shape, sort_by_row):
         data, row, col = rows_in_order(data, row, col, rmax)
     prepared = PreparedCoo(data, row, col.to(torch.int32), shape)
     prepared.use_seg_kernel = True
-    prepared._layout = SliceLayout(data, prepared.col, row_pointers(row, n_rows))
+    prepared._layout = SliceLayout(data, prepared.col, row_pointers(row, n_rows), one_shot=True)
     return prepared
 
 

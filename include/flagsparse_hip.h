@@ -222,16 +222,20 @@ int fsp_spmv_csr(int dtype, int acc_f64, const void* vals, const int32_t* cols,
  * added in order by a second pass.  Replaces the same launches as fsp_spmv_csr.
  *   vals, cols, rowptr, x, y, dtype, acc_f64   as fsp_spmv_csr (no row_map); n_rows < 2^31
  *   table      device scratch, 2 * (slices + 1) int64: the slices' boundaries {row, entry}
+ *   table_built  1: table holds fsp_slice_table(.., fsp_spmv_slice_items(),
+ *              fsp_spmv_slice_keep(), table); 0: the call builds it (a launch more)
  *   sums       device scratch, 2 * slices doubles: the pieces of cut rows
  *   cut_rows   0: no row is longer than fsp_spmv_slice_keep() (the second pass is left out)
- * table and sums need no initial value; calls sharing them must not overlap.
+ * sums (and table when the call builds it) need no initial value; calls sharing them must not
+ * overlap.
  */
 int64_t fsp_spmv_slices(int64_t n_rows, int64_t nnz);
 int64_t fsp_spmv_slice_keep(void);
+int64_t fsp_spmv_slice_items(void);
 int fsp_spmv_sliced(int dtype, int acc_f64, const void* vals, const int32_t* cols,
                     const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t nnz,
-                    const void* x, void* y, int64_t* table, void* sums, int cut_rows,
-                    void* stream);
+                    const void* x, void* y, int64_t* table, int table_built, void* sums,
+                    int cut_rows, void* stream);
 
 /*
  * fsp_spmv_csr without a caller workspace, for callers that cannot allocate device memory
@@ -436,9 +440,20 @@ int fsp_slice_table(const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t
                     int64_t items, int64_t keep, int64_t* table, void* stream);
 
 /*
+ * A launch order of the slices for products whose dense operand (n_cols rows) is larger than an
+ * L2: slices that lie inside one long row come last, by the column they start at.  order: n_slices
+ * int32, order[b] = the slice of workgroup b; scratch: fsp_slice_order_scratch(n_slices) int32.
+ * A product's result does not depend on it.
+ */
+int64_t fsp_slice_order_scratch(int64_t n_slices);
+int fsp_slice_order(const int64_t* table, int64_t n_slices, const int32_t* cols, int64_t n_cols,
+                    int32_t* order, int32_t* scratch, void* stream);
+
+/*
  * C[n_rows, N] = A @ B over the slices of fsp_slice_table, otherwise as fsp_spmm_csr.
  *   table, items, keep  the slices' boundaries and what they were built with; items + keep <=
  *                  2042
+ *   order          NULL (row order), or fsp_slice_order's order
  *   sums           2 * slices * N slots of the accumulation type, 16-byte aligned: the pieces
  *                  of cut rows.  Calls sharing sums must not overlap.
  *   cut_rows       0: no row is longer than keep (sums may be NULL, and the second pass that
@@ -451,8 +466,8 @@ int fsp_slice_table(const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t
 int fsp_spmm_sliced(int dtype, int acc_f64, const void* vals, const int32_t* cols,
                     const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t nnz,
                     const void* B, int64_t ldb, int64_t N, void* C, int64_t ldc,
-                    const int64_t* table, int64_t items, int64_t keep, void* sums, int cut_rows,
-                    int lanes_per_row, int vec, int xcd_remap, void* stream);
+                    const int64_t* table, const int32_t* order, int64_t items, int64_t keep,
+                    void* sums, int cut_rows, int lanes_per_row, int vec, int xcd_remap, void* stream);
 
 /*
  * COO entries into row order (stable), in place of the lexicographic sorts of
@@ -526,6 +541,7 @@ int fsp_sddmm_csr(int dtype, int acc_f64, int out_f64, const int32_t* cols,
  * The same over the slices of fsp_slice_table(rowptr, .., items, 0, table): no plan, row by row,
  * for vec <= K <= 4 * lanes_per_entry * vec, K >= 1.
  *   items          rows + entries per slice, at most 4096
+ *   order          NULL (row order), or fsp_slice_order's order
  *   vec            elements per lane per load: 1, 2 or 4 (fp32) / 1 or 2 (fp64); needs no
  *                  alignment of x, y, ldx or ldy beyond the element's own
  *   cols           16-byte aligned; the other arguments as fsp_sddmm_csr
@@ -534,8 +550,8 @@ int fsp_sddmm_sliced(int dtype, int acc_f64, int out_f64, const int32_t* cols,
                      const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t nnz,
                      const void* x, int64_t ldx, const void* y, int64_t ldy, int64_t K,
                      const void* data_in, double alpha, double beta, void* out,
-                     const int64_t* table, int64_t items, int lanes_per_entry, int vec,
-                     void* stream);
+                     const int64_t* table, const int32_t* order, int64_t items,
+                     int lanes_per_entry, int vec, void* stream);
 
 /*
  * Matrix Market coordinate file reader (host only, no GPU): the format of the reference's

@@ -125,3 +125,17 @@ def test_sddmm_row_ids(dev):
     out = fs.flagsparse_sddmm_csr(x=x.to(dev), y=y.to(dev), prepared=q)
     assert not q._tables
     assert oracle.rel_l2(out, oracle.sddmm_csr(ip, cols, x, y)) <= 1e-5
+
+
+@pytest.mark.parametrize("name", sorted(LENGTHS))
+def test_sliced_sddmm_by_column(dev, monkeypatch, name):
+    ip, cols, data, x, y, shape = _case(name, 503, 40, torch.float64, dev)
+    args = dict(x=x.to(dev), y=y.to(dev))
+    out = fs.flagsparse_sddmm_csr(
+        prepared=fs.prepare_sddmm_csr(cols.to(dev), ip.to(dev), shape), **args)
+    monkeypatch.setattr(sddmm_csr._slices, "ordered", lambda *a: True)
+    p = fs.prepare_sddmm_csr(cols.to(dev), ip.to(dev), shape)
+    assert torch.equal(fs.flagsparse_sddmm_csr(prepared=p, **args), out)
+    (_, order), = p._tables.values()
+    assert torch.equal(torch.sort(order.cpu()).values.to(torch.int64),
+                       torch.arange(order.numel()))

@@ -119,3 +119,26 @@ def test_spmm_capture_needs_a_first_call(dev):
     torch.cuda.synchronize()
     ref = oracle.spmm_csr(ip, cols, vals, B)
     assert oracle.rel_l2(fs.flagsparse_spmm_csr_opt(B=Bd, prepared=p), ref) <= 1e-5
+
+
+@pytest.mark.parametrize("name", sorted(set(LENGTHS) - {"empty"}))
+def test_slices_by_column(dev, monkeypatch, name):
+    # any launch order gives the same sums; the order is a permutation with the slices inside one
+    # row last, by column within each XCD's part
+    vals, cols, ip, B, shape = _case(name, 901, 20, torch.float32, dev)
+    C, _ = _run(vals, cols, ip, B, shape, dev, False)
+    shape_of = spmm_csr._spmm_slice_shape
+    monkeypatch.setattr(spmm_csr._slices, "ordered", lambda *a: True)
+    monkeypatch.setattr(spmm_csr, "_spmm_slice_shape", lambda l, p, by=False: shape_of(l, p))
+    Co, kc = _run(vals, cols, ip, B, shape, dev, False)
+    assert torch.equal(C, Co)
+    (table, order), = kc._tables.values()
+    t, o = table.view(-1, 2).cpu(), order.cpu().to(torch.int64)
+    n = t.shape[0] - 1
+    assert torch.equal(torch.sort(o).values, torch.arange(n))
+    inside = (t[:-1, 0] == t[1:, 0]) & (t[1:, 1] > t[:-1, 1])
+    others = int((~inside).sum())
+    assert not bool(inside[o[:others]].any()) and bool(inside[o[others:]].all())
+    k = cols[t[o[others:], 1]] * 255 // shape[1]
+    for x in range(8):  # slots 8 apart are one XCD's, in column bins that rise
+        assert bool((k[x::8][1:] >= k[x::8][:-1]).all())
