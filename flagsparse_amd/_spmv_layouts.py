@@ -8,6 +8,11 @@ The layouts below, chosen once per matrix at prepare time:
     chunk order.  Right when the x entries a block gathers lie close together (banded,
     stencil, locally clustered columns) or x fits in one XCD's L2.
 
+``SliceLayout`` (csrc/slices.hip, ``spmv_slices_kernel``)
+    The CSR arrays cut into slices of equal rows + entries, found by a search in the row pointers.
+    Right for matrices used once (nothing is planned) and for those with rows longer than a row
+    block, where the row-block layout would be taken.
+
 ``XcsLayout`` (csrc/spmv_xcs.hip, ``spmv_xcs_kernel``, ``xcs_window_combine_kernel``)
     Columns split into panels of about equal nnz (P of them, P / 8 per XCD in turn, or shared
     by two XCDs when P = 4); entries regrouped by (row tile, panel) so that every workgroup
@@ -1426,7 +1431,8 @@ def build_layout(data, cols, rowptr, n_cols, one_shot=False, max_row_nnz=None):
     one_shot: the layout serves a single call (no prepared object) and is asked for no run to
     row map, so the slices, which need no plan, are taken; the row blocks' plan alone takes 0.6
     ms for a million rows and the staged-x layout tens of milliseconds (a power law of 8.4M rows:
-    28 ms for a 0.2 ms product).  max_row_nnz: the longest row, where the caller knows it."""
+    28 ms for a 0.2 ms product).  max_row_nnz: the longest row of a CSR matrix, where the caller
+    knows it and asks for no row map."""
     mode = FORCE
     nnz = int(data.numel())
     if mode is None and one_shot:
@@ -1459,6 +1465,15 @@ def build_layout(data, cols, rowptr, n_cols, one_shot=False, max_row_nnz=None):
             return xcs_layout(data, cols, rowptr, n_cols, FORCE_PANELS_PER_XCD)
         except ValueError:
             pass  # too large for the packing: row blocks
+    if FORCE is None and max_row_nnz is not None and \
+            max_row_nnz > _abi.lib().fsp_spmv_stream_nnz_cap():
+        # Rows longer than a row block go through chunk workgroups and a second pass there, and a
+        # skewed matrix's blocks sum rows of very different lengths with the same lanes.  Measured
+        # on MI355X, row blocks / slices, power laws: float32, 40k rows of mean 12 29.7 / 8.7 us,
+        # 300k of 20 48.0 / 29.9, 900k of 6 56.2 / 34.2; float64, 300k of 20 51.4 / 35.7.  Without
+        # such rows they are level (900k rows of 0 to 12 entries 32.8 / 32.9), stencils apart,
+        # whose row blocks have a launch order of their own (float64 2048 x 2048 58.1 / 82.4).
+        return SliceLayout(data, cols, rowptr, max_row_nnz)
     return RowBlockLayout(data, cols, rowptr)
 
 

@@ -66,6 +66,23 @@ def test_sliced_spmv(dev, monkeypatch, name, dtype, opt, bits64):
     assert oracle.rel_l2(fs.flagsparse_spmv_csr(x=args[3], prepared=p, use_opt=opt), ref) <= tol
 
 
+@pytest.mark.parametrize("name,kind", [("crossing", "slices"), ("mixed", "rowblock"),
+                                       ("one_row", "slices"), ("short", "rowblock")])
+def test_prepared_layout(dev, name, kind):
+    # rows longer than a row block: the prepared matrix runs on slices whose table it keeps
+    vals, cols, ip = _csr(LENGTHS[name], 3001, 8, torch.float32)
+    shape = (len(LENGTHS[name]), 3001)
+    p = fs.prepare_spmv_csr(vals.to(dev), cols.to(dev), ip.to(dev), shape)
+    assert p._kernel(False).kind == kind
+    for k in range(3):
+        x = synthetic.uniform_values(9 + k, 3, 3001, torch.float32, "cpu")
+        y = fs.flagsparse_spmv_csr(x=x.to(dev), prepared=p)
+        assert oracle.rel_l2(y, oracle.spmv_csr(ip, cols, vals, x)) <= 1e-5
+    one = fs.flagsparse_spmv_csr(vals.to(dev), cols.to(dev), ip.to(dev), x.to(dev), shape)
+    if kind == "slices":
+        assert torch.equal(one, y)
+
+
 def test_sliced_spmv_nonfinite(dev):
     # an infinity and a NaN of x reach the rows that name them and no others
     vals, cols, ip = _csr(LENGTHS["crossing"], 3001, 6, torch.float32)
