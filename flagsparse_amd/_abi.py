@@ -100,6 +100,16 @@ SIGNATURES = {
     "fsp_probe_rows": (_i32, [_p, _i64, _i64, _p, _i64, _p, _p]),
     "fsp_probe_stream_blocks": (_i64, [_i64]),
     "fsp_probe_stream": (_i32, [_p, _i64, _p, _p]),
+    "fsp_bound_bytes": (_i64, []),
+    "fsp_bind_spmv_csr": (_i32, [_p, _i32, _i32, _p, _p, _p, _i32, _i64, _i64, _p, _i64, _p, _p,
+                                 _i64, _i64, _p, _p, _p, _p, _i64, _i32]),
+    "fsp_bind_spmv_sliced": (_i32, [_p, _i32, _i32, _p, _p, _p, _i32, _i64, _i64, _p, _i32, _p,
+                                    _i32]),
+    "fsp_bind_spmm_csr": (_i32, [_p, _i32, _i32, _p, _p, _p, _i32, _i64, _i64, _i64, _p, _i64,
+                                 _i64, _i32, _i32, _p, _p, _p, _p, _i64, _i32]),
+    "fsp_bind_spmm_sliced": (_i32, [_p, _i32, _i32, _p, _p, _p, _i32, _i64, _i64, _i64, _p, _p,
+                                    _i64, _i64, _p, _i32, _i32, _i32, _i32]),
+    "fsp_run": (_i32, [_p, _p, _p, _p]),
 }
 
 
@@ -144,6 +154,23 @@ def dtype_code(dtype):
 def ptr(t):
     """Device (or host) address of a tensor's first element; None for absent tensors."""
     return None if t is None else ctypes.c_void_p(t.data_ptr())
+
+
+def bind(name, *args):
+    """The call ``name`` with every argument but its input, output and stream filled in
+    (fsp_bind_*): ``run(bound, input, output, stream)`` makes it, with plain addresses.  The
+    caller keeps what the arguments point to."""
+    L = lib()
+    buf = ctypes.create_string_buffer(int(L.fsp_bound_bytes()) + 8)
+    at = (ctypes.addressof(buf) + 7) & ~7
+    check(getattr(L, "fsp_bind_" + name)(at, *args), "fsp_bind_" + name)
+    return buf, at
+
+
+def run(bound, inp, out, stream):
+    status = _lib.fsp_run(bound[1], inp, out, stream)
+    if status != 0:
+        check(status, "fsp_run")
 
 
 def stream_handle(device):

@@ -20,7 +20,7 @@ LIB_DIR = os.path.join(PKG_DIR, "_lib")
 LIB_NAME = "libflagsparse_hip.so"
 LIB_PATH = os.path.join(LIB_DIR, LIB_NAME)
 
-SOURCES = ("abi.cpp", "mtx.cpp", "plan.hip", "spmv.hip", "spmv_xcs.hip", "spmm.hip", "sddmm.hip",
+SOURCES = ("abi.cpp", "bound.cpp", "mtx.cpp", "plan.hip", "spmv.hip", "spmv_xcs.hip", "spmm.hip", "sddmm.hip",
            "index_stats.hip", "check.hip", "slices.hip",
            "spmm_slices.hip", "sddmm_slices.hip", "coo_sort.hip", "probe.hip")
 ARCH = "gfx950"

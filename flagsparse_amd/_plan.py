@@ -91,6 +91,8 @@ class StreamOrder:
         """The raw handle of torch's current stream on ``device``, ordered after the previous
         user's work when it differs."""
         s = _abi.raw_stream(device)
+        if s == self._last:
+            return s  # ordered by the stream itself, captured or not
         if torch.cuda.is_current_stream_capturing():
             # A graph being captured: nothing runs now, and a wait on an event recorded
             # outside the capture cannot be recorded into it.  Replays run in the order of
@@ -98,7 +100,7 @@ class StreamOrder:
             # same object on other streams is the caller's (as for the graph's inputs).
             return s
         last = self._last
-        if last is not None and s != last:
+        if last is not None:
             old = torch.cuda.ExternalStream(last, device=device)
             new = torch.cuda.ExternalStream(s, device=device)
             ev = torch.cuda.Event()

@@ -204,31 +204,26 @@ class RowBlockLayout:
                 "band_block_offset": self.band_offset}
 
     def launch(self, x, y, acc_f64, row_map=None, n_out=0):
-        # The arguments that do not change between calls are converted once (per accumulation
-        # mode); a call fills in x, y, the row map and the stream.
-        args = self._args.get(bool(acc_f64))
-        if args is None:
+        # The arguments that do not change between calls are bound once, per accumulation mode
+        # and row map (a matrix has one or none; the bound call keeps it).
+        key = (bool(acc_f64), row_map is None, n_out)
+        bound = self._args.get(key)
+        if bound is None or bound[2] is not row_map:
             plan = self.plan
             groups, group_base, split_rows = plan.split_groups()
-            keep = (plan.workspace(), groups, group_base, split_rows, plan.desc, plan.ranges,
-                    self.data, self.cols, self.rowptr)
-            args = [_abi.dtype_code(self.data.dtype), int(acc_f64), self.data.data_ptr(),
-                    self.cols.data_ptr(), self.rowptr.data_ptr(), self.rowptr_bits,
-                    self.n_rows, self.nnz, None, None, None, 0, plan.desc.data_ptr(),
-                    plan.ranges.data_ptr(), plan.n_desc, plan.chunk, keep[0].data_ptr(),
-                    groups.data_ptr() if groups.numel() else None,
-                    group_base.data_ptr() if group_base.numel() else None,
-                    split_rows.data_ptr() if split_rows.numel() else None,
-                    int(groups.shape[0]), 0, None]
-            self._args[bool(acc_f64)] = args
-            self._keep = keep
-        a = list(args)
-        a[8], a[9] = x.data_ptr(), y.data_ptr()
-        a[10] = None if row_map is None else row_map.data_ptr()
-        a[11] = n_out
-        a[21] = XCD_REMAP_ROWBLOCK
-        a[22] = self._order.stream(y.device, self._keep)
-        _abi.check(_abi.lib().fsp_spmv_csr(*a), "fsp_spmv_csr")
+            self._keep = (plan.workspace(), groups, group_base, split_rows, plan.desc,
+                          plan.ranges, self.data, self.cols, self.rowptr)
+            bound = _abi.bind(
+                "spmv_csr", _abi.dtype_code(self.data.dtype), int(acc_f64), self.data.data_ptr(),
+                self.cols.data_ptr(), self.rowptr.data_ptr(), self.rowptr_bits, self.n_rows,
+                self.nnz, None if row_map is None else row_map.data_ptr(), n_out,
+                plan.desc.data_ptr(), plan.ranges.data_ptr(), plan.n_desc, plan.chunk,
+                self._keep[0].data_ptr(), groups.data_ptr() if groups.numel() else None,
+                group_base.data_ptr() if group_base.numel() else None,
+                split_rows.data_ptr() if split_rows.numel() else None, int(groups.shape[0]),
+                XCD_REMAP_ROWBLOCK) + (row_map,)
+            self._args[key] = bound
+        _abi.run(bound, x.data_ptr(), y.data_ptr(), self._order.stream(y.device, self._keep))
         return y
 
 
@@ -258,10 +253,9 @@ class SliceLayout:
                                          _abi.raw_stream(scratch.device)), "fsp_slice_table")
         self.cut_rows = cut_rows
         self._keep = (scratch, self.data, self.cols, self.rowptr)
-        self._args = [_abi.dtype_code(self.data.dtype), None, self.data.data_ptr(),
-                      self.cols.data_ptr(), self.rowptr.data_ptr(), self.rowptr_bits,
-                      self.n_rows, self.nnz, None, None, scratch.data_ptr(), int(not one_shot),
-                      scratch.data_ptr() + 16 * (n + 1), int(cut_rows), None]
+        self._sums = scratch.data_ptr() + 16 * (n + 1)
+        self._table_built = int(not one_shot)
+        self._args = {}
         self._order = StreamOrder(self.data.device)
 
     def kernel_name(self):
@@ -278,10 +272,15 @@ class SliceLayout:
 
     def launch(self, x, y, acc_f64, row_map=None, n_out=0):
         assert row_map is None, "slices write every row"
-        a = list(self._args)
-        a[1], a[8], a[9] = int(acc_f64), x.data_ptr(), y.data_ptr()
-        a[14] = self._order.stream(y.device, self._keep)
-        _abi.check(_abi.lib().fsp_spmv_sliced(*a), "fsp_spmv_sliced")
+        bound = self._args.get(bool(acc_f64))
+        if bound is None:
+            bound = _abi.bind(
+                "spmv_sliced", _abi.dtype_code(self.data.dtype), int(acc_f64),
+                self.data.data_ptr(), self.cols.data_ptr(), self.rowptr.data_ptr(),
+                self.rowptr_bits, self.n_rows, self.nnz, self._keep[0].data_ptr(),
+                self._table_built, self._sums, int(self.cut_rows))
+            self._args[bool(acc_f64)] = bound
+        _abi.run(bound, x.data_ptr(), y.data_ptr(), self._order.stream(y.device, self._keep))
         return y
 
 

@@ -38,7 +38,7 @@ class SDDMMPrepared:
     (block_k, num_warps)."""
 
     __slots__ = ("indices", "indptr", "shape", "n_rows", "n_cols", "nnz", "_row_ids", "block_k",
-                 "num_warps", "_tables", "_kernel_ptr", "_one_call", "_max_row_nnz")
+                 "num_warps", "_tables", "_shapes", "_kernel_ptr", "_one_call", "_max_row_nnz")
 
     def __init__(self, indices, indptr, shape, row_ids, block_k, num_warps):
         self.indices = indices
@@ -51,6 +51,7 @@ class SDDMMPrepared:
         self.block_k = int(block_k)
         self.num_warps = int(num_warps)
         self._tables = {}
+        self._shapes = {}
         self._kernel_ptr = None
         self._one_call = False  # made by and for a single call
         self._max_row_nnz = None  # where known
@@ -270,13 +271,21 @@ def _launch_sddmm(prepared, x, y, data, alpha, beta, out, acc_f64):
     code = _abi.dtype_code(x.dtype)
     out_f64 = int(out.dtype == torch.float64 and x.dtype == torch.float32)
     cols = prepared.indices
-    lanes, vec = _sddmm_slice_lanes(K, x.dtype)
-    if 1 <= K <= 4 * lanes * vec and cols.data_ptr() % 16 == 0:
-        items = _sddmm_slice_items(lanes, prepared.n_rows + prepared.nnz)
-        row_bytes = K * x.element_size()
-        by_column = _slices.ordered(prepared._max_row_nnz, items, prepared.n_cols * row_bytes,
-                                    prepared.nnz * row_bytes, prepared._one_call)
-        table, order = prepared.slices(items, by_column)
+    shape = prepared._shapes.get((K, x.dtype))
+    if shape is None:  # what a launch needs for this K
+        lanes, vec = _sddmm_slice_lanes(K, x.dtype)
+        if 1 <= K <= 4 * lanes * vec and cols.data_ptr() % 16 == 0:
+            items = _sddmm_slice_items(lanes, prepared.n_rows + prepared.nnz)
+            row_bytes = K * x.element_size()
+            by_column = _slices.ordered(prepared._max_row_nnz, items,
+                                        prepared.n_cols * row_bytes, prepared.nnz * row_bytes,
+                                        prepared._one_call)
+            shape = (lanes, vec, items) + prepared.slices(items, by_column)
+        else:
+            shape = ()
+        prepared._shapes[(K, x.dtype)] = shape
+    if shape:
+        lanes, vec, items, table, order = shape
         rp = prepared._kernel_ptr
         _abi.check(
             L.fsp_sddmm_sliced(code, int(acc_f64), out_f64, cols.data_ptr(), rp.data_ptr(),
@@ -383,13 +392,18 @@ def flagsparse_sddmm_csr(data=None, indices=None, indptr=None, x=None, y=None, s
         if return_meta:
             return out, meta
         return out
+    x, y = x.contiguous(), y.contiguous()
+    data = data.contiguous() if data is not None else None
+    if not timed and not allow_fallback:
+        out = _prepare_validated_sddmm_out(prepared, x, out)
+        if prepared.nnz > 0:
+            _launch_sddmm(prepared, x, y, data, alpha, beta, out, x.dtype == torch.float64)
+        return out
     if timed:
         torch.cuda.synchronize()
     t0 = time.perf_counter()
-    out_tensor, launch_meta = _run_sddmm_prepared(
-        prepared, x.contiguous(), y.contiguous(),
-        data.contiguous() if data is not None else None, alpha, beta, out,
-        allow_fallback=allow_fallback)
+    out_tensor, launch_meta = _run_sddmm_prepared(prepared, x, y, data, alpha, beta, out,
+                                                  allow_fallback=allow_fallback)
     if timed:
         torch.cuda.synchronize()
     elapsed_ms = (time.perf_counter() - t0) * 1000.0

@@ -394,72 +394,66 @@ def _auto_tile_cols(B):
     return t if t < n else None
 
 
-def _run_spmm_sliced(kc, B, C, acc_f64, lanes, vec):
+def _bind_sliced(kc, B, C, acc_f64, lanes, vec):
+    n_dense_cols, n_cols, positions = int(B.shape[1]), int(B.shape[0]), kc.n_rows + kc.nnz
+    row_bytes = min(n_dense_cols, lanes * vec) * B.element_size()  # of one column tile
+    items, keep = _spmm_slice_shape(lanes, positions, True)
+    by_column = _slices.ordered(kc.max_row_nnz, items, n_cols * row_bytes, kc.nnz * row_bytes,
+                                kc.one_shot)
+    if not by_column:
+        items, keep = _spmm_slice_shape(lanes, positions)
+    table, order = kc.slices(items, keep, n_cols, by_column)
+    cut = kc.max_row_nnz is None or kc.max_row_nnz > keep
+    sums = None
+    if cut:  # the pieces of cut rows: a carry and a head per slice
+        n = int(table.numel()) // 2 - 1
+        sums = torch.empty(2 * n * n_dense_cols, device=C.device,
+                           dtype=torch.float64 if acc_f64 else B.dtype)
+    kc._keep.extend((table, order, sums))
+    return _abi.bind(
+        "spmm_sliced", _abi.dtype_code(B.dtype), 1 if acc_f64 else 0, kc.data.data_ptr(),
+        kc.cols.data_ptr(), kc.rowptr.data_ptr(), kc.rowptr_bits, kc.n_rows, kc.nnz,
+        n_dense_cols, table.data_ptr(), None if order is None else order.data_ptr(), items, keep,
+        None if sums is None else sums.data_ptr(), int(cut), lanes, vec, XCD_REMAP)
+
+
+def _bind_row_blocks(kc, B, acc_f64, lanes, vec):
     n_dense_cols = int(B.shape[1])
-    key = ("slices", lanes, vec, n_dense_cols, bool(acc_f64), B.dtype)
-    stream = kc._order.stream(C.device, kc._keep)
-    args = kc._args.get(key)
-    if args is None:  # the arguments that do not change between calls, converted once
-        n_cols, positions = int(B.shape[0]), kc.n_rows + kc.nnz
-        row_bytes = min(n_dense_cols, lanes * vec) * B.element_size()  # of one column tile
-        items, keep = _spmm_slice_shape(lanes, positions, True)
-        by_column = _slices.ordered(kc.max_row_nnz, items, n_cols * row_bytes,
-                                    kc.nnz * row_bytes, kc.one_shot)
-        if not by_column:
-            items, keep = _spmm_slice_shape(lanes, positions)
-        table, order = kc.slices(items, keep, n_cols, by_column)
-        cut = kc.max_row_nnz is None or kc.max_row_nnz > keep
-        sums = None
-        if cut:  # the pieces of cut rows: a carry and a head per slice
-            n = int(table.numel()) // 2 - 1
-            sums = torch.empty(2 * n * n_dense_cols, device=C.device,
-                               dtype=torch.float64 if acc_f64 else B.dtype)
-        args = [_abi.dtype_code(B.dtype), 1 if acc_f64 else 0, kc.data.data_ptr(),
-                kc.cols.data_ptr(), kc.rowptr.data_ptr(), kc.rowptr_bits, kc.n_rows, kc.nnz,
-                None, 0, n_dense_cols, None, 0, table.data_ptr(),
-                None if order is None else order.data_ptr(), items, keep,
-                None if sums is None else sums.data_ptr(), int(cut), lanes, vec, XCD_REMAP, None]
-        kc._args[key] = args
-        kc._keep.extend((table, order, sums))
-    a = list(args)
-    a[8], a[9], a[11], a[12] = B.data_ptr(), B.stride(0), C.data_ptr(), C.stride(0)
-    a[22] = stream
-    _abi.check(_abi.lib().fsp_spmm_sliced(*a), "fsp_spmm_sliced")
-    return C
+    plan = kc.plan(lanes)
+    partials = plan.workspace(n_dense_cols)
+    groups, group_base, split_rows = plan.split_groups()
+    p = lambda t: t.data_ptr() if t.numel() else None  # noqa: E731
+    kc._keep.extend((partials, plan.desc, groups, group_base, split_rows))
+    return _abi.bind(
+        "spmm_csr", _abi.dtype_code(B.dtype), 1 if acc_f64 else 0, p(kc.data), p(kc.cols),
+        p(kc.rowptr), kc.rowptr_bits, kc.n_rows, kc.nnz, n_dense_cols, p(plan.desc), plan.n_desc,
+        plan.chunk, lanes, vec, p(partials), p(groups), p(group_base), p(split_rows),
+        int(groups.shape[0]), XCD_REMAP)
 
 
 def _run_spmm(kc, B, C, acc_f64, tile_cols=None):
     """C[n_rows, N] = A @ B (B, C contiguous row-major) on slices or row blocks (kc.sliced).
     Without an explicit tile (the reference's block_n), a B over SPMM_B_TILE_BYTES is tiled by
     columns."""
-    n_dense_cols = int(B.shape[1])
+    n_dense_cols = B.shape[1]
     if kc.n_rows == 0 or n_dense_cols == 0:
         return C
-    if tile_cols is None:
+    if tile_cols is None and 2 * B.numel() * B.element_size() > SPMM_B_TILE_BYTES:
         tile_cols = _auto_tile_cols(B)
-    dtype = B.dtype
-    slice_lanes, slice_vec = _spmm_slice_lanes(n_dense_cols, dtype, tile_cols)
-    lanes, vec = _spmm_lane_shape(n_dense_cols, dtype, B, C, tile_cols)
-    if kc.sliced() or vec < slice_vec:  # the row-block kernel's loads need aligned vectors
-        return _run_spmm_sliced(kc, B, C, acc_f64, slice_lanes, slice_vec)
-    key = (lanes, vec, n_dense_cols, bool(acc_f64), dtype)
-    args = kc._args.get(key)
-    if args is None:  # the arguments that do not change between calls, converted once
-        plan = kc.plan(lanes)
-        partials = plan.workspace(n_dense_cols)
-        groups, group_base, split_rows = plan.split_groups()
-        p = lambda t: t.data_ptr() if t.numel() else None  # noqa: E731
-        args = [_abi.dtype_code(dtype), 1 if acc_f64 else 0, p(kc.data), p(kc.cols),
-                p(kc.rowptr), kc.rowptr_bits, kc.n_rows, kc.nnz, None, 0, n_dense_cols, None, 0,
-                p(plan.desc), plan.n_desc, plan.chunk, lanes, vec, p(partials), p(groups),
-                p(group_base), p(split_rows), int(groups.shape[0]), 0, None]
-        kc._args[key] = args
-        kc._keep.extend((partials, plan.desc, groups, group_base, split_rows))
-    a = list(args)
-    a[8], a[9], a[11], a[12] = B.data_ptr(), B.stride(0), C.data_ptr(), C.stride(0)
-    a[23] = XCD_REMAP
-    a[24] = kc._order.stream(C.device, kc._keep)
-    _abi.check(_abi.lib().fsp_spmm_csr(*a), "fsp_spmm_csr")
+    b, c = B.data_ptr(), C.data_ptr()
+    stream = kc._order.stream(C.device, kc._keep)
+    # what a launch is bound to follows from the matrix and these
+    key = (n_dense_cols, B.dtype, bool(acc_f64), tile_cols, (b | c) & 15 == 0)
+    bound = kc._args.get(key)
+    if bound is None:
+        slice_lanes, slice_vec = _spmm_slice_lanes(n_dense_cols, B.dtype, tile_cols)
+        lanes, vec = _spmm_lane_shape(n_dense_cols, B.dtype, B, C, tile_cols)
+        if kc.sliced() or vec < slice_vec:  # the row-block kernel's loads need aligned vectors
+            bound = _bind_sliced(kc, B, C, acc_f64, slice_lanes, slice_vec)
+        else:
+            bound = _bind_row_blocks(kc, B, acc_f64, lanes, vec)
+        kc._args[key] = bound
+    _abi.run(bound, b, c, stream)
     return C
 
 
@@ -521,10 +515,10 @@ class PreparedCsrSpmmOpt:
         self._ref_meta = None
         self._kernel = None
 
-    def _kernel_csr(self):
+    def _kernel_csr(self, one_shot=False):
         if self._kernel is None:
             self._kernel = _SpmmKernelCsr(self.data, self.kernel_indices, self.kernel_indptr,
-                                          self.max_row_nnz)
+                                          self.max_row_nnz, one_shot)
         return self._kernel
 
     def _reference_metadata(self):
@@ -599,13 +593,19 @@ class PreparedCsrSpmmOpt:
 
 
 def prepare_spmm_csr_opt(data, indices, indptr, shape):
-    """spmm_csr.py:480-522: validation plus the gfx950 row-block plan for common widths."""
+    """spmm_csr.py:480-522: validation and narrowing; plans and slices are built by the first call
+    of each width."""
+    return _prepare_spmm_csr_opt(data, indices, indptr, shape, False)
+
+
+def _prepare_spmm_csr_opt(data, indices, indptr, shape, one_shot):
+    """prepare_spmm_csr_opt; one_shot: for a single call, so nothing is planned."""
     (data, kernel_indices, kernel_indptr, n_rows, n_cols, row_lengths,
      max_row_nnz) = _prepare_spmm_csr_matrix(data, indices, indptr, shape)
     prepared = PreparedCsrSpmmOpt(data, kernel_indices, kernel_indptr, shape, n_rows, n_cols,
                                   row_lengths, max_row_nnz)
     if prepared.supports_opt and n_rows > 0:
-        prepared._kernel_csr()
+        prepared._kernel_csr(one_shot)
     return prepared
 
 
@@ -635,7 +635,7 @@ def flagsparse_spmm_csr_opt(data=None, indices=None, indptr=None, B=None, shape=
         if any(arg is None for arg in (data, indices, indptr, shape)):
             raise ValueError(
                 "data, indices, indptr, and shape are required when prepared is not provided")
-        prepared = prepare_spmm_csr_opt(data, indices, indptr, shape)
+        prepared = _prepare_spmm_csr_opt(data, indices, indptr, shape, True)
     elif shape is not None:
         resolved_shape = (int(shape[0]), int(shape[1]))
         if resolved_shape != prepared.shape:

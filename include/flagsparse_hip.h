@@ -589,6 +589,37 @@ int fsp_probe_rows(const float* b, int64_t n_rows, int64_t row_floats, const int
 int64_t fsp_probe_stream_blocks(int64_t n16);
 int fsp_probe_stream(const void* src, int64_t n16, float* out, void* stream);
 
+/*
+ * Bound calls: fsp_bind_* writes a call's arguments, all but the input (x or B), the output (y or
+ * C) and the stream, into call - fsp_bound_bytes() bytes of host memory, 8-byte aligned, the
+ * caller's - and fsp_run makes the call with the three.  The arguments are checked by fsp_run, as
+ * the entry point checks them.  B and C are N columns wide (ldb = ldc = N).  What the arguments
+ * point to must live as long as the bound call is run; one may be run from several threads.
+ */
+int64_t fsp_bound_bytes(void);
+int fsp_bind_spmv_csr(void* call, int dtype, int acc_f64, const void* vals, const int32_t* cols,
+                      const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t nnz,
+                      const int32_t* row_map, int64_t n_out, const int32_t* desc,
+                      const int64_t* ranges, int64_t n_desc, int64_t chunk, void* partials,
+                      const int32_t* groups, const int64_t* group_base,
+                      const int32_t* split_rows, int64_t n_groups, int xcd_remap);
+int fsp_bind_spmv_sliced(void* call, int dtype, int acc_f64, const void* vals,
+                         const int32_t* cols, const void* rowptr, int rowptr_bits,
+                         int64_t n_rows, int64_t nnz, int64_t* table, int table_built,
+                         void* sums, int cut_rows);
+int fsp_bind_spmm_csr(void* call, int dtype, int acc_f64, const void* vals, const int32_t* cols,
+                      const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t nnz,
+                      int64_t N, const int32_t* desc, int64_t n_desc, int64_t chunk,
+                      int lanes_per_row, int vec, void* partials, const int32_t* groups,
+                      const int64_t* group_base, const int32_t* split_rows, int64_t n_groups,
+                      int xcd_remap);
+int fsp_bind_spmm_sliced(void* call, int dtype, int acc_f64, const void* vals,
+                         const int32_t* cols, const void* rowptr, int rowptr_bits,
+                         int64_t n_rows, int64_t nnz, int64_t N, const int64_t* table,
+                         const int32_t* order, int64_t items, int64_t keep, void* sums,
+                         int cut_rows, int lanes_per_row, int vec, int xcd_remap);
+int fsp_run(const void* call, const void* in, void* out, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

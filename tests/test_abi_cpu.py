@@ -323,3 +323,27 @@ def test_build_flags_kernels_with_scratch():
     ])
     assert _build._scratch_kernels(log) == {"_Z3badPf"}
     assert _build._scratch_kernels("") == set()
+
+
+def test_bound_calls_check_like_their_entry_points():
+    # fsp_run hands a bound call's arguments to the entry point, which refuses what it refuses
+    L = _abi.lib()
+    buf = ctypes.create_string_buffer(int(L.fsp_bound_bytes()) + 8)
+    at = (ctypes.addressof(buf) + 7) & ~7
+    assert L.fsp_run(None, None, None, None) == -1
+    assert L.fsp_run(at, None, None, None) == -1 and b"bound call" in L.fsp_last_error()
+    assert L.fsp_bind_spmm_csr(None, *[0] * 20) == -1  # no memory
+    assert L.fsp_bind_spmm_csr(at + 4, *[0] * 20) == -1  # not 8-byte aligned
+    for name, args, text in (
+            ("spmv_csr", (9, 0, None, None, None, 32, 0, 0, None, 0, None, None, 0, 1, None, None,
+                          None, None, 0, 0), b"fsp_spmv_csr: dtype"),
+            ("spmv_sliced", (0, 0, None, None, None, 16, 0, 0, None, 0, None, 0),
+             b"fsp_spmv_sliced: rowptr_bits"),
+            ("spmm_csr", (0, 0, None, None, None, 32, 1, 0, -4, None, 0, 1, 1, 1, None, None, None,
+                          None, 0, 0), b"fsp_spmm_csr: negative size"),
+            ("spmm_sliced", (0, 0, None, None, None, 32, 1, 0, 8, None, None, 0, 0, None, 0, 1, 1,
+                             0), b"fsp_spmm_sliced: a slice must hold")):
+        bound = _abi.bind(name, *args)
+        assert bound[1] % 8 == 0
+        assert L.fsp_run(bound[1], None, None, None) < 0
+        assert text in L.fsp_last_error(), (name, L.fsp_last_error())
