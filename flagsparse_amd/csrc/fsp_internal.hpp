@@ -19,7 +19,7 @@ constexpr int64_t kSpmvChunkCap = kSpmvChunkUnitsPerThread * 4 * 256 - 3;
 constexpr int64_t kSpmmSlots = 2048;                     // LDS (col, val) slots per SpMM block
 constexpr int64_t kSpmmNnzCap = kSpmmSlots - 3;
 constexpr int64_t kIndexStatsBlocks = 1024;             // first-pass workgroups of fsp_index_stats
-constexpr int64_t kCsrCheckBlocks = 2048;               // first-pass workgroups of fsp_csr_check
+constexpr int64_t kCheckBlocks = 512;                   // most workgroups of an index check
 // Sliced SpMV: positions (rows + entries) per slice, and the longest row that no boundary cuts.
 constexpr int64_t kSpmvSliceSlots = 1024;               // LDS product slots per slice
 constexpr int64_t kSpmvSliceItems = 760;

@@ -20,7 +20,7 @@ import torch
 
 from . import _abi
 from ._coo_order import row_pointers, rows_in_order
-from ._index_stats import index_stats
+from ._csr_check import coo_check
 from ._common import (
     SUPPORTED_INDEX_DTYPES,
     _INDEX_LIMIT_INT32,
@@ -42,7 +42,7 @@ from .synthetic import build_random_coo, build_random_dense
 
 def _check_spmm_coo_inputs(data, row, col, B, shape):
     """The checks of spmm_coo.py:312-371 (same order, messages and types): (data, row, col, B) as
-    contiguous arrays, the sizes, and whether the rows are already in order (from the same pass
+    contiguous arrays, the indices int32 where there are entries, the sizes, and whether the rows are already in order (from the same pass
     over the indices)."""
     if len(shape) != 2:
         raise ValueError("shape must be a 2-tuple: (n_rows, n_cols)")
@@ -77,8 +77,8 @@ def _check_spmm_coo_inputs(data, row, col, B, shape):
     row, col = row.contiguous(), col.contiguous()
     row_sorted = True
     if nnz > 0:
-        # one pass over both arrays and one host sync for the four bounds and the row order
-        min_row, max_row, min_col, max_col, descents = index_stats(row, col)
+        # one pass over both arrays: the four bounds, the row order, int32 copies
+        (min_row, max_row, min_col, max_col, descents), row, col = coo_check(row, col)
         row_sorted = descents == 0
         if min_row < 0 or max_row >= n_rows:
             raise IndexError("row indices out of range for n_rows")

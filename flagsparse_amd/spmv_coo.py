@@ -18,7 +18,7 @@ import torch
 from . import _abi, _spmv_layouts
 from ._common import _INDEX_LIMIT_INT32
 from ._coo_order import row_pointers, rows_in_order
-from ._index_stats import index_stats
+from ._csr_check import coo_check
 from ._spmv_layouts import RowBlockLayout, SliceLayout, build_layout
 
 
@@ -187,12 +187,12 @@ def _prepare_one_call(data, row, col, shape, sort_by_row):
     if nnz == 0 or n_rows > max(1 << 26, 4 * nnz) or not data.device == row.device == col.device:
         return _prepare_spmv_coo(data, row, col, shape, sort_by_row, True)
     data, row, col = data.contiguous(), row.contiguous(), col.contiguous()
-    # one pass over both index arrays and one host synchronisation: bounds and row order
-    rmin, rmax, cmin, cmax, descents = index_stats(row, col)
+    # one pass over both index arrays: bounds, row order, int32 copies
+    (rmin, rmax, cmin, cmax, descents), row, col = coo_check(row, col)
     _check_coo_bounds(rmin, rmax, cmin, cmax, n_rows, n_cols)
     if descents:
         data, row, col = rows_in_order(data, row, col, rmax)
-    prepared = PreparedCoo(data, row, col.to(torch.int32), shape)
+    prepared = PreparedCoo(data, row, col, shape)
     prepared.use_seg_kernel = True
     prepared._layout = SliceLayout(data, prepared.col, row_pointers(row, n_rows), one_shot=True)
     return prepared

@@ -145,16 +145,24 @@ int fsp_plan_panel_chunks_device(const int64_t* panel_runs, int64_t n_panels,
  *   indptr, ptr_bits   n_rows + 1 row pointers, int32 or int64
  *   idx32              NULL, or nnz int32 (16-byte aligned): the columns, narrowed
  *   ptr_out            NULL, or n_rows + 1 row pointers of ptr_out_bits (32 / 64)
- *   partial            device scratch, fsp_csr_check_partial_len() int64
- *   out                6 int64 (device, or host memory the device can write): indptr[0],
- *                      indptr[n_rows], the number of decreases, the longest row, the smallest
- *                      and the largest column (INT64_MAX and INT64_MIN when nnz is 0)
- * The narrowed copies hold meaningless values where the checks fail.
+ *   pinned             pinned host memory the device can write, fsp_check_pinned_len() int64; in
+ *                      use until the call returns
+ *   out                6 int64 (host): indptr[0], indptr[n_rows], the number of decreases, the
+ *                      longest row, the smallest and the largest column (INT64_MAX and INT64_MIN
+ *                      when nnz is 0)
+ * The call returns when the results are there (it waits for the check, not for later work of the
+ * stream; it cannot be captured).  The narrowed copies are complete for work queued after it on
+ * the stream, and hold meaningless values where the checks fail.
+ * fsp_coo_check: the same for nnz >= 1 row and column indices; row32, col32 NULL or nnz int32
+ * (16-byte aligned) for the narrowed arrays; out: smallest and largest row, smallest and largest
+ * column, the number of places where the rows decrease.
  */
-int64_t fsp_csr_check_partial_len(void);
+int64_t fsp_check_pinned_len(void);
 int fsp_csr_check(const void* indices, int idx_bits, int64_t nnz, const void* indptr,
                   int ptr_bits, int64_t n_rows, int32_t* idx32, void* ptr_out, int ptr_out_bits,
-                  int64_t* partial, int64_t* out, void* stream);
+                  int64_t* pinned, int64_t* out, void* stream);
+int fsp_coo_check(const void* rows, int row_bits, const void* cols, int col_bits, int64_t nnz,
+                  int32_t* row32, int32_t* col32, int64_t* pinned, int64_t* out, void* stream);
 
 /*
  * The same plan built on the device in two passes (no host copy of rowptr, no host loop):

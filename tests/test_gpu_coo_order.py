@@ -8,6 +8,7 @@ import torch
 import flagsparse_amd as fs
 from flagsparse_amd import _common, spmv_coo, synthetic
 from flagsparse_amd._coo_order import row_pointers, rows_in_order
+from flagsparse_amd._csr_check import coo_check
 from oracle import oracle
 
 pytestmark = pytest.mark.gpu
@@ -104,3 +105,52 @@ def test_coo_one_call_routes(dev):
     for bad, exc in (((row - 1, col), "row indices"), ((row, col + 50), "col indices")):
         with pytest.raises(IndexError, match=exc):
             fs.flagsparse_spmv_coo(data, *bad, x, (100, 50))
+
+
+@pytest.mark.parametrize("nnz", [1, 3, 4, 1023, 1024, 1025, 2047, 70001, 5000003])
+@pytest.mark.parametrize("rt", [torch.int32, torch.int64])
+@pytest.mark.parametrize("ct", [torch.int32, torch.int64])
+def test_coo_check(dev, nnz, rt, ct):
+    row = synthetic.randint(6, 1, nnz, 50001, "cpu") - 7
+    col = synthetic.randint(6, 2, nnz, 90001, "cpu")
+    for order in ("any", "sorted", "one"):
+        r = row if order == "any" else torch.sort(row).values
+        if order == "one" and nnz > 1:  # a single decrease, across a quad or workgroup step
+            r[-1] = r[0] - 1
+        want = [int(r.min()), int(r.max()), int(col.min()), int(col.max()),
+                int((r[1:] < r[:-1]).sum())]
+        for shift in (0, 1):
+            rd = torch.cat([r.new_zeros(shift), r]).to(rt).to(dev)[shift:]
+            cd = torch.cat([col.new_zeros(shift), col]).to(ct).to(dev)[shift:]
+            stats, r32, c32 = coo_check(rd, cd)
+            assert stats == want, (order, shift)
+            assert r32.dtype == c32.dtype == torch.int32
+            assert torch.equal(r32.cpu().to(torch.int64), r)
+            assert torch.equal(c32.cpu().to(torch.int64), col)
+
+
+def test_checks_wait_for_queued_work(dev):
+    # indices still being written by earlier work of the stream, longer than the host watches for
+    row = torch.zeros(40000, dtype=torch.int64, device=dev)
+    big = torch.randn(4096, 4096, device=dev)
+    for _ in range(2):
+        out = big
+        for _ in range(12):
+            out = out @ big * 1e-3
+        row.copy_(torch.arange(40000, device=dev) + (out[0, 0] * 0).to(torch.int64))
+        stats, r32, _ = coo_check(row, row)
+        assert stats == [0, 39999, 0, 39999, 0]
+        assert torch.equal(r32.to(torch.int64), torch.arange(40000, device=dev))
+        row.zero_()
+
+
+def test_checks_refuse_capture(dev):
+    row = torch.zeros(10, dtype=torch.int32, device=dev)
+    data = torch.ones(10, device=dev)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with pytest.raises(RuntimeError, match="captured"):
+        with torch.cuda.graph(g):
+            fs.flagsparse_spmv_coo(data, row, row, data, (10, 10))
+    torch.cuda.synchronize()
+    assert float(fs.flagsparse_spmv_coo(data, row, row, data, (10, 10))[0]) == 10.0
