@@ -11,7 +11,7 @@
 // for 1.65M entries of 150k rows, 240 us for 1.2M of 60k).  Here only the bits that the rows have
 // are sorted, up to 9 a pass (two passes to 262,144 rows, three to 134M), 16 bytes an entry.
 // A pass is three launches:
-//   coo_hist_kernel     digits of each tile of 4096 entries -> counts[digit][tile]
+//   coo_hist_kernel     digits of each tile of 2048 or 4096 entries -> counts[digit][tile]
 //   coo_scan_kernel     a workgroup per digit: exclusive sums over the tiles, the digit's total
 //   coo_scatter_kernel  each tile ranks its entries (wave ballots, one digit bit at a time; LDS
 //                       counters per wave keep the order), puts them in digit order in LDS and
@@ -28,10 +28,16 @@ namespace {
 
 constexpr int kSortBlock = 512;
 constexpr int kSortWaves = kSortBlock / kWave;
-constexpr int kSortSteps = 8;  // entries per thread
-constexpr int kTile = kSortBlock * kSortSteps;
+// Entries per thread of a tile: 4 for short sorts, whose tiles would not fill the CUs, else 8 (runs
+// of equal digits twice as long).  Measured on MI355X, a sort with 4 / 8: 16k entries 20.2 / 24.5
+// us, 400k 26.4 / 33.7, 1.65M 56.4 / 52.4, 12M 336 / 285.
+constexpr int kShortSteps = 4, kLongSteps = 8;
+constexpr int64_t kShortNnz = 1 << 20;
 constexpr int kMaxDigits = 512;  // one per thread in the scatter kernel's scans
 static_assert(kMaxDigits == kSortBlock, "a thread per digit");
+// Up to this many tiles the scatter kernel reads all their counts itself: a launch less, which a
+// small sort is made of (two passes of 16k entries: 29.4 -> 20.8 us of host time with the launches).
+constexpr int kFewTiles = 32;
 
 __device__ __forceinline__ int wave_inclusive(int v) {
   const int lane = threadIdx.x & (kWave - 1);
@@ -62,24 +68,25 @@ __device__ __forceinline__ int block_exclusive(int v, int* s_w, int* total) {
   return before + incl - v;
 }
 
-template <typename R>
+template <typename R, int STEPS>
 __global__ __launch_bounds__(kSortBlock) void coo_hist_kernel(const R* __restrict__ rows, int n,
                                                               int shift, int bits, int n_tiles,
                                                               int* __restrict__ counts) {
+  constexpr int TILE = kSortBlock * STEPS;
   __shared__ int s_cnt[kMaxDigits];
   const int tile = xcd_logical_block(blockIdx.x, n_tiles);  // neighbours share lines of counts
   const int D = 1 << bits;
   if ((int)threadIdx.x < D) s_cnt[threadIdx.x] = 0;
   __syncthreads();
-  const int base = tile * kTile;
-  int d[kSortSteps];
+  const int base = tile * TILE;
+  int d[STEPS];
 #pragma unroll
-  for (int q = 0; q < kSortSteps; ++q) {
-    const int i = base + q * kSortBlock + threadIdx.x;  // < 2^31: n <= 2^31 - 1 - kTile
+  for (int q = 0; q < STEPS; ++q) {
+    const int i = base + q * kSortBlock + threadIdx.x;  // < 2^31: n <= 2^31 - 1 - TILE
     d[q] = i < n ? (int)((uint32_t)rows[i] >> shift) & (D - 1) : -1;
   }
 #pragma unroll
-  for (int q = 0; q < kSortSteps; ++q)
+  for (int q = 0; q < STEPS; ++q)
     if (d[q] >= 0) atomicAdd(&s_cnt[d[q]], 1);
   __syncthreads();
   if ((int)threadIdx.x < D) counts[(int64_t)threadIdx.x * n_tiles + tile] = s_cnt[threadIdx.x];
@@ -100,28 +107,29 @@ __global__ __launch_bounds__(kBlock) void coo_scan_kernel(int* __restrict__ coun
   if (threadIdx.x == 0) totals[blockIdx.x] = run;
 }
 
-template <typename R, typename C, typename T>
+template <typename R, typename C, typename T, int STEPS>
 __global__ __launch_bounds__(kSortBlock) void coo_scatter_kernel(
     const R* __restrict__ rows, const C* __restrict__ cols, const T* __restrict__ vals, int n,
     int shift, int bits, int n_tiles, const int* __restrict__ counts,
     const int* __restrict__ totals, int* __restrict__ out_rows, int* __restrict__ out_cols,
     T* __restrict__ out_vals) {
-  __shared__ int s_key[kTile];
-  __shared__ T s_buf[kTile];  // the columns, then the values, in digit order
+  constexpr int TILE = kSortBlock * STEPS;
+  __shared__ int s_key[TILE];
+  __shared__ T s_buf[TILE];  // the columns, then the values, in digit order
   __shared__ uint16_t s_cnt[kSortWaves][kMaxDigits];
   __shared__ int s_start[kMaxDigits];  // a digit's first position in the tile's digit order
   __shared__ int s_dst[kMaxDigits];    // its place in the output, less s_start
   __shared__ int s_w[kSortWaves];
   const int tid = threadIdx.x, lane = tid & (kWave - 1), w = tid / kWave;
   const int tile = xcd_logical_block(blockIdx.x, n_tiles);
-  const int D = 1 << bits, base = tile * kTile;
-  const int m = n - base < kTile ? n - base : kTile;
-  int key[kSortSteps], col[kSortSteps];
-  T val[kSortSteps];
-  int at[kSortSteps];  // wave w holds entries [w * 512, w * 512 + 512) in order, 64 a step
+  const int D = 1 << bits, base = tile * TILE;
+  const int m = n - base < TILE ? n - base : TILE;
+  int key[STEPS], col[STEPS];
+  T val[STEPS];
+  int at[STEPS];  // wave w holds entries [w * 512, w * 512 + 512) in order, 64 a step
 #pragma unroll
-  for (int q = 0; q < kSortSteps; ++q) {
-    const int i = w * (kTile / kSortWaves) + q * kWave + lane;
+  for (int q = 0; q < STEPS; ++q) {
+    const int i = w * (TILE / kSortWaves) + q * kWave + lane;
     const bool ok = i < m;
     key[q] = ok ? (int)rows[base + i] : 0;
     col[q] = ok ? (int)cols[base + i] : 0;
@@ -133,8 +141,8 @@ __global__ __launch_bounds__(kSortBlock) void coo_scatter_kernel(
   volatile uint16_t* cnt = s_cnt[w];
   const uint64_t below = (uint64_t(1) << lane) - 1;
 #pragma unroll
-  for (int q = 0; q < kSortSteps; ++q) {
-    const bool ok = w * (kTile / kSortWaves) + q * kWave + lane < m;
+  for (int q = 0; q < STEPS; ++q) {
+    const bool ok = w * (TILE / kSortWaves) + q * kWave + lane < m;
     const int d = (int)((uint32_t)key[q] >> shift) & (D - 1);
     uint64_t same = __ballot(ok);  // the lanes of this step that hold the same digit
     for (int b = 0; b < bits; ++b) {
@@ -161,18 +169,33 @@ __global__ __launch_bounds__(kSortBlock) void coo_scatter_kernel(
       mine += c;
     }
   }
+  // The digit's entries in all tiles and in those before this one: from coo_scan_kernel, or,
+  // where tiles are few (totals NULL), added up here.
+  int in_all = 0, in_before = 0;
+  if (tid < D) {
+    if (totals) {
+      in_all = totals[tid];
+      in_before = counts[(int64_t)tid * n_tiles + tile];
+    } else {
+      for (int t = 0; t < n_tiles; ++t) {
+        const int c = counts[(int64_t)tid * n_tiles + t];
+        in_all += c;
+        in_before += t < tile ? c : 0;
+      }
+    }
+  }
   int all;
   const int start = block_exclusive<kSortWaves>(mine, s_w, &all);
-  const int place = block_exclusive<kSortWaves>(tid < D ? totals[tid] : 0, s_w, &all);
+  const int place = block_exclusive<kSortWaves>(in_all, s_w, &all);
   if (tid < D) {
     s_start[tid] = start;
-    s_dst[tid] = place + counts[(int64_t)tid * n_tiles + tile] - start;
+    s_dst[tid] = place + in_before - start;
   }
   __syncthreads();
   int* s_col = reinterpret_cast<int*>(s_buf);
 #pragma unroll
-  for (int q = 0; q < kSortSteps; ++q) {
-    if (w * (kTile / kSortWaves) + q * kWave + lane < m) {
+  for (int q = 0; q < STEPS; ++q) {
+    if (w * (TILE / kSortWaves) + q * kWave + lane < m) {
       const int d = (int)((uint32_t)key[q] >> shift) & (D - 1);
       at[q] += s_start[d] + s_cnt[w][d];
       s_key[at[q]] = key[q];
@@ -180,9 +203,9 @@ __global__ __launch_bounds__(kSortBlock) void coo_scatter_kernel(
     }
   }
   __syncthreads();
-  int dst[kSortSteps];
+  int dst[STEPS];
 #pragma unroll
-  for (int q = 0; q < kSortSteps; ++q) {
+  for (int q = 0; q < STEPS; ++q) {
     const int i = q * kSortBlock + tid;
     dst[q] = -1;
     if (i < m) {
@@ -194,11 +217,11 @@ __global__ __launch_bounds__(kSortBlock) void coo_scatter_kernel(
   }
   __syncthreads();
 #pragma unroll
-  for (int q = 0; q < kSortSteps; ++q)
-    if (w * (kTile / kSortWaves) + q * kWave + lane < m) s_buf[at[q]] = val[q];
+  for (int q = 0; q < STEPS; ++q)
+    if (w * (TILE / kSortWaves) + q * kWave + lane < m) s_buf[at[q]] = val[q];
   __syncthreads();
 #pragma unroll
-  for (int q = 0; q < kSortSteps; ++q)
+  for (int q = 0; q < STEPS; ++q)
     if (dst[q] >= 0) out_vals[dst[q]] = s_buf[q * kSortBlock + tid];
 }
 
@@ -218,7 +241,7 @@ __global__ __launch_bounds__(kBlock) void coo_rowptr_kernel(const R* __restrict_
 }
 
 struct SortPlan {
-  int passes, bits, n_tiles;  // bits per pass
+  int passes, bits, steps, n_tiles;  // bits per pass, entries per thread
 };
 
 SortPlan sort_plan(int64_t nnz, int64_t max_row) {
@@ -227,29 +250,46 @@ SortPlan sort_plan(int64_t nnz, int64_t max_row) {
   SortPlan p;
   p.passes = (bits + 8) / 9;
   p.bits = (bits + p.passes - 1) / p.passes;
-  p.n_tiles = (int)((nnz + kTile - 1) / kTile);
+  p.steps = nnz < kShortNnz ? kShortSteps : kLongSteps;
+  const int64_t tile = (int64_t)kSortBlock * p.steps;
+  p.n_tiles = (int)((nnz + tile - 1) / tile);
   return p;
 }
 
 int64_t align16(int64_t b) { return (b + 15) & ~int64_t(15); }
 
+template <typename R, typename C, typename T, int STEPS>
+int sort_pass_steps(const R* rows, const C* cols, const T* vals, int n, int shift, const SortPlan& p,
+              int* counts, int* totals, int* out_rows, int* out_cols, T* out_vals,
+              hipStream_t st) {
+  const unsigned tiles = (unsigned)p.n_tiles;
+  hipLaunchKernelGGL((coo_hist_kernel<R, STEPS>), dim3(tiles), dim3(kSortBlock), 0, st, rows, n, shift,
+                     p.bits, p.n_tiles, counts);
+  int rc = check_hip(hipGetLastError(), "coo_hist_kernel launch");
+  if (rc) return rc;
+  if (p.n_tiles <= kFewTiles) {
+    totals = nullptr;  // the scatter kernel adds the counts up
+  } else {
+    hipLaunchKernelGGL(coo_scan_kernel, dim3(1u << p.bits), dim3(kBlock), 0, st, counts,
+                       p.n_tiles, totals);
+    rc = check_hip(hipGetLastError(), "coo_scan_kernel launch");
+    if (rc) return rc;
+  }
+  hipLaunchKernelGGL((coo_scatter_kernel<R, C, T, STEPS>), dim3(tiles), dim3(kSortBlock), 0, st, rows,
+                     cols, vals, n, shift, p.bits, p.n_tiles, counts, totals, out_rows, out_cols,
+                     out_vals);
+  return check_hip(hipGetLastError(), "coo_scatter_kernel launch");
+}
+
 template <typename R, typename C, typename T>
 int sort_pass(const R* rows, const C* cols, const T* vals, int n, int shift, const SortPlan& p,
               int* counts, int* totals, int* out_rows, int* out_cols, T* out_vals,
               hipStream_t st) {
-  const unsigned tiles = (unsigned)p.n_tiles;
-  hipLaunchKernelGGL((coo_hist_kernel<R>), dim3(tiles), dim3(kSortBlock), 0, st, rows, n, shift,
-                     p.bits, p.n_tiles, counts);
-  int rc = check_hip(hipGetLastError(), "coo_hist_kernel launch");
-  if (rc) return rc;
-  hipLaunchKernelGGL(coo_scan_kernel, dim3(1u << p.bits), dim3(kBlock), 0, st, counts, p.n_tiles,
-                     totals);
-  rc = check_hip(hipGetLastError(), "coo_scan_kernel launch");
-  if (rc) return rc;
-  hipLaunchKernelGGL((coo_scatter_kernel<R, C, T>), dim3(tiles), dim3(kSortBlock), 0, st, rows,
-                     cols, vals, n, shift, p.bits, p.n_tiles, counts, totals, out_rows, out_cols,
-                     out_vals);
-  return check_hip(hipGetLastError(), "coo_scatter_kernel launch");
+  if (p.steps == kShortSteps)
+    return sort_pass_steps<R, C, T, kShortSteps>(rows, cols, vals, n, shift, p, counts, totals,
+                                                 out_rows, out_cols, out_vals, st);
+  return sort_pass_steps<R, C, T, kLongSteps>(rows, cols, vals, n, shift, p, counts, totals,
+                                              out_rows, out_cols, out_vals, st);
 }
 
 template <typename R, typename C, typename T>
@@ -305,7 +345,7 @@ int sort_any(int row_bits, int col_bits, const void* rows, const void* cols, con
 
 using namespace fsp;
 
-extern "C" int64_t fsp_coo_sort_max_nnz(void) { return 0x7fffffffLL - kTile; }
+extern "C" int64_t fsp_coo_sort_max_nnz(void) { return 0x7fffffffLL - kSortBlock * kLongSteps; }
 
 extern "C" int64_t fsp_coo_sort_scratch(int dtype, int64_t nnz, int64_t max_row) {
   if (nnz < 1 || nnz > fsp_coo_sort_max_nnz() || max_row < 0) return 0;

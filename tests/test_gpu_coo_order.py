@@ -13,10 +13,11 @@ from oracle import oracle
 
 pytestmark = pytest.mark.gpu
 
-TILE = 4096
+TILE = 2048  # entries of a tile below 2^20 entries, 4096 from there on; 32 tiles need no scan
 
 
-@pytest.mark.parametrize("nnz", [1, 63, 64, TILE - 1, TILE, TILE + 1, 5 * TILE + 17, 300001])
+@pytest.mark.parametrize("nnz", [1, 63, 64, TILE - 1, TILE, TILE + 1, 5 * TILE + 17, 32 * TILE,
+                                 32 * TILE + 1, (1 << 20) - 1, 1 << 20])
 @pytest.mark.parametrize("max_row", [1, 255, 511, 512, 70000, 262143, 262144, (1 << 27) + 5,
                                      2**31 - 2])
 def test_rows_in_order(dev, nnz, max_row):
@@ -24,7 +25,7 @@ def test_rows_in_order(dev, nnz, max_row):
     row[nnz // 2] = max_row
     kinds = [(torch.int32, torch.int32, torch.float32), (torch.int64, torch.int64, torch.float64),
              (torch.int32, torch.int64, torch.float64), (torch.int64, torch.int32, torch.float32)]
-    for rt, ct, vt in kinds if nnz < 2 * TILE else kinds[:2]:
+    for rt, ct, vt in kinds if nnz < 2 * TILE else kinds[1:3]:
         col = torch.arange(nnz, dtype=ct)  # the input position: shows the order inside a row
         val = torch.arange(nnz, dtype=vt)
         print(f"sort nnz={nnz} max_row={max_row} {rt} {ct} {vt}", flush=True)
