@@ -277,8 +277,8 @@ extern "C" int fsp_sddmm_sliced(int dtype, int acc_f64, int out_f64, const int32
     return set_error(FSP_EINVAL, "fsp_sddmm_sliced: vec must be 1, 2 or 4 (fp32) / 1, 2 (fp64)");
   if (K < vec || K > 4 * ((int64_t)vec << lg))
     return set_error(FSP_EINVAL, "fsp_sddmm_sliced: needs vec <= K <= 4 * lanes * vec");
-  if (items < 1 || items > 4096)
-    return set_error(FSP_EINVAL, "fsp_sddmm_sliced: items outside [1, 4096]");
+  if (items < 1 || items > 2048)  // 33 KB of LDS with float64 results
+    return set_error(FSP_EINVAL, "fsp_sddmm_sliced: items outside [1, 2048]");
   if (ldx < K || ldy < K)
     return set_error(FSP_EINVAL, "fsp_sddmm_sliced: ldx/ldy smaller than K");
   if (out_f64 && dtype != FSP_F32)

@@ -149,6 +149,8 @@ def _prepare_sddmm(indices, indptr, shape, k_hint, one_call):
     if one_call:
         prepared._one_call = True
         prepared._kernel_ptr = indptr
+    else:  # calls may come from other streams than the one the copies are made on
+        torch.cuda.current_stream(indices.device).synchronize()
     return prepared
 
 
@@ -257,7 +259,7 @@ def _sddmm_slice_items(lanes, positions):
     positions, 8 lanes: 674 / 689 / 739 us with 256 / 512 / 1024; 16 lanes: 818 / 676 / 704 with
     128 / 256 / 512), and fewer where the slices would not fill the 256 CUs."""
     items = {1: 1024, 2: 1024, 4: 512, 8: 256}.get(lanes, 128)
-    while positions > 150000 * items and items < 4096:
+    while positions > 150000 * items and items < 2048:
         items <<= 1
     while items > 64 and positions < 256 * items:
         items >>= 1

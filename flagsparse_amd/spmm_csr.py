@@ -39,6 +39,10 @@ XCD_REMAP = 1
 # prepared: fp32 N=16 380 / 329 / 327 us with windows of 1 / 4 / 16 blocks, N=64 663 / 663 / 662
 # (the planner takes longer on wide windows: one thread each).
 SPMM_PLAN_WINDOW_BLOCKS = 4
+# A one-off COO matrix's longest row is not known.  Up to this many values its slices get room for
+# the pieces of cut rows unseen; beyond it (32 MB of float64) the row pointers are looked at first
+# (25 us with its host wait, on products of milliseconds).
+_SUMS_UNSEEN = 1 << 22
 # Rows longer than this go to the part path (several lane groups per row).
 _SPMM_ROW_SPLIT_THRESHOLD = 128
 
@@ -403,11 +407,13 @@ def _bind_sliced(kc, B, C, acc_f64, lanes, vec):
     if not by_column:
         items, keep = _spmm_slice_shape(lanes, positions)
     table, order = kc.slices(items, keep, n_cols, by_column)
+    # the pieces of cut rows: a carry and a head per slice
+    sums, sums_len = None, (int(table.numel()) - 2) * n_dense_cols
+    if kc.max_row_nnz is None and sums_len > _SUMS_UNSEEN:
+        kc.max_row_nnz = int((kc.rowptr[1:] - kc.rowptr[:-1]).max())
     cut = kc.max_row_nnz is None or kc.max_row_nnz > keep
-    sums = None
-    if cut:  # the pieces of cut rows: a carry and a head per slice
-        n = int(table.numel()) // 2 - 1
-        sums = torch.empty(2 * n * n_dense_cols, device=C.device,
+    if cut:
+        sums = torch.empty(sums_len, device=C.device,
                            dtype=torch.float64 if acc_f64 else B.dtype)
     kc._keep.extend((table, order, sums))
     return _abi.bind(

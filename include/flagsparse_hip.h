@@ -548,7 +548,7 @@ int fsp_sddmm_csr(int dtype, int acc_f64, int out_f64, const int32_t* cols,
 /*
  * The same over the slices of fsp_slice_table(rowptr, .., items, 0, table): no plan, row by row,
  * for vec <= K <= 4 * lanes_per_entry * vec, K >= 1.
- *   items          rows + entries per slice, at most 4096
+ *   items          rows + entries per slice, at most 2048
  *   order          NULL (row order), or fsp_slice_order's order
  *   vec            elements per lane per load: 1, 2 or 4 (fp32) / 1 or 2 (fp64); needs no
  *                  alignment of x, y, ldx or ldy beyond the element's own

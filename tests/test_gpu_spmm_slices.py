@@ -142,3 +142,19 @@ def test_slices_by_column(dev, monkeypatch, name):
     k = cols[t[o[others:], 1]] * 255 // shape[1]
     for x in range(8):  # slots 8 apart are one XCD's, in column bins that rise
         assert bool((k[x::8][1:] >= k[x::8][:-1]).all())
+
+
+def test_unknown_longest_row(dev, monkeypatch):
+    # a one-off COO matrix: room for cut rows' pieces is only taken unseen while it is small
+    for name, cut in (("crossing", True), ("short", False)):
+        vals, cols, ip, B, shape = _case(name, 901, 24, torch.float32, dev)
+        row = torch.repeat_interleave(torch.arange(shape[0]), ip[1:] - ip[:-1])
+        args = [t.to(dev) for t in (vals, row, cols, B)]
+        C = fs.flagsparse_spmm_coo(*args, shape)
+        monkeypatch.setattr(spmm_csr, "_SUMS_UNSEEN", 0)
+        assert torch.equal(fs.flagsparse_spmm_coo(*args, shape), C)
+        kc = spmm_csr._SpmmKernelCsr(args[0], args[2].to(torch.int32), ip.to(dev), one_shot=True)
+        spmm_csr._run_spmm(kc, args[3], torch.empty_like(C), True)
+        assert (kc.max_row_nnz > 256) == cut and (kc._keep[-1] is not None) == cut
+        monkeypatch.undo()
+        assert oracle.rel_l2(C, oracle.spmm_csr(ip, cols, vals, B)) <= 1e-5

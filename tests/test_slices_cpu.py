@@ -35,7 +35,7 @@ def test_sddmm_slice_lanes(dtype):
         lanes, vec = sddmm_csr._sddmm_slice_lanes(K, dtype)
         assert vec <= K and vec == (vmax if K >= vmax else min(K, 2))
         assert K <= 4 * lanes * vec or lanes == 64
-        assert 64 <= sddmm_csr._sddmm_slice_items(lanes, 1 << 40) <= 4096
+        assert 64 <= sddmm_csr._sddmm_slice_items(lanes, 1 << 40) <= 2048
 
 
 def test_ordered_rule():
