@@ -225,19 +225,116 @@ __global__ __launch_bounds__(kSortBlock) void coo_scatter_kernel(
     if (dst[q] >= 0) out_vals[dst[q]] = s_buf[q * kSortBlock + tid];
 }
 
-// ptr[r] = the number of entries whose row is below r: one binary search per row.
-template <typename R, typename P>
-__global__ __launch_bounds__(kBlock) void coo_rowptr_kernel(const R* __restrict__ rows, int64_t n,
-                                                            int64_t n_rows, P* __restrict__ ptr) {
-  const int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (r > n_rows) return;
-  int64_t lo = 0, hi = n;
+// The number of entries in rows[lo, hi) whose row is below r, plus lo, by one wave: 64 probes at a
+// time, so a search of n entries is log65(n) loads deep instead of log2(n).
+template <typename R>
+__device__ inline int64_t wave_lower_bound(const R* __restrict__ rows, int64_t lo, int64_t hi,
+                                           int64_t r, int lane) {
+  while (lo < hi) {
+    const int64_t step = (hi - lo + 64) / 65;
+    const int64_t probe = lo + (lane + 1) * step - 1;
+    const bool below = probe < hi && (int64_t)rows[probe] < r;
+    const int64_t c = __popcll(__ballot(below));
+    const int64_t end = lo + (c + 1) * step - 1;
+    lo += c * step;
+    if (c < 64 && end < hi) hi = end;  // rows[end] >= r; after 64 probes nothing is known of hi
+  }
+  return lo;
+}
+
+template <typename R>
+__device__ inline int64_t lower_bound(const R* __restrict__ rows, int64_t lo, int64_t hi, int64_t r) {
   while (lo < hi) {
     const int64_t mid = (lo + hi) >> 1;
     if ((int64_t)rows[mid] < r) lo = mid + 1;
     else hi = mid;
   }
-  ptr[r] = (P)lo;
+  return lo;
+}
+
+// ptr[r] = the number of entries whose row is below r: one binary search per row.
+template <typename R, typename P>
+__global__ __launch_bounds__(kBlock) void coo_rowptr_search_kernel(const R* __restrict__ rows,
+                                                                   int64_t n, int64_t n_rows,
+                                                                   P* __restrict__ ptr) {
+  const int64_t r = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (r <= n_rows) ptr[r] = (P)lower_bound(rows, (int64_t)0, n, r);
+}
+
+// The same pointers from one read of the entries.  A workgroup takes 256 pointers: two waves search
+// for the first and the last, then the entries between them are read in order, four to a lane, and
+// each place where the row rises writes the pointers up to the new row.  More than kRowptrScan
+// entries between them (a long row, or rows far above the average) are searched by a thread per
+// pointer instead, so no workgroup reads a long row alone.
+// MI355X, int32, us, a search per row -> this kernel:
+//   33.5M entries in 1M rows     62.7 -> 34.8  (one read at the copy's rate: 27)
+//   the same, power-law lengths  36.0 -> 24.0
+//   2M entries in 2M rows        20.1 -> 17.0
+//   1.2M entries in 150,000 rows  6.0 -> 5.4
+// It is not used where it was slower: below kRowptrScanRows rows a search per row finds its first
+// steps in L2 and the launch is all latency (600,000 entries in 60,000 rows 4.3 against 4.5, 16.8M
+// in 1000 rows 5.3 against 6.3), and with more rows than entries the runs of empty rows are
+// written by the one lane that meets them (400,000 entries in 4M rows 31.6 against 46.6).
+constexpr int64_t kRowptrScan = 64 * kBlock;
+constexpr int64_t kRowptrScanRows = int64_t(1) << 17;
+
+template <typename R, typename P>
+__global__ __launch_bounds__(kBlock) void coo_rowptr_kernel(const R* __restrict__ rows, int64_t n,
+                                                            int64_t n_rows, P* __restrict__ ptr) {
+  __shared__ int64_t s_ends[2];
+  __shared__ int s_at[kBlock];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t r0 = (int64_t)blockIdx.x * kBlock;
+  const int64_t last = r0 + kBlock - 1 < n_rows ? r0 + kBlock - 1 : n_rows;
+  if (wave < 2) {
+    const int64_t e = wave_lower_bound(rows, (int64_t)0, n, wave == 0 ? r0 : last, lane);
+    if (lane == 0) s_ends[wave] = e;
+  }
+  __syncthreads();
+  const int64_t lo = s_ends[0], hi = s_ends[1];
+  const int64_t r = r0 + tid;
+  if (hi - lo > kRowptrScan) {
+    if (r > n_rows) return;
+    ptr[r] = (P)lower_bound(rows, lo, hi, r);
+    return;
+  }
+  s_at[tid] = tid == 0 ? 0 : (int)(hi - lo);
+  __syncthreads();
+  // every entry here lies in a row of [r0, last), so the pointers written are those of (r0, last)
+  for (int64_t p = lo + 4 * tid; p < hi; p += 4 * kBlock) {
+    R row[4];
+    if (p + 4 <= hi) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) row[j] = rows[p + j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) row[j] = rows[p + j < hi ? p + j : hi - 1];
+    }
+    R before = p > lo ? rows[p - 1] : (R)r0;
+    if (before == row[3]) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      // for rows in order r0 <= before <= row < r0 + kBlock; held to that, no write leaves s_at
+      const int from = before < (R)r0 ? 0 : before < (R)last ? (int)(before - (R)r0) : kBlock - 1;
+      const int to = row[j] < (R)r0 ? 0 : row[j] < (R)last ? (int)(row[j] - (R)r0) : kBlock - 1;
+      for (int k = from + 1; k <= to; ++k) s_at[k] = (int)(p + j - lo);
+      before = row[j];
+    }
+  }
+  __syncthreads();
+  if (r <= n_rows) ptr[r] = (P)(lo + s_at[tid]);
+}
+
+template <typename R, typename P>
+int launch_rowptr(const void* rows, int64_t nnz, int64_t n_rows, void* ptr, hipStream_t st) {
+  const dim3 grid((unsigned)(n_rows / kBlock + 1)), block(kBlock);
+  const R* r = static_cast<const R*>(rows);
+  P* p = static_cast<P*>(ptr);
+  if (n_rows >= kRowptrScanRows && nnz >= n_rows)
+    hipLaunchKernelGGL((coo_rowptr_kernel<R, P>), grid, block, 0, st, r, nnz, n_rows, p);
+  else
+    hipLaunchKernelGGL((coo_rowptr_search_kernel<R, P>), grid, block, 0, st, r, nnz, n_rows, p);
+  return check_hip(hipGetLastError(), "coo_rowptr_kernel launch");
 }
 
 struct SortPlan {
@@ -385,18 +482,9 @@ extern "C" int fsp_coo_rowptr(const void* rows, int row_bits, int64_t nnz, int64
     return set_error(FSP_EINVAL, "fsp_coo_rowptr: size out of range");
   if (!ptr || (nnz > 0 && !rows)) return set_error(FSP_EINVAL, "fsp_coo_rowptr: null pointer");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)(n_rows / kBlock + 1)), block(kBlock);
   if (row_bits == 32 && ptr_bits == 32)
-    hipLaunchKernelGGL((coo_rowptr_kernel<int32_t, int32_t>), grid, block, 0, st,
-                       static_cast<const int32_t*>(rows), nnz, n_rows, static_cast<int32_t*>(ptr));
-  else if (row_bits == 32)
-    hipLaunchKernelGGL((coo_rowptr_kernel<int32_t, int64_t>), grid, block, 0, st,
-                       static_cast<const int32_t*>(rows), nnz, n_rows, static_cast<int64_t*>(ptr));
-  else if (ptr_bits == 32)
-    hipLaunchKernelGGL((coo_rowptr_kernel<int64_t, int32_t>), grid, block, 0, st,
-                       static_cast<const int64_t*>(rows), nnz, n_rows, static_cast<int32_t*>(ptr));
-  else
-    hipLaunchKernelGGL((coo_rowptr_kernel<int64_t, int64_t>), grid, block, 0, st,
-                       static_cast<const int64_t*>(rows), nnz, n_rows, static_cast<int64_t*>(ptr));
-  return check_hip(hipGetLastError(), "coo_rowptr_kernel launch");
+    return launch_rowptr<int32_t, int32_t>(rows, nnz, n_rows, ptr, st);
+  if (row_bits == 32) return launch_rowptr<int32_t, int64_t>(rows, nnz, n_rows, ptr, st);
+  if (ptr_bits == 32) return launch_rowptr<int64_t, int32_t>(rows, nnz, n_rows, ptr, st);
+  return launch_rowptr<int64_t, int64_t>(rows, nnz, n_rows, ptr, st);
 }

@@ -61,6 +61,24 @@ def test_row_pointers(dev, monkeypatch, dtype, bits64):
         assert torch.equal(ptr.cpu().to(torch.int64), want)
 
 
+@pytest.mark.parametrize("n_rows", [(1 << 17) - 1, 1 << 17, (1 << 17) + 1, (1 << 17) + 255])
+@pytest.mark.parametrize("lengths", [
+    [1], [65], [0] * 255 + [300], [64] * 256, [64] * 255 + [65], [3] + [0] * 1000, [0] * 511 + [2000],
+    [16384, 0, 1] + [0] * 997, [16385] + [0] * 255 + [3], [5] * 254 + [20000, 7, 0, 0, 2],
+    [150000] + [0] * 200000],
+    ids=lambda v: f"{len(v)}rows_{sum(v)}")
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+def test_row_pointers_blocks(dev, n_rows, lengths, dtype):
+    """Around the rows from which the entries are read once, around 256 pointers and 64 * 256
+    entries of a workgroup, and multiples of the 65 parts that a search step cuts its range into;
+    ``lengths`` is repeated over the rows."""
+    n = torch.tensor((lengths * (n_rows // len(lengths) + 1))[:n_rows])
+    n[-1] += max(0, n_rows - int(n.sum()))  # as many entries as rows, or more
+    row = torch.repeat_interleave(torch.arange(n_rows), n).to(dtype)
+    want = torch.cat([torch.zeros(1, dtype=torch.int64), n.cumsum(0)])
+    assert torch.equal(row_pointers(row.to(dev), n_rows).cpu().to(torch.int64), want)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("index", [torch.int32, torch.int64])
 @pytest.mark.parametrize("order", ["sorted", "rows", "any"])
