@@ -21,7 +21,7 @@ class RowBlockPlan:
     """A descriptor table on the device plus the partial-sum workspace its split rows need."""
 
     __slots__ = ("desc", "desc_host", "ranges", "n_desc", "n_parts", "n_split_rows", "chunk",
-                 "rows_cap", "nnz_cap", "long_threshold", "_workspaces", "_groups")
+                 "rows_cap", "nnz_cap", "long_threshold", "by_column", "_workspaces", "_groups")
 
     def __init__(self, desc, n_parts, n_split_rows, chunk, rows_cap, nnz_cap, long_threshold,
                  desc_host=None, ranges=None, groups=None):
@@ -35,6 +35,7 @@ class RowBlockPlan:
         self.rows_cap = int(rows_cap)
         self.nnz_cap = int(nnz_cap)
         self.long_threshold = int(long_threshold)
+        self.by_column = False  # desc in a launch order of its own (spmm_csr.py)
         self._workspaces = {}
         self._groups = groups
 

@@ -6,9 +6,12 @@ Public API and error behaviour mirror ``src/flagsparse/sparse_operations/spmm_cs
 precision), the validation metrics (:6-90, :1186-1192) and the benchmark cases
 (:1195-1562).
 
-Both paths run ``spmm_rowblock_kernel`` (flagsparse_amd/csrc/spmm.hip): G lanes share each
-B row with 16-byte loads along N, short rows are one row per lane group, rows longer than
-128 entries are cut into parts whose sums are added in part order (deterministic).
+Two kernels, both with G lanes sharing each B row by 16-byte loads along N:
+``spmm_rowblock_kernel`` (flagsparse_amd/csrc/spmm.hip) for prepared matrices whose rows are all
+short (at most 128 entries), one row per lane group over a planned table, or so long that the
+order of additions shows (over 8192); ``spmm_slices_kernel``
+(csrc/spmm_slices.hip) for everything else: slices of equal work found by a search in the row
+pointers, the pieces of a cut row added in slice order (deterministic).
 """
 
 import time
@@ -310,6 +313,36 @@ def _spmm_slice_shape(lanes, positions, by_column=False):
     return items, 256 if items >= 128 else 128
 
 
+# Sums of more than this many products depend visibly on the order of addition: in float32 two
+# orders differ by up to 4.6e-5 of the result's root mean square (200k rows of power-law lengths,
+# N = 47), against 1e-6 below.  Prepared products on such rows keep the order of the row-block
+# kernel, 128-entry parts added one after another, bit for bit, and change only the launch order
+# of the parts (slices would take 55 / 119 / 211 us where that takes 64 / 279 / 302: fp32, N = 16 / 47
+# / 128).
+_SPMM_SUMS_KEPT = 8192
+
+
+def _xcd_places(n, device):
+    """Which of n items in order each launch slot takes, so that each of the 8 XCDs (slot mod 8)
+    gets one contiguous eighth of them."""
+    slot = torch.arange(n, device=device)
+    x = slot % 8
+    return x * (n // 8) + torch.clamp(x, max=n % 8) + slot // 8
+
+
+def _parts_by_column(desc, cols, rowptr, chunk):
+    """The descriptor table in launch order: row blocks as they are, then the parts of long rows
+    by the first column they hold, each XCD a contiguous eighth of either.  Parts of different
+    rows over the same columns then read the same rows of B while they are in that XCD's L2.
+    Measured on MI355X, us, in row order / in this order: 200k rows of power-law lengths, fp32
+    N=16 92 / 64, N=47 320 / 279, N=128 468 / 302; fp64 N=33 402 / 368, N=64 462 / 331."""
+    part = desc[:, 2] > 0
+    blocks, parts = desc[~part], desc[part]
+    first = rowptr[parts[:, 0].long()].long() + parts[:, 1].long() * chunk
+    parts = parts[torch.argsort(cols[first], stable=True)]
+    return torch.cat([t[_xcd_places(int(t.shape[0]), t.device)] for t in (blocks, parts)])
+
+
 class _SpmmKernelCsr:
     """Kernel-facing CSR arrays (aligned, int32 offsets when they fit), their row-block plans per
     G and their slices.  max_row_nnz: the longest row, where known; one_shot: the object serves
@@ -336,10 +369,11 @@ class _SpmmKernelCsr:
         self._order = StreamOrder(self.data.device)
 
     def kernel_name(self):
-        return "spmm_rowblock_kernel"
+        return "spmm_rowblock_kernel" if self._plans or not self.sliced() \
+            else "spmm_slices_kernel"
 
     def describe(self):
-        return {"layout": "rowblock", "plans": {g: {"descriptors": p.n_desc,
+        return {"layout": "rowblock" if self._plans or not self.sliced() else "slices", "plans": {g: {"descriptors": p.n_desc,
                                                     "split_rows": p.n_split_rows}
                                                 for g, p in self._plans.items()},
                 "slices": {k[0]: int(t[0].numel()) // 2 - 1 for k, t in self._tables.items()}}
@@ -349,10 +383,11 @@ class _SpmmKernelCsr:
         the faster: prepared, every row one group's work (and, in _run_spmm, N, B and C whole
         vectors).  Measured on MI355X, row blocks / slices: fp32 N=16, 100k rows of 0 to 32
         entries 18.4 / 20.8 us; N=33, 3M entries 80.6 / 53.0; a power law, N=128 457 / 316, N=47
-        326 / 214.  A matrix used once has no plan to use."""
+        326 / 214.  A matrix used once has no plan to use.  A prepared one with rows of more than
+        _SPMM_SUMS_KEPT entries keeps the row blocks' order of additions (see there)."""
         if self.one_shot or self.max_row_nnz is None:
             return True
-        return self.max_row_nnz > _SPMM_ROW_SPLIT_THRESHOLD
+        return _SPMM_ROW_SPLIT_THRESHOLD < self.max_row_nnz <= _SPMM_SUMS_KEPT
 
     def slices(self, items, keep, n_cols, by_column):
         """The slices' boundaries and launch order (built on the current stream, once)."""
@@ -364,7 +399,7 @@ class _SpmmKernelCsr:
             self._tables[key] = t
         return t
 
-    def plan(self, lanes):
+    def plan(self, lanes, row_bytes=0, n_cols=0):
         p = self._plans.get(lanes)
         if p is None:
             ngrp = 256 // lanes
@@ -373,6 +408,10 @@ class _SpmmKernelCsr:
             chunk = min(cap, max(threshold, 16 * ngrp))
             p = build_row_block_plan_device(self.rowptr, cap, ngrp, threshold, chunk,
                                             window_rows=SPMM_PLAN_WINDOW_BLOCKS * ngrp)
+            p.by_column = _slices.ordered(self.max_row_nnz, chunk, n_cols * row_bytes,
+                                          self.nnz * row_bytes, False)
+            if p.by_column:
+                p.desc = _parts_by_column(p.desc, self.cols, self.rowptr, chunk)
             self._plans[lanes] = p
         return p
 
@@ -425,7 +464,7 @@ def _bind_sliced(kc, B, C, acc_f64, lanes, vec):
 
 def _bind_row_blocks(kc, B, acc_f64, lanes, vec):
     n_dense_cols = int(B.shape[1])
-    plan = kc.plan(lanes)
+    plan = kc.plan(lanes, min(n_dense_cols, lanes * vec) * B.element_size(), int(B.shape[0]))
     partials = plan.workspace(n_dense_cols)
     groups, group_base, split_rows = plan.split_groups()
     p = lambda t: t.data_ptr() if t.numel() else None  # noqa: E731
@@ -434,7 +473,7 @@ def _bind_row_blocks(kc, B, acc_f64, lanes, vec):
         "spmm_csr", _abi.dtype_code(B.dtype), 1 if acc_f64 else 0, p(kc.data), p(kc.cols),
         p(kc.rowptr), kc.rowptr_bits, kc.n_rows, kc.nnz, n_dense_cols, p(plan.desc), plan.n_desc,
         plan.chunk, lanes, vec, p(partials), p(groups), p(group_base), p(split_rows),
-        int(groups.shape[0]), XCD_REMAP)
+        int(groups.shape[0]), 0 if plan.by_column else XCD_REMAP)
 
 
 def _run_spmm(kc, B, C, acc_f64, tile_cols=None):
@@ -454,7 +493,9 @@ def _run_spmm(kc, B, C, acc_f64, tile_cols=None):
     if bound is None:
         slice_lanes, slice_vec = _spmm_slice_lanes(n_dense_cols, B.dtype, tile_cols)
         lanes, vec = _spmm_lane_shape(n_dense_cols, B.dtype, B, C, tile_cols)
-        if kc.sliced() or vec < slice_vec:  # the row-block kernel's loads need aligned vectors
+        kept = not kc.one_shot and (kc.max_row_nnz or 0) > _SPMM_SUMS_KEPT
+        # the row-block kernel's loads need aligned vectors
+        if kc.sliced() or (vec < slice_vec and not kept):
             bound = _bind_sliced(kc, B, C, acc_f64, slice_lanes, slice_vec)
         else:
             bound = _bind_row_blocks(kc, B, acc_f64, lanes, vec)

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import flagsparse_amd as fs
-from flagsparse_amd import _common, spmm_csr, synthetic
+from flagsparse_amd import _common, _slices, spmm_csr, synthetic
 from oracle import oracle
 
 pytestmark = pytest.mark.gpu
@@ -158,3 +158,27 @@ def test_unknown_longest_row(dev, monkeypatch):
         assert (kc.max_row_nnz > 256) == cut and (kc._keep[-1] is not None) == cut
         monkeypatch.undo()
         assert oracle.rel_l2(C, oracle.spmm_csr(ip, cols, vals, B)) <= 1e-5
+
+
+@pytest.mark.parametrize("n", [1, 16, 47, 64])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_long_rows_keep_their_order_of_additions(dev, monkeypatch, n, dtype):
+    """Over 8192 entries in a row: row blocks, whose parts in column order give the same bits as in
+    row order."""
+    lengths = torch.tensor([3, 0, 9000, 127, 128, 129, 40] * 20 + [20000, 1])
+    ptr = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
+    cols = torch.cat([torch.sort(synthetic.randint(7, k, int(m), 60000, "cpu")).values
+                      for k, m in enumerate(lengths)]).to(torch.int32)
+    data = (torch.arange(cols.numel()) % 17 - 8).to(dtype) / 7
+    B = ((torch.arange(60000 * n) % 1013).to(dtype) / 1013 - 0.5).reshape(60000, n)
+    shape = (lengths.numel(), 60000)
+    out = []
+    for order in (True, False):
+        monkeypatch.setattr(_slices, "ordered", lambda *a: order)
+        p = fs.prepare_spmm_csr_opt(data.to(dev), cols.to(dev), ptr.to(dev), shape)
+        out.append(fs.flagsparse_spmm_csr_opt(B=B.to(dev), prepared=p).cpu())
+        assert p._kernel_csr().kernel_name() == "spmm_rowblock_kernel"
+        assert all(q.by_column == order for q in p._kernel_csr()._plans.values())
+    assert torch.equal(out[0], out[1])
+    ref = oracle.spmm_csr(ptr, cols, data, B)
+    assert oracle.rel_l2(out[0], ref) <= oracle.REL_L2_BOUND[str(dtype)[6:]]
