@@ -91,8 +91,8 @@ WORKLOADS = {
     "cfg5": "CSR SpMM A 1M x 1M, 32 nnz/row (16 in a 512-wide band + 16 uniform), B row-major "
             "1M x N, int32, U(-1,1)",
     "coo5": "COO SpMM: cfg5's matrix as row-sorted COO (int32 row/col), B row-major 1M x N, "
-            "through flagsparse_spmm_coo (per-call row-order check, bincount row pointer and "
-            "plan inside the step, as the reference's per-call coalesce/sort)",
+            "through flagsparse_spmm_coo (per-call index and row-order checks, row pointer and "
+            "slices inside the step, as the reference's per-call coalesce/sort)",
     "sddmm": "CSR SDDMM on cfg5's pattern (1M x 1M, 32 nnz/row), x [1M, K] and y [1M, K] "
              "row-major ~U(-1,1), alpha 1, beta 0, fp32 accumulation (the reference's baseline)",
     "copy": "plain device copy of 1 GiB (PMC calibration kernel)",

@@ -1,5 +1,6 @@
-"""Index checks of the per-call COO paths in one device pass (fsp_index_stats in
-csrc/index_stats.hip): the bounds of two index arrays and whether the first is in order."""
+"""Bounds of two index arrays and whether the first is in order, in one device pass
+(fsp_index_stats in csrc/index_stats.hip).  The package's own calls check their indices with
+_csr_check.py, which also narrows them; this is the C library's general form."""
 
 import torch
 

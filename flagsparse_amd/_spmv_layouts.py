@@ -39,7 +39,7 @@ The layouts below, chosen once per matrix at prepare time:
     staged x, placed in LDS in (row, panel) order, and each row's products summed in that
     fixed order (deterministic), beside the long rows' partial sums.
 
-Both replace the reference's per-bucket launches (spmv_csr.py:281-376) and produce the same
+All replace the reference's per-bucket launches (spmv_csr.py:281-376) and produce the same
 row sums up to floating-point summation order.
 """
 

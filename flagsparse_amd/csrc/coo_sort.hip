@@ -17,9 +17,9 @@
 //                       counters per wave keep the order), puts them in digit order in LDS and
 //                       writes runs of equal digits to their places
 // Bound: the entries' bytes, read and written once a pass, and at these sizes the launches.
-// Measured there: 59 us for the 1.65M float64 entries (histograms 12, scans 8, scatters 39, 2.7
-// TB/s of what they read and write) and 51 us for the 1.2M float32 ones; the whole SpMV call 1551
-// -> 119 us, the SpMM call of N = 32 452 -> 117 us.
+// Measured there: 57 us for the 1.65M float64 entries (histograms 11, scans 8, scatters 37, 2.8
+// TB/s of what they read and write) and 47 us for the 1.2M float32 ones; the whole SpMV call 1551
+// -> 111 us, the SpMM call of N = 32 452 -> 111 us.
 #include "fsp_device.hpp"
 #include "fsp_internal.hpp"
 

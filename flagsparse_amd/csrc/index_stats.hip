@@ -2,7 +2,9 @@
 // maximum of each and the number of places where the first one decreases.  The validation of
 // a COO call needs exactly these (indices in range, int32-representable, rows already in
 // order); as separate torch reductions they were four passes plus a fifth for the order, each
-// reading the arrays again (cfg5-shape COO SpMM: 226 us of a 1.2 ms call).
+// reading the arrays again (226 us of a 1.2 ms COO SpMM call on 33.5M entries).  The package's
+// calls now take these with the narrowed indices from one launch (check.hip); this entry point is
+// for callers that want the bounds alone.
 //
 // Reference behaviour replaced: the per-call checks of spmm_coo.py:312-371
 // (_prepare_spmm_coo_inputs: min/max of row and col) and the sortedness test that decides

@@ -1,6 +1,6 @@
-// Row-block plans built on the device, for the paths that plan on every call (CSR SpMM
-// without a prepared object, COO SpMM) and for the SpMM prepare step: no copy of the row
-// pointers to the host and no host loop over rows.
+// Row-block plans built on the device, for the prepare steps of SpMV and SpMM: no copy of the row
+// pointers to the host and no host loop over rows.  (Calls without a prepared object need no plan:
+// they run on slices, slices.hip.)
 //
 // The rows are cut into windows of window_rows rows.  One thread plans its window with the
 // rules of the host planner fsp_plan_row_blocks (abi.cpp): a block takes at most rows_cap

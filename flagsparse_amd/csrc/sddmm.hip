@@ -10,6 +10,9 @@
 // G lanes share one entry, each holding VW consecutive elements (16-byte loads for VW = 4 fp32
 // / 2 fp64) of the x row and the y row, so a group covers G*VW elements of K per step.
 //
+// The package runs K <= 4*64*VW on slices (sddmm_slices.hip) and larger K on the flat kernel; the
+// row-block kernel serves callers of the C entry point that hold a plan.
+//
 // sddmm_rowblock_kernel (K <= 4*G*VW): one launch over a row-block plan.  A workgroup stages
 // its entries' columns into LDS with 16-byte loads; in a short-row block each lane group owns
 // one row, keeps that row of x in registers (loaded once) and walks the row's entries four at

@@ -5,8 +5,9 @@ Public API mirrors ``src/flagsparse/sparse_operations/spmv_coo.py``: ``PreparedC
 
 * ``sort_by_row=True``: entries sorted by (row, col) (skipped when already sorted), constant-row
   runs ``seg_starts`` (:167-179); one sum per run, rows without a run are 0.  The runs are fed
-  to the same row-block kernel as CSR SpMV with a run -> row map (identity, and then omitted,
-  when every row has entries).
+  to the same kernels as CSR SpMV with a run -> row map (identity, and then omitted, when every
+  row has entries).  A call without a prepared object puts the entries in row order only
+  (_coo_order.py) and runs the slices of CSR SpMV over all rows.
 * ``sort_by_row=False``: one atomic add per entry into a zeroed y (:111-150); the summation
   order, and so the last bits of y, vary from call to call, as in the reference.
 """

@@ -10,8 +10,9 @@ as the reference's base path does (:498-536); ``use_opt=True`` accumulates in th
 (:161-279).  float64 always accumulates in float64.  A caller's ``max_segments`` truncates
 rows exactly where the reference's static tile loop stops (:111-118 base, :308-314 opt).
 
-The kernel is one launch over a layout built once per matrix (flagsparse_amd/_spmv_layouts.py):
-row blocks (csrc/spmv.hip) or, when x gathers would miss L2, the XCD column split
+The kernels run over a layout built once per matrix (flagsparse_amd/_spmv_layouts.py): row blocks
+(csrc/spmv.hip); slices of equal work (csrc/slices.hip) where rows are longer than a row block or
+the matrix serves one call; or, when x gathers would miss L2, the staged-x layout
 (csrc/spmv_xcs.hip).
 """
 

@@ -16,7 +16,7 @@
  *                          per-bucket row lists.
  *   fsp_plan_windows_count / fsp_plan_windows_emit
  *                        - the same planning on the device (spmm_csr.py:417-477, the host
- *                          Python loop over long rows included), for per-call plans.
+ *                          Python loop over long rows included).
  *   fsp_spmv_csr         - the Triton launches of spmv_csr.py:329-376
  *                          (_triton_spmv_csr_impl_opt_prepared, use_opt=True) and
  *                          spmv_csr.py:510-536 (_triton_spmv_csr_impl_prepared, default
@@ -44,6 +44,15 @@
  *   fsp_spmm_coo_atomic  - spmm_coo.py:464-523 (_triton_spmm_coo_atomic_impl).
  *   fsp_sddmm_csr        - sddmm_csr.py:107-151 (_sddmm_csr_real_kernel) and its launch in
  *                          _run_sddmm_prepared (:271-347).
+ *   fsp_spmv_sliced, fsp_spmm_sliced, fsp_sddmm_sliced
+ *                        - the launches of fsp_spmv_csr, fsp_spmm_csr and fsp_sddmm_csr over slices
+ *                          of equal rows + entries (fsp_slice_table) instead of a planned table.
+ *   fsp_csr_check, fsp_coo_check
+ *                        - the per-call checks of spmv_csr.py:379-436, spmm_csr.py:197-255,
+ *                          sddmm_csr.py:46-79 and spmm_coo.py:312-371, with the narrowed indices.
+ *   fsp_coo_sort_rows, fsp_coo_rowptr
+ *                        - the sorts of spmv_coo.py:153-164 and spmm_coo.py:136-180 before a
+ *                          product, by row alone.
  *   fsp_index_stats      - the per-call index checks of spmm_coo.py:312-371 (min/max of row
  *                          and col) and the row-order test of the row-run route (:394-461).
  *   fsp_mtx_read         - the .mtx parsing of the reference's test loaders
