@@ -317,7 +317,7 @@ def _spmm_slice_shape(lanes, positions, by_column=False):
 # orders differ by up to 4.6e-5 of the result's root mean square (200k rows of power-law lengths,
 # N = 47), against 1e-6 below.  Prepared products on such rows keep the order of the row-block
 # kernel, 128-entry parts added one after another, bit for bit, and change only the launch order
-# of the parts (slices would take 55 / 119 / 211 us where that takes 64 / 279 / 302: fp32, N = 16 / 47
+# of the parts (slices would take 56 / 119 / 207 us where that takes 61 / 195 / 219: fp32, N = 16 / 47
 # / 128).
 _SPMM_SUMS_KEPT = 8192
 
@@ -335,7 +335,7 @@ def _parts_by_column(desc, cols, rowptr, chunk):
     by the first column they hold, each XCD a contiguous eighth of either.  Parts of different
     rows over the same columns then read the same rows of B while they are in that XCD's L2.
     Measured on MI355X, us, in row order / in this order: 200k rows of power-law lengths, fp32
-    N=16 92 / 64, N=47 320 / 279, N=128 468 / 302; fp64 N=33 402 / 368, N=64 462 / 331."""
+    N=16 86 / 61, N=47 238 / 195, N=128 382 / 219; fp64 N=33 316 / 287, N=64 376 / 246."""
     part = desc[:, 2] > 0
     blocks, parts = desc[~part], desc[part]
     first = rowptr[parts[:, 0].long()].long() + parts[:, 1].long() * chunk
