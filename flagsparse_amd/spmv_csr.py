@@ -278,6 +278,8 @@ def _prepare_spmv_csr(data, indices, indptr, shape, block_nnz, max_segments, one
     prepared._one_shot = bool(one_shot)
     if prepared.supports_opt and n_rows > 0 and not one_shot:
         prepared._kernel(False)  # build the descriptor table now, outside the timed calls
+    if not one_shot:  # the narrowed copies may be read on other streams than this one
+        torch.cuda.current_stream(data.device).synchronize()
     return prepared
 
 

@@ -83,6 +83,19 @@ def test_prepared_layout(dev, name, kind):
         assert torch.equal(one, y)
 
 
+def test_prepare_leaves_nothing_queued(dev):
+    """A prepared matrix's narrowed copies may be read on any stream, by what orders nothing
+    (rows truncated later, the row lengths), so prepare waits for the stream that wrote them."""
+    d, c, ip = (t.to(dev) for t in _csr([5000] + [12] * 300000, 100000, 5, torch.float32))
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream(dev)
+    with torch.cuda.stream(side):
+        prepared = fs.prepare_spmv_csr(d, c, ip, (300001, 100000))
+        done = side.query()
+    assert done
+    assert prepared._kernel(False).kind == "slices"
+
+
 def test_sliced_spmv_nonfinite(dev):
     # an infinity and a NaN of x reach the rows that name them and no others
     vals, cols, ip = _csr(LENGTHS["crossing"], 3001, 6, torch.float32)
