@@ -77,6 +77,7 @@ SIGNATURES = {
     "fsp_slice_table": (_i32, [_p, _i32, _i64, _i64, _i64, _i64, _p, _p]),
     "fsp_slice_order_scratch": (_i64, [_i64]),
     "fsp_slice_order": (_i32, [_p, _i64, _p, _i64, _p, _p, _p]),
+    "fsp_part_order": (_i32, [_p, _i64, _p, _i32, _i64, _p, _i64, _p, _p, _p]),
     "fsp_spmm_sliced": (_i32, [_i32, _i32, _p, _p, _p, _i32, _i64, _i64, _p, _i64, _i64, _p, _i64,
                                _p, _p, _i64, _i64, _p, _i32, _i32, _i32, _i32, _p]),
     "fsp_coo_sort_max_nnz": (_i64, []),

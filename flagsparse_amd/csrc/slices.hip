@@ -96,24 +96,53 @@ constexpr int kBins = 256;  // bin 0: not inside one row
 // for the three launches instead of 14), more where the counts would make the scan long.
 int64_t order_tile(int64_t n) { return n <= (1 << 14) ? kBlock : 4 * kBlock; }
 
-__device__ __forceinline__ int order_bin(const int64_t* table, int64_t k, const int* cols,
-                                         int64_t n_cols) {
-  const int64_t i0 = table[2 * k], p0 = table[2 * k + 1];
-  if (table[2 * k + 2] != i0 || table[2 * k + 3] <= p0) return 0;
-  const int64_t b = (int64_t)cols[p0] * (kBins - 1) / n_cols;
+__device__ __forceinline__ int column_bin(int col, int64_t n_cols) {
+  const int64_t b = (int64_t)col * (kBins - 1) / n_cols;
   return 1 + (int)(b < 0 ? 0 : b > kBins - 2 ? kBins - 2 : b);
 }
 
-__global__ __launch_bounds__(kBlock) void order_hist_kernel(const int64_t* __restrict__ table,
-                                                            int64_t n, const int* __restrict__ cols,
-                                                            int64_t n_cols, int tile, int n_tiles,
+// What is ordered: slices (the order is of their numbers) ...
+struct Slices {
+  const int64_t* table;
+  const int* cols;
+  int64_t n_cols;
+  int* order;
+  __device__ __forceinline__ int bin(int64_t k) const {
+    const int64_t i0 = table[2 * k], p0 = table[2 * k + 1];
+    if (table[2 * k + 2] != i0 || table[2 * k + 3] <= p0) return 0;
+    return column_bin(cols[p0], n_cols);
+  }
+  __device__ __forceinline__ void put(int64_t slot, int64_t k) const { order[slot] = (int)k; }
+};
+
+// ... or a row-block plan's descriptors {first row, .., 0, ..} and {long row, part, parts, ..},
+// of which the parts go by column (moved themselves: out must be another array).
+template <typename P>
+struct Descriptors {
+  const i32x4* desc;
+  const P* rowptr;
+  int64_t chunk;
+  const int* cols;
+  int64_t n_cols;
+  i32x4* out;
+  __device__ __forceinline__ int bin(int64_t k) const {
+    const i32x4 d = desc[k];
+    if (d.z <= 0) return 0;
+    return column_bin(cols[(int64_t)rowptr[d.x] + d.y * chunk], n_cols);
+  }
+  __device__ __forceinline__ void put(int64_t slot, int64_t k) const { out[slot] = desc[k]; }
+};
+
+template <typename S>
+__global__ __launch_bounds__(kBlock) void order_hist_kernel(S what, int64_t n, int tile,
+                                                            int n_tiles,
                                                             int* __restrict__ counts) {
   __shared__ int s_cnt[kBins];
   s_cnt[threadIdx.x] = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < tile; i += kBlock) {
     const int64_t k = (int64_t)blockIdx.x * tile + i;
-    if (k < n) atomicAdd(&s_cnt[order_bin(table, k, cols, n_cols)], 1);
+    if (k < n) atomicAdd(&s_cnt[what.bin(k)], 1);
   }
   __syncthreads();
   counts[(int64_t)threadIdx.x * n_tiles + blockIdx.x] = s_cnt[threadIdx.x];
@@ -167,9 +196,10 @@ __device__ __forceinline__ int64_t xcd_slot(int64_t p, int64_t q) {
   return 8 * j + x;
 }
 
-__global__ __launch_bounds__(kBlock) void order_scatter_kernel(
-    const int64_t* __restrict__ table, int64_t n, const int* __restrict__ cols, int64_t n_cols,
-    int tile, int n_tiles, const int* __restrict__ places, int* __restrict__ order) {
+template <typename S>
+__global__ __launch_bounds__(kBlock) void order_scatter_kernel(S what, int64_t n, int tile,
+                                                               int n_tiles,
+                                                               const int* __restrict__ places) {
   __shared__ int s_cnt[kBins];
   s_cnt[threadIdx.x] = places[(int64_t)threadIdx.x * n_tiles + blockIdx.x];
   __syncthreads();
@@ -177,12 +207,29 @@ __global__ __launch_bounds__(kBlock) void order_scatter_kernel(
   for (int i = threadIdx.x; i < tile; i += kBlock) {
     const int64_t k = (int64_t)blockIdx.x * tile + i;
     if (k < n) {
-      const int64_t p = atomicAdd(&s_cnt[order_bin(table, k, cols, n_cols)], 1);
+      const int64_t p = atomicAdd(&s_cnt[what.bin(k)], 1);
       const int64_t slot = p < others ? xcd_slot(p, others)
                                       : others + xcd_slot(p - others, n - others);
-      order[slot] = (int)k;
+      what.put(slot, k);
     }
   }
+}
+
+template <typename S>
+int launch_order(const S& what, int64_t n, int32_t* scratch, hipStream_t st) {
+  const int tile = (int)order_tile(n);
+  const int tiles = (int)((n + tile - 1) / tile);
+  hipLaunchKernelGGL((order_hist_kernel<S>), dim3((unsigned)tiles), dim3(kBlock), 0, st, what, n,
+                     tile, tiles, scratch);
+  int rc = check_hip(hipGetLastError(), "order_hist_kernel launch");
+  if (rc) return rc;
+  hipLaunchKernelGGL(order_scan_kernel, dim3(1), dim3(1024), 0, st, scratch,
+                     (int64_t)kBins * tiles);
+  rc = check_hip(hipGetLastError(), "order_scan_kernel launch");
+  if (rc) return rc;
+  hipLaunchKernelGGL((order_scatter_kernel<S>), dim3((unsigned)tiles), dim3(kBlock), 0, st, what,
+                     n, tile, tiles, scratch);
+  return check_hip(hipGetLastError(), "order_scatter_kernel launch");
 }
 
 template <typename T, typename A, typename P>
@@ -370,20 +417,31 @@ extern "C" int fsp_slice_order(const int64_t* table, int64_t n_slices, const int
   if (n_slices == 0) return FSP_OK;
   if (!table || !cols || !order || !scratch)
     return set_error(FSP_EINVAL, "fsp_slice_order: null pointer");
+  return launch_order(Slices{table, cols, n_cols, order}, n_slices, scratch,
+                      static_cast<hipStream_t>(stream));
+}
+
+extern "C" int fsp_part_order(const int32_t* desc, int64_t n_desc, const void* rowptr,
+                              int rowptr_bits, int64_t chunk, const int32_t* cols, int64_t n_cols,
+                              int32_t* out, int32_t* scratch, void* stream) {
+  if (rowptr_bits != 32 && rowptr_bits != 64)
+    return set_error(FSP_EINVAL, "fsp_part_order: rowptr_bits must be 32 or 64");
+  if (n_desc < 0 || n_desc > 0x7fffffffLL || n_cols < 1 || chunk < 1)
+    return set_error(FSP_EINVAL, "fsp_part_order: size out of range");
+  if (n_desc == 0) return FSP_OK;
+  if (!desc || !rowptr || !cols || !out || !scratch || desc == out)
+    return set_error(FSP_EINVAL, "fsp_part_order: null pointer, or out is desc");
+  if (!aligned16(desc) || !aligned16(out))
+    return set_error(FSP_EINVAL, "fsp_part_order: desc and out must be 16-byte aligned");
+  const i32x4* d = reinterpret_cast<const i32x4*>(desc);
+  i32x4* o = reinterpret_cast<i32x4*>(out);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int tile = (int)order_tile(n_slices);
-  const int tiles = (int)((n_slices + tile - 1) / tile);
-  hipLaunchKernelGGL(order_hist_kernel, dim3((unsigned)tiles), dim3(kBlock), 0, st, table,
-                     n_slices, cols, n_cols, tile, tiles, scratch);
-  int rc = check_hip(hipGetLastError(), "order_hist_kernel launch");
-  if (rc) return rc;
-  hipLaunchKernelGGL(order_scan_kernel, dim3(1), dim3(1024), 0, st, scratch,
-                     (int64_t)kBins * tiles);
-  rc = check_hip(hipGetLastError(), "order_scan_kernel launch");
-  if (rc) return rc;
-  hipLaunchKernelGGL(order_scatter_kernel, dim3((unsigned)tiles), dim3(kBlock), 0, st, table,
-                     n_slices, cols, n_cols, tile, tiles, scratch, order);
-  return check_hip(hipGetLastError(), "order_scatter_kernel launch");
+  if (rowptr_bits == 32)
+    return launch_order(Descriptors<int>{d, static_cast<const int*>(rowptr), chunk, cols, n_cols, o},
+                        n_desc, scratch, st);
+  return launch_order(
+      Descriptors<int64_t>{d, static_cast<const int64_t*>(rowptr), chunk, cols, n_cols, o}, n_desc,
+      scratch, st);
 }
 
 extern "C" int64_t fsp_spmv_slices(int64_t n_rows, int64_t nnz) {

@@ -322,25 +322,23 @@ def _spmm_slice_shape(lanes, positions, by_column=False):
 _SPMM_SUMS_KEPT = 8192
 
 
-def _xcd_places(n, device):
-    """Which of n items in order each launch slot takes, so that each of the 8 XCDs (slot mod 8)
-    gets one contiguous eighth of them."""
-    slot = torch.arange(n, device=device)
-    x = slot % 8
-    return x * (n // 8) + torch.clamp(x, max=n % 8) + slot // 8
-
-
-def _parts_by_column(desc, cols, rowptr, chunk):
+def _parts_by_column(desc, cols, n_cols, rowptr, chunk):
     """The descriptor table in launch order: row blocks as they are, then the parts of long rows
     by the first column they hold, each XCD a contiguous eighth of either.  Parts of different
     rows over the same columns then read the same rows of B while they are in that XCD's L2.
     Measured on MI355X, us, in row order / in this order: 200k rows of power-law lengths, fp32
-    N=16 86 / 61, N=47 238 / 195, N=128 382 / 219; fp64 N=33 316 / 287, N=64 376 / 246."""
-    part = desc[:, 2] > 0
-    blocks, parts = desc[~part], desc[part]
-    first = rowptr[parts[:, 0].long()].long() + parts[:, 1].long() * chunk
-    parts = parts[torch.argsort(cols[first], stable=True)]
-    return torch.cat([t[_xcd_places(int(t.shape[0]), t.device)] for t in (blocks, parts)])
+    N=16 86 / 61, N=47 238 / 195, N=128 382 / 219; fp64 N=33 316 / 287, N=64 376 / 246.  Ordered
+    by 256 column bins in three launches (csrc/slices.hip): a full sort and gathers by torch took
+    0.34 ms more of a matrix's first product (N=47: 815 / 479 us) for the same 195 us after it."""
+    L = _abi.lib()
+    n, dev = int(desc.shape[0]), desc.device
+    out = torch.empty_like(desc)
+    scratch = torch.empty(int(L.fsp_slice_order_scratch(n)), dtype=torch.int32, device=dev)
+    _abi.check(L.fsp_part_order(desc.data_ptr(), n, rowptr.data_ptr(),
+                                32 if rowptr.dtype == torch.int32 else 64, chunk, cols.data_ptr(),
+                                n_cols, out.data_ptr(), scratch.data_ptr(), _abi.raw_stream(dev)),
+               "fsp_part_order")
+    return out
 
 
 class _SpmmKernelCsr:
@@ -411,7 +409,7 @@ class _SpmmKernelCsr:
             p.by_column = _slices.ordered(self.max_row_nnz, chunk, n_cols * row_bytes,
                                           self.nnz * row_bytes, False)
             if p.by_column:
-                p.desc = _parts_by_column(p.desc, self.cols, self.rowptr, chunk)
+                p.desc = _parts_by_column(p.desc, self.cols, n_cols, self.rowptr, chunk)
             self._plans[lanes] = p
         return p
 

@@ -467,6 +467,16 @@ int fsp_slice_order(const int64_t* table, int64_t n_slices, const int32_t* cols,
                     int32_t* order, int32_t* scratch, void* stream);
 
 /*
+ * The same for a row-block plan's descriptors: out (n_desc quadruples, not desc itself) holds the
+ * row blocks, then the parts of long rows by the column they start at.  chunk: entries per part, as
+ * the plan was made with; scratch: fsp_slice_order_scratch(n_desc) int32.  desc and out 16-byte
+ * aligned.
+ */
+int fsp_part_order(const int32_t* desc, int64_t n_desc, const void* rowptr, int rowptr_bits,
+                   int64_t chunk, const int32_t* cols, int64_t n_cols, int32_t* out,
+                   int32_t* scratch, void* stream);
+
+/*
  * C[n_rows, N] = A @ B over the slices of fsp_slice_table, otherwise as fsp_spmm_csr.
  *   table, items, keep  the slices' boundaries and what they were built with; items + keep <=
  *                  2042

@@ -182,3 +182,27 @@ def test_long_rows_keep_their_order_of_additions(dev, monkeypatch, n, dtype):
     assert torch.equal(out[0], out[1])
     ref = oracle.spmm_csr(ptr, cols, data, B)
     assert oracle.rel_l2(out[0], ref) <= oracle.REL_L2_BOUND[str(dtype)[6:]]
+
+
+@pytest.mark.parametrize("ptr", [torch.int32, torch.int64])
+@pytest.mark.parametrize("lengths", [[9000], [3, 0, 5], [3, 9000, 0, 300] * 9 + [1],
+                                     [1] * 40 + [2000] * 1100])
+def test_part_order(dev, ptr, lengths):
+    """A permutation of the plan's descriptors: the row blocks first, then the parts, by column
+    within each XCD's share."""
+    lengths = torch.tensor(lengths)
+    rowptr = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)]).to(ptr).to(dev)
+    nnz, n_cols = int(lengths.sum()), 40000
+    cols = synthetic.randint(3, 1, nnz, n_cols, "cpu").to(torch.int32)
+    plan = spmm_csr.build_row_block_plan_device(rowptr, 1024, 16, 128, 256, window_rows=256)
+    out = spmm_csr._parts_by_column(plan.desc, cols.to(dev), n_cols, rowptr, 256).cpu().long()
+    desc = plan.desc.cpu().long()
+    key = lambda t: (t[:, 0] << 32) + (t[:, 1] << 1) + (t[:, 2] > 0)  # noqa: E731
+    assert torch.equal(key(out).sort().values, key(desc).sort().values)
+    part = out[:, 2] > 0
+    n = int((~part).sum())
+    assert not bool(part[:n].any()) and bool(part[n:].all())
+    first = rowptr.cpu().long()[out[n:, 0]] + out[n:, 1] * 256
+    k = cols[first].long() * 255 // n_cols
+    for x in range(8):
+        assert bool((k[x::8][1:] >= k[x::8][:-1]).all())
