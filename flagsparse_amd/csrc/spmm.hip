@@ -80,6 +80,38 @@ constexpr int spmm_scratch_bytes() {
                                                                    : kBlock * VW * (int)sizeof(A);
 }
 
+// B rows requested together per lane of a long row's part, and before kRowsInFlight of a short
+// row where they are 16.  With single elements a lane's chain of requests is what bounds both: a
+// part of 128 entries over 4 groups of 64 lanes was 8 dependent steps of 4, a short row up to 32.
+// Measured on MI355X, us, 4 rows everywhere / these: 200k power-law rows, fp32 N = 33 188 / 163,
+// N = 47 192 / 176, N = 101 388 / 351, fp64 N = 33 284 / 273, bit-identical.  Whole vectors gain
+// little (N = 16 62.1 / 61.3, N = 64 and 128 level), pairs of float32 nothing (4 kept); a wider
+// accumulator would lose waves to registers (58 -> 87) and keeps 4.
+template <typename T, typename A, int VW>
+constexpr int kPartRows = sizeof(A) != sizeof(T) || (sizeof(T) == 4 && VW == 2) ? 4
+                          : VW * sizeof(T) == 4                                 ? 16
+                                                                                : 8;
+
+// Adds entries i, i + step, ... of a part to acc, Q at a time while Q are left, in that order
+// whatever Q is.
+template <typename T, typename A, int VW, int Q>
+__device__ __forceinline__ void part_rows(const T* __restrict__ Bc, int64_t ldb, const int* s_col,
+                                          const T* s_val, int& i, int step, int len,
+                                          A (&acc)[VW]) {
+  for (; i + (Q - 1) * step < len; i += Q * step) {
+    T bv[Q][VW];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) load_vec<T, VW>(Bc + (int64_t)s_col[i + q * step] * ldb, bv[q]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const A av = A(s_val[i + q * step]);
+#pragma unroll
+      for (int j = 0; j < VW; ++j) acc[j] += av * A(bv[q][j]);
+    }
+  }
+}
+
 template <typename T, typename A, typename P, int VW, bool NT>
 __global__ __launch_bounds__(kBlock) void spmm_rowblock_kernel(
     const T* __restrict__ vals, const int* __restrict__ cols, const P* __restrict__ rowptr,
@@ -158,6 +190,8 @@ __global__ __launch_bounds__(kBlock) void spmm_rowblock_kernel(
       const int a = (int)(s_ptr[grp] - lo), e = (int)(s_ptr[grp + 1] - lo);
       const T* Bc = B + ncol;
       int i = a;
+      if constexpr (kPartRows<T, A, VW> == 16)
+        part_rows<T, A, VW, 16>(Bc, ldb, s_col, s_val, i, 1, e, acc);
       for (; i + kRowsInFlight <= e; i += kRowsInFlight) {
         T bv[kRowsInFlight][VW];
 #pragma unroll
@@ -188,18 +222,8 @@ __global__ __launch_bounds__(kBlock) void spmm_rowblock_kernel(
   if (col_ok) {
     const T* Bc = B + ncol;
     int i = grp;
-    for (; i + 3 * ngrp < len; i += 4 * ngrp) {
-      T bv[4][VW];
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-        load_vec<T, VW>(Bc + (int64_t)s_col[i + q * ngrp] * ldb, bv[q]);
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const A av = A(s_val[i + q * ngrp]);
-#pragma unroll
-        for (int j = 0; j < VW; ++j) acc[j] += av * A(bv[q][j]);
-      }
-    }
+    part_rows<T, A, VW, kPartRows<T, A, VW>>(Bc, ldb, s_col, s_val, i, ngrp, len, acc);
+    part_rows<T, A, VW, 4>(Bc, ldb, s_col, s_val, i, ngrp, len, acc);
     for (; i < len; i += ngrp) {
       T bv[VW];
       load_vec<T, VW>(Bc + (int64_t)s_col[i] * ldb, bv);
