@@ -7,8 +7,8 @@
 //   spmm_csr.py:778-919    opt long-row split: per-part sums, then parts added in index order
 //
 // The package runs it for prepared matrices of short rows with N, B and C in whole vectors, and for
-// those with rows so long that the order of additions shows; other products run on slices
-// (spmm_slices.hip).
+// those with rows so long that the order of additions shows (spmm_ragged_kernel below where their N
+// is odd or B unaligned); other products run on slices (spmm_slices.hip).
 //
 // Mapping (a gather-bound contraction, so no MFMA):
 //   * G lanes share one B row; each lane owns VW consecutive columns (16-byte loads for
@@ -83,8 +83,8 @@ constexpr int spmm_scratch_bytes() {
 // B rows requested together per lane of a long row's part, and before kRowsInFlight of a short
 // row where they are 16.  With single elements a lane's chain of requests is what bounds both: a
 // part of 128 entries over 4 groups of 64 lanes was 8 dependent steps of 4, a short row up to 32.
-// Measured on MI355X, us, 4 rows everywhere / these: 200k power-law rows, fp32 N = 33 188 / 163,
-// N = 47 192 / 176, N = 101 388 / 351, fp64 N = 33 284 / 273, bit-identical.  Whole vectors gain
+// Measured on MI355X, us, 4 rows everywhere / these: 200k power-law rows, fp32 N = 1 35.2 / 33.9,
+// N = 3 41.6 / 38.6, N = 47 192 / 176 (spmm_ragged_kernel takes 130 there), bit-identical.  Whole vectors gain
 // little (N = 16 62.1 / 61.3, N = 64 and 128 level), pairs of float32 nothing (4 kept); a wider
 // accumulator would lose waves to registers (58 -> 87) and keeps 4.
 template <typename T, typename A, int VW>
@@ -247,6 +247,134 @@ __global__ __launch_bounds__(kBlock) void spmm_rowblock_kernel(
   else partials[(int64_t)(part + k) * N + col] = sum;
 }
 
+// part_rows with VW elements at any alignment.
+template <typename T, int VW, int Q>
+__device__ __forceinline__ void ragged_rows(const T* __restrict__ Bc, int64_t ldb,
+                                            const int* s_col, const T* s_val, int& i, int step,
+                                            int len, T (&acc)[VW]) {
+  for (; i + (Q - 1) * step < len; i += Q * step) {
+    T bv[Q][VW];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) load_any<T, VW>(Bc + (int64_t)s_col[i + q * step] * ldb, bv[q]);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const T av = s_val[i + q * step];
+#pragma unroll
+      for (int j = 0; j < VW; ++j) acc[j] += av * bv[q][j];
+    }
+  }
+}
+
+// The same sums where N is no whole number of vectors, B or C are unaligned: what
+// spmm_rowblock_kernel does with 2^lg lanes of one element, here with 2^lg / VW lanes of VW
+// consecutive ones in workgroups of kBlock / VW, so a workgroup keeps its count of groups and
+// every sum its order of additions, bit for bit, with a VW-th of the load instructions.  The
+// last lane of a row moves back to end at N and keeps only the elements its neighbour lacks.
+// slots: entries that fit the LDS (more, from a plan of other rows, are read where they lie).
+// Bound: requests for B rows, L2-miss fills among them.  Measured on MI355X, us, single elements /
+// here, 200k power-law rows: fp32 N = 33 165 / 107, N = 47 175 / 130, N = 101 353 / 262; 900k
+// rows, N = 47 798 / 564; fp64 N = 33 272 / 180.
+template <typename T, typename P, int VW>
+__global__ __launch_bounds__(kBlock / VW) void spmm_ragged_kernel(
+    const T* __restrict__ vals, const int* __restrict__ cols, const P* __restrict__ rowptr,
+    P nnz_total, const T* __restrict__ B, int64_t ldb, int N, T* __restrict__ C, int64_t ldc,
+    const i32x4* __restrict__ desc, int n_desc, P chunk, int lg, T* __restrict__ partials,
+    int slots, int xcd_remap) {
+  constexpr int kThreads = kBlock / VW;
+  constexpr int kMaxGroups = 8;  // lg >= 5
+  extern __shared__ __attribute__((aligned(16))) unsigned char s_raw[];
+  T* s_val = reinterpret_cast<T*>(s_raw);  // [slots], then s_col [slots]
+  int* s_col = reinterpret_cast<int*>(s_val + slots);
+  T* s_red = s_val;  // [ngrp][W], reused after the entries are consumed
+  __shared__ P s_ptr[kMaxGroups + 1];
+
+  const int tid = threadIdx.x;
+  int b = blockIdx.x;
+  if (xcd_remap) b = xcd_logical_block(b, n_desc);
+  const int W = 1 << lg, G = W / VW, ngrp = kBlock >> lg;
+  const int grp = tid / G, lane = tid & (G - 1);
+  const int first = blockIdx.y * W + lane * VW;  // the columns [first, first + VW) below N
+  const bool col_ok = first < N;
+  const int shift = first + VW > N ? first + VW - N : 0;  // N >= VW (host check)
+  const int ncol = col_ok ? first - shift : 0;
+  const i32x4 d = desc[b];
+
+  P lo, hi;
+  int R = 0;
+  if (d.z == 0) {
+    R = d.y - d.x;
+    if (R <= 0 || R > ngrp) return;  // not a planner descriptor; uniform per block
+    if (tid <= R) s_ptr[tid] = rowptr[d.x + tid];
+    __syncthreads();
+    lo = s_ptr[0];
+    hi = s_ptr[R];
+  } else {
+    const P rs = rowptr[d.x], re = rowptr[d.x + 1];
+    lo = rs + P(d.y) * chunk;
+    hi = (lo + chunk < re) ? lo + chunk : re;
+  }
+  if (hi - lo > P(kSpmmNnzCap)) return;  // uniform per block
+  const int len = (int)(hi - lo);
+  const bool staged = len <= slots;
+  if (staged) {
+    for (P base = (lo & ~P(3)) + P(4) * tid; base < hi; base += P(4) * kThreads) {
+      T v[4];
+      int c[4];
+      QuadLoader<true, T>::load(vals, cols, base, lo, hi, nnz_total, v, c);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (c[j] >= 0) {
+          const int o = (int)(base + j - lo);
+          s_col[o] = c[j];
+          s_val[o] = v[j];
+        }
+    }
+  }
+  __syncthreads();
+
+  const T* Bc = B + ncol;
+  T acc[VW];
+#pragma unroll
+  for (int j = 0; j < VW; ++j) acc[j] = T(0);
+  // entries i, i + step, ... below e, in that order
+  auto add = [&](int i, int step, int e) {
+    if (staged) {
+      ragged_rows<T, VW, 8>(Bc, ldb, s_col, s_val, i, step, e, acc);
+      ragged_rows<T, VW, 4>(Bc, ldb, s_col, s_val, i, step, e, acc);
+      ragged_rows<T, VW, 1>(Bc, ldb, s_col, s_val, i, step, e, acc);
+    } else {
+      ragged_rows<T, VW, 1>(Bc, ldb, cols + lo, vals + lo, i, step, e, acc);
+    }
+  };
+
+  if (d.z == 0) {  // short rows: group grp owns row d.x + grp
+    if (grp >= R || !col_ok) return;
+    add((int)(s_ptr[grp] - lo), 1, (int)(s_ptr[grp + 1] - lo));
+    T* c = C + (int64_t)(d.x + grp) * ldc + ncol;
+    if (shift == 0) {
+      store_any<T, T, VW>(c, acc);
+    } else {
+#pragma unroll
+      for (int j = 0; j < VW; ++j)
+        if (j >= shift) c[j] = acc[j];
+    }
+    return;
+  }
+  if (col_ok) add(grp, ngrp, len);
+  __syncthreads();  // every group is done with s_val before s_red (same bytes) is written
+#pragma unroll
+  for (int j = 0; j < VW; ++j)
+    if (col_ok && j >= shift) s_red[grp * W + lane * VW + j - shift] = acc[j];
+  __syncthreads();
+  const int col = blockIdx.y * W + tid;
+  if (tid >= W || col >= N) return;
+  T sum = T(0);
+  for (int g = 0; g < ngrp; ++g) sum += s_red[g * W + tid];
+  if (d.z == 1) C[(int64_t)d.x * ldc + col] = sum;
+  else partials[(int64_t)(d.w + d.y) * N + col] = sum;
+}
+
 // Second pass for rows cut into parts: C[row, :] = sum over k < nch of the part sums, k in
 // increasing order.  One workgroup per split row (group {g, 1, nch, 0}, first part
 // group_base[g]); a separate launch, so the first pass needs no device-scope fence.
@@ -306,12 +434,30 @@ int launch_spmm(const void* vals, const int32_t* cols, const void* rowptr, int64
                 const void* B, int64_t ldb, int64_t N, void* C, int64_t ldc, const int32_t* desc,
                 int64_t n_desc, int64_t chunk, int lg, void* partials, const SplitGroups& sg,
                 int64_t n_tiles, int xcd_remap, hipStream_t st) {
-  hipLaunchKernelGGL((spmm_rowblock_kernel<T, A, P, VW, true>),
-                     dim3((unsigned)n_desc, (unsigned)n_tiles), dim3(kBlock), 0, st,
-                     static_cast<const T*>(vals), cols, static_cast<const P*>(rowptr), (P)nnz,
-                     static_cast<const T*>(B), ldb, (int)N, static_cast<T*>(C), ldc,
-                     reinterpret_cast<const i32x4*>(desc), (int)n_desc, (P)chunk, lg,
-                     static_cast<A*>(partials), xcd_remap);
+  // Single elements give way to vectors from 32 lanes on.  With 16, 2048 staged entries a workgroup
+  // leave room for few workgroups: fp32 N = 15 83.0 us with single elements, 86.5 with vectors
+  // (900k rows, N = 13: 384 / 400); fp64 N = 15 141 / 134.
+  bool ragged = false;
+  if constexpr (VW == 1 && sizeof(A) == sizeof(T)) {
+    constexpr int kVec = 16 / sizeof(T);
+    ragged = lg >= 5 && N >= kVec;
+    if (ragged) {
+      const int slots = (kBlock >> lg) * 128;  // rows and parts of at most 128 entries
+      hipLaunchKernelGGL((spmm_ragged_kernel<T, P, kVec>),
+                         dim3((unsigned)n_desc, (unsigned)n_tiles), dim3(kBlock / kVec),
+                         slots * (sizeof(T) + sizeof(int)), st, static_cast<const T*>(vals), cols,
+                         static_cast<const P*>(rowptr), (P)nnz, static_cast<const T*>(B), ldb,
+                         (int)N, static_cast<T*>(C), ldc, reinterpret_cast<const i32x4*>(desc),
+                         (int)n_desc, (P)chunk, lg, static_cast<T*>(partials), slots, xcd_remap);
+    }
+  }
+  if (!ragged)
+    hipLaunchKernelGGL((spmm_rowblock_kernel<T, A, P, VW, true>),
+                       dim3((unsigned)n_desc, (unsigned)n_tiles), dim3(kBlock), 0, st,
+                       static_cast<const T*>(vals), cols, static_cast<const P*>(rowptr), (P)nnz,
+                       static_cast<const T*>(B), ldb, (int)N, static_cast<T*>(C), ldc,
+                       reinterpret_cast<const i32x4*>(desc), (int)n_desc, (P)chunk, lg,
+                       static_cast<A*>(partials), xcd_remap);
   int rc = check_hip(hipGetLastError(), "spmm_rowblock_kernel launch");
   if (rc || sg.n == 0) return rc;
   hipLaunchKernelGGL((spmm_split_combine_kernel<T, A>), dim3((unsigned)sg.n), dim3(kBlock), 0, st,

@@ -9,7 +9,7 @@ precision), the validation metrics (:6-90, :1186-1192) and the benchmark cases
 Two kernels, both with G lanes sharing each B row by 16-byte loads along N:
 ``spmm_rowblock_kernel`` (flagsparse_amd/csrc/spmm.hip) for prepared matrices whose rows are all
 short (at most 128 entries), one row per lane group over a planned table, or so long that the
-order of additions shows (over 8192); ``spmm_slices_kernel``
+order of additions shows (over 8192; ``spmm_ragged_kernel`` where N is odd and over 16); ``spmm_slices_kernel``
 (csrc/spmm_slices.hip) for everything else: slices of equal work found by a search in the row
 pointers, the pieces of a cut row added in slice order (deterministic).
 """
@@ -317,7 +317,7 @@ def _spmm_slice_shape(lanes, positions, by_column=False):
 # orders differ by up to 4.6e-5 of the result's root mean square (200k rows of power-law lengths,
 # N = 47), against 1e-6 below.  Prepared products on such rows keep the order of the row-block
 # kernel, 128-entry parts added one after another, bit for bit, and change only the launch order
-# of the parts (slices would take 56 / 119 / 207 us where that takes 61 / 195 / 219: fp32, N = 16 / 47
+# of the parts (slices would take 56 / 119 / 207 us where that takes 61 / 130 / 219: fp32, N = 16 / 47
 # / 128).
 _SPMM_SUMS_KEPT = 8192
 
@@ -327,7 +327,7 @@ def _parts_by_column(desc, cols, n_cols, rowptr, chunk):
     by the first column they hold, each XCD a contiguous eighth of either.  Parts of different
     rows over the same columns then read the same rows of B while they are in that XCD's L2.
     Measured on MI355X, us, in row order / in this order: 200k rows of power-law lengths, fp32
-    N=16 86 / 61, N=47 238 / 195, N=128 382 / 219; fp64 N=33 316 / 287, N=64 376 / 246.  Ordered
+    N=16 89 / 61, N=47 231 / 130, N=128 382 / 234; fp64 N=33 287 / 176, N=64 379 / 256.  Ordered
     by 256 column bins in three launches (csrc/slices.hip): a full sort and gathers by torch took
     0.34 ms more of a matrix's first product (N=47: 815 / 479 us) for the same 195 us after it."""
     L = _abi.lib()

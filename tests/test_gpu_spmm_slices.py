@@ -208,19 +208,26 @@ def test_part_order(dev, ptr, lengths):
         assert bool((k[x::8][1:] >= k[x::8][:-1]).all())
 
 
-@pytest.mark.parametrize("n", [1, 3, 16, 47, 64, 128])
+@pytest.mark.parametrize("n", [1, 3, 16, 17, 31, 33, 47, 64, 65, 101, 128, 129])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-def test_parts_of_every_length(dev, n, dtype):
+@pytest.mark.parametrize("offset, longest", [(0, 128), (1, 128), (0, 250)])
+def test_parts_of_every_length(dev, monkeypatch, n, dtype, offset, longest):
     """Rows over 8192 entries whose last parts leave every remainder to the rows of B requested
-    together.  Whole numbers with sums below 2^24, so the result is exact in any order."""
+    together; single columns in a last tile, B off a vector's alignment, blocks of more entries
+    than the odd widths' kernel stages (rows of over 128 uncut).  Whole numbers with sums below
+    2^24, so the result is exact in any order."""
+    monkeypatch.setattr(spmm_csr, "_SPMM_ROW_SPLIT_THRESHOLD", longest)
     tails = [1, 2, 3, 4, 5, 12, 15, 16, 17, 31, 32, 33, 60, 61, 63, 64, 65, 100, 127, 128]
-    lengths = torch.tensor([1024 * 9 + t for t in tails] + [129, 192, 200, 0, 7])
+    lengths = torch.tensor([1024 * 9 + t for t in tails] + [129, 192, 200, 0, 7, 1, 2] + [250] * 9)
     ptr = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
     cols = synthetic.randint(5, 1, int(ptr[-1]), 3000, "cpu").to(torch.int32)
     data = (torch.arange(cols.numel()) % 13 - 6).to(dtype)
     B = (torch.arange(3000 * n) % 101 - 50).to(dtype).reshape(3000, n)
+    room = torch.empty(3000 * n + offset, dtype=dtype, device=dev)
+    Bd = room[offset:].view(3000, n)
+    Bd.copy_(B)
     p = fs.prepare_spmm_csr_opt(data.to(dev), cols.to(dev), ptr.to(dev), (lengths.numel(), 3000))
-    out = fs.flagsparse_spmm_csr_opt(B=B.to(dev), prepared=p).cpu()
+    out = fs.flagsparse_spmm_csr_opt(B=Bd, prepared=p).cpu()
     assert p._kernel_csr().kernel_name() == "spmm_rowblock_kernel"
     ref = oracle.spmm_csr(ptr, cols, data, B)
     assert torch.equal(out.double(), torch.as_tensor(ref).double())
