@@ -272,7 +272,8 @@ __device__ __forceinline__ void ragged_rows(const T* __restrict__ Bc, int64_t ld
 // every sum its order of additions, bit for bit, with a VW-th of the load instructions.  The
 // last lane of a row moves back to end at N and keeps only the elements its neighbour lacks.
 // slots: entries that fit the LDS (more, from a plan of other rows, are read where they lie).
-// Bound: requests for B rows, L2-miss fills among them.  Measured on MI355X, us, single elements /
+// Bound: L2 line requests for B rows and the fills of those that miss (N = 47: 13M lines, 68 % hits,
+// 4.5 TB/s filled, 118 us).  Measured on MI355X, us per call, single elements /
 // here, 200k power-law rows: fp32 N = 33 165 / 107, N = 47 175 / 130, N = 101 353 / 262; 900k
 // rows, N = 47 798 / 564; fp64 N = 33 272 / 180.
 template <typename T, typename P, int VW>
