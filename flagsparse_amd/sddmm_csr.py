@@ -59,8 +59,17 @@ class SDDMMPrepared:
     @property
     def row_ids(self):
         if self._row_ids is None:
-            self._row_ids = _build_row_ids(self.indptr)
+            ids = _build_row_ids(self.indptr)
+            self._built()
+            self._row_ids = ids
         return self._row_ids
+
+    def _built(self):
+        """Waits for what was just queued to fill an array that this object is about to keep: the
+        next call may come from another stream, which nothing orders after this one.  An object of
+        one call has one stream."""
+        if not self._one_call:
+            torch.cuda.current_stream(self.indices.device).synchronize()
 
     def slices(self, items, by_column):
         """The boundaries of slices of ``items`` rows + entries and their launch order (built once
@@ -72,8 +81,7 @@ class SDDMMPrepared:
                     torch.int32 if self.nnz <= _common.ROWPTR32_MAX_NNZ else torch.int64)
             t = _slices.build(self._kernel_ptr, self.n_rows, self.nnz, items, 0, "SDDMM",
                               self.indices if by_column else None, self.n_cols)
-            if not self._one_call:  # later calls may come from other streams
-                torch.cuda.current_stream(self.indices.device).synchronize()
+            self._built()
             self._tables[(items, by_column)] = t
         return t
 

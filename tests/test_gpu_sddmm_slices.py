@@ -139,3 +139,20 @@ def test_sliced_sddmm_by_column(dev, monkeypatch, name):
     (_, order), = p._tables.values()
     assert torch.equal(torch.sort(order.cpu()).values.to(torch.int64),
                        torch.arange(order.numel()))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_wide_sddmm_two_streams(dev, dtype):
+    # the kernel of very wide K reads the row ids, which the first call makes on its own stream
+    ip, cols, data, x, y, shape = _case("crossing", 503, 2051, dtype, dev)
+    xd, yd = x.to(dev), y.to(dev)
+    p = fs.prepare_sddmm_csr(cols.to(dev), ip.to(dev), shape, k_hint=2051)
+    outs = []
+    for _ in range(2):
+        for s in (torch.cuda.Stream(device=dev), torch.cuda.Stream(device=dev)):
+            with torch.cuda.stream(s):
+                outs.append(fs.flagsparse_sddmm_csr(x=xd, y=yd, prepared=p))
+    torch.cuda.synchronize()
+    assert not p._tables
+    ref = oracle.sddmm_csr(ip, cols, x, y)
+    assert all(oracle.rel_l2(o, ref) <= oracle.REL_L2_BOUND[str(dtype)[6:]] for o in outs)
