@@ -76,12 +76,14 @@ class SDDMMPrepared:
         per size)."""
         t = self._tables.get((items, by_column))
         if t is None:
-            if self._kernel_ptr is None:
-                self._kernel_ptr = self.indptr.to(
+            ptr = self._kernel_ptr
+            if ptr is None:
+                ptr = self.indptr.to(
                     torch.int32 if self.nnz <= _common.ROWPTR32_MAX_NNZ else torch.int64)
-            t = _slices.build(self._kernel_ptr, self.n_rows, self.nnz, items, 0, "SDDMM",
+            t = _slices.build(ptr, self.n_rows, self.nnz, items, 0, "SDDMM",
                               self.indices if by_column else None, self.n_cols)
             self._built()
+            self._kernel_ptr = ptr
             self._tables[(items, by_column)] = t
         return t
 

@@ -38,6 +38,15 @@ def test_row_ids_wait_before_they_are_kept(prepared):
     assert p.row_ids is p.row_ids and len(stream.held) == 1
 
 
+def test_slices_wait_before_they_are_kept(prepared):
+    p, stream = prepared
+    assert p.slices(64, False) == ("table", "order")
+    assert stream.held == [(None, None, {})]
+    assert p._kernel_ptr.dtype == torch.int32
+    p.slices(64, False)
+    assert len(stream.held) == 1
+
+
 def test_one_call_waits_for_nothing(prepared):
     p, stream = prepared
     p._one_call = True
