@@ -276,9 +276,39 @@ def _sddmm_slice_items(lanes, positions):
     return items
 
 
+class _Launch:
+    """What launches of one K and type share: the sliced kernel's arguments (None: the flat kernel),
+    the arrays a launch reads, and the streams those are marked as used on."""
+
+    __slots__ = ("sliced", "arrays", "streams")
+
+    def __init__(self, sliced, arrays):
+        self.sliced = sliced
+        self.arrays = arrays
+        self.streams = set()
+
+    def __reduce__(self):  # a copy's arrays are other arrays, marked nowhere
+        return _Launch, (self.sliced, self.arrays)
+
+    def mark(self, stream, device):
+        """Marks the arrays as used on ``stream``, the current one: they belong to the stream that
+        made them, and calls do not wait, so without the mark the caching allocator could hand
+        their memory out while a kernel of this stream still reads it.  Once per stream: the
+        allocator keeps the mark until the memory is given back.  Not while a graph is captured:
+        nothing runs then, and keeping the pattern for the replays is the caller's."""
+        if torch.cuda.is_current_stream_capturing():
+            return
+        current = torch.cuda.current_stream(device)
+        for t in self.arrays:
+            if t is not None:
+                t.record_stream(current)
+        self.streams.add(stream)
+
+
 def _launch_sddmm(prepared, x, y, data, alpha, beta, out, acc_f64):
     """The sliced kernel when K fits four steps of a lane group, else one lane group per entry."""
     K = int(x.shape[1])
+    stream = _abi.raw_stream(x.device)
     L = _abi.lib()
     code = _abi.dtype_code(x.dtype)
     out_f64 = int(out.dtype == torch.float64 and x.dtype == torch.float32)
@@ -292,27 +322,31 @@ def _launch_sddmm(prepared, x, y, data, alpha, beta, out, acc_f64):
             by_column = _slices.ordered(prepared._max_row_nnz, items,
                                         prepared.n_cols * row_bytes, prepared.nnz * row_bytes,
                                         prepared._one_call)
-            shape = (lanes, vec, items) + prepared.slices(items, by_column)
+            table, order = prepared.slices(items, by_column)
+            rp = prepared._kernel_ptr
+            shape = _Launch((lanes, vec, items, rp, table, order), (cols, rp, table, order))
         else:
-            shape = ()
+            shape = _Launch(None, (cols, prepared.row_ids))
         prepared._shapes[(K, x.dtype)] = shape
-    if shape:
-        lanes, vec, items, table, order = shape
-        rp = prepared._kernel_ptr
+    if not prepared._one_call and stream not in shape.streams:
+        shape.mark(stream, x.device)
+    if shape.sliced is not None:
+        lanes, vec, items, rp, table, order = shape.sliced
         _abi.check(
             L.fsp_sddmm_sliced(code, int(acc_f64), out_f64, cols.data_ptr(), rp.data_ptr(),
                                32 if rp.dtype == torch.int32 else 64, prepared.n_rows,
                                prepared.nnz, x.data_ptr(), x.stride(0), y.data_ptr(),
                                y.stride(0), K, None if data is None else data.data_ptr(),
                                float(alpha), float(beta), out.data_ptr(), table.data_ptr(),
-                               None if order is None else order.data_ptr(), items, lanes, vec, _abi.raw_stream(x.device)), "fsp_sddmm_sliced")
+                               None if order is None else order.data_ptr(), items, lanes, vec,
+                               stream), "fsp_sddmm_sliced")
         return
     lanes, vec = _sddmm_lane_shape(K, x, y)
     _abi.check(
         L.fsp_sddmm_csr(code, int(acc_f64), out_f64, _abi.ptr(cols), _abi.ptr(prepared.row_ids),
                         None, 32, prepared.nnz, _abi.ptr(x), x.stride(0), _abi.ptr(y),
                         y.stride(0), K, _abi.ptr(data), float(alpha), float(beta), _abi.ptr(out),
-                        None, None, 0, lanes, vec, _abi.stream_handle(x.device)),
+                        None, None, 0, lanes, vec, stream),
         "fsp_sddmm_csr")
 
 

@@ -156,3 +156,33 @@ def test_wide_sddmm_two_streams(dev, dtype):
     assert not p._tables
     ref = oracle.sddmm_csr(ip, cols, x, y)
     assert all(oracle.rel_l2(o, ref) <= oracle.REL_L2_BOUND[str(dtype)[6:]] for o in outs)
+
+
+@pytest.mark.parametrize("K", [40, 2051])  # the sliced kernel, the flat one
+def test_sddmm_keeps_its_arrays_from_other_streams(dev, monkeypatch, K):
+    """A prepared pattern dropped after a call on another stream: the memory of its arrays is not
+    given out while that stream is busy."""
+    ip, cols, data, x, y, shape = _case("crossing", 503, K, torch.float32, dev)
+    if K == 40:
+        monkeypatch.setattr(sddmm_csr._slices, "ordered", lambda *a: True)
+    xd, yd, mat = x.to(dev), y.to(dev), torch.ones(8192, 8192, device=dev)
+    p = fs.prepare_sddmm_csr(cols.to(dev), ip.to(dev), shape, k_hint=K)
+    fs.flagsparse_sddmm_csr(x=xd, y=yd, prepared=p)  # its arrays belong to this stream
+    side = torch.cuda.Stream(device=dev)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(20):  # about 10 ms each
+            mat = mat @ mat
+        out = fs.flagsparse_sddmm_csr(x=xd, y=yd, prepared=p)
+    (launch,) = p._shapes.values()
+    arrays = [t for t in launch.arrays if t is not None]
+    assert len(arrays) == (4 if K == 40 else 2)
+    sizes = [t.untyped_storage().nbytes() for t in arrays]
+    held = {t.untyped_storage().data_ptr() for t in arrays}
+    del p, launch, arrays
+    taken = [torch.empty(n, dtype=torch.uint8, device=dev) for n in sizes * 4]
+    busy = not side.query()
+    assert not held & {t.untyped_storage().data_ptr() for t in taken}
+    assert busy  # else the allocator was free to give them out
+    torch.cuda.synchronize()
+    assert oracle.rel_l2(out, oracle.sddmm_csr(ip, cols, x, y)) <= 1e-5

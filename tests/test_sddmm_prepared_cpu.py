@@ -2,6 +2,9 @@
 come from other streams, which nothing orders after the one that built it (no GPU: the stream is a
 recorder)."""
 
+import copy
+import pickle
+
 import pytest
 import torch
 
@@ -52,3 +55,13 @@ def test_one_call_waits_for_nothing(prepared):
     p._one_call = True
     p.row_ids, p.slices(64, False)
     assert stream.held == []
+
+
+def test_copied_launch_is_marked_nowhere():
+    table = torch.arange(4)
+    launch = sddmm_csr._Launch((8, 4, 256, table, table, None), (table, None))
+    launch.streams.add(17)
+    for other in (copy.deepcopy(launch), pickle.loads(pickle.dumps(launch))):
+        assert other.streams == set() and other.sliced[:3] == (8, 4, 256)
+        assert other.arrays[0] is other.sliced[3] and torch.equal(other.arrays[0], table)
+        assert other.arrays[0].data_ptr() != table.data_ptr()
