@@ -147,20 +147,21 @@ __global__ __launch_bounds__(kBlock) void spmm_rowblock_kernel(
   } else {
     const P rs = rowptr[d.x], re = rowptr[d.x + 1];
     lo = rs + P(d.y) * chunk;
-    hi = (lo + chunk < re) ? lo + chunk : re;
+    hi = re - lo > chunk ? lo + chunk : re;
   }
   if (hi - lo > P(kSpmmNnzCap)) return;  // uniform per block
 
   // Stage the (col, val) entries [lo, hi) into LDS with 16-byte loads.
   {
     const P s0 = lo & ~P(3);
+    const int span = (int)(hi - s0), head = (int)(lo - s0);
     T v[kStageUPT][4];
     int c[kStageUPT][4];
 #pragma unroll
     for (int u = 0; u < kStageUPT; ++u) {
-      const P base = s0 + P(4) * (tid + u * kBlock);
-      if (base < hi) {
-        QuadLoader<NT, T>::load(vals, cols, base, lo, hi, nnz_total, v[u], c[u]);
+      const int off = 4 * (tid + u * kBlock);
+      if (off < span) {
+        QuadLoader<NT, T>::load(vals, cols, P(s0 + off), lo, hi, nnz_total, v[u], c[u]);
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) { v[u][j] = T(0); c[u][j] = -1; }
@@ -168,11 +169,11 @@ __global__ __launch_bounds__(kBlock) void spmm_rowblock_kernel(
     }
 #pragma unroll
     for (int u = 0; u < kStageUPT; ++u) {
-      const P base = s0 + P(4) * (tid + u * kBlock);
+      const int off = 4 * (tid + u * kBlock) - head;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (c[u][j] >= 0) {
-          const int o = (int)(base + j - lo);
+          const int o = off + j;
           s_col[o] = c[u][j];
           s_val[o] = v[u][j];
         }
@@ -313,20 +314,22 @@ __global__ __launch_bounds__(kBlock / VW) void spmm_ragged_kernel(
   } else {
     const P rs = rowptr[d.x], re = rowptr[d.x + 1];
     lo = rs + P(d.y) * chunk;
-    hi = (lo + chunk < re) ? lo + chunk : re;
+    hi = re - lo > chunk ? lo + chunk : re;
   }
   if (hi - lo > P(kSpmmNnzCap)) return;  // uniform per block
   const int len = (int)(hi - lo);
   const bool staged = len <= slots;
   if (staged) {
-    for (P base = (lo & ~P(3)) + P(4) * tid; base < hi; base += P(4) * kThreads) {
+    const P s0 = lo & ~P(3);
+    const int span = (int)(hi - s0), head = (int)(lo - s0);
+    for (int off = 4 * tid; off < span; off += 4 * kThreads) {
       T v[4];
       int c[4];
-      QuadLoader<true, T>::load(vals, cols, base, lo, hi, nnz_total, v, c);
+      QuadLoader<true, T>::load(vals, cols, P(s0 + off), lo, hi, nnz_total, v, c);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (c[j] >= 0) {
-          const int o = (int)(base + j - lo);
+          const int o = off - head + j;
           s_col[o] = c[j];
           s_val[o] = v[j];
         }

@@ -56,14 +56,15 @@ __global__ __launch_bounds__(kBlock) void spmv_rowblock_kernel(
     if (R <= 0 || R > kStreamRows || hi - lo > P(kSpmvStreamNnzCap) || hi < lo)
       return;  // not a planner descriptor; uniform per block
     const P s0 = lo & ~P(3);
+    const int span = (int)(hi - s0), head = (int)(lo - s0);
 
     T v[kStreamUPT][4];
     int c[kStreamUPT][4];
 #pragma unroll
     for (int u = 0; u < kStreamUPT; ++u) {
-      const P base = s0 + P(4) * (tid + u * kBlock);
-      if (base < hi) {
-        QuadLoader<NT, T>::load(vals, cols, base, lo, hi, nnz_total, v[u], c[u]);
+      const int off = 4 * (tid + u * kBlock);
+      if (off < span) {
+        QuadLoader<NT, T>::load(vals, cols, P(s0 + off), lo, hi, nnz_total, v[u], c[u]);
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) { v[u][j] = T(0); c[u][j] = -1; }
@@ -80,10 +81,10 @@ __global__ __launch_bounds__(kBlock) void spmv_rowblock_kernel(
     gather_x<kStreamUPT, A>(x, c, hi > lo, xv);
 #pragma unroll
     for (int u = 0; u < kStreamUPT; ++u) {
-      const P base = s0 + P(4) * (tid + u * kBlock);
+      const int off = 4 * (tid + u * kBlock) - head;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (c[u][j] >= 0) s_prod[(int)(base + j - lo)] = A(v[u][j]) * A(xv[u][j]);
+        if (c[u][j] >= 0) s_prod[off + j] = A(v[u][j]) * A(xv[u][j]);
     }
 #pragma unroll
     for (int u = 0; u < kPtrPT; ++u) {
@@ -122,14 +123,15 @@ __global__ __launch_bounds__(kBlock) void spmv_rowblock_kernel(
   const int row = d.x, k = d.y, nch = d.z, part = d.w;
   if (hi - lo > chunk || hi < lo) return;  // not a planner descriptor; uniform per block
   const P s0 = lo & ~P(3);
+  const int span = (int)(hi - s0);
 
   T v[kChunkUPT][4];
   int c[kChunkUPT][4];
 #pragma unroll
   for (int u = 0; u < kChunkUPT; ++u) {
-    const P base = s0 + P(4) * (tid + u * kBlock);
-    if (base < hi) {
-      QuadLoader<NT, T>::load(vals, cols, base, lo, hi, nnz_total, v[u], c[u]);
+    const int off = 4 * (tid + u * kBlock);
+    if (off < span) {
+      QuadLoader<NT, T>::load(vals, cols, P(s0 + off), lo, hi, nnz_total, v[u], c[u]);
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j) { v[u][j] = T(0); c[u][j] = -1; }
