@@ -15,7 +15,8 @@ LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "lib
 
 FSP_F32 = 0
 FSP_F64 = 1
-ABI_VERSION = 18
+FSP_CUT_PIECES = 2
+ABI_VERSION = 19
 
 _lib = None
 
@@ -75,6 +76,7 @@ SIGNATURES = {
                             _i64, _i64, _i32, _i32, _p, _p, _p, _p, _i64, _i32, _p]),
     "fsp_slice_count": (_i64, [_i64, _i64, _i64]),
     "fsp_slice_table": (_i32, [_p, _i32, _i64, _i64, _i64, _i64, _p, _p]),
+    "fsp_slice_pieces": (_i32, [_p, _i32, _i64, _p, _p]),
     "fsp_slice_order_scratch": (_i64, [_i64]),
     "fsp_slice_order": (_i32, [_p, _i64, _p, _i64, _p, _p, _p]),
     "fsp_part_order": (_i32, [_p, _i64, _p, _i32, _i64, _p, _i64, _p, _p, _p]),

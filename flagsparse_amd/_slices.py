@@ -37,3 +37,16 @@ def build(rowptr, n_rows, nnz, items, keep, what, cols=None, n_cols=0):
     _abi.check(L.fsp_slice_order(table.data_ptr(), n, cols.data_ptr(), n_cols, order.data_ptr(),
                                  order[n:].data_ptr(), stream), "fsp_slice_order")
     return table, order[:n]
+
+
+def pieces(rowptr, table):
+    """(``table`` with the first piece of a cut row in each slice behind it, the number of pieces):
+    for sums that take room only where rows are cut.  Waits for the device."""
+    n = table.numel() // 2 - 1
+    both = torch.empty(2 * (n + 1) + n // 2 + 1, dtype=torch.int64, device=table.device)
+    both[:2 * (n + 1)].copy_(table)
+    _abi.check(_abi.lib().fsp_slice_pieces(rowptr.data_ptr(),
+                                           32 if rowptr.dtype == torch.int32 else 64, n,
+                                           both.data_ptr(), _abi.raw_stream(table.device)),
+               "fsp_slice_pieces")
+    return both, int(both[2 * (n + 1):].view(torch.int32)[n])

@@ -148,7 +148,8 @@ __global__ __launch_bounds__(kBlock) void order_hist_kernel(S what, int64_t n, i
   counts[(int64_t)threadIdx.x * n_tiles + blockIdx.x] = s_cnt[threadIdx.x];
 }
 
-// Exclusive sums over all (bin, tile) counts, bins outer: one workgroup.
+// Exclusive sums over all (bin, tile) counts, bins outer (or over the slices' pieces): one
+// workgroup.
 __global__ __launch_bounds__(1024) void order_scan_kernel(int* __restrict__ counts, int64_t m) {
   __shared__ int s_w[1024 / kWave];
   int run = 0;
@@ -230,6 +231,25 @@ int launch_order(const S& what, int64_t n, int32_t* scratch, hipStream_t st) {
   hipLaunchKernelGGL((order_scatter_kernel<S>), dim3((unsigned)tiles), dim3(kBlock), 0, st, what,
                      n, tile, tiles, scratch);
   return check_hip(hipGetLastError(), "order_scatter_kernel launch");
+}
+
+// The pieces of cut rows that slice k holds: the end of a row begun earlier, the start of a row that
+// goes on in the next slice.  What spmm_slices_kernel puts into head[k] and carry[k].
+template <typename P>
+__global__ __launch_bounds__(kBlock) void slice_piece_count_kernel(
+    const P* __restrict__ rowptr, const int64_t* __restrict__ table, int64_t n,
+    int* __restrict__ counts) {
+  const int64_t k = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (k > n) return;
+  int c = 0;
+  if (k < n) {
+    const int64_t i0 = table[2 * k], p0 = table[2 * k + 1];
+    const int64_t i1 = table[2 * k + 2], p1 = table[2 * k + 3];
+    if (i1 > i0 && (int64_t)rowptr[i0] < p0) ++c;
+    const int64_t a = (int64_t)rowptr[i1];
+    if (p1 > (a > p0 ? a : p0)) ++c;
+  }
+  counts[k] = c;
 }
 
 template <typename T, typename A, typename P>
@@ -443,6 +463,28 @@ extern "C" int fsp_part_order(const int32_t* desc, int64_t n_desc, const void* r
   return launch_order(
       Descriptors<int64_t>{d, static_cast<const int64_t*>(rowptr), chunk, cols, n_cols, o}, n_desc,
       scratch, st);
+}
+
+extern "C" int fsp_slice_pieces(const void* rowptr, int rowptr_bits, int64_t n_slices,
+                                int64_t* table, void* stream) {
+  if (rowptr_bits != 32 && rowptr_bits != 64)
+    return set_error(FSP_EINVAL, "fsp_slice_pieces: rowptr_bits must be 32 or 64");
+  if (n_slices < 0 || n_slices > 0x3fffffffLL)  // two pieces a slice in 32 bits
+    return set_error(FSP_EINVAL, "fsp_slice_pieces: size out of range");
+  if (!rowptr || !table) return set_error(FSP_EINVAL, "fsp_slice_pieces: null pointer");
+  int* counts = reinterpret_cast<int*>(table + 2 * (n_slices + 1));
+  const dim3 grid((unsigned)(n_slices / kBlock + 1));
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (rowptr_bits == 32)
+    hipLaunchKernelGGL((slice_piece_count_kernel<int>), grid, dim3(kBlock), 0, st,
+                       static_cast<const int*>(rowptr), table, n_slices, counts);
+  else
+    hipLaunchKernelGGL((slice_piece_count_kernel<int64_t>), grid, dim3(kBlock), 0, st,
+                       static_cast<const int64_t*>(rowptr), table, n_slices, counts);
+  const int rc = check_hip(hipGetLastError(), "slice_piece_count_kernel launch");
+  if (rc) return rc;
+  hipLaunchKernelGGL(order_scan_kernel, dim3(1), dim3(1024), 0, st, counts, n_slices + 1);
+  return check_hip(hipGetLastError(), "order_scan_kernel launch");
 }
 
 extern "C" int64_t fsp_spmv_slices(int64_t n_rows, int64_t nnz) {

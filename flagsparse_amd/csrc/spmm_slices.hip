@@ -18,7 +18,9 @@
 //   * a row much longer than the groups' share of the slice is left to a second step, where all
 //     groups take its entries in turn and their sums are added through LDS in a fixed order.
 //   * the piece of a row that goes on in the next slice goes to carry[k], the end of a row begun
-//     earlier to head[k]; spmm_slice_fixup_kernel adds the pieces in slice order.
+//     earlier to head[k]; spmm_slice_fixup_kernel adds the pieces in slice order.  A slot for either
+//     of every slice needs no count; where that is much room (wide N, few cut rows), the pieces are
+//     counted (fsp_slice_pieces) and lie one after the other: slice k's from pieces[k].
 //
 // Bound: the B rows' fills from outside L2 (whole 128-byte lines), as spmm_rowblock_kernel.
 // Measured on MI355X, row blocks / slices: a power law of 200k rows and 4.8M entries, fp32 N=47
@@ -76,7 +78,8 @@ __global__ __launch_bounds__(kBlock, 8) void spmm_slices_kernel(
     const T* __restrict__ vals, const int* __restrict__ cols, const P* __restrict__ rowptr,
     P nnz_total, const T* __restrict__ B, uint32_t ldb, int N, T* __restrict__ C, int64_t ldc,
     const int64_t* __restrict__ table, const int* __restrict__ order, int n_slices, int cap,
-    int rows_cap, int lg, A* __restrict__ carry, A* __restrict__ head, int xcd_remap) {
+    int rows_cap, int lg, A* __restrict__ carry, A* __restrict__ head,
+    const int* __restrict__ pieces, int xcd_remap) {
   extern __shared__ __attribute__((aligned(16))) unsigned char s_raw[];
   // s_red [4 waves][G * VW] | s_val [cap] | s_col [cap] | s_ptr [rows_cap + 2] | s_list | s_n
   const int G = 1 << lg, ngrp = kBlock >> lg, W = G * VW;
@@ -142,9 +145,11 @@ __global__ __launch_bounds__(kBlock, 8) void spmm_slices_kernel(
   const T* Bc = B + ncol;
   auto put = [&](int s, const A(&acc)[VW]) {
     if (s == R) {
-      store_any<A, A, VW>(carry + (int64_t)k * N + ncol, acc);
+      const int64_t slot = pieces ? pieces[k] + (begun ? 1 : 0) : k;
+      store_any<A, A, VW>(carry + slot * N + ncol, acc);
     } else if (s == 0 && begun) {
-      store_any<A, A, VW>(head + (int64_t)k * N + ncol, acc);
+      const int64_t slot = pieces ? pieces[k] : k;
+      store_any<A, A, VW>(head + slot * N + ncol, acc);
     } else {
       store_any<T, A, VW>(C + (i0 + s) * ldc + ncol, acc);
     }
@@ -227,8 +232,8 @@ __global__ __launch_bounds__(kBlock, 8) void spmm_slices_kernel(
 template <typename T, typename A, typename P>
 __global__ __launch_bounds__(kBlock) void spmm_slice_fixup_kernel(
     const P* __restrict__ rowptr, const int64_t* __restrict__ table, int64_t Wpos,
-    const A* __restrict__ carry, const A* __restrict__ head, int N, int cw,
-    T* __restrict__ C, int64_t ldc) {
+    const A* __restrict__ carry, const A* __restrict__ head, const int* __restrict__ pieces, int N,
+    int cw, T* __restrict__ C, int64_t ldc) {
   __shared__ A s_red[kBlock];
   const int tid = threadIdx.x;
   const int64_t k = blockIdx.x, row = table[2 * k], p0 = table[2 * k + 1];
@@ -237,6 +242,10 @@ __global__ __launch_bounds__(kBlock) void spmm_slice_fixup_kernel(
   if (a >= p0) return;  // it begins here
   int64_t j0 = (a + row) / Wpos;  // the slice the row began in (spmv_slice_fixup_kernel)
   if (table[2 * j0 + 3] <= a) ++j0;
+  if (pieces) {  // counted: the row's pieces lie one after the other, up to pieces[k]
+    carry += (pieces[k] - k) * N;
+    head += (pieces[k] - k) * N;
+  }
   const int c0 = tid & (cw - 1), pg = tid / cw, npg = kBlock / cw;
   for (int cb = 0; cb < N; cb += cw) {
     const int c = cb + c0;
@@ -289,20 +298,22 @@ int launch_upt(const SliceArgs& a) {
   const int64_t tiles = (a.N + W - 1) / W;
   const size_t lds = (size_t)kWavesPerBlock * W * sizeof(A) + (size_t)cap * (sizeof(T) + 4) +
                      4 * (size_t)(rows_cap + 2 + (kBlock >> a.lg) + 1);
+  const bool counted = a.cut_rows == FSP_CUT_PIECES;
   A* carry = static_cast<A*>(a.sums);
-  A* head = carry + n * a.N;
+  A* head = counted ? carry : carry + n * a.N;
+  const int* pieces = counted ? reinterpret_cast<const int*>(a.table + 2 * (n + 1)) : nullptr;
   hipLaunchKernelGGL((spmm_slices_kernel<T, A, P, VW, UPT>), dim3((unsigned)n, (unsigned)tiles),
                      dim3(kBlock), lds, a.st, static_cast<const T*>(a.vals), a.cols,
                      static_cast<const P*>(a.rowptr), (P)a.nnz, static_cast<const T*>(a.B),
                      (uint32_t)a.ldb, (int)a.N, static_cast<T*>(a.C), a.ldc, a.table, a.order, (int)n, cap,
-                     rows_cap, a.lg, carry, head, a.xcd_remap);
+                     rows_cap, a.lg, carry, head, pieces, a.xcd_remap);
   int rc = check_hip(hipGetLastError(), "spmm_slices_kernel launch");
   if (rc || !a.cut_rows) return rc;
   int cw = 1;
   while (cw < a.N && cw < kBlock) cw <<= 1;
   hipLaunchKernelGGL((spmm_slice_fixup_kernel<T, A, P>),
                      dim3((unsigned)n), dim3(kBlock), 0, a.st,
-                     static_cast<const P*>(a.rowptr), a.table, a.items, carry, head, (int)a.N,
+                     static_cast<const P*>(a.rowptr), a.table, a.items, carry, head, pieces, (int)a.N,
                      cw, static_cast<T*>(a.C), a.ldc);
   return check_hip(hipGetLastError(), "spmm_slice_fixup_kernel launch");
 }

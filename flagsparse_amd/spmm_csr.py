@@ -46,6 +46,12 @@ SPMM_PLAN_WINDOW_BLOCKS = 4
 # the pieces of cut rows unseen; beyond it (32 MB of float64) the row pointers are looked at first
 # (25 us with its host wait, on products of milliseconds).
 _SUMS_UNSEEN = 1 << 22
+# Room for the pieces of cut rows, two for every slice, is taken without a count up to this many bytes.
+# One row over the longest uncut length is enough for it, and it grows with N: 1M rows of 32 entries
+# with one of 300, N = 256, would take 1.06 GB for three pieces.  Beyond the limit the pieces are
+# counted, once per matrix and slice size (two launches and a host wait: 0.1 ms of a 4.8 ms product
+# without a prepared object there).
+_SUMS_ROOM = 256 << 20
 # Rows longer than this go to the part path (several lane groups per row).
 _SPMM_ROW_SPLIT_THRESHOLD = 128
 
@@ -347,7 +353,7 @@ class _SpmmKernelCsr:
     one call, so nothing is planned."""
 
     __slots__ = ("data", "cols", "rowptr", "rowptr_bits", "nnz", "n_rows", "_plans", "_args",
-                 "_keep", "_order", "max_row_nnz", "one_shot", "_tables")
+                 "_keep", "_order", "max_row_nnz", "one_shot", "_tables", "_pieces", "_sums")
 
     def __init__(self, data, cols, indptr, max_row_nnz=None, one_shot=False):
         self.max_row_nnz = max_row_nnz
@@ -361,6 +367,8 @@ class _SpmmKernelCsr:
         else:
             self.rowptr, self.rowptr_bits = indptr.to(torch.int64).contiguous(), 64
         self._tables = {}
+        self._pieces = {}
+        self._sums = {}
         self._plans = {}
         self._args = {}
         self._keep = [self.data, self.cols, self.rowptr]  # what a launch reads or writes
@@ -396,6 +404,24 @@ class _SpmmKernelCsr:
                               self.cols if by_column else None, n_cols)
             self._tables[key] = t
         return t
+
+    def piece_slots(self, items, table, n_dense_cols, dtype):
+        """(the table to launch with, room for the pieces of cut rows, the kind of cut): a slot for
+        either end of every slice, or, where that is too much, for each piece.  Calls are ordered
+        (StreamOrder), so those of one size share it."""
+        length, cut = (int(table.numel()) - 2) * n_dense_cols, 1
+        if length * dtype.itemsize > _SUMS_ROOM:
+            if items not in self._pieces:
+                self._pieces[items] = _slices.pieces(self.rowptr, table)
+            table, n = self._pieces[items]
+            if n == 0:
+                return table, None, 0
+            length, cut = n * n_dense_cols, _abi.FSP_CUT_PIECES
+        sums = self._sums.get((length, dtype))
+        if sums is None:
+            sums = self._sums[length, dtype] = torch.empty(length, dtype=dtype,
+                                                           device=table.device)
+        return table, sums, cut
 
     def plan(self, lanes, row_bytes=0, n_cols=0):
         p = self._plans.get(lanes)
@@ -435,7 +461,7 @@ def _auto_tile_cols(B):
     return t if t < n else None
 
 
-def _bind_sliced(kc, B, C, acc_f64, lanes, vec):
+def _bind_sliced(kc, B, acc_f64, lanes, vec):
     n_dense_cols, n_cols, positions = int(B.shape[1]), int(B.shape[0]), kc.n_rows + kc.nnz
     row_bytes = min(n_dense_cols, lanes * vec) * B.element_size()  # of one column tile
     items, keep = _spmm_slice_shape(lanes, positions, True)
@@ -444,20 +470,18 @@ def _bind_sliced(kc, B, C, acc_f64, lanes, vec):
     if not by_column:
         items, keep = _spmm_slice_shape(lanes, positions)
     table, order = kc.slices(items, keep, n_cols, by_column)
-    # the pieces of cut rows: a carry and a head per slice
-    sums, sums_len = None, (int(table.numel()) - 2) * n_dense_cols
-    if kc.max_row_nnz is None and sums_len > _SUMS_UNSEEN:
+    if kc.max_row_nnz is None and (int(table.numel()) - 2) * n_dense_cols > _SUMS_UNSEEN:
         kc.max_row_nnz = int((kc.rowptr[1:] - kc.rowptr[:-1]).max())
-    cut = kc.max_row_nnz is None or kc.max_row_nnz > keep
-    if cut:
-        sums = torch.empty(sums_len, device=C.device,
-                           dtype=torch.float64 if acc_f64 else B.dtype)
+    sums, cut = None, 0
+    if kc.max_row_nnz is None or kc.max_row_nnz > keep:
+        table, sums, cut = kc.piece_slots((items, keep), table, n_dense_cols,
+                                          torch.float64 if acc_f64 else B.dtype)
     kc._keep.extend((table, order, sums))
     return _abi.bind(
         "spmm_sliced", _abi.dtype_code(B.dtype), 1 if acc_f64 else 0, kc.data.data_ptr(),
         kc.cols.data_ptr(), kc.rowptr.data_ptr(), kc.rowptr_bits, kc.n_rows, kc.nnz,
         n_dense_cols, table.data_ptr(), None if order is None else order.data_ptr(), items, keep,
-        None if sums is None else sums.data_ptr(), int(cut), lanes, vec, XCD_REMAP)
+        None if sums is None else sums.data_ptr(), cut, lanes, vec, XCD_REMAP)
 
 
 def _bind_row_blocks(kc, B, acc_f64, lanes, vec):
@@ -494,7 +518,7 @@ def _run_spmm(kc, B, C, acc_f64, tile_cols=None):
         kept = not kc.one_shot and (kc.max_row_nnz or 0) > _SPMM_SUMS_KEPT
         # the row-block kernel's loads need aligned vectors
         if kc.sliced() or (vec < slice_vec and not kept):
-            bound = _bind_sliced(kc, B, C, acc_f64, slice_lanes, slice_vec)
+            bound = _bind_sliced(kc, B, acc_f64, slice_lanes, slice_vec)
         else:
             bound = _bind_row_blocks(kc, B, acc_f64, lanes, vec)
         kc._args[key] = bound

@@ -71,6 +71,9 @@ extern "C" {
 /* Value type of data / x / y / B / C. */
 enum fsp_dtype { FSP_F32 = 0, FSP_F64 = 1 };
 
+/* Value of fsp_spmm_sliced's cut_rows (see there). */
+#define FSP_CUT_PIECES 2
+
 enum fsp_status {
   FSP_OK = 0,
   FSP_EINVAL = -1,   /* bad argument (sizes, null pointers, alignment, unsupported combo) */
@@ -457,6 +460,14 @@ int fsp_slice_table(const void* rowptr, int rowptr_bits, int64_t n_rows, int64_t
                     int64_t items, int64_t keep, int64_t* table, void* stream);
 
 /*
+ * For fsp_spmm_sliced with cut_rows = FSP_CUT_PIECES: behind the 2 * (n_slices + 1) boundaries of
+ * table, n_slices + 1 int32 (room for them is the caller's): the first piece of a cut row that each
+ * slice holds, counted through all slices, and at last the number of pieces.
+ */
+int fsp_slice_pieces(const void* rowptr, int rowptr_bits, int64_t n_slices, int64_t* table,
+                     void* stream);
+
+/*
  * A launch order of the slices for products whose dense operand (n_cols rows) is larger than an
  * L2: slices that lie inside one long row come last, by the column they start at.  order: n_slices
  * int32, order[b] = the slice of workgroup b; scratch: fsp_slice_order_scratch(n_slices) int32.
@@ -484,7 +495,8 @@ int fsp_part_order(const int32_t* desc, int64_t n_desc, const void* rowptr, int 
  *   sums           2 * slices * N slots of the accumulation type, 16-byte aligned: the pieces
  *                  of cut rows.  Calls sharing sums must not overlap.
  *   cut_rows       0: no row is longer than keep (sums may be NULL, and the second pass that
- *                  adds the pieces is left out)
+ *                  adds the pieces is left out); FSP_CUT_PIECES: sums holds N slots for each piece
+ *                  and no more, and table is followed by what fsp_slice_pieces writes
  *   lanes_per_row  G in {1,2,4,...,64}: lanes sharing one B row; a workgroup covers G * vec
  *                  columns
  *   vec            elements per lane per load: 1, 2 or 4 (fp32) / 1 or 2 (fp64), at most N;

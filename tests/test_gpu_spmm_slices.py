@@ -231,3 +231,59 @@ def test_parts_of_every_length(dev, monkeypatch, n, dtype, offset, longest):
     assert p._kernel_csr().kernel_name() == "spmm_rowblock_kernel"
     ref = oracle.spmm_csr(ptr, cols, data, B)
     assert torch.equal(out.double(), torch.as_tensor(ref).double())
+
+
+@pytest.mark.parametrize("name", sorted(set(LENGTHS) - {"empty"}))
+@pytest.mark.parametrize("N,dtype,acc", [(3, torch.float32, False), (47, torch.float32, True),
+                                         (130, torch.float64, True)])
+def test_room_for_cut_rows_only(dev, monkeypatch, name, N, dtype, acc):
+    """Where a slot for both ends of every slice is too much room: a slot for each piece of a cut
+    row, counted, and the same bits."""
+    vals, cols, ip, B, shape = _case(name, 901, N, dtype, dev)
+    C, plain = _run(vals, cols, ip, B, shape, dev, acc)
+    monkeypatch.setattr(spmm_csr, "_SUMS_ROOM", 0)
+    for one_shot in (True, False):
+        Cp, kc = _run(vals, cols, ip, B, shape, dev, acc, one_shot=one_shot)
+        if kc._tables:
+            assert torch.equal(C, Cp)
+        elif name != "one_row":
+            continue  # short rows, prepared: row blocks
+    (table, _), = plain._tables.values()
+    t = table.view(-1, 2).cpu()
+    inside = ip[t[1:-1, 0]] < t[1:-1, 1]  # boundaries inside a row: a piece before each, and
+    rows = t[1:-1, 0][inside]             # one after the row's last
+    want = int(inside.sum()) + int(torch.unique(rows).numel())
+    _, kc = _run(vals, cols, ip, B, shape, dev, acc)
+    cut = int((ip[1:] - ip[:-1]).max()) > next(iter(plain._tables))[1]
+    sums = kc._keep[-1]
+    assert (0 if sums is None else sums.numel()) == (want * N if cut else 0)
+    if cut:
+        (counted, n), = kc._pieces.values()
+        assert n == want and sums.numel() < plain._keep[-1].numel()
+
+
+def test_room_is_shared(dev):
+    # one width with B aligned and not, and again: one workspace
+    vals, cols, ip, B, shape = _case("at_keep", 901, 130, torch.float32, dev)
+    p = fs.prepare_spmm_csr_opt(vals.to(dev), cols.to(dev), ip.to(dev), shape)
+    flat = torch.empty(B.numel() + 1, device=dev)
+    Bu = flat[1:].view(B.shape)
+    Bu.copy_(B)
+    outs = [fs.flagsparse_spmm_csr_opt(B=b, prepared=p) for b in (B.to(dev), Bu, B.to(dev))]
+    assert len(p._kernel_csr()._args) == 2 and len(p._kernel_csr()._sums) == 1
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+def test_room_at_size(dev):
+    """A million rows with one that is cut, N = 256: three pieces take their own room, not 1 GB."""
+    n = 1_000_000
+    lengths = torch.full((n,), 32, dtype=torch.int64)
+    lengths[777] = 300
+    ptr = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
+    cols = torch.arange(int(ptr[-1]), dtype=torch.int32) % 1000
+    data = torch.ones(cols.numel())
+    p = fs.prepare_spmm_csr_opt(data.to(dev), cols.to(dev), ptr.to(dev), (n, 1000))
+    C = fs.flagsparse_spmm_csr_opt(B=torch.ones(1000, 256, device=dev), prepared=p)
+    assert torch.equal(C, lengths.float().to(dev)[:, None].expand_as(C))
+    (sums,) = p._kernel_csr()._sums.values()
+    assert 2 * 256 <= sums.numel() <= 5 * 256
