@@ -410,8 +410,9 @@ class _SpmmKernelCsr:
         either end of every slice, or, where that is too much, for each piece.  Calls are ordered
         (StreamOrder), so those of one size share it."""
         length, cut = (int(table.numel()) - 2) * n_dense_cols, 1
-        if length * dtype.itemsize > _SUMS_ROOM:
-            if items not in self._pieces:
+        if length * dtype.itemsize > _SUMS_ROOM and (
+                items in self._pieces or not torch.cuda.is_current_stream_capturing()):
+            if items not in self._pieces:  # the count is waited for, which a capture may not do
                 self._pieces[items] = _slices.pieces(self.rowptr, table)
             table, n = self._pieces[items]
             if n == 0:

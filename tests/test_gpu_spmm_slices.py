@@ -287,3 +287,22 @@ def test_room_at_size(dev):
     assert torch.equal(C, lengths.float().to(dev)[:, None].expand_as(C))
     (sums,) = p._kernel_csr()._sums.values()
     assert 2 * 256 <= sums.numel() <= 5 * 256
+
+
+def test_room_of_a_new_width_while_capturing(dev, monkeypatch):
+    # a width first used in a capture, on slices that exist: nothing is counted (a host wait)
+    vals, cols, ip, B, shape = _case("at_keep", 901, 33, torch.float32, dev)
+    p = fs.prepare_spmm_csr_opt(vals.to(dev), cols.to(dev), ip.to(dev), shape)
+    fs.flagsparse_spmm_csr_opt(B=torch.ones(901, 36, device=dev), prepared=p)
+    monkeypatch.setattr(spmm_csr, "_SUMS_ROOM", 0)
+    Bd = B.to(dev)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        C = fs.flagsparse_spmm_csr_opt(B=Bd, prepared=p)
+    for _ in range(3):
+        C.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert oracle.rel_l2(C, oracle.spmm_csr(ip, cols, vals, B)) <= 1e-5
+    assert torch.equal(fs.flagsparse_spmm_csr_opt(B=Bd.clone(), prepared=p), C)
