@@ -59,6 +59,8 @@ SIGNATURES = {
     "fsp_check_pinned_len": (_i64, []),
     "fsp_coo_check": (_i32, [_p, _i32, _p, _i32, _i64, _p, _p, _p, _p, _p]),
     "fsp_csr_check": (_i32, [_p, _i32, _i64, _p, _i32, _i64, _p, _p, _i32, _p, _p, _p]),
+    "fsp_csr_check_rows": (_i32, [_p, _i32, _i64, _p, _i32, _i64, _p, _p, _i32, _i64, _i64, _i64,
+                                  _p, _p, _p]),
     "fsp_spmv_scratch_slots": (_i64, []),
     "fsp_spmv_csr_static": (_i32, [_i32, _i32, _p, _p, _p, _i32, _i64, _i64, _p, _p, _p, _i64, _p,
                                    _p, _i64, _i64, _i64, _p, _p, _p, _i64, _i32, _p]),

@@ -22,10 +22,12 @@ def _pinned():
     return torch.empty(int(_abi.lib().fsp_check_pinned_len()), dtype=torch.int64, pin_memory=True)
 
 
-def csr_check(indices, indptr, ptr_bits=None):
+def csr_check(indices, indptr, ptr_bits=None, classes=None):
     """([first, last, decreases, longest row, min column, max column] as Python ints, the columns
     as int32, the row pointers at ``ptr_bits``) of contiguous 1-D device arrays (columns int32 or
-    int64; row pointers of another type are converted first).
+    int64; row pointers of another type are converted first).  ``classes`` (uneven, block, chunk):
+    two more ints, the rows of more than ``uneven`` and at most ``block`` entries and the entries in
+    rows of more than ``chunk``.
 
     The two arrays are the arguments themselves where they already have that width (or where
     ``ptr_bits`` is None); the column bounds are meaningless without entries.  Copies are made
@@ -47,14 +49,15 @@ def csr_check(indices, indptr, ptr_bits=None):
         ptr = torch.empty(n_rows + 1, dtype=torch.int32 if ptr_bits == 32 else torch.int64,
                           device=dev)
     pinned = _pinned()
-    out = (ctypes.c_int64 * 6)()
-    _abi.check(
-        L.fsp_csr_check(indices.data_ptr() if nnz else None, idx_bits, nnz, indptr.data_ptr(),
-                        have_bits, n_rows,
-                        idx32.data_ptr() if idx32 is not indices and nnz else None,
-                        None if ptr is indptr else ptr.data_ptr(), ptr_bits or have_bits,
-                        pinned.data_ptr(), ctypes.addressof(out), _abi.raw_stream(dev)),
-        "fsp_csr_check")
+    out = (ctypes.c_int64 * (6 if classes is None else 8))()
+    args = (indices.data_ptr() if nnz else None, idx_bits, nnz, indptr.data_ptr(), have_bits, n_rows,
+            idx32.data_ptr() if idx32 is not indices and nnz else None,
+            None if ptr is indptr else ptr.data_ptr(), ptr_bits or have_bits)
+    to = (pinned.data_ptr(), ctypes.addressof(out), _abi.raw_stream(dev))
+    if classes is None:
+        _abi.check(L.fsp_csr_check(*args, *to), "fsp_csr_check")
+    else:
+        _abi.check(L.fsp_csr_check_rows(*args, *classes, *to), "fsp_csr_check_rows")
     return list(out), idx32, ptr
 
 

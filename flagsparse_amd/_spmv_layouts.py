@@ -10,8 +10,8 @@ The layouts below, chosen once per matrix at prepare time:
 
 ``SliceLayout`` (csrc/slices.hip, ``spmv_slices_kernel``)
     The CSR arrays cut into slices of equal rows + entries, found by a search in the row pointers.
-    Right for matrices used once (nothing is planned) and for those with rows longer than a row
-    block, where the row-block layout would be taken.
+    Right for matrices used once (nothing is planned) and for skewed ones, where the row-block
+    layout would be taken (slices_pay).
 
 ``XcsLayout`` (csrc/spmv_xcs.hip, ``spmv_xcs_kernel``, ``xcs_window_combine_kernel``)
     Columns split into panels of about equal nnz (P of them, P / 8 per XCD in turn, or shared
@@ -1425,13 +1425,13 @@ def xcs_layout(data, cols, rowptr, n_cols, panels_per_xcd=None):
     return XcsLayout(data, cols, rowptr, n_cols, panels_per_xcd, item_format=0)
 
 
-def build_layout(data, cols, rowptr, n_cols, one_shot=False, max_row_nnz=None):
+def build_layout(data, cols, rowptr, n_cols, one_shot=False, max_row_nnz=None, row_classes=None):
     """The layout for one CSR (or COO row-run) matrix: XCS when it pays, else row blocks.
     one_shot: the layout serves a single call (no prepared object) and is asked for no run to
     row map, so the slices, which need no plan, are taken; the row blocks' plan alone takes 0.6
     ms for a million rows and the staged-x layout tens of milliseconds (a power law of 8.4M rows:
     28 ms for a 0.2 ms product).  max_row_nnz: the longest row of a CSR matrix, where the caller
-    knows it and asks for no row map."""
+    knows it and asks for no row map; row_classes: what the check counted by row_class_bounds."""
     mode = FORCE
     nnz = int(data.numel())
     if mode is None and one_shot:
@@ -1464,16 +1464,57 @@ def build_layout(data, cols, rowptr, n_cols, one_shot=False, max_row_nnz=None):
             return xcs_layout(data, cols, rowptr, n_cols, FORCE_PANELS_PER_XCD)
         except ValueError:
             pass  # too large for the packing: row blocks
-    if FORCE is None and max_row_nnz is not None and \
-            max_row_nnz > _abi.lib().fsp_spmv_stream_nnz_cap():
-        # Rows longer than a row block go through chunk workgroups and a second pass there, and a
-        # skewed matrix's blocks sum rows of very different lengths with the same lanes.  Measured
-        # on MI355X, row blocks / slices, power laws: float32, 40k rows of mean 12 29.7 / 8.7 us,
-        # 300k of 20 48.0 / 29.9, 900k of 6 56.2 / 34.2; float64, 300k of 20 51.4 / 35.7.  Without
-        # such rows they are level (900k rows of 0 to 12 entries 32.8 / 32.9), stencils apart,
-        # whose row blocks have a launch order of their own (float64 2048 x 2048 58.1 / 82.4).
+    if FORCE is None and row_classes is not None and \
+            slices_pay(cols, rowptr, n_cols, max_row_nnz, *row_classes):
         return SliceLayout(data, cols, rowptr, max_row_nnz)
     return RowBlockLayout(data, cols, rowptr)
+
+
+# When a prepared matrix that would run on row blocks runs on slices instead (slices_pay).
+SLICE_SKEW = 16          # a row this many times the mean, and at least SLICE_SKEW_MIN entries,
+SLICE_SKEW_MIN = 64      # holds up its row block, ...
+SLICE_SKEW_BLOCKS = 0.1  # ... and this many such rows to a block slow down the product
+SLICE_LONG_SHARE = 0.1   # share of the entries in rows of more than one chunk
+
+
+def row_class_bounds(n_rows, nnz):
+    """(uneven, block, chunk): the bounds whose counts slices_pay goes by."""
+    L = _abi.lib()
+    return (max(SLICE_SKEW_MIN, SLICE_SKEW * nnz // max(n_rows, 1)), L.fsp_spmv_stream_nnz_cap(),
+            L.fsp_spmv_chunk_nnz_cap())
+
+
+def slices_pay(cols, rowptr, n_cols, max_row_nnz, uneven_rows, cut_entries):
+    """Whether a prepared matrix runs on slices rather than row blocks, by the rows and entries of
+    its row_class_bounds.  Row blocks are the faster
+    where rows are alike: a block sums its rows with the same lanes each, nothing is searched, and
+    it can run in the order of its band.  They lose where
+    * rows of very different lengths share a block, whose other lanes wait for the longest: power
+      laws.  Row blocks / slices on MI355X, us, float32: 40k rows of mean 12 30.2 / 8.5, 300k of 20
+      49.8 / 28.0, 900k of 6 60.4 / 35.1, all with over 0.6 such rows to a block; 900k rows of 0 to
+      6 entries, one in 1000 of 400 (0.3 to a block) 38.0 / 25.2, 900k of 0 to 12 (0.16) 43.0 / 38.9;
+    * much of the matrix lies in rows that are cut into chunks, whose sums are a second pass: rows of
+      5000 among 1M of 12, 0.05 / 0.08 / 0.25 of the entries: 34.9 / 38.9, 43.6 / 41.4, 68.3 / 56.9.
+    One such row is no reason: a 2048 x 2048 stencil with a row of 20000 51.1 / 61.4 (float64 60.6 /
+    78.5), 1M rows of 12 31.2 / 35.2 (32.1 / 40.9), 300k random ones with a row of 1100 19.7 / 22.7.
+    Only where the columns are spread out they are level (300k random rows, a row of 20000: 22.6 /
+    22.6), and the slices stay.  Without a row longer than a block nothing is cut: row blocks."""
+    nnz = int(cols.numel())
+    _, block, chunk = row_class_bounds(int(rowptr.numel()) - 1, nnz)
+    if max_row_nnz <= block:
+        return False
+    if uneven_rows * block >= SLICE_SKEW_BLOCKS * nnz or cut_entries >= SLICE_LONG_SHARE * nnz:
+        return True
+    return max_row_nnz > chunk and not columns_local(cols, rowptr, n_cols)
+
+
+def columns_local(cols, rowptr, n_cols):
+    """Whether most entries lie within a sixteenth of the columns around their row's place."""
+    n_rows, nnz = int(rowptr.numel()) - 1, int(cols.numel())
+    at = sample_indices(nnz, 1 << 12, cols.device)
+    rows = torch.searchsorted(rowptr.to(torch.int64), at, right=True) - 1
+    place = (rows + 1) * (n_cols / (n_rows + 1))
+    return bool(((cols[at] - place).abs() <= n_cols / 16).double().mean() > 0.5)
 
 
 __all__ = ["RowBlockLayout", "SliceLayout", "XcsLayout", "PanelLayout", "XcsHybridLayout", "XstageLayout",

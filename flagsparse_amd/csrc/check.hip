@@ -34,6 +34,7 @@ constexpr int kThreads = 1024;
 constexpr int kWaves = kThreads / kWave;
 constexpr int64_t kStep = 4 * kThreads;  // elements a workgroup takes in one step
 constexpr int kCsrWords = 2;  // per workgroup: {min, ~max} of columns or {decreases, longest}
+constexpr int kRowWords = 4;  // the same, and from row pointers {uneven rows, entries in cut rows}
 constexpr int kCooWords = 5;  // {min, ~max} of rows, {min, ~max} of columns, decreases
 // What a word holds until its workgroup has stored it.
 constexpr int64_t kPending = LLONG_MIN + 0x5bd1e995;
@@ -112,15 +113,22 @@ __device__ __forceinline__ void publish(int64_t* host, int64_t v) {
   __hip_atomic_store(host, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// host: [0] = ptr[0], [1] = ptr[n_rows], then kCsrWords per workgroup.
+// What else is counted of the rows: those of more than `uneven` and at most `block` entries, and the
+// entries of those of more than `chunk`.  words: per workgroup, kCsrWords where nothing is.
+struct RowClasses {
+  int64_t uneven, block, chunk;
+  int words;
+};
+
+// host: [0] = ptr[0], [1] = ptr[n_rows], then rows.words per workgroup.
 template <typename I, typename P>
 __global__ __launch_bounds__(kThreads) void csr_check_kernel(
     const I* __restrict__ idx, int64_t nnz, const P* __restrict__ ptr, int64_t n_rows,
     int32_t* __restrict__ idx32, void* __restrict__ ptr_out, int ptr_out_bits, int idx_vec,
-    int idx_blocks, int64_t* host) {
+    int idx_blocks, RowClasses rows, int64_t* host) {
   __shared__ int64_t s_w[kWaves];
   const int tid = threadIdx.x;
-  int64_t a, b;
+  int64_t a, b, uneven = 0, cut = 0;
   if ((int)blockIdx.x < idx_blocks) {
     Bounds<I> c;
     const int64_t stride = (int64_t)idx_blocks * kStep;
@@ -158,13 +166,20 @@ __global__ __launch_bounds__(kThreads) void csr_check_kernel(
         const int64_t len = (int64_t)((uint64_t)q - (uint64_t)p);
         dec += q < p ? 1 : 0;
         longest = len > longest ? len : longest;
+        uneven += len > rows.uneven && len <= rows.block ? 1 : 0;
+        cut += len > rows.chunk ? len : 0;
       }
     }
     a = block_reduce<true>(dec, s_w);
     b = block_reduce<false>(~longest, s_w);
+    if (rows.words == kRowWords) {
+      uneven = block_reduce<true>(uneven, s_w);
+      cut = block_reduce<true>(cut, s_w);
+    }
   }
-  if (tid < kCsrWords)  // one store
-    publish(host + 2 + (int64_t)blockIdx.x * kCsrWords + tid, tid == 0 ? a : b);
+  if (tid < rows.words)  // one store
+    publish(host + 2 + (int64_t)blockIdx.x * rows.words + tid,
+            tid == 0 ? a : tid == 1 ? b : tid == 2 ? uneven : cut);
 }
 
 // host: kCooWords per workgroup.  row32 / col32: NULL, or the narrowed arrays.
@@ -243,22 +258,27 @@ int wait_words(const int64_t* host, int64_t n, hipStream_t st) {
 
 template <typename I, typename P>
 int run_csr_check(const void* idx, int64_t nnz, const void* ptr, int64_t n_rows, int32_t* idx32,
-                  void* ptr_out, int ptr_out_bits, int64_t* pinned, int64_t* out,
-                  hipStream_t st) {
+                  void* ptr_out, int ptr_out_bits, const RowClasses& rows, int64_t* pinned,
+                  int64_t* out, hipStream_t st) {
   const int64_t ib = nnz > 0 ? blocks_for(nnz, kStep, kCheckBlocks) : 0;
   const int64_t pb = blocks_for(n_rows + 1, 2 * kThreads, kCheckBlocks / 4);
-  const int64_t n = 2 + (ib + pb) * kCsrWords;
+  const int64_t n = 2 + (ib + pb) * rows.words;
   for (int64_t i = 0; i < n; ++i) pinned[i] = kPending;
   const int vec = reinterpret_cast<uintptr_t>(idx) % 16 == 0;
   hipLaunchKernelGGL((csr_check_kernel<I, P>), dim3((unsigned)(ib + pb)), dim3(kThreads), 0, st,
                      static_cast<const I*>(idx), nnz, static_cast<const P*>(ptr), n_rows, idx32,
-                     ptr_out, ptr_out_bits, vec, (int)ib, pinned);
+                     ptr_out, ptr_out_bits, vec, (int)ib, rows, pinned);
   int rc = check_hip(hipGetLastError(), "csr_check_kernel launch");
   if (!rc) rc = wait_words(pinned, n, st);
   if (rc) return rc;
-  int64_t mn = LLONG_MAX, nmx = LLONG_MAX, dec = 0, nlong = ~int64_t(0);
+  int64_t mn = LLONG_MAX, nmx = LLONG_MAX, dec = 0, nlong = ~int64_t(0), uneven = 0, cut = 0;
   for (int64_t b = 0; b < ib + pb; ++b) {
-    const int64_t u = pinned[2 + b * kCsrWords], v = pinned[2 + b * kCsrWords + 1];
+    const int64_t* w = pinned + 2 + b * rows.words;
+    const int64_t u = w[0], v = w[1];
+    if (rows.words == kRowWords) {
+      uneven += w[2];
+      cut += w[3];
+    }
     if (b < ib) {
       mn = u < mn ? u : mn;
       nmx = v < nmx ? v : nmx;
@@ -273,6 +293,10 @@ int run_csr_check(const void* idx, int64_t nnz, const void* ptr, int64_t n_rows,
   out[3] = ~nlong;
   out[4] = mn;
   out[5] = ~nmx;
+  if (rows.words == kRowWords) {
+    out[6] = uneven;
+    out[7] = cut;
+  }
   return FSP_OK;
 }
 
@@ -311,13 +335,15 @@ int run_coo_check(const void* row, const void* col, int64_t nnz, int32_t* row32,
 using namespace fsp;
 
 extern "C" int64_t fsp_check_pinned_len(void) {
-  const int64_t csr = 2 + 2 * kCheckBlocks * kCsrWords, coo = kCheckBlocks * kCooWords;
+  const int64_t csr = 2 + 2 * kCheckBlocks * kRowWords, coo = kCheckBlocks * kCooWords;
   return csr > coo ? csr : coo;
 }
 
-extern "C" int fsp_csr_check(const void* indices, int idx_bits, int64_t nnz, const void* indptr,
-                             int ptr_bits, int64_t n_rows, int32_t* idx32, void* ptr_out,
-                             int ptr_out_bits, int64_t* pinned, int64_t* out, void* stream) {
+namespace {
+
+int csr_check(const void* indices, int idx_bits, int64_t nnz, const void* indptr, int ptr_bits,
+              int64_t n_rows, int32_t* idx32, void* ptr_out, int ptr_out_bits,
+              const RowClasses& rows, int64_t* pinned, int64_t* out, void* stream) {
   if ((idx_bits != 32 && idx_bits != 64) || (ptr_bits != 32 && ptr_bits != 64) ||
       (ptr_out && ptr_out_bits != 32 && ptr_out_bits != 64))
     return set_error(FSP_EINVAL, "fsp_csr_check: index widths must be 32 or 64");
@@ -327,13 +353,31 @@ extern "C" int fsp_csr_check(const void* indices, int idx_bits, int64_t nnz, con
   if (reinterpret_cast<uintptr_t>(idx32) % 16)
     return set_error(FSP_EINVAL, "fsp_csr_check: idx32 must be 16-byte aligned");
   hipStream_t st = static_cast<hipStream_t>(stream);
-#define FSP_CHECK_ARGS indices, nnz, indptr, n_rows, idx32, ptr_out, ptr_out_bits, pinned, out, st
+#define FSP_CHECK_ARGS indices, nnz, indptr, n_rows, idx32, ptr_out, ptr_out_bits, rows, pinned, out, st
   if (idx_bits == 32)
     return ptr_bits == 32 ? run_csr_check<int32_t, int32_t>(FSP_CHECK_ARGS)
                           : run_csr_check<int32_t, int64_t>(FSP_CHECK_ARGS);
   return ptr_bits == 32 ? run_csr_check<int64_t, int32_t>(FSP_CHECK_ARGS)
                         : run_csr_check<int64_t, int64_t>(FSP_CHECK_ARGS);
 #undef FSP_CHECK_ARGS
+}
+
+}  // namespace
+
+extern "C" int fsp_csr_check(const void* indices, int idx_bits, int64_t nnz, const void* indptr,
+                             int ptr_bits, int64_t n_rows, int32_t* idx32, void* ptr_out,
+                             int ptr_out_bits, int64_t* pinned, int64_t* out, void* stream) {
+  return csr_check(indices, idx_bits, nnz, indptr, ptr_bits, n_rows, idx32, ptr_out, ptr_out_bits,
+                   RowClasses{0, 0, 0, kCsrWords}, pinned, out, stream);
+}
+
+extern "C" int fsp_csr_check_rows(const void* indices, int idx_bits, int64_t nnz,
+                                  const void* indptr, int ptr_bits, int64_t n_rows,
+                                  int32_t* idx32, void* ptr_out, int ptr_out_bits, int64_t uneven,
+                                  int64_t block, int64_t chunk, int64_t* pinned, int64_t* out,
+                                  void* stream) {
+  return csr_check(indices, idx_bits, nnz, indptr, ptr_bits, n_rows, idx32, ptr_out, ptr_out_bits,
+                   RowClasses{uneven, block, chunk, kRowWords}, pinned, out, stream);
 }
 
 extern "C" int fsp_coo_check(const void* rows, int row_bits, const void* cols, int col_bits,

@@ -11,8 +11,8 @@ as the reference's base path does (:498-536); ``use_opt=True`` accumulates in th
 rows exactly where the reference's static tile loop stops (:111-118 base, :308-314 opt).
 
 The kernels run over a layout built once per matrix (flagsparse_amd/_spmv_layouts.py): row blocks
-(csrc/spmv.hip); slices of equal work (csrc/slices.hip) where rows are longer than a row block or
-the matrix serves one call; or, when x gathers would miss L2, the staged-x layout
+(csrc/spmv.hip); slices of equal work (csrc/slices.hip) where rows are very uneven or the matrix
+serves one call; or, when x gathers would miss L2, the staged-x layout
 (csrc/spmv_xcs.hip).
 """
 
@@ -28,7 +28,7 @@ from ._common import (
 )
 from ._csr_check import csr_check
 from ._plan import truncate_rows
-from ._spmv_layouts import build_layout
+from ._spmv_layouts import build_layout, row_class_bounds
 
 # Opt-path buckets of the reference (max_row_nnz, block_size, num_warps, num_stages,
 # batch_rows) - spmv_csr.py:64-89.  Only their truncation effect under a caller's
@@ -88,6 +88,7 @@ class PreparedCsrSpmv:
         "_baseline_compute_dtype",
         "_baseline_data",
         "_one_shot",
+        "_row_classes",
     )
 
     def __init__(self, data, kernel_indices, kernel_indptr, shape, n_rows, n_cols, block_nnz,
@@ -102,6 +103,7 @@ class PreparedCsrSpmv:
         self.max_segments = max_segments
         self.max_row_nnz = max_row_nnz
         self._one_shot = False
+        self._row_classes = None
         self.supports_opt = data.dtype in (torch.float32, torch.float64)
         if data.dtype in (torch.float16, torch.bfloat16):
             self._baseline_compute_dtype = torch.float32
@@ -185,7 +187,8 @@ class PreparedCsrSpmv:
             if kc is None:
                 kc = build_layout(self.data, self.kernel_indices, self.kernel_indptr,
                                   self.n_cols, one_shot=self._one_shot,
-                                  max_row_nnz=self.max_row_nnz)
+                                  max_row_nnz=self.max_row_nnz,
+                                  row_classes=self._row_classes)
                 self._kernels["full"] = kc
         else:
             d, c, ip = truncate_rows(self.data, self.kernel_indices, self.kernel_indptr, caps)
@@ -194,8 +197,9 @@ class PreparedCsrSpmv:
         return kc
 
 
-def _prepare_spmv_csr_matrix(data, indices, indptr, shape):
-    """Validation and narrowing - spmv_csr.py:379-436 (same checks, order and exceptions)."""
+def _check_spmv_csr_matrix(data, indices, indptr, shape, one_shot):
+    """Validation and narrowing - spmv_csr.py:379-436 (same checks, order and exceptions), and, for a
+    matrix that is kept, the counts by which its layout is chosen (row_class_bounds)."""
     if not all(torch.is_tensor(t) for t in (data, indices, indptr)):
         raise TypeError("data, indices, indptr must all be torch.Tensor")
     if data.ndim != 1 or indices.ndim != 1 or indptr.ndim != 1:
@@ -221,8 +225,10 @@ def _prepare_spmv_csr_matrix(data, indices, indptr, shape):
     # one pass over the index arrays, one host synchronisation
     ptr_bits = 32 if nnz <= _INDEX_LIMIT_INT32 else 64
     no_rows = indptr.numel() == 0  # n_rows of -1: nothing to check in the row pointers
-    (first, last, decreases, max_row_nnz, min_index, max_index), kernel_indices, kernel_indptr = \
-        csr_check(indices, indptr.new_zeros(1) if no_rows else indptr, ptr_bits)
+    stats, kernel_indices, kernel_indptr = csr_check(
+        indices, indptr.new_zeros(1) if no_rows else indptr, ptr_bits,
+        None if one_shot else row_class_bounds(n_rows, nnz))
+    first, last, decreases, max_row_nnz, min_index, max_index = stats[:6]
     if not no_rows:
         if first != 0:
             raise ValueError("indptr must start at zero")
@@ -235,7 +241,8 @@ def _prepare_spmv_csr_matrix(data, indices, indptr, shape):
             raise IndexError("indices out of range for n_cols")
         if max_index > _INDEX_LIMIT_INT32:
             raise ValueError(f"int64 column index {max_index} exceeds Triton int32 kernel range")
-    return data, kernel_indices, kernel_indptr, n_rows, n_cols, max_row_nnz
+    return (data, kernel_indices, kernel_indptr, n_rows, n_cols, max_row_nnz,
+            None if one_shot else stats[6:])
 
 
 def _validate_spmv_x(x, prepared):
@@ -263,8 +270,8 @@ def prepare_spmv_csr(data, indices, indptr, shape, block_nnz=256, max_segments=N
 def _prepare_spmv_csr(data, indices, indptr, shape, block_nnz, max_segments, one_shot):
     """prepare_spmv_csr; one_shot marks a prepared object made for a single call (the layout
     that builds fastest)."""
-    (data, kernel_indices, kernel_indptr, n_rows, n_cols,
-     max_row_nnz) = _prepare_spmv_csr_matrix(data, indices, indptr, shape)
+    (data, kernel_indices, kernel_indptr, n_rows, n_cols, max_row_nnz,
+     row_classes) = _check_spmv_csr_matrix(data, indices, indptr, shape, one_shot)
     block_nnz_use = block_nnz
     if max_segments is None:
         max_segments_use = max((max_row_nnz + block_nnz_use - 1) // block_nnz_use, 1)
@@ -276,6 +283,7 @@ def _prepare_spmv_csr(data, indices, indptr, shape, block_nnz, max_segments, one
     prepared = PreparedCsrSpmv(data, kernel_indices, kernel_indptr, shape, n_rows, n_cols,
                                block_nnz_use, max_segments_use, max_row_nnz, max_segments)
     prepared._one_shot = bool(one_shot)
+    prepared._row_classes = row_classes
     if prepared.supports_opt and n_rows > 0 and not one_shot:
         prepared._kernel(False)  # build the descriptor table now, outside the timed calls
     if not one_shot:  # the narrowed copies may be read on other streams than this one

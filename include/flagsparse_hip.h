@@ -165,6 +165,8 @@ int fsp_plan_panel_chunks_device(const int64_t* panel_runs, int64_t n_panels,
  * The call returns when the results are there (it waits for the check, not for later work of the
  * stream; it cannot be captured).  The narrowed copies are complete for work queued after it on
  * the stream, and hold meaningless values where the checks fail.
+ * fsp_csr_check_rows: the same with 8 int64 in out: behind those six, the number of rows of more
+ * than `uneven` and at most `block` entries, and the entries in rows of more than `chunk`.
  * fsp_coo_check: the same for nnz >= 1 row and column indices; row32, col32 NULL or nnz int32
  * (16-byte aligned) for the narrowed arrays; out: smallest and largest row, smallest and largest
  * column, the number of places where the rows decrease.
@@ -173,6 +175,10 @@ int64_t fsp_check_pinned_len(void);
 int fsp_csr_check(const void* indices, int idx_bits, int64_t nnz, const void* indptr,
                   int ptr_bits, int64_t n_rows, int32_t* idx32, void* ptr_out, int ptr_out_bits,
                   int64_t* pinned, int64_t* out, void* stream);
+int fsp_csr_check_rows(const void* indices, int idx_bits, int64_t nnz, const void* indptr,
+                       int ptr_bits, int64_t n_rows, int32_t* idx32, void* ptr_out,
+                       int ptr_out_bits, int64_t uneven, int64_t block, int64_t chunk,
+                       int64_t* pinned, int64_t* out, void* stream);
 int fsp_coo_check(const void* rows, int row_bits, const void* cols, int col_bits, int64_t nnz,
                   int32_t* row32, int32_t* col32, int64_t* pinned, int64_t* out, void* stream);
 

@@ -151,3 +151,35 @@ def test_one_call_errors(dev):
         with pytest.raises(kind, match=text):
             fs.flagsparse_spmv_csr(vals.to(dev), c.to(dev), p.to(dev), x, (4, 10), out=y)
         assert bool((y == 7.0).all())
+
+
+@pytest.mark.parametrize("ptr", [torch.int32, torch.int64])
+@pytest.mark.parametrize("n_rows", [0, 1, 2047, 2048, 300001])
+def test_csr_check_row_classes(dev, ptr, n_rows):
+    lengths = synthetic.randint(4, n_rows, n_rows, 40, "cpu") ** 2
+    ip = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
+    cols = torch.zeros(int(ip[-1]), dtype=torch.int32)
+    stats, _, _ = csr_check(cols.to(dev), ip.to(ptr).to(dev), 32, (100, 1000, 1200))
+    plain, _, _ = csr_check(cols.to(dev), ip.to(ptr).to(dev), 32)
+    assert stats[:6] == plain and len(plain) == 6
+    assert stats[6:] == [int(((lengths > 100) & (lengths <= 1000)).sum()),
+                         int(lengths[lengths > 1200].sum())]
+
+
+@pytest.mark.parametrize("long_row", [1100, 20000])
+def test_stencil_with_a_dense_row_keeps_its_band_order(dev, long_row):
+    side = 700
+    i = torch.arange(side * side)
+    r, c = i // side, i % side
+    valid = torch.stack([r > 0, c > 0, r >= 0, c < side - 1, r < side - 1], 1)
+    cols = (i[:, None] + torch.tensor([-side, -1, 0, 1, side])[None, :])[valid]
+    more = torch.arange(long_row) * (side * side // long_row)
+    lengths = torch.cat([valid.sum(1), torch.tensor([long_row])])
+    ip = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
+    cols = torch.cat([cols, more])
+    vals = synthetic.uniform_values(5, 2, cols.numel(), torch.float64, "cpu")
+    x = synthetic.uniform_values(5, 3, side * side, torch.float64, "cpu")
+    p = fs.prepare_spmv_csr(vals.to(dev), cols.to(dev), ip.to(dev), (ip.numel() - 1, side * side))
+    assert p._kernel(False).kind == "rowblock" and p._kernel(False).band_offset is not None
+    y = fs.flagsparse_spmv_csr(x=x.to(dev), prepared=p)
+    assert oracle.rel_l2(y, oracle.spmv_csr(ip, cols, vals, x)) <= 1e-12

@@ -1,9 +1,10 @@
 """The rules that pick slice sizes and launch orders (no GPU)."""
 
+import numpy as np
 import pytest
 import torch
 
-from flagsparse_amd import _slices, sddmm_csr, spmm_csr
+from flagsparse_amd import _slices, _spmv_layouts, sddmm_csr, spmm_csr
 
 
 @pytest.mark.parametrize("n,dtype,tile,want", [
@@ -46,3 +47,55 @@ def test_ordered_rule():
     assert not _slices.ordered(5000, 256, 4 << 20, big, True)  # fits an L2
     assert not _slices.ordered(5000, 256, big, 200 << 20, True)
     assert _slices.ordered(5000, 256, big, 200 << 20, False)
+
+
+def _stencil(side):
+    i = torch.arange(side * side)
+    r, c = i // side, i % side
+    valid = torch.stack([r > 0, c > 0, r >= 0, c < side - 1, r < side - 1], 1)
+    cols = (i[:, None] + torch.tensor([-side, -1, 0, 1, side])[None, :])[valid]
+    return valid.sum(1), cols, side * side
+
+
+def _random(lengths, n_cols):
+    gen = torch.Generator().manual_seed(1)
+    lengths = torch.as_tensor(lengths)
+    return lengths, torch.randint(0, n_cols, (int(lengths.sum()),), generator=gen), n_cols
+
+
+def _with_rows(matrix, rows, length):
+    """``rows`` rows of ``length`` spread-out entries in the middle of a matrix."""
+    lengths, cols, n_cols = matrix
+    half = lengths.numel() // 2
+    entries = int(lengths[:half].sum())
+    _, more, _ = _random([length] * rows, n_cols)
+    return (torch.cat([lengths[:half], torch.full((rows,), length), lengths[half:]]),
+            torch.cat([cols[:entries], more, cols[entries:]]), n_cols)
+
+
+_ZIPF = torch.as_tensor(np.minimum(np.random.default_rng(2).zipf(1.8, 40000), 9000))
+
+
+@pytest.mark.parametrize("matrix,want", [
+    # local or alike rows with a few long ones keep the row blocks and their launch order
+    (_with_rows(_stencil(300), 1, 1100), False), (_with_rows(_stencil(300), 1, 20000), False),
+    (_with_rows(_random([12] * 40000, 40000), 1, 1100), False),
+    (_with_rows(_random([12] * 40000, 40000), 20, 2000), False),
+    # no row longer than a block
+    (_with_rows(_random([2] * 40000, 40000), 2000, 400), False),
+    # rows of very different lengths side by side
+    (_random(_ZIPF, 40000), True),
+    (_with_rows(_with_rows(_random([6] * 40000, 40000), 60, 400), 1, 3000), True),
+    # a large share in rows cut into chunks; spread-out columns with one of those
+    (_with_rows(_stencil(300), 20, 5000), True),
+    (_with_rows(_random([12] * 40000, 40000), 1, 5000), True),
+])
+def test_prepared_spmv_layout_rule(matrix, want):
+    lengths, cols, n_cols = matrix
+    rowptr = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)]).to(torch.int32)
+    cols = cols.to(torch.int32)
+    uneven, block, chunk = _spmv_layouts.row_class_bounds(lengths.numel(), cols.numel())
+    assert _spmv_layouts.slices_pay(
+        cols, rowptr, n_cols, int(lengths.max()),
+        int(((lengths > uneven) & (lengths <= block)).sum()),
+        int(lengths[lengths > chunk].sum())) == want
