@@ -162,6 +162,14 @@ def ptr(t):
     return None if t is None else ctypes.c_void_p(t.data_ptr())
 
 
+class Calls(dict):
+    """Calls with their arguments converted once, by mode; they hold plain addresses.  A copy of the
+    object that keeps them (copy, pickle) has other arrays, so it starts without any."""
+
+    def __reduce__(self):
+        return Calls, ()
+
+
 def bind(name, *args):
     """The call ``name`` with every argument but its input, output and stream filled in
     (fsp_bind_*): ``run(bound, input, output, stream)`` makes it, with plain addresses.  The

@@ -183,7 +183,7 @@ class RowBlockLayout:
                 self.plan.desc = self.plan.desc[order].contiguous()
                 self.plan.ranges = self.plan.ranges[order].contiguous()
                 self.band_offset = off
-        self._args = {}
+        self._args = _abi.Calls()
         self._keep = None
         self._order = StreamOrder(self.data.device)
 
@@ -253,9 +253,9 @@ class SliceLayout:
                                          _abi.raw_stream(scratch.device)), "fsp_slice_table")
         self.cut_rows = cut_rows
         self._keep = (scratch, self.data, self.cols, self.rowptr)
-        self._sums = scratch.data_ptr() + 16 * (n + 1)
+        self._sums_at = 16 * (n + 1)  # in scratch, behind the table
         self._table_built = int(not one_shot)
-        self._args = {}
+        self._args = _abi.Calls()
         self._order = StreamOrder(self.data.device)
 
     def kernel_name(self):
@@ -278,7 +278,7 @@ class SliceLayout:
                 "spmv_sliced", _abi.dtype_code(self.data.dtype), int(acc_f64),
                 self.data.data_ptr(), self.cols.data_ptr(), self.rowptr.data_ptr(),
                 self.rowptr_bits, self.n_rows, self.nnz, self._keep[0].data_ptr(),
-                self._table_built, self._sums, int(self.cut_rows))
+                self._table_built, self._keep[0].data_ptr() + self._sums_at, int(self.cut_rows))
             self._args[bool(acc_f64)] = bound
         _abi.run(bound, x.data_ptr(), y.data_ptr(), self._order.stream(y.device, self._keep))
         return y
@@ -730,7 +730,7 @@ class XcsLayout:
         args = self._args.get(bool(acc_f64)) if hasattr(self, "_args") else None
         if args is None:
             if not hasattr(self, "_args"):
-                self._args = {}
+                self._args = _abi.Calls()
             p = lambda t: t.data_ptr() if t is not None and t.numel() else None  # noqa: E731
             args = [_abi.dtype_code(self.vals.dtype), int(acc_f64), p(self.vals), p(self.pidx),
                     self.n_entries, self.col_bits, None, None, None, 0, p(self.items),
@@ -975,7 +975,7 @@ class PanelLayout:
         # every array a launch reads or writes (marked as used on a new caller stream)
         self._keep = (self.partials, self.vals, self.pcol, self.jobs, self.job_panel,
                       self.chunk_info, self.rows, self.row_ptr, self.slots)
-        self._args = {}
+        self._args = _abi.Calls()
         self._order = StreamOrder(dev)
 
     def kernel_name(self):
@@ -1055,7 +1055,7 @@ class XcsHybridLayout:
         # the long rows have no sums in the XCS part: its windows leave them to the panel rows
         if long_rows.numel():
             self.short.row_count[long_rows] = ROW_SKIP
-        self._args = {}
+        self._args = _abi.Calls()
 
     def kernel_name(self):
         return "spmv_xcs_kernel+spmv_panel_kernel"
@@ -1322,7 +1322,7 @@ class XstageLayout:
                       self.stage_jobs)
         if self.long is not None:
             self._keep = self._keep + self.long._keep
-        self._args = {}
+        self._args = _abi.Calls()
         self._order = StreamOrder(dev)
 
     def kernel_name(self):

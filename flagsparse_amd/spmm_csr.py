@@ -370,7 +370,7 @@ class _SpmmKernelCsr:
         self._pieces = {}
         self._sums = {}
         self._plans = {}
-        self._args = {}
+        self._args = _abi.Calls()
         self._keep = [self.data, self.cols, self.rowptr]  # what a launch reads or writes
         self._order = StreamOrder(self.data.device)
 

@@ -1,10 +1,13 @@
 """The rules that pick slice sizes and launch orders (no GPU)."""
 
+import copy
+import pickle
+
 import numpy as np
 import pytest
 import torch
 
-from flagsparse_amd import _slices, _spmv_layouts, sddmm_csr, spmm_csr
+from flagsparse_amd import _abi, _slices, _spmv_layouts, sddmm_csr, spmm_csr
 
 
 @pytest.mark.parametrize("n,dtype,tile,want", [
@@ -99,3 +102,9 @@ def test_prepared_spmv_layout_rule(matrix, want):
         cols, rowptr, n_cols, int(lengths.max()),
         int(((lengths > uneven) & (lengths <= block)).sum()),
         int(lengths[lengths > chunk].sum())) == want
+
+
+def test_copies_start_without_calls():
+    calls = _abi.Calls(base=("buffer", 4096))
+    assert dict(calls) and not copy.deepcopy({"a": calls})["a"]
+    assert not copy.copy(calls) and not pickle.loads(pickle.dumps(calls))
