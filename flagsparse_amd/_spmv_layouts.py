@@ -203,26 +203,30 @@ class RowBlockLayout:
                 "split_rows": self.plan.n_split_rows, "partials": self.plan.n_parts,
                 "band_block_offset": self.band_offset}
 
+    def bind(self, acc_f64, row_map=None, n_out=0):
+        """The call with the arguments that do not change, converted once per accumulation mode and
+        row map (a matrix has one or none; the bound call keeps it): by prepare for the mode that is
+        the default, by the first launch for the other."""
+        plan = self.plan
+        groups, group_base, split_rows = plan.split_groups()
+        self._keep = (plan.workspace(), groups, group_base, split_rows, plan.desc, plan.ranges,
+                      self.data, self.cols, self.rowptr, row_map)
+        bound = _abi.bind(
+            "spmv_csr", _abi.dtype_code(self.data.dtype), int(acc_f64), self.data.data_ptr(),
+            self.cols.data_ptr(), self.rowptr.data_ptr(), self.rowptr_bits, self.n_rows, self.nnz,
+            None if row_map is None else row_map.data_ptr(), n_out, plan.desc.data_ptr(),
+            plan.ranges.data_ptr(), plan.n_desc, plan.chunk, self._keep[0].data_ptr(),
+            groups.data_ptr() if groups.numel() else None,
+            group_base.data_ptr() if group_base.numel() else None,
+            split_rows.data_ptr() if split_rows.numel() else None, int(groups.shape[0]),
+            XCD_REMAP_ROWBLOCK) + (row_map,)
+        self._args[bool(acc_f64), row_map is None, n_out] = bound
+        return bound
+
     def launch(self, x, y, acc_f64, row_map=None, n_out=0):
-        # The arguments that do not change between calls are bound once, per accumulation mode
-        # and row map (a matrix has one or none; the bound call keeps it).
-        key = (bool(acc_f64), row_map is None, n_out)
-        bound = self._args.get(key)
+        bound = self._args.get((bool(acc_f64), row_map is None, n_out))
         if bound is None or bound[2] is not row_map:
-            plan = self.plan
-            groups, group_base, split_rows = plan.split_groups()
-            self._keep = (plan.workspace(), groups, group_base, split_rows, plan.desc,
-                          plan.ranges, self.data, self.cols, self.rowptr)
-            bound = _abi.bind(
-                "spmv_csr", _abi.dtype_code(self.data.dtype), int(acc_f64), self.data.data_ptr(),
-                self.cols.data_ptr(), self.rowptr.data_ptr(), self.rowptr_bits, self.n_rows,
-                self.nnz, None if row_map is None else row_map.data_ptr(), n_out,
-                plan.desc.data_ptr(), plan.ranges.data_ptr(), plan.n_desc, plan.chunk,
-                self._keep[0].data_ptr(), groups.data_ptr() if groups.numel() else None,
-                group_base.data_ptr() if group_base.numel() else None,
-                split_rows.data_ptr() if split_rows.numel() else None, int(groups.shape[0]),
-                XCD_REMAP_ROWBLOCK) + (row_map,)
-            self._args[key] = bound
+            bound = self.bind(acc_f64, row_map, n_out)
         _abi.run(bound, x.data_ptr(), y.data_ptr(), self._order.stream(y.device, self._keep))
         return y
 
@@ -270,16 +274,20 @@ class SliceLayout:
     def describe(self):
         return {"layout": self.kind, "cut_rows": self.cut_rows}
 
+    def bind(self, acc_f64):
+        """See RowBlockLayout.bind."""
+        bound = self._args[bool(acc_f64)] = _abi.bind(
+            "spmv_sliced", _abi.dtype_code(self.data.dtype), int(acc_f64), self.data.data_ptr(),
+            self.cols.data_ptr(), self.rowptr.data_ptr(), self.rowptr_bits, self.n_rows, self.nnz,
+            self._keep[0].data_ptr(), self._table_built, self._keep[0].data_ptr() + self._sums_at,
+            int(self.cut_rows))
+        return bound
+
     def launch(self, x, y, acc_f64, row_map=None, n_out=0):
         assert row_map is None, "slices write every row"
         bound = self._args.get(bool(acc_f64))
         if bound is None:
-            bound = _abi.bind(
-                "spmv_sliced", _abi.dtype_code(self.data.dtype), int(acc_f64),
-                self.data.data_ptr(), self.cols.data_ptr(), self.rowptr.data_ptr(),
-                self.rowptr_bits, self.n_rows, self.nnz, self._keep[0].data_ptr(),
-                self._table_built, self._keep[0].data_ptr() + self._sums_at, int(self.cut_rows))
-            self._args[bool(acc_f64)] = bound
+            bound = self.bind(acc_f64)
         _abi.run(bound, x.data_ptr(), y.data_ptr(), self._order.stream(y.device, self._keep))
         return y
 

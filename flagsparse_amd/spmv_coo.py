@@ -169,7 +169,9 @@ def _prepare_spmv_coo(data, row, col, shape, sort_by_row, one_shot):
     prepared = PreparedCoo(d, kr, kc, shape, seg_starts=seg)
     prepared._one_shot = bool(one_shot)
     if prepared.use_seg_kernel:
-        prepared._run_layout()
+        layout = prepared._run_layout()
+        if not one_shot and isinstance(layout, RowBlockLayout):
+            layout.bind(d.dtype == torch.float64, prepared._run_rows, prepared.n_rows)
     return prepared
 
 

@@ -28,7 +28,7 @@ from ._common import (
 )
 from ._csr_check import csr_check
 from ._plan import truncate_rows
-from ._spmv_layouts import build_layout, row_class_bounds
+from ._spmv_layouts import RowBlockLayout, SliceLayout, build_layout, row_class_bounds
 
 # Opt-path buckets of the reference (max_row_nnz, block_size, num_warps, num_stages,
 # batch_rows) - spmv_csr.py:64-89.  Only their truncation effect under a caller's
@@ -285,7 +285,9 @@ def _prepare_spmv_csr(data, indices, indptr, shape, block_nnz, max_segments, one
     prepared._one_shot = bool(one_shot)
     prepared._row_classes = row_classes
     if prepared.supports_opt and n_rows > 0 and not one_shot:
-        prepared._kernel(False)  # build the descriptor table now, outside the timed calls
+        layout = prepared._kernel(False)  # build the descriptor table now, outside the timed calls
+        if isinstance(layout, (RowBlockLayout, SliceLayout)):
+            layout.bind(True)  # the default sums in float64
     if not one_shot:  # the narrowed copies may be read on other streams than this one
         torch.cuda.current_stream(data.device).synchronize()
     return prepared

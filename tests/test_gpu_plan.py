@@ -14,6 +14,7 @@ import numpy as np
 import pytest
 import torch
 
+import flagsparse_amd as fs
 from flagsparse_amd import _abi
 from flagsparse_amd._plan import build_row_block_plan_device
 
@@ -153,3 +154,27 @@ def test_device_panel_chunk_plan_matches_host(dev, seed):
             auto = _spmv_layouts.plan_panel_chunks(pr.to(dev), rl.to(dev), chunk, cap)
             for got in (kern, auto):
                 assert torch.equal(got[0].cpu(), host[0]) and torch.equal(got[1].cpu(), host[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("lengths", [[3, 0, 5, 7] * 300, [3, 9000, 5] * 30])
+def test_prepare_converts_the_default_call(dev, monkeypatch, dtype, lengths):
+    """The first product of a prepared matrix converts no arguments: prepare did, for the default
+    accumulation (CSR: float64; COO: the values' type)."""
+    ip = torch.cat([torch.zeros(1, dtype=torch.int64), torch.as_tensor(lengths).cumsum(0)])
+    cols = torch.arange(int(ip[-1])) % 3000
+    vals = torch.ones(cols.numel(), dtype=dtype)
+    row = torch.repeat_interleave(torch.arange(len(lengths)), ip[1:] - ip[:-1])
+    shape, x = (len(lengths), 3000), torch.ones(3000, dtype=dtype, device=dev)
+    csr = fs.prepare_spmv_csr(vals.to(dev), cols.to(dev), ip.to(dev), shape)
+    coo = fs.prepare_spmv_coo(vals.to(dev), row.to(dev), cols.to(dev), shape)
+
+    def refuse(*args):
+        raise AssertionError("arguments converted by a call")
+
+    monkeypatch.setattr(_abi, "bind", refuse)
+    want = torch.as_tensor(lengths, dtype=dtype, device=dev)
+    assert torch.equal(fs.flagsparse_spmv_csr(x=x, prepared=csr), want)
+    assert torch.equal(fs.flagsparse_spmv_coo(x=x, prepared=coo), want)
+    monkeypatch.undo()
+    assert torch.equal(fs.flagsparse_spmv_csr(x=x, prepared=csr, use_opt=True), want)
