@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace fsp {
 
 constexpr int kWave = 64;
@@ -31,8 +33,11 @@ __device__ __forceinline__ V ld_stream(const V* p) {
 // Four consecutive matrix entries ("a quad"): values converted to the accumulator type.
 // base is a multiple of 4, so the 16-byte vector loads are aligned when the array base is.
 // Entries outside [lo, hi) are returned with val = 0 and col = -1.  P counts to nnz_total and no
-// further (a 32-bit P reaches 2^31 - 1), so nothing past the entries is computed in it: a caller
-// compares a quad's offset with the length of its range and adds the offset only inside it.
+// further (a 32-bit P reaches 2^31 - 1), so a position that may lie past the entries is computed
+// and compared as Wide<P>, which the span of a workgroup cannot take past its end.
+template <typename P>
+using Wide = std::make_unsigned_t<P>;
+
 template <bool NT, typename T>
 struct QuadLoader;
 
@@ -42,7 +47,7 @@ struct QuadLoader<NT, float> {
   __device__ __forceinline__ static void load(const float* __restrict__ vals,
                                               const int* __restrict__ cols, P base, P lo,
                                               P hi, P nnz_total, float (&v)[4], int (&c)[4]) {
-    if (base <= nnz_total - 4) {
+    if (Wide<P>(base) + 4 <= Wide<P>(nnz_total)) {
       f32x4 vv = ld_stream<NT>(reinterpret_cast<const f32x4*>(vals + base));
       i32x4 cc = ld_stream<NT>(reinterpret_cast<const i32x4*>(cols + base));
       v[0] = vv.x; v[1] = vv.y; v[2] = vv.z; v[3] = vv.w;
@@ -69,7 +74,7 @@ struct QuadLoader<NT, double> {
   __device__ __forceinline__ static void load(const double* __restrict__ vals,
                                               const int* __restrict__ cols, P base, P lo,
                                               P hi, P nnz_total, double (&v)[4], int (&c)[4]) {
-    if (base <= nnz_total - 4) {
+    if (Wide<P>(base) + 4 <= Wide<P>(nnz_total)) {
       f64x2 v01 = ld_stream<NT>(reinterpret_cast<const f64x2*>(vals + base));
       f64x2 v23 = ld_stream<NT>(reinterpret_cast<const f64x2*>(vals + base + 2));
       i32x4 cc = ld_stream<NT>(reinterpret_cast<const i32x4*>(cols + base));

@@ -270,15 +270,14 @@ __global__ __launch_bounds__(kBlock) void spmv_slices_kernel(
   if (R64 < 0 || R64 > kSlots || p1 < p0 || p1 - p0 > P(kSlots - 3)) return;  // uniform
   const int R = (int)R64, n = (int)(p1 - p0);
   const P s0 = p0 & ~P(3);
-  const int span = (int)(p1 - s0), lead = (int)(p0 - s0);
 
   T v[kUPT][4];
   int c[kUPT][4];
 #pragma unroll
   for (int u = 0; u < kUPT; ++u) {
-    const int off = 4 * (tid + u * kBlock);
-    if (off < span) {
-      QuadLoader<false, T>::load(vals, cols, P(s0 + off), p0, p1, nnz_total, v[u], c[u]);
+    const Wide<P> base = Wide<P>(s0) + 4 * (tid + u * kBlock);
+    if (base < Wide<P>(p1)) {
+      QuadLoader<false, T>::load(vals, cols, P(base), p0, p1, nnz_total, v[u], c[u]);
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j) { v[u][j] = T(0); c[u][j] = -1; }
@@ -300,10 +299,10 @@ __global__ __launch_bounds__(kBlock) void spmv_slices_kernel(
   gather_x<kUPT, A>(x, c, n > 0, xv);
 #pragma unroll
   for (int u = 0; u < kUPT; ++u) {
-    const int off = 4 * (tid + u * kBlock) - lead;
+    const Wide<P> base = Wide<P>(s0) + 4 * (tid + u * kBlock);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
-      if (c[u][j] >= 0) s_prod[off + j] = A(v[u][j]) * A(xv[u][j]);
+      if (c[u][j] >= 0) s_prod[(int)(base + j - Wide<P>(p0))] = A(v[u][j]) * A(xv[u][j]);
   }
 #pragma unroll
   for (int u = 0; u < kPtrPT; ++u) {

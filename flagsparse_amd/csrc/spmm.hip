@@ -154,14 +154,13 @@ __global__ __launch_bounds__(kBlock) void spmm_rowblock_kernel(
   // Stage the (col, val) entries [lo, hi) into LDS with 16-byte loads.
   {
     const P s0 = lo & ~P(3);
-    const int span = (int)(hi - s0), head = (int)(lo - s0);
     T v[kStageUPT][4];
     int c[kStageUPT][4];
 #pragma unroll
     for (int u = 0; u < kStageUPT; ++u) {
-      const int off = 4 * (tid + u * kBlock);
-      if (off < span) {
-        QuadLoader<NT, T>::load(vals, cols, P(s0 + off), lo, hi, nnz_total, v[u], c[u]);
+      const Wide<P> base = Wide<P>(s0) + 4 * (tid + u * kBlock);
+      if (base < Wide<P>(hi)) {
+        QuadLoader<NT, T>::load(vals, cols, P(base), lo, hi, nnz_total, v[u], c[u]);
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) { v[u][j] = T(0); c[u][j] = -1; }
@@ -169,11 +168,11 @@ __global__ __launch_bounds__(kBlock) void spmm_rowblock_kernel(
     }
 #pragma unroll
     for (int u = 0; u < kStageUPT; ++u) {
-      const int off = 4 * (tid + u * kBlock) - head;
+      const Wide<P> base = Wide<P>(s0) + 4 * (tid + u * kBlock);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (c[u][j] >= 0) {
-          const int o = off + j;
+          const int o = (int)(base + j - Wide<P>(lo));
           s_col[o] = c[u][j];
           s_val[o] = v[u][j];
         }
@@ -320,16 +319,14 @@ __global__ __launch_bounds__(kBlock / VW) void spmm_ragged_kernel(
   const int len = (int)(hi - lo);
   const bool staged = len <= slots;
   if (staged) {
-    const P s0 = lo & ~P(3);
-    const int span = (int)(hi - s0), head = (int)(lo - s0);
-    for (int off = 4 * tid; off < span; off += 4 * kThreads) {
+    for (Wide<P> base = Wide<P>(lo & ~P(3)) + 4 * tid; base < Wide<P>(hi); base += 4 * kThreads) {
       T v[4];
       int c[4];
-      QuadLoader<true, T>::load(vals, cols, P(s0 + off), lo, hi, nnz_total, v, c);
+      QuadLoader<true, T>::load(vals, cols, P(base), lo, hi, nnz_total, v, c);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (c[j] >= 0) {
-          const int o = off - head + j;
+          const int o = (int)(base + j - Wide<P>(lo));
           s_col[o] = c[j];
           s_val[o] = v[j];
         }

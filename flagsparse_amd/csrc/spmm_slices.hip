@@ -103,14 +103,13 @@ __global__ __launch_bounds__(kBlock, 8) void spmm_slices_kernel(
   const int R = (int)R64, n = (int)(p1 - p0);
   {
     const P s0 = p0 & ~P(3);
-    const int span = (int)(p1 - s0), lead = (int)(p0 - s0);
     T v[UPT][4];
     int c[UPT][4];
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
-      const int off = 4 * (tid + u * kBlock);
-      if (off < span) {
-        QuadLoader<true, T>::load(vals, cols, P(s0 + off), p0, p1, nnz_total, v[u], c[u]);
+      const Wide<P> base = Wide<P>(s0) + 4 * (tid + u * kBlock);
+      if (base < Wide<P>(p1)) {
+        QuadLoader<true, T>::load(vals, cols, P(base), p0, p1, nnz_total, v[u], c[u]);
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) { v[u][j] = T(0); c[u][j] = -1; }
@@ -126,11 +125,11 @@ __global__ __launch_bounds__(kBlock, 8) void spmm_slices_kernel(
     }
 #pragma unroll
     for (int u = 0; u < UPT; ++u) {
-      const int off = 4 * (tid + u * kBlock) - lead;
+      const Wide<P> base = Wide<P>(s0) + 4 * (tid + u * kBlock);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (c[u][j] >= 0) {
-          const int o = off + j;
+          const int o = (int)(base + j - Wide<P>(p0));
           s_col[o] = c[u][j];
           s_val[o] = v[u][j];
         }

@@ -56,15 +56,14 @@ __global__ __launch_bounds__(kBlock) void spmv_rowblock_kernel(
     if (R <= 0 || R > kStreamRows || hi - lo > P(kSpmvStreamNnzCap) || hi < lo)
       return;  // not a planner descriptor; uniform per block
     const P s0 = lo & ~P(3);
-    const int span = (int)(hi - s0), head = (int)(lo - s0);
 
     T v[kStreamUPT][4];
     int c[kStreamUPT][4];
 #pragma unroll
     for (int u = 0; u < kStreamUPT; ++u) {
-      const int off = 4 * (tid + u * kBlock);
-      if (off < span) {
-        QuadLoader<NT, T>::load(vals, cols, P(s0 + off), lo, hi, nnz_total, v[u], c[u]);
+      const Wide<P> base = Wide<P>(s0) + 4 * (tid + u * kBlock);
+      if (base < Wide<P>(hi)) {
+        QuadLoader<NT, T>::load(vals, cols, P(base), lo, hi, nnz_total, v[u], c[u]);
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j) { v[u][j] = T(0); c[u][j] = -1; }
@@ -81,10 +80,10 @@ __global__ __launch_bounds__(kBlock) void spmv_rowblock_kernel(
     gather_x<kStreamUPT, A>(x, c, hi > lo, xv);
 #pragma unroll
     for (int u = 0; u < kStreamUPT; ++u) {
-      const int off = 4 * (tid + u * kBlock) - head;
+      const Wide<P> base = Wide<P>(s0) + 4 * (tid + u * kBlock);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (c[u][j] >= 0) s_prod[off + j] = A(v[u][j]) * A(xv[u][j]);
+        if (c[u][j] >= 0) s_prod[(int)(base + j - Wide<P>(lo))] = A(v[u][j]) * A(xv[u][j]);
     }
 #pragma unroll
     for (int u = 0; u < kPtrPT; ++u) {
@@ -123,15 +122,14 @@ __global__ __launch_bounds__(kBlock) void spmv_rowblock_kernel(
   const int row = d.x, k = d.y, nch = d.z, part = d.w;
   if (hi - lo > chunk || hi < lo) return;  // not a planner descriptor; uniform per block
   const P s0 = lo & ~P(3);
-  const int span = (int)(hi - s0);
 
   T v[kChunkUPT][4];
   int c[kChunkUPT][4];
 #pragma unroll
   for (int u = 0; u < kChunkUPT; ++u) {
-    const int off = 4 * (tid + u * kBlock);
-    if (off < span) {
-      QuadLoader<NT, T>::load(vals, cols, P(s0 + off), lo, hi, nnz_total, v[u], c[u]);
+    const Wide<P> base = Wide<P>(s0) + 4 * (tid + u * kBlock);
+    if (base < Wide<P>(hi)) {
+      QuadLoader<NT, T>::load(vals, cols, P(base), lo, hi, nnz_total, v[u], c[u]);
     } else {
 #pragma unroll
       for (int j = 0; j < 4; ++j) { v[u][j] = T(0); c[u][j] = -1; }
