@@ -22,7 +22,7 @@ def _pinned():
     return torch.empty(int(_abi.lib().fsp_check_pinned_len()), dtype=torch.int64, pin_memory=True)
 
 
-def csr_check(indices, indptr, ptr_bits=None, classes=None):
+def csr_check(indices, indptr, ptr_bits=None, classes=()):
     """([first, last, decreases, longest row, min column, max column] as Python ints, the columns
     as int32, the row pointers at ``ptr_bits``) of contiguous 1-D device arrays (columns int32 or
     int64; row pointers of another type are converted first).  ``classes`` (uneven, block, chunk):
@@ -49,15 +49,14 @@ def csr_check(indices, indptr, ptr_bits=None, classes=None):
         ptr = torch.empty(n_rows + 1, dtype=torch.int32 if ptr_bits == 32 else torch.int64,
                           device=dev)
     pinned = _pinned()
-    out = (ctypes.c_int64 * (6 if classes is None else 8))()
-    args = (indices.data_ptr() if nnz else None, idx_bits, nnz, indptr.data_ptr(), have_bits, n_rows,
-            idx32.data_ptr() if idx32 is not indices and nnz else None,
-            None if ptr is indptr else ptr.data_ptr(), ptr_bits or have_bits)
-    to = (pinned.data_ptr(), ctypes.addressof(out), _abi.raw_stream(dev))
-    if classes is None:
-        _abi.check(L.fsp_csr_check(*args, *to), "fsp_csr_check")
-    else:
-        _abi.check(L.fsp_csr_check_rows(*args, *classes, *to), "fsp_csr_check_rows")
+    out = (ctypes.c_int64 * (6 + (2 if classes else 0)))()
+    call = L.fsp_csr_check_rows if classes else L.fsp_csr_check
+    _abi.check(
+        call(indices.data_ptr() if nnz else None, idx_bits, nnz, indptr.data_ptr(), have_bits,
+             n_rows, idx32.data_ptr() if idx32 is not indices and nnz else None,
+             None if ptr is indptr else ptr.data_ptr(), ptr_bits or have_bits, *classes,
+             pinned.data_ptr(), ctypes.addressof(out), _abi.raw_stream(dev)),
+        "fsp_csr_check")
     return list(out), idx32, ptr
 
 

@@ -113,15 +113,14 @@ __device__ __forceinline__ void publish(int64_t* host, int64_t v) {
   __hip_atomic_store(host, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// What else is counted of the rows: those of more than `uneven` and at most `block` entries, and the
-// entries of those of more than `chunk`.  words: per workgroup, kCsrWords where nothing is.
+// What else is counted of the rows (COUNT): those of more than `uneven` and at most `block` entries,
+// and the entries of those of more than `chunk`.
 struct RowClasses {
   int64_t uneven, block, chunk;
-  int words;
 };
 
-// host: [0] = ptr[0], [1] = ptr[n_rows], then rows.words per workgroup.
-template <typename I, typename P>
+// host: [0] = ptr[0], [1] = ptr[n_rows], then kCsrWords or, with COUNT, kRowWords per workgroup.
+template <typename I, typename P, bool COUNT>
 __global__ __launch_bounds__(kThreads) void csr_check_kernel(
     const I* __restrict__ idx, int64_t nnz, const P* __restrict__ ptr, int64_t n_rows,
     int32_t* __restrict__ idx32, void* __restrict__ ptr_out, int ptr_out_bits, int idx_vec,
@@ -166,20 +165,23 @@ __global__ __launch_bounds__(kThreads) void csr_check_kernel(
         const int64_t len = (int64_t)((uint64_t)q - (uint64_t)p);
         dec += q < p ? 1 : 0;
         longest = len > longest ? len : longest;
-        uneven += len > rows.uneven && len <= rows.block ? 1 : 0;
-        cut += len > rows.chunk ? len : 0;
+        if constexpr (COUNT) {
+          uneven += len > rows.uneven && len <= rows.block ? 1 : 0;
+          cut += len > rows.chunk ? len : 0;
+        }
       }
     }
     a = block_reduce<true>(dec, s_w);
     b = block_reduce<false>(~longest, s_w);
-    if (rows.words == kRowWords) {
+    if constexpr (COUNT) {
       uneven = block_reduce<true>(uneven, s_w);
       cut = block_reduce<true>(cut, s_w);
     }
   }
-  if (tid < rows.words)  // one store
-    publish(host + 2 + (int64_t)blockIdx.x * rows.words + tid,
-            tid == 0 ? a : tid == 1 ? b : tid == 2 ? uneven : cut);
+  constexpr int kWords = COUNT ? kRowWords : kCsrWords;
+  if (tid < kWords)  // one store
+    publish(host + 2 + (int64_t)blockIdx.x * kWords + tid,
+            tid == 0 ? a : !COUNT || tid == 1 ? b : tid == 2 ? uneven : cut);
 }
 
 // host: kCooWords per workgroup.  row32 / col32: NULL, or the narrowed arrays.
@@ -256,16 +258,17 @@ int wait_words(const int64_t* host, int64_t n, hipStream_t st) {
   return FSP_OK;
 }
 
-template <typename I, typename P>
+template <typename I, typename P, bool COUNT>
 int run_csr_check(const void* idx, int64_t nnz, const void* ptr, int64_t n_rows, int32_t* idx32,
                   void* ptr_out, int ptr_out_bits, const RowClasses& rows, int64_t* pinned,
                   int64_t* out, hipStream_t st) {
   const int64_t ib = nnz > 0 ? blocks_for(nnz, kStep, kCheckBlocks) : 0;
   const int64_t pb = blocks_for(n_rows + 1, 2 * kThreads, kCheckBlocks / 4);
-  const int64_t n = 2 + (ib + pb) * rows.words;
+  constexpr int kWords = COUNT ? kRowWords : kCsrWords;
+  const int64_t n = 2 + (ib + pb) * kWords;
   for (int64_t i = 0; i < n; ++i) pinned[i] = kPending;
   const int vec = reinterpret_cast<uintptr_t>(idx) % 16 == 0;
-  hipLaunchKernelGGL((csr_check_kernel<I, P>), dim3((unsigned)(ib + pb)), dim3(kThreads), 0, st,
+  hipLaunchKernelGGL((csr_check_kernel<I, P, COUNT>), dim3((unsigned)(ib + pb)), dim3(kThreads), 0, st,
                      static_cast<const I*>(idx), nnz, static_cast<const P*>(ptr), n_rows, idx32,
                      ptr_out, ptr_out_bits, vec, (int)ib, rows, pinned);
   int rc = check_hip(hipGetLastError(), "csr_check_kernel launch");
@@ -273,9 +276,9 @@ int run_csr_check(const void* idx, int64_t nnz, const void* ptr, int64_t n_rows,
   if (rc) return rc;
   int64_t mn = LLONG_MAX, nmx = LLONG_MAX, dec = 0, nlong = ~int64_t(0), uneven = 0, cut = 0;
   for (int64_t b = 0; b < ib + pb; ++b) {
-    const int64_t* w = pinned + 2 + b * rows.words;
+    const int64_t* w = pinned + 2 + b * kWords;
     const int64_t u = w[0], v = w[1];
-    if (rows.words == kRowWords) {
+    if constexpr (COUNT) {
       uneven += w[2];
       cut += w[3];
     }
@@ -293,7 +296,7 @@ int run_csr_check(const void* idx, int64_t nnz, const void* ptr, int64_t n_rows,
   out[3] = ~nlong;
   out[4] = mn;
   out[5] = ~nmx;
-  if (rows.words == kRowWords) {
+  if constexpr (COUNT) {
     out[6] = uneven;
     out[7] = cut;
   }
@@ -341,6 +344,7 @@ extern "C" int64_t fsp_check_pinned_len(void) {
 
 namespace {
 
+template <bool COUNT>
 int csr_check(const void* indices, int idx_bits, int64_t nnz, const void* indptr, int ptr_bits,
               int64_t n_rows, int32_t* idx32, void* ptr_out, int ptr_out_bits,
               const RowClasses& rows, int64_t* pinned, int64_t* out, void* stream) {
@@ -355,10 +359,10 @@ int csr_check(const void* indices, int idx_bits, int64_t nnz, const void* indptr
   hipStream_t st = static_cast<hipStream_t>(stream);
 #define FSP_CHECK_ARGS indices, nnz, indptr, n_rows, idx32, ptr_out, ptr_out_bits, rows, pinned, out, st
   if (idx_bits == 32)
-    return ptr_bits == 32 ? run_csr_check<int32_t, int32_t>(FSP_CHECK_ARGS)
-                          : run_csr_check<int32_t, int64_t>(FSP_CHECK_ARGS);
-  return ptr_bits == 32 ? run_csr_check<int64_t, int32_t>(FSP_CHECK_ARGS)
-                        : run_csr_check<int64_t, int64_t>(FSP_CHECK_ARGS);
+    return ptr_bits == 32 ? run_csr_check<int32_t, int32_t, COUNT>(FSP_CHECK_ARGS)
+                          : run_csr_check<int32_t, int64_t, COUNT>(FSP_CHECK_ARGS);
+  return ptr_bits == 32 ? run_csr_check<int64_t, int32_t, COUNT>(FSP_CHECK_ARGS)
+                        : run_csr_check<int64_t, int64_t, COUNT>(FSP_CHECK_ARGS);
 #undef FSP_CHECK_ARGS
 }
 
@@ -367,8 +371,8 @@ int csr_check(const void* indices, int idx_bits, int64_t nnz, const void* indptr
 extern "C" int fsp_csr_check(const void* indices, int idx_bits, int64_t nnz, const void* indptr,
                              int ptr_bits, int64_t n_rows, int32_t* idx32, void* ptr_out,
                              int ptr_out_bits, int64_t* pinned, int64_t* out, void* stream) {
-  return csr_check(indices, idx_bits, nnz, indptr, ptr_bits, n_rows, idx32, ptr_out, ptr_out_bits,
-                   RowClasses{0, 0, 0, kCsrWords}, pinned, out, stream);
+  return csr_check<false>(indices, idx_bits, nnz, indptr, ptr_bits, n_rows, idx32, ptr_out,
+                          ptr_out_bits, RowClasses{0, 0, 0}, pinned, out, stream);
 }
 
 extern "C" int fsp_csr_check_rows(const void* indices, int idx_bits, int64_t nnz,
@@ -376,8 +380,8 @@ extern "C" int fsp_csr_check_rows(const void* indices, int idx_bits, int64_t nnz
                                   int32_t* idx32, void* ptr_out, int ptr_out_bits, int64_t uneven,
                                   int64_t block, int64_t chunk, int64_t* pinned, int64_t* out,
                                   void* stream) {
-  return csr_check(indices, idx_bits, nnz, indptr, ptr_bits, n_rows, idx32, ptr_out, ptr_out_bits,
-                   RowClasses{uneven, block, chunk, kRowWords}, pinned, out, stream);
+  return csr_check<true>(indices, idx_bits, nnz, indptr, ptr_bits, n_rows, idx32, ptr_out,
+                         ptr_out_bits, RowClasses{uneven, block, chunk}, pinned, out, stream);
 }
 
 extern "C" int fsp_coo_check(const void* rows, int row_bits, const void* cols, int col_bits,

@@ -227,7 +227,7 @@ def _check_spmv_csr_matrix(data, indices, indptr, shape, one_shot):
     no_rows = indptr.numel() == 0  # n_rows of -1: nothing to check in the row pointers
     stats, kernel_indices, kernel_indptr = csr_check(
         indices, indptr.new_zeros(1) if no_rows else indptr, ptr_bits,
-        None if one_shot else row_class_bounds(n_rows, nnz))
+        () if one_shot else row_class_bounds(n_rows, nnz))
     first, last, decreases, max_row_nnz, min_index, max_index = stats[:6]
     if not no_rows:
         if first != 0:
