@@ -9,6 +9,7 @@ rows (spmm_csr.py:417-441):
                           nch > 1 go to partial slots part .. part+nch-1
 """
 
+import copy
 import ctypes
 
 import numpy as np
@@ -38,6 +39,12 @@ class RowBlockPlan:
         self.by_column = False  # desc in a launch order of its own (spmm_csr.py)
         self._workspaces = {}
         self._groups = groups
+
+    def in_order(self, desc):
+        """The same plan with its descriptors in another launch order; all else is shared."""
+        other = copy.copy(self)
+        other.desc, other.by_column = desc, True
+        return other
 
     def workspace(self, width=1):
         """Partial-sum buffer for ``width`` values per row part, kept on the plan and reused by

@@ -353,7 +353,8 @@ class _SpmmKernelCsr:
     one call, so nothing is planned."""
 
     __slots__ = ("data", "cols", "rowptr", "rowptr_bits", "nnz", "n_rows", "_plans", "_args",
-                 "_keep", "_order", "max_row_nnz", "one_shot", "_tables", "_pieces", "_sums")
+                 "_keep", "_order", "max_row_nnz", "one_shot", "_tables", "_pieces", "_sums",
+                 "_row_order")
 
     def __init__(self, data, cols, indptr, max_row_nnz=None, one_shot=False):
         self.max_row_nnz = max_row_nnz
@@ -369,7 +370,8 @@ class _SpmmKernelCsr:
         self._tables = {}
         self._pieces = {}
         self._sums = {}
-        self._plans = {}
+        self._plans = {}      # by lanes and whether in column order; in use
+        self._row_order = {}  # by lanes, in row order
         self._args = _abi.Calls()
         self._keep = [self.data, self.cols, self.rowptr]  # what a launch reads or writes
         self._order = StreamOrder(self.data.device)
@@ -379,9 +381,11 @@ class _SpmmKernelCsr:
             else "spmm_slices_kernel"
 
     def describe(self):
-        return {"layout": "rowblock" if self._plans or not self.sliced() else "slices", "plans": {g: {"descriptors": p.n_desc,
-                                                    "split_rows": p.n_split_rows}
-                                                for g, p in self._plans.items()},
+        plans = {f"{lanes} by column" if by_column else lanes:
+                 {"descriptors": p.n_desc, "split_rows": p.n_split_rows}
+                 for (lanes, by_column), p in self._plans.items()}
+        return {"layout": "rowblock" if self._plans or not self.sliced() else "slices",
+                "plans": plans,
                 "slices": {k[0]: int(t[0].numel()) // 2 - 1 for k, t in self._tables.items()}}
 
     def sliced(self):
@@ -425,19 +429,26 @@ class _SpmmKernelCsr:
         return table, sums, cut
 
     def plan(self, lanes, row_bytes=0, n_cols=0):
-        p = self._plans.get(lanes)
+        """The row-block plan for ``lanes``, in the launch order that suits rows of B of
+        ``row_bytes`` (widths of several sizes can share a lane count)."""
+        ngrp = 256 // lanes
+        cap = _abi.caps()["spmm_block_nnz"]
+        threshold = min(_SPMM_ROW_SPLIT_THRESHOLD, cap)
+        chunk = min(cap, max(threshold, 16 * ngrp))
+        by_column = _slices.ordered(self.max_row_nnz, chunk, n_cols * row_bytes,
+                                    self.nnz * row_bytes, False)
+        p = self._plans.get((lanes, by_column))
         if p is None:
-            ngrp = 256 // lanes
-            cap = _abi.caps()["spmm_block_nnz"]
-            threshold = min(_SPMM_ROW_SPLIT_THRESHOLD, cap)
-            chunk = min(cap, max(threshold, 16 * ngrp))
-            p = build_row_block_plan_device(self.rowptr, cap, ngrp, threshold, chunk,
-                                            window_rows=SPMM_PLAN_WINDOW_BLOCKS * ngrp)
-            p.by_column = _slices.ordered(self.max_row_nnz, chunk, n_cols * row_bytes,
-                                          self.nnz * row_bytes, False)
-            if p.by_column:
-                p.desc = _parts_by_column(p.desc, self.cols, n_cols, self.rowptr, chunk)
-            self._plans[lanes] = p
+            p = self._row_order.get(lanes)
+            if p is None:
+                p = self._row_order[lanes] = build_row_block_plan_device(
+                    self.rowptr, cap, ngrp, threshold, chunk,
+                    window_rows=SPMM_PLAN_WINDOW_BLOCKS * ngrp)
+            if by_column:
+                if torch.cuda.is_current_stream_capturing():
+                    return p  # the order would only be written by a replay; the sums are the same
+                p = p.in_order(_parts_by_column(p.desc, self.cols, n_cols, self.rowptr, chunk))
+            self._plans[lanes, by_column] = p
         return p
 
 

@@ -306,3 +306,48 @@ def test_room_of_a_new_width_while_capturing(dev, monkeypatch):
         torch.cuda.synchronize()
         assert oracle.rel_l2(C, oracle.spmm_csr(ip, cols, vals, B)) <= 1e-5
     assert torch.equal(fs.flagsparse_spmm_csr_opt(B=Bd.clone(), prepared=p), C)
+
+
+@pytest.mark.parametrize("widths", [(47, 256), (256, 47)])
+def test_launch_order_follows_the_width(dev, widths):
+    """Two widths of one lane count, of which the wider B does not fit an L2: each has the launch
+    order of its own size, whichever comes first, on one plan."""
+    lengths = torch.tensor([40, 9000, 3, 128] * 12)
+    ptr = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
+    cols = synthetic.randint(7, 1, int(ptr[-1]), 10000, "cpu").to(torch.int32)
+    data = synthetic.uniform_values(7, 2, cols.numel(), torch.float32, "cpu")
+    shape = (lengths.numel(), 10000)
+    p = fs.prepare_spmm_csr_opt(data.to(dev), cols.to(dev), ptr.to(dev), shape)
+    kc = p._kernel_csr()
+    for n in widths:
+        B = synthetic.dense_uniform(10000, n, torch.float32, seed=n, device="cpu")
+        out = fs.flagsparse_spmm_csr_opt(B=B.to(dev), prepared=p)
+        assert oracle.rel_l2(out, oracle.spmm_csr(ptr, cols, data, B)) <= 1e-5
+    assert set(kc._plans) == {(64, False), (64, True)} and set(kc._row_order) == {64}
+    assert kc._plans[64, True].by_column and not kc._plans[64, False].by_column
+    assert kc._plans[64, True]._workspaces is kc._plans[64, False]._workspaces
+    assert len(kc.describe()["plans"]) == 2
+
+
+def test_launch_order_is_not_built_in_a_capture(dev):
+    lengths = torch.tensor([40, 9000, 3, 128] * 12)
+    ptr = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
+    cols = synthetic.randint(7, 1, int(ptr[-1]), 10000, "cpu").to(torch.int32)
+    data = synthetic.uniform_values(7, 2, cols.numel(), torch.float32, "cpu")
+    p = fs.prepare_spmm_csr_opt(data.to(dev), cols.to(dev), ptr.to(dev), (48, 10000))
+    fs.flagsparse_spmm_csr_opt(B=torch.ones(10000, 47, device=dev), prepared=p)  # row order
+    B = synthetic.dense_uniform(10000, 256, torch.float32, seed=3, device="cpu")
+    Bd = B.to(dev)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        C = fs.flagsparse_spmm_csr_opt(B=Bd, prepared=p)
+    assert set(p._kernel_csr()._plans) == {(64, False)}
+    eager = fs.flagsparse_spmm_csr_opt(B=Bd, prepared=p)  # before any replay
+    ref = oracle.spmm_csr(ptr, cols, data, B)
+    assert oracle.rel_l2(eager, ref) <= 1e-5
+    for _ in range(3):
+        C.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(C, eager)
