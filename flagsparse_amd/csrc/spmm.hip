@@ -319,14 +319,16 @@ __global__ __launch_bounds__(kBlock / VW) void spmm_ragged_kernel(
   const int len = (int)(hi - lo);
   const bool staged = len <= slots;
   if (staged) {
-    for (Wide<P> base = Wide<P>(lo & ~P(3)) + 4 * tid; base < Wide<P>(hi); base += 4 * kThreads) {
+    const P s0 = lo & ~P(3);
+    const int span = (int)(hi - s0), head = (int)(lo - s0);
+    for (int off = 4 * tid; off < span; off += 4 * kThreads) {
       T v[4];
       int c[4];
-      QuadLoader<true, T>::load(vals, cols, P(base), lo, hi, nnz_total, v, c);
+      QuadLoader<true, T>::load(vals, cols, P(s0 + off), lo, hi, nnz_total, v, c);
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         if (c[j] >= 0) {
-          const int o = (int)(base + j - Wide<P>(lo));
+          const int o = off - head + j;
           s_col[o] = c[j];
           s_val[o] = v[j];
         }
