@@ -6,6 +6,9 @@ import torch
 from . import _abi
 
 _L2_BYTES = 4 << 20  # one XCD's L2
+# A launch holds fewer than 2^32 threads, so this many workgroups of 256 at most, a slice each.  More
+# are not refused by the runtime: it launches the number modulo 2^32, and rows stay unwritten.
+MAX_SLICES = (2**32 - 1) // 256
 
 
 def ordered(longest_row, items, dense_bytes, gathered_bytes, one_call):

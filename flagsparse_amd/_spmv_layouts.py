@@ -48,6 +48,7 @@ import torch
 
 from . import _abi
 from . import _common
+from . import _slices
 from ._common import _INDEX_LIMIT_INT32, _aligned
 from ._plan import StreamOrder, build_row_block_plan_windows
 
@@ -1442,8 +1443,11 @@ def build_layout(data, cols, rowptr, n_cols, one_shot=False, max_row_nnz=None, r
     knows it and asks for no row map; row_classes: what the check counted by row_class_bounds."""
     mode = FORCE
     nnz = int(data.numel())
-    if mode is None and one_shot:
+    few = _abi.lib().fsp_spmv_slices(int(rowptr.numel()) - 1, nnz) <= _slices.MAX_SLICES
+    if mode is None and one_shot and few:  # else the row blocks, of which there are fewer
         return SliceLayout(data, cols, rowptr, max_row_nnz, one_shot=True)
+    if mode is None and one_shot:
+        mode = "rowblock"
     if mode is None:
         mode = ("xstage" if STAGED else "xcs") \
             if prefers_xcs(cols, rowptr, n_cols, data.element_size()) else "rowblock"
@@ -1472,7 +1476,7 @@ def build_layout(data, cols, rowptr, n_cols, one_shot=False, max_row_nnz=None, r
             return xcs_layout(data, cols, rowptr, n_cols, FORCE_PANELS_PER_XCD)
         except ValueError:
             pass  # too large for the packing: row blocks
-    if FORCE is None and row_classes is not None and \
+    if FORCE is None and row_classes is not None and few and \
             slices_pay(cols, rowptr, n_cols, max_row_nnz, *row_classes):
         return SliceLayout(data, cols, rowptr, max_row_nnz)
     return RowBlockLayout(data, cols, rowptr)

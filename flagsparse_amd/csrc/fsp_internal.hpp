@@ -10,6 +10,9 @@
 
 namespace fsp {
 
+// A launch holds fewer than 2^32 threads; a larger grid is launched modulo 2^32 without an error.
+constexpr int64_t kMaxBlocks = 0xffffffffLL / 256;       // workgroups of 256 threads
+
 // Kernel capacities (see the kernels for why each value is what it is).
 constexpr int64_t kSpmvStreamSlots = 1024;               // LDS product slots per short-row block
 constexpr int64_t kSpmvStreamNnzCap = kSpmvStreamSlots - 3;

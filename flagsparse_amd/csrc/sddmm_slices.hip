@@ -283,8 +283,8 @@ extern "C" int fsp_sddmm_sliced(int dtype, int acc_f64, int out_f64, const int32
     return set_error(FSP_EINVAL, "fsp_sddmm_sliced: ldx/ldy smaller than K");
   if (out_f64 && dtype != FSP_F32)
     return set_error(FSP_EINVAL, "fsp_sddmm_sliced: out_f64 applies to fp32 inputs only");
-  if (slice_count(n_rows, nnz, items) > 0x7fffffffLL)
-    return set_error(FSP_EINVAL, "fsp_sddmm_sliced: more than 2^31-1 slices");
+  if (slice_count(n_rows, nnz, items) > kMaxBlocks)
+    return set_error(FSP_EINVAL, "fsp_sddmm_sliced: more slices than a launch holds");
   if (nnz == 0) return FSP_OK;
   if (!cols || !rowptr || !x || !y || !out || !table)
     return set_error(FSP_EINVAL, "fsp_sddmm_sliced: null pointer");

@@ -502,8 +502,10 @@ extern "C" int fsp_spmv_sliced(int dtype, int acc_f64, const void* vals, const i
   if (rowptr_bits != 32 && rowptr_bits != 64)
     return set_error(FSP_EINVAL, "fsp_spmv_sliced: rowptr_bits must be 32 or 64");
   if (n_rows < 0 || nnz < 0) return set_error(FSP_EINVAL, "fsp_spmv_sliced: negative size");
-  if (n_rows > 0x7fffffffLL || slice_count(n_rows, nnz, kSpmvSliceItems) > 0x7fffffffLL)
-    return set_error(FSP_EINVAL, "fsp_spmv_sliced: more than 2^31-1 rows or slices");
+  if (n_rows > 0x7fffffffLL)
+    return set_error(FSP_EINVAL, "fsp_spmv_sliced: more than 2^31-1 rows");
+  if (slice_count(n_rows, nnz, kSpmvSliceItems) > kMaxBlocks)
+    return set_error(FSP_EINVAL, "fsp_spmv_sliced: more slices than a launch holds");
   if (rowptr_bits == 32 && nnz > 0x7fffffffLL)
     return set_error(FSP_EINVAL, "fsp_spmv_sliced: nnz exceeds int32 rowptr range");
   if (n_rows == 0) return FSP_OK;

@@ -393,8 +393,8 @@ extern "C" int fsp_spmm_sliced(int dtype, int acc_f64, const void* vals, const i
   const int64_t W = (int64_t)lanes_per_row * vec;
   if ((N + W - 1) / W > 65535)
     return set_error(FSP_EINVAL, "fsp_spmm_sliced: too many column tiles");
-  if (slice_count(n_rows, nnz, items) > 0x7fffffffLL)
-    return set_error(FSP_EINVAL, "fsp_spmm_sliced: more than 2^31-1 slices");
+  if (slice_count(n_rows, nnz, items) > kMaxBlocks)
+    return set_error(FSP_EINVAL, "fsp_spmm_sliced: more slices than a launch holds");
   const SliceArgs a{vals, cols, rowptr, n_rows, nnz,   B,    ldb,      N,  C,
                     ldc,  table, order, sums,  items,  keep,  cut_rows, lg, xcd_remap,
                     static_cast<hipStream_t>(stream)};

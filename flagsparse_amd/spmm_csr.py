@@ -316,6 +316,8 @@ def _spmm_slice_shape(lanes, positions, by_column=False):
         items = {64: 128, 32: 256, 16: 512, 8: 1024}.get(lanes, 1536)
     while items > 64 and positions < 1024 * items:
         items = max(64, items >> 1)
+    while items < 1536 and positions > _slices.MAX_SLICES * items:
+        items = min(1536, items << 1)
     return items, 256 if items >= 128 else 128
 
 

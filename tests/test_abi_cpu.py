@@ -347,3 +347,21 @@ def test_bound_calls_check_like_their_entry_points():
         assert bound[1] % 8 == 0
         assert L.fsp_run(bound[1], None, None, None) < 0
         assert text in L.fsp_last_error(), (name, L.fsp_last_error())
+
+
+def test_more_slices_than_a_launch_holds():
+    """Refused before any launch: the runtime would launch the threads modulo 2^32."""
+    L = _abi.lib()
+    limit = (2**32 - 1) // 256
+    at = 4096  # an aligned address that no refused call follows
+    n_rows, nnz, items = 1, 64 * limit, 64
+    assert L.fsp_slice_count(n_rows, nnz, items) == limit + 1
+    rc = L.fsp_spmm_sliced(0, 0, at, at, at, 64, n_rows, nnz, at, 4, 4, at, 4, at, None, items, 128,
+                           None, 0, 1, 4, 1, None)
+    assert rc == -1 and b"launch holds" in L.fsp_last_error()
+    rc = L.fsp_sddmm_sliced(0, 0, 0, at, at, 64, n_rows, nnz, at, 4, at, 4, 4, None, 1.0, 0.0, at, at,
+                            None, items, 1, 4, None)
+    assert rc == -1 and b"launch holds" in L.fsp_last_error()
+    nnz = int(L.fsp_spmv_slice_items()) * limit
+    rc = L.fsp_spmv_sliced(0, 1, at, at, at, 64, 1, nnz, at, at, at, 1, at, 1, None)
+    assert rc == -1 and b"launch holds" in L.fsp_last_error()

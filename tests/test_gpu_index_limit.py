@@ -62,3 +62,13 @@ def test_spmm_last_entries(dev, entries, length, n):
     C = fs.flagsparse_spmm_csr_opt(B=B, prepared=p)
     assert p._kernel_csr()._plans and p._kernel_csr().rowptr_bits == 32
     assert torch.equal(C, want[:, None].expand_as(C))
+
+
+def test_spmm_many_slices(dev, entries):
+    # 64 lanes take the smallest slices: 2^31 rows + entries of them must still fit one launch (a
+    # larger grid runs modulo 2^32 threads, and leaves rows unwritten)
+    data, cols, ptr, shape, want = _matrix(entries, 64, dev)
+    C = fs.flagsparse_spmm_csr_opt(data, cols, ptr, torch.ones(COLS, 256, device=dev), shape)
+    for k in range(0, shape[0], 1 << 22):
+        part = C[k:k + (1 << 22)]
+        assert torch.equal(part, want[k:k + (1 << 22), None].expand_as(part))

@@ -108,3 +108,27 @@ def test_copies_start_without_calls():
     calls = _abi.Calls(base=("buffer", 4096))
     assert dict(calls) and not copy.deepcopy({"a": calls})["a"]
     assert not copy.copy(calls) and not pickle.loads(pickle.dumps(calls))
+
+
+@pytest.mark.parametrize("by_column", [False, True])
+@pytest.mark.parametrize("lanes", [1, 2, 4, 8, 16, 32, 64])
+def test_spmm_slices_fit_a_launch(lanes, by_column):
+    for positions in (1 << 31, (1 << 31) + (1 << 25), 10**10, 1 << 34, _slices.MAX_SLICES * 128,
+                      _slices.MAX_SLICES * 128 + 1):
+        items, keep = spmm_csr._spmm_slice_shape(lanes, positions, by_column)
+        assert -(-positions // items) <= _slices.MAX_SLICES and items + keep + 6 <= 2048
+
+
+def test_spmv_slices_fit_a_launch(monkeypatch):
+    lengths, cols, n_cols = _random([12] * 2000, 2000)
+    rowptr = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
+    built = []
+    monkeypatch.setattr(_spmv_layouts, "SliceLayout", lambda *a, **k: built.append("slices"))
+    monkeypatch.setattr(_spmv_layouts, "RowBlockLayout", lambda *a, **k: built.append("rowblock"))
+    data, cols = torch.ones(cols.numel()), cols.to(torch.int32)
+    for limit in (_slices.MAX_SLICES, 10):  # the matrix has 35 slices
+        monkeypatch.setattr(_slices, "MAX_SLICES", limit)
+        _spmv_layouts.build_layout(data, cols, rowptr, n_cols, one_shot=True)
+        _spmv_layouts.build_layout(data, cols, rowptr, n_cols, max_row_nnz=5000,
+                                   row_classes=[0, cols.numel()])
+    assert built == ["slices", "slices", "rowblock", "rowblock"]
