@@ -368,8 +368,8 @@ extern "C" int fsp_sddmm_csr(int dtype, int acc_f64, int out_f64, const int32_t*
                                  "16-byte aligned x, y");
   if (out_f64 && dtype != FSP_F32)
     return set_error(FSP_EINVAL, "fsp_sddmm_csr: out_f64 applies to fp32 inputs only");
-  if (n_desc < 0 || n_desc > 0x7fffffffLL)
-    return set_error(FSP_EINVAL, "fsp_sddmm_csr: n_desc outside [0, 2^31-1]");
+  if (n_desc < 0 || n_desc > kMaxBlocks)
+    return set_error(FSP_EINVAL, "fsp_sddmm_csr: n_desc negative or more than a launch holds");
   if (n_desc > 0) {
     if (!desc || !ranges || !rowptr)
       return set_error(FSP_EINVAL, "fsp_sddmm_csr: row-block plan without desc/ranges/rowptr");

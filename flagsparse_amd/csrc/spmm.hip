@@ -518,10 +518,11 @@ extern "C" int fsp_spmm_csr(int dtype, int acc_f64, const void* vals, const int3
     return set_error(FSP_EINVAL, "fsp_spmm_csr: rowptr_bits must be 32 or 64");
   if (n_rows < 0 || nnz < 0 || N < 0 || n_desc < 0 || n_groups < 0)
     return set_error(FSP_EINVAL, "fsp_spmm_csr: negative size");
-  if (n_groups > 0x7fffffffLL) return set_error(FSP_EINVAL, "fsp_spmm_csr: too many groups");
+  if (n_desc > kMaxBlocks || n_groups > kMaxBlocks)
+    return set_error(FSP_EINVAL, "fsp_spmm_csr: more descriptors or groups than a launch holds");
   if (n_groups > 0 && (!groups || !group_base || !split_rows || !partials))
     return set_error(FSP_EINVAL, "fsp_spmm_csr: null split-row pointer");
-  if (n_desc > 0x7fffffffLL || n_rows > 0x7fffffffLL || N > 0x7fffffffLL)
+  if (n_rows > 0x7fffffffLL || N > 0x7fffffffLL)
     return set_error(FSP_EINVAL, "fsp_spmm_csr: size exceeds 2^31-1");
   if (rowptr_bits == 32 && nnz > 0x7fffffffLL)
     return set_error(FSP_EINVAL, "fsp_spmm_csr: nnz exceeds int32 rowptr range");

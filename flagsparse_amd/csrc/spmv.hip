@@ -248,8 +248,9 @@ int spmv_csr_checked(const char* who, int dtype, int acc_f64, const void* vals,
     return set_error(FSP_EINVAL, w + ": rowptr_bits must be 32 or 64");
   if (n_rows < 0 || nnz < 0 || n_desc < 0 || n_out < 0 || n_groups < 0)
     return set_error(FSP_EINVAL, w + ": negative size");
-  if (n_desc > 0x7fffffffLL || n_rows > 0x7fffffffLL || n_groups > 0x7fffffffLL)
-    return set_error(FSP_EINVAL, w + ": more than 2^31-1 rows, descriptors or groups");
+  if (n_rows > 0x7fffffffLL) return set_error(FSP_EINVAL, w + ": more than 2^31-1 rows");
+  if (n_desc > kMaxBlocks || n_groups > kMaxBlocks)
+    return set_error(FSP_EINVAL, w + ": more descriptors or groups than a launch holds");
   if (rowptr_bits == 32 && nnz > 0x7fffffffLL)
     return set_error(FSP_EINVAL, w + ": nnz exceeds int32 rowptr range");
   if (chunk < 1 || chunk > kSpmvChunkCap)
@@ -357,8 +358,12 @@ extern "C" int fsp_spmv_coo_atomic(int dtype, const void* vals, const int32_t* r
   if (nnz > 0 && (!vals || !rows || !cols || !x))
     return set_error(FSP_EINVAL, "fsp_spmv_coo_atomic: null pointer");
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const int64_t blocks = (nnz + nnz_per_block - 1) / nnz_per_block;
+  int64_t blocks = (nnz + nnz_per_block - 1) / nnz_per_block;
   if (blocks > 0x7fffffffLL) return set_error(FSP_EINVAL, "fsp_spmv_coo_atomic: grid too large");
+  while (blocks > kMaxBlocks) {  // more entries to a workgroup until a launch holds them
+    nnz_per_block *= 2;
+    blocks = (nnz + nnz_per_block - 1) / nnz_per_block;
+  }
   if (dtype == FSP_F32) {
     int rc = fill_zero<float>(static_cast<float*>(y), n_rows, st);
     if (rc || nnz == 0) return rc;

@@ -501,6 +501,8 @@ def _bind_sliced(kc, B, acc_f64, lanes, vec):
 def _bind_row_blocks(kc, B, acc_f64, lanes, vec):
     n_dense_cols = int(B.shape[1])
     plan = kc.plan(lanes, min(n_dense_cols, lanes * vec) * B.element_size(), int(B.shape[0]))
+    if plan.n_desc > _slices.MAX_SLICES:
+        return None  # more workgroups than a launch holds (four rows each with 64 lanes)
     partials = plan.workspace(n_dense_cols)
     groups, group_base, split_rows = plan.split_groups()
     p = lambda t: t.data_ptr() if t.numel() else None  # noqa: E731
@@ -531,10 +533,11 @@ def _run_spmm(kc, B, C, acc_f64, tile_cols=None):
         lanes, vec = _spmm_lane_shape(n_dense_cols, B.dtype, B, C, tile_cols)
         kept = not kc.one_shot and (kc.max_row_nnz or 0) > _SPMM_SUMS_KEPT
         # the row-block kernel's loads need aligned vectors
-        if kc.sliced() or (vec < slice_vec and not kept):
-            bound = _bind_sliced(kc, B, acc_f64, slice_lanes, slice_vec)
-        else:
+        bound = None
+        if not (kc.sliced() or (vec < slice_vec and not kept)):
             bound = _bind_row_blocks(kc, B, acc_f64, lanes, vec)
+        if bound is None:
+            bound = _bind_sliced(kc, B, acc_f64, slice_lanes, slice_vec)
         kc._args[key] = bound
     _abi.run(bound, b, c, stream)
     return C

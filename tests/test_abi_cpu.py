@@ -365,3 +365,16 @@ def test_more_slices_than_a_launch_holds():
     nnz = int(L.fsp_spmv_slice_items()) * limit
     rc = L.fsp_spmv_sliced(0, 1, at, at, at, 64, 1, nnz, at, at, at, 1, at, 1, None)
     assert rc == -1 and b"launch holds" in L.fsp_last_error()
+
+
+def test_more_row_blocks_than_a_launch_holds():
+    L, at, limit = _abi.lib(), 4096, (2**32 - 1) // 256
+    rc = L.fsp_spmv_csr(0, 1, at, at, at, 32, 1 << 30, 4, at, at, None, 0, at, at, limit + 1, 64, at,
+                        None, None, None, 0, 0, None)
+    assert rc == -1 and b"launch holds" in L.fsp_last_error()
+    rc = L.fsp_spmm_csr(0, 0, at, at, at, 32, 1 << 30, 4, at, 4, 4, at, 4, at, limit + 1, 64, 1, 4, at,
+                        None, None, None, 0, 1, None)
+    assert rc == -1 and b"launch holds" in L.fsp_last_error()
+    rc = L.fsp_sddmm_csr(0, 0, 0, at, at, at, 32, 4, at, 4, at, 4, 4, None, 1.0, 0.0, at, at, at,
+                         limit + 1, 1, 4, None)
+    assert rc == -1 and b"launch holds" in L.fsp_last_error()

@@ -351,3 +351,13 @@ def test_launch_order_is_not_built_in_a_capture(dev):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(C, eager)
+
+
+def test_more_row_blocks_than_a_launch_holds(dev, monkeypatch):
+    # the prepared product runs on slices instead (here with a limit that 1200 rows reach)
+    vals, cols, ip, B, shape = _case("short", 901, 16, torch.float32, dev)
+    p = fs.prepare_spmm_csr_opt(vals.to(dev), cols.to(dev), ip.to(dev), shape)
+    monkeypatch.setattr(_slices, "MAX_SLICES", 12)
+    C = fs.flagsparse_spmm_csr_opt(B=B.to(dev), prepared=p)
+    assert p._kernel_csr()._tables
+    assert oracle.rel_l2(C, oracle.spmm_csr(ip, cols, vals, B)) <= 1e-5

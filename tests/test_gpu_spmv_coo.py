@@ -104,3 +104,13 @@ def test_api_knobs_out_and_errors(dev):
                                device=dev), torch.empty(0, dtype=torch.int32, device=dev),
                                torch.ones(4, device=dev), (6, 4))
     assert e.shape == (6,) and torch.count_nonzero(e) == 0
+
+
+def test_atomic_route_with_one_entry_per_workgroup(dev):
+    # 20M workgroups of 256 threads would be more than a launch holds: they take more entries each
+    nnz, n = 20_000_000, 1000
+    i = torch.arange(nnz, device=dev, dtype=torch.int32)
+    y = fs.flagsparse_spmv_coo(torch.ones(nnz, dtype=torch.float64, device=dev), i % n, i % 7,
+                               torch.ones(7, dtype=torch.float64, device=dev), (n, 7),
+                               sort_by_row=False, block_size=1)
+    assert torch.equal(y, torch.full_like(y, nnz / n))
