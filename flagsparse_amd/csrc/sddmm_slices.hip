@@ -140,9 +140,12 @@ __global__ __launch_bounds__(kBlock) void sddmm_slices_kernel(
     A acc[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      // Pairs, then vectors, then steps: no running sum is longer than two products, so fewer
-      // lanes (more steps) lose no precision.  A dropped element is 0 in both rows (an infinity
-      // or a NaN next to 0 would show).
+      // A vector's products in a chain of fused steps, which rounds one product where pairs would
+      // round two; then vectors, then lanes: no running sum is longer than a vector, so fewer
+      // lanes (more steps) lose no precision.  Error against 64 bits, in 1e-8 of the result's norm,
+      // row blocks / pairs / so: fp32 K=8 4.829 / 4.920 / 4.829, K=64 6.766 / 6.832 / 6.766, K=256
+      // 9.61 / 7.84 / 7.78.  A dropped element is 0 in both rows (an infinity or a NaN next to 0
+      // would show).
       A part[KC];
 #pragma unroll
       for (int c = 0; c < KC; ++c) {
@@ -154,7 +157,7 @@ __global__ __launch_bounds__(kBlock) void sddmm_slices_kernel(
         }
         if constexpr (VW == 1) part[c] = a[0] * b[0];
         else if constexpr (VW == 2) part[c] = fma(a[1], b[1], a[0] * b[0]);
-        else part[c] = fma(a[1], b[1], a[0] * b[0]) + fma(a[3], b[3], a[2] * b[2]);
+        else part[c] = fma(a[3], b[3], fma(a[2], b[2], fma(a[1], b[1], a[0] * b[0])));
       }
       if constexpr (KC == 1) acc[q] = part[0];
       else if constexpr (KC == 2) acc[q] = part[0] + part[1];

@@ -186,3 +186,28 @@ def test_sddmm_keeps_its_arrays_from_other_streams(dev, monkeypatch, K):
     assert busy  # else the allocator was free to give them out
     torch.cuda.synchronize()
     assert oracle.rel_l2(out, oracle.sddmm_csr(ip, cols, x, y)) <= 1e-5
+
+
+@pytest.mark.parametrize("K", [4, 8, 16, 64, 128])
+def test_sliced_sddmm_order_of_additions(dev, K):
+    """float32, bit for bit: a vector's four products in a chain of fused multiply-adds, a lane's
+    vectors and then the lanes added in a tree.  The chain rounds one product of a vector where pairs
+    would round two.  (The oracle's fused step rounds an extended-precision sum, which differs from a
+    fused float32 step only where that sum lies half-way between two floats to 2^-63.)"""
+    ip, cols, _, x, y, shape = _case("crossing", 503, K, torch.float32, dev)
+    p = fs.prepare_sddmm_csr(cols.to(dev), ip.to(dev), shape, k_hint=K)
+    out = fs.flagsparse_sddmm_csr(x=x.to(dev), y=y.to(dev), prepared=p).cpu().numpy()
+    lanes, vec = sddmm_csr._sddmm_slice_lanes(K, torch.float32)
+    steps = K // (lanes * vec)
+    assert vec == 4 and K == steps * lanes * vec and steps in (1, 2, 4)
+    row = torch.repeat_interleave(torch.arange(shape[0]), ip[1:] - ip[:-1])
+    X = x[row].numpy().reshape(-1, steps, lanes, 4).astype(np.longdouble)
+    Y = y[cols.long()].numpy().reshape(-1, steps, lanes, 4).astype(np.longdouble)
+    v = np.zeros(X.shape[:3], dtype=np.float32)
+    for j in range(4):
+        v = (X[..., j] * Y[..., j] + v).astype(np.float32)
+    for axis in (1, 2):
+        while v.shape[axis] > 1:
+            a, b = (np.take(v, range(k, v.shape[axis], 2), axis) for k in (0, 1))
+            v = a + b
+    np.testing.assert_array_equal(out, v[:, 0, 0])
