@@ -485,8 +485,8 @@ def _spmm_workload(dev, dtype_name, N, torch, fs, synthetic, part="all"):
         shape[0] * N * v,
         "nbytes": nbytes, "flops": 2 * nnz * N, "info": info, "cpu": cpu,
         "cpu_lib": _cpu_lib("csr", (ptr, idx, data), B, shape, nbytes, 2 * nnz * N, torch),
-        "dtype": dtype_name, "kernel": kc.kernel_name(),
-        "tag": f"{kc.kernel_name()}_cfg5_{dtype_name}_n{N}" + ("" if part == "all" else
+        "dtype": dtype_name, "kernel": kc.kernel_name(N),
+        "tag": f"{kc.kernel_name(N)}_cfg5_{dtype_name}_n{N}" + ("" if part == "all" else
                                                                 f"_{part}_half"),
     }
 
@@ -538,8 +538,8 @@ def _spmm_coo_workload(dev, dtype_name, N, torch, fs, synthetic):
         "step": lambda: fs.flagsparse_spmm_coo(data, row, col, B, shape, out=C),
         "launch": lambda: mod._run_spmm(kc, B, C, acc_f64=True),
         "nbytes": nbytes, "flops": 2 * nnz * N, "info": info, "cpu": cpu,
-        "dtype": dtype_name, "kernel": kc.kernel_name(),
-        "tag": f"{kc.kernel_name()}_coo5_{dtype_name}_n{N}",
+        "dtype": dtype_name, "kernel": kc.kernel_name(N),
+        "tag": f"{kc.kernel_name(N)}_coo5_{dtype_name}_n{N}",
     }
 
 

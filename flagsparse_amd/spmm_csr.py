@@ -356,7 +356,7 @@ class _SpmmKernelCsr:
 
     __slots__ = ("data", "cols", "rowptr", "rowptr_bits", "nnz", "n_rows", "_plans", "_args",
                  "_keep", "_order", "max_row_nnz", "one_shot", "_tables", "_pieces", "_sums",
-                 "_row_order")
+                 "_row_order", "_names")
 
     def __init__(self, data, cols, indptr, max_row_nnz=None, one_shot=False):
         self.max_row_nnz = max_row_nnz
@@ -372,15 +372,18 @@ class _SpmmKernelCsr:
         self._tables = {}
         self._pieces = {}
         self._sums = {}
+        self._names = {}  # the kernel of each width's latest bound call
         self._plans = {}      # by lanes and whether in column order; in use
         self._row_order = {}  # by lanes, in row order
         self._args = _abi.Calls()
         self._keep = [self.data, self.cols, self.rowptr]  # what a launch reads or writes
         self._order = StreamOrder(self.data.device)
 
-    def kernel_name(self):
-        return "spmm_rowblock_kernel" if self._plans or not self.sliced() \
-            else "spmm_slices_kernel"
+    def kernel_name(self, n_dense_cols=None):
+        """The kernel that the latest product of this width ran; without a width, or before a
+        product of it, the kernel of the matrix's layout for whole vectors."""
+        layout = "spmm_rowblock_kernel" if self._plans or not self.sliced() else "spmm_slices_kernel"
+        return self._names.get(n_dense_cols, layout)
 
     def describe(self):
         plans = {f"{lanes} by column" if by_column else lanes:
@@ -490,6 +493,7 @@ def _bind_sliced(kc, B, acc_f64, lanes, vec):
     if kc.max_row_nnz is None or kc.max_row_nnz > keep:
         table, sums, cut = kc.piece_slots((items, keep), table, n_dense_cols,
                                           torch.float64 if acc_f64 else B.dtype)
+    kc._names[n_dense_cols] = "spmm_slices_kernel"
     kc._keep.extend((table, order, sums))
     return _abi.bind(
         "spmm_sliced", _abi.dtype_code(B.dtype), 1 if acc_f64 else 0, kc.data.data_ptr(),
@@ -506,6 +510,10 @@ def _bind_row_blocks(kc, B, acc_f64, lanes, vec):
     partials = plan.workspace(n_dense_cols)
     groups, group_base, split_rows = plan.split_groups()
     p = lambda t: t.data_ptr() if t.numel() else None  # noqa: E731
+    # launch_spmm's rule (csrc/spmm.hip)
+    ragged = (vec == 1 and lanes >= 32 and n_dense_cols * B.element_size() >= 16
+              and (not acc_f64 or B.dtype == torch.float64))
+    kc._names[n_dense_cols] = "spmm_ragged_kernel" if ragged else "spmm_rowblock_kernel"
     kc._keep.extend((partials, plan.desc, groups, group_base, split_rows))
     return _abi.bind(
         "spmm_csr", _abi.dtype_code(B.dtype), 1 if acc_f64 else 0, p(kc.data), p(kc.cols),

@@ -160,6 +160,43 @@ def test_unknown_longest_row(dev, monkeypatch):
         assert oracle.rel_l2(C, oracle.spmm_csr(ip, cols, vals, B)) <= 1e-5
 
 
+def _row_block_kernel(n, dtype, aligned=True):
+    """The kernel of a prepared matrix with rows over 8192 entries: vectors of any alignment from 32
+    lanes of single elements on, which N takes that is no whole number of pairs or not aligned."""
+    single = n % 2 == 1 or not aligned
+    return "spmm_ragged_kernel" if single and n > 16 else "spmm_rowblock_kernel"
+
+
+@pytest.mark.parametrize("n,wide", [(17, 2), (31, 2), (33, 4), (47, 4), (101, 4), (130, 4)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_odd_widths_keep_their_order_of_additions(dev, n, wide, dtype):
+    """spmm_ragged_kernel adds as spmm_rowblock_kernel does, bit for bit: the first n columns of a
+    wider B, whose whole vectors take as many lanes and so as many groups and the same plan, come out
+    the same.  Rows over 8192 entries, short ones, single and several parts; 130 columns from B off a
+    vector's alignment, in three tiles."""
+    lengths = torch.tensor([3, 0, 9000, 127, 128, 129, 40, 250, 700] * 20 + [20000, 1])
+    ptr = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
+    cols = synthetic.randint(7, 1, int(ptr[-1]), 3000, "cpu").to(torch.int32)
+    data = synthetic.uniform_values(7, 2, cols.numel(), dtype, "cpu")
+    p = fs.prepare_spmm_csr_opt(data.to(dev), cols.to(dev), ptr.to(dev), (lengths.numel(), 3000))
+    # 2 * 16 or 4 * 16 lanes of 16 bytes: 32 or 64 lanes
+    N = max(n, (64 if wide == 4 else 32) * (16 // dtype.itemsize))
+    Bw = synthetic.dense_uniform(3000, N, dtype, seed=5, device=dev)
+    want = fs.flagsparse_spmm_csr_opt(B=Bw, prepared=p)[:, :n]
+    kc = p._kernel_csr()
+    assert kc.kernel_name(N) == "spmm_rowblock_kernel"
+    room = torch.empty(3000 * n + 1, dtype=dtype, device=dev)
+    B = room[n == 130:][:3000 * n].view(3000, n)
+    B.copy_(Bw[:, :n])
+    got = fs.flagsparse_spmm_csr_opt(B=B, prepared=p)
+    if N != n:
+        assert kc.kernel_name(n) == "spmm_ragged_kernel"
+    assert {k[0] for k in kc._plans} == {32 if wide == 2 else 64}  # one plan for both
+    assert torch.equal(got, want)
+    ref = oracle.spmm_csr(ptr, cols, data, B.cpu())
+    assert oracle.rel_l2(got, ref) <= oracle.REL_L2_BOUND[str(dtype)[6:]]
+
+
 @pytest.mark.parametrize("n", [1, 16, 47, 64])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_long_rows_keep_their_order_of_additions(dev, monkeypatch, n, dtype):
@@ -178,6 +215,7 @@ def test_long_rows_keep_their_order_of_additions(dev, monkeypatch, n, dtype):
         p = fs.prepare_spmm_csr_opt(data.to(dev), cols.to(dev), ptr.to(dev), shape)
         out.append(fs.flagsparse_spmm_csr_opt(B=B.to(dev), prepared=p).cpu())
         assert p._kernel_csr().kernel_name() == "spmm_rowblock_kernel"
+        assert p._kernel_csr().kernel_name(n) == _row_block_kernel(n, dtype)
         assert all(q.by_column == order for q in p._kernel_csr()._plans.values())
     assert torch.equal(out[0], out[1])
     ref = oracle.spmm_csr(ptr, cols, data, B)
@@ -229,6 +267,7 @@ def test_parts_of_every_length(dev, monkeypatch, n, dtype, offset, longest):
     p = fs.prepare_spmm_csr_opt(data.to(dev), cols.to(dev), ptr.to(dev), (lengths.numel(), 3000))
     out = fs.flagsparse_spmm_csr_opt(B=Bd, prepared=p).cpu()
     assert p._kernel_csr().kernel_name() == "spmm_rowblock_kernel"
+    assert p._kernel_csr().kernel_name(n) == _row_block_kernel(n, dtype, offset == 0)
     ref = oracle.spmm_csr(ptr, cols, data, B)
     assert torch.equal(out.double(), torch.as_tensor(ref).double())
 
