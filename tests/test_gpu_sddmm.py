@@ -1,6 +1,6 @@
-"""CSR SDDMM on the GPU (sddmm_csr_kernel) against the fp64 C oracle, plus the reference's API
-checks (tests/test_sddmm.py:514-557), its diagnostic variants (sddmm_csr.py:243-268) and the
-benchmark case's result dictionary (:552-572).
+"""CSR SDDMM on the GPU (the slices, the flat and the row-block kernel) against the fp64 C oracle,
+plus the reference's API checks (tests/test_sddmm.py:514-557), its diagnostic variants
+(sddmm_csr.py:243-268) and the benchmark case's result dictionary (:552-572).
 
 Bars: fp64, and fp32 with float64 accumulation ("acc64"): relative L2 <= 1e-12 / 1e-5 against
 the oracle.  fp32 accumulated in fp32 (the reference's baseline): the reference script's
@@ -12,7 +12,8 @@ import pytest
 import torch
 
 import flagsparse_amd as fs
-from flagsparse_amd import sddmm_csr, synthetic
+from flagsparse_amd import _abi, sddmm_csr, synthetic
+from flagsparse_amd._plan import build_row_block_plan_device
 from oracle import oracle
 
 pytestmark = pytest.mark.gpu
@@ -57,8 +58,8 @@ def test_sddmm_random(dev, dtype, K):
 
 
 def test_sddmm_long_rows_and_both_schedules(dev):
-    # rows far longer than the 128-entry split threshold (chunks shared by a workgroup) next to
-    # empty and short rows; the row-block schedule against the one-group-per-entry schedule
+    # rows of many slices next to empty and short rows; the slices against the
+    # one-group-per-entry schedule
     n_rows, n_cols, K = 40, 3000, 64
     lengths = torch.zeros(n_rows, dtype=torch.int64)
     lengths[3], lengths[7], lengths[20:30] = 5000, 129, 3
@@ -75,7 +76,6 @@ def test_sddmm_long_rows_and_both_schedules(dev):
     # the one-group-per-entry schedule agrees (same lane split of K and reduction; the compiler
     # may contract the multiply-adds differently, so equality is up to rounding)
     flat = torch.empty_like(out)
-    from flagsparse_amd import _abi
     lanes, vec = sddmm_csr._sddmm_lane_shape(K, x, y)
     _abi.check(_abi.lib().fsp_sddmm_csr(0, 0, 0, _abi.ptr(p.indices), _abi.ptr(p.row_ids), None,
                                         32, p.nnz, _abi.ptr(x), K, _abi.ptr(y), K, K, None, 1.0,
@@ -83,6 +83,35 @@ def test_sddmm_long_rows_and_both_schedules(dev):
                                         _abi.stream_handle(dev)), "fsp_sddmm_csr")
     _check(flat, indptr, indices, x, y, None, 1.0, 0.0)
     torch.testing.assert_close(out, flat, rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("K", [0, 1, 7, 16, 33, 64, 100, 256])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("ptr", [torch.int32, torch.int64])
+def test_sddmm_over_a_row_block_plan(dev, K, dtype, ptr):
+    """The row-block schedule of fsp_sddmm_csr, which the package itself no longer takes, with a plan
+    in the limits that the entry point names: short-row blocks, rows of several chunks, empty rows."""
+    lengths = torch.tensor([3, 0, 5000, 1, 129, 128, 2, 40] * 5 + [0] * 300 + [2] * 700)
+    ip = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
+    nnz, n_rows, n_cols = int(ip[-1]), lengths.numel(), 2000
+    cols = synthetic.randint(8, 1, nnz, n_cols, "cpu").to(torch.int32).to(dev)
+    x = synthetic.dense_uniform(n_rows, max(K, 1), dtype, seed=8, device=dev)
+    y = synthetic.dense_uniform(n_cols, max(K, 1), dtype, seed=9, device=dev)
+    data = synthetic.uniform_values(8, 2, nnz, dtype, "cpu").to(dev)
+    rowptr = ip.to(ptr).to(dev)
+    lanes, vec = sddmm_csr._sddmm_lane_shape(max(K, 1), x, y)
+    assert K <= 4 * lanes * vec
+    cap = _abi.caps()["spmm_block_nnz"]
+    plan = build_row_block_plan_device(rowptr, cap, 256 // lanes, 128, cap,
+                                       window_rows=4 * (256 // lanes))
+    out = torch.empty(nnz, dtype=dtype, device=dev)
+    print(f"row-block sddmm K={K} {dtype} {ptr}", flush=True)
+    _abi.check(_abi.lib().fsp_sddmm_csr(
+        _abi.dtype_code(dtype), 0, 0, _abi.ptr(cols), None, _abi.ptr(rowptr),
+        32 if ptr == torch.int32 else 64, nnz, _abi.ptr(x), x.stride(0), _abi.ptr(y), y.stride(0),
+        K, _abi.ptr(data), 0.5, 2.0, _abi.ptr(out), _abi.ptr(plan.desc), _abi.ptr(plan.ranges),
+        plan.n_desc, lanes, vec, _abi.stream_handle(dev)), "fsp_sddmm_csr")
+    _check(out, ip, cols, x[:, :K], y[:, :K], data, 0.5, 2.0)
 
 
 def test_sddmm_strided_and_unaligned_dense(dev):
