@@ -555,8 +555,13 @@ def _sddmm_workload(dev, dtype_name, K, torch, fs, synthetic):
     out = torch.empty(prepared.nnz, dtype=vdt, device=dev)
     v = x.element_size()
     nnz = prepared.nnz
-    # per entry: column, row id, result; x and y rows once each
-    nbytes = nnz * (4 + 4 + v) + shape[0] * K * v + shape[1] * K * v
+    # per entry: column and result; x and y rows once each; the row pointers, or, past four steps
+    # of 64 lanes of 16 bytes, where the flat kernel runs, a row id per entry
+    sliced = K <= 4 * 64 * (16 // v)
+    kernel = "sddmm_slices_kernel" if sliced else "sddmm_flat_kernel"
+    p_k = 4 if nnz <= 2**31 - 1 else 8
+    nbytes = nnz * (4 + v) + ((shape[0] + 1) * p_k if sliced else nnz * 4) + \
+        shape[0] * K * v + shape[1] * K * v
     info = {"n_rows": shape[0], "n_cols": shape[1], "nnz": nnz, "K": K,
             "path": "flagsparse_sddmm_csr (baseline variant)", "prepare_ms": prep_ms,
             "inputs": {"indices": idx, "indptr": ptr, "x": x, "y": y}}
@@ -585,10 +590,10 @@ def _sddmm_workload(dev, dtype_name, K, torch, fs, synthetic):
     return {
         "step": lambda: fs.flagsparse_sddmm_csr(x=x, y=y, prepared=prepared, out=out),
         "launch": lambda: mod._launch_sddmm(prepared, x, y, None, 1.0, 0.0, out, False),
-        "bytes_gather_inclusive": nnz * (4 + 4 + v + 2 * K * v),
+        "bytes_gather_inclusive": nnz * (4 + v + 2 * K * v) + (0 if sliced else 4 * nnz),
         "nbytes": nbytes, "flops": 2 * nnz * K, "info": info, "cpu": cpu,
-        "dtype": dtype_name, "kernel": "sddmm_csr_kernel",
-        "tag": f"sddmm_csr_kernel_{dtype_name}_k{K}",
+        "dtype": dtype_name, "kernel": kernel,
+        "tag": f"{kernel}_{dtype_name}_k{K}",
     }
 
 

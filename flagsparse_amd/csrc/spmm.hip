@@ -384,7 +384,7 @@ __global__ __launch_bounds__(kBlock / VW) void spmm_ragged_kernel(
 // Bound by latency: a thread's sums depend on each other, its loads need not, so 32 of them are
 // requested before the first is added (held apart by the barrier), in the same order of additions.
 // MI355X, fp32, 200k power-law rows, the longest of 50,000 entries (390 parts): N = 47 one load at a
-// time 94 us, so 12.7; the product 279 -> 195 us, N = 128 302 -> 219.
+// time 94 us, so 13; the product 279 -> 195 us, N = 128 302 -> 233.
 constexpr int kPartsInFlight = 32;
 template <typename T, typename A>
 __global__ __launch_bounds__(kBlock) void spmm_split_combine_kernel(
@@ -439,7 +439,10 @@ int launch_spmm(const void* vals, const int32_t* cols, const void* rowptr, int64
                 int64_t n_tiles, int xcd_remap, hipStream_t st) {
   // Single elements give way to vectors from 32 lanes on.  With 16, 2048 staged entries a workgroup
   // leave room for few workgroups: fp32 N = 15 83.0 us with single elements, 86.5 with vectors
-  // (900k rows, N = 13: 384 / 400); fp64 N = 15 141 / 134.
+  // (900k rows, N = 13: 384 / 400); fp64 N = 15 141 / 134.  Pairs of float32 (N = 2 mod 4, B and C
+  // aligned) stay with their lanes and so their order of additions, though vectors, in the lanes of
+  // single elements, take less: N = 34 146 / 106 us, 50 161 / 133, 66 230 / 225, 130 497 / 356 (from
+  // N = 66 on with the same groups).
   bool ragged = false;
   if constexpr (VW == 1 && sizeof(A) == sizeof(T)) {
     constexpr int kVec = 16 / sizeof(T);

@@ -325,7 +325,7 @@ def _spmm_slice_shape(lanes, positions, by_column=False):
 # orders differ by up to 4.6e-5 of the result's root mean square (200k rows of power-law lengths,
 # N = 47), against 1e-6 below.  Prepared products on such rows keep the order of the row-block
 # kernel, 128-entry parts added one after another, bit for bit, and change only the launch order
-# of the parts (slices would take 56 / 119 / 207 us where that takes 61 / 130 / 219: fp32, N = 16 / 47
+# of the parts (slices would take 57 / 122 / 214 us where that takes 60 / 130 / 233: fp32, N = 16 / 47
 # / 128).
 _SPMM_SUMS_KEPT = 8192
 
@@ -335,7 +335,7 @@ def _parts_by_column(desc, cols, n_cols, rowptr, chunk):
     by the first column they hold, each XCD a contiguous eighth of either.  Parts of different
     rows over the same columns then read the same rows of B while they are in that XCD's L2.
     Measured on MI355X, us, in row order / in this order: 200k rows of power-law lengths, fp32
-    N=16 89 / 61, N=47 231 / 130, N=128 382 / 234; fp64 N=33 287 / 176, N=64 379 / 256.  Ordered
+    N=16 89 / 60, N=47 231 / 130, N=128 382 / 233; fp64 N=33 287 / 176, N=64 379 / 256.  Ordered
     by 256 column bins in three launches (csrc/slices.hip): a full sort and gathers by torch took
     0.34 ms more of a matrix's first product (N=47: 815 / 479 us) for the same 195 us after it."""
     L = _abi.lib()
