@@ -20,7 +20,9 @@
 //   * the piece of a row that goes on in the next slice goes to carry[k], the end of a row begun
 //     earlier to head[k]; spmm_slice_fixup_kernel adds the pieces in slice order.  A slot for either
 //     of every slice needs no count; where that is much room (wide N, few cut rows), the pieces are
-//     counted (fsp_slice_pieces) and lie one after the other: slice k's from pieces[k].
+//     counted (fsp_slice_pieces) and lie one after the other: slice k's from pieces[k] (COUNTED,
+//     a kernel of its own: as a test in the other it cost single elements 13 %, 50k rows of 200,
+//     fp32 N=3 33.5 / 38.1 us).
 //
 // Bound: the B rows' fills from outside L2 (whole 128-byte lines), as spmm_rowblock_kernel.
 // Measured on MI355X, row blocks / slices: a power law of 200k rows and 4.8M entries, fp32 N=47
@@ -73,7 +75,7 @@ __device__ __forceinline__ void add_entries(const int* s_col, const T* s_val, in
 }
 
 // UPT: quads of entries per thread (a slice holds at most UPT * 1024 - 3 entries).
-template <typename T, typename A, typename P, int VW, int UPT>
+template <typename T, typename A, typename P, int VW, int UPT, bool COUNTED>
 __global__ __launch_bounds__(kBlock, 8) void spmm_slices_kernel(
     const T* __restrict__ vals, const int* __restrict__ cols, const P* __restrict__ rowptr,
     P nnz_total, const T* __restrict__ B, uint32_t ldb, int N, T* __restrict__ C, int64_t ldc,
@@ -144,10 +146,10 @@ __global__ __launch_bounds__(kBlock, 8) void spmm_slices_kernel(
   const T* Bc = B + ncol;
   auto put = [&](int s, const A(&acc)[VW]) {
     if (s == R) {
-      const int64_t slot = pieces ? pieces[k] + (begun ? 1 : 0) : k;
+      const int64_t slot = COUNTED ? pieces[k] + (begun ? 1 : 0) : k;
       store_any<A, A, VW>(carry + slot * N + ncol, acc);
     } else if (s == 0 && begun) {
-      const int64_t slot = pieces ? pieces[k] : k;
+      const int64_t slot = COUNTED ? pieces[k] : k;
       store_any<A, A, VW>(head + slot * N + ncol, acc);
     } else {
       store_any<T, A, VW>(C + (i0 + s) * ldc + ncol, acc);
@@ -228,7 +230,7 @@ __global__ __launch_bounds__(kBlock, 8) void spmm_slices_kernel(
 // such end: cw threads side by side over the columns, the 256 / cw groups over the pieces, their
 // sums added in a fixed tree.  (64 slices to a workgroup: a power law's many rows of a few
 // pieces then wait for each other, 32 instead of 8 us at N = 47.)
-template <typename T, typename A, typename P>
+template <typename T, typename A, typename P, bool COUNTED>
 __global__ __launch_bounds__(kBlock) void spmm_slice_fixup_kernel(
     const P* __restrict__ rowptr, const int64_t* __restrict__ table, int64_t Wpos,
     const A* __restrict__ carry, const A* __restrict__ head, const int* __restrict__ pieces, int N,
@@ -241,7 +243,7 @@ __global__ __launch_bounds__(kBlock) void spmm_slice_fixup_kernel(
   if (a >= p0) return;  // it begins here
   int64_t j0 = (a + row) / Wpos;  // the slice the row began in (spmv_slice_fixup_kernel)
   if (table[2 * j0 + 3] <= a) ++j0;
-  if (pieces) {  // counted: the row's pieces lie one after the other, up to pieces[k]
+  if constexpr (COUNTED) {  // the row's pieces lie one after the other, up to pieces[k]
     carry += (pieces[k] - k) * N;
     head += (pieces[k] - k) * N;
   }
@@ -288,7 +290,7 @@ struct SliceArgs {
   hipStream_t st;
 };
 
-template <typename T, typename A, typename P, int VW, int UPT>
+template <typename T, typename A, typename P, int VW, int UPT, bool COUNTED>
 int launch_upt(const SliceArgs& a) {
   const int64_t n = slice_count(a.n_rows, a.nnz, a.items);
   const int cap = (int)((a.items + a.keep + 6 + 3) & ~int64_t(3));
@@ -297,11 +299,11 @@ int launch_upt(const SliceArgs& a) {
   const int64_t tiles = (a.N + W - 1) / W;
   const size_t lds = (size_t)kWavesPerBlock * W * sizeof(A) + (size_t)cap * (sizeof(T) + 4) +
                      4 * (size_t)(rows_cap + 2 + (kBlock >> a.lg) + 1);
-  const bool counted = a.cut_rows == FSP_CUT_PIECES;
   A* carry = static_cast<A*>(a.sums);
-  A* head = counted ? carry : carry + n * a.N;
-  const int* pieces = counted ? reinterpret_cast<const int*>(a.table + 2 * (n + 1)) : nullptr;
-  hipLaunchKernelGGL((spmm_slices_kernel<T, A, P, VW, UPT>), dim3((unsigned)n, (unsigned)tiles),
+  A* head = COUNTED ? carry : carry + n * a.N;
+  const int* pieces = COUNTED ? reinterpret_cast<const int*>(a.table + 2 * (n + 1)) : nullptr;
+  hipLaunchKernelGGL((spmm_slices_kernel<T, A, P, VW, UPT, COUNTED>),
+                     dim3((unsigned)n, (unsigned)tiles),
                      dim3(kBlock), lds, a.st, static_cast<const T*>(a.vals), a.cols,
                      static_cast<const P*>(a.rowptr), (P)a.nnz, static_cast<const T*>(a.B),
                      (uint32_t)a.ldb, (int)a.N, static_cast<T*>(a.C), a.ldc, a.table, a.order, (int)n, cap,
@@ -310,7 +312,7 @@ int launch_upt(const SliceArgs& a) {
   if (rc || !a.cut_rows) return rc;
   int cw = 1;
   while (cw < a.N && cw < kBlock) cw <<= 1;
-  hipLaunchKernelGGL((spmm_slice_fixup_kernel<T, A, P>),
+  hipLaunchKernelGGL((spmm_slice_fixup_kernel<T, A, P, COUNTED>),
                      dim3((unsigned)n), dim3(kBlock), 0, a.st,
                      static_cast<const P*>(a.rowptr), a.table, a.items, carry, head, pieces, (int)a.N,
                      cw, static_cast<T*>(a.C), a.ldc);
@@ -319,8 +321,10 @@ int launch_upt(const SliceArgs& a) {
 
 template <typename T, typename A, typename P, int VW>
 int launch_vec(const SliceArgs& a) {
-  if (a.items + a.keep + 6 <= 4 * kBlock) return launch_upt<T, A, P, VW, 1>(a);
-  return launch_upt<T, A, P, VW, 2>(a);
+  const bool counted = a.cut_rows == FSP_CUT_PIECES;
+  if (a.items + a.keep + 6 <= 4 * kBlock)
+    return counted ? launch_upt<T, A, P, VW, 1, true>(a) : launch_upt<T, A, P, VW, 1, false>(a);
+  return counted ? launch_upt<T, A, P, VW, 2, true>(a) : launch_upt<T, A, P, VW, 2, false>(a);
 }
 
 template <typename T, typename A, typename P>
