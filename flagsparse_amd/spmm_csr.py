@@ -355,8 +355,7 @@ class _SpmmKernelCsr:
     one call, so nothing is planned."""
 
     __slots__ = ("data", "cols", "rowptr", "rowptr_bits", "nnz", "n_rows", "_plans", "_args",
-                 "_keep", "_order", "max_row_nnz", "one_shot", "_tables", "_pieces", "_sums",
-                 "_row_order", "_names")
+                 "_keep", "_order", "max_row_nnz", "one_shot", "_tables", "_shared")
 
     def __init__(self, data, cols, indptr, max_row_nnz=None, one_shot=False):
         self.max_row_nnz = max_row_nnz
@@ -370,12 +369,11 @@ class _SpmmKernelCsr:
         else:
             self.rowptr, self.rowptr_bits = indptr.to(torch.int64).contiguous(), 64
         self._tables = {}
-        self._pieces = {}
-        self._sums = {}
-        self._names = {}  # the kernel of each width's latest bound call
-        self._plans = {}      # by lanes and whether in column order; in use
-        self._row_order = {}  # by lanes, in row order
-        self._args = _abi.Calls()
+        # what products of several widths share: ("pieces", slice size), ("sums", length, dtype),
+        # ("row order", lanes), and ("name", N), the kernel of that width's latest bound call
+        self._shared = {}
+        self._plans = {}  # by lanes and whether in column order
+        self._args = {} if one_shot else _abi.Calls()
         self._keep = [self.data, self.cols, self.rowptr]  # what a launch reads or writes
         self._order = StreamOrder(self.data.device)
 
@@ -383,7 +381,7 @@ class _SpmmKernelCsr:
         """The kernel that the latest product of this width ran; without a width, or before a
         product of it, the kernel of the matrix's layout for whole vectors."""
         layout = "spmm_rowblock_kernel" if self._plans or not self.sliced() else "spmm_slices_kernel"
-        return self._names.get(n_dense_cols, layout)
+        return self._shared.get(("name", n_dense_cols), layout)
 
     def describe(self):
         plans = {f"{lanes} by column" if by_column else lanes:
@@ -418,19 +416,21 @@ class _SpmmKernelCsr:
         """(the table to launch with, room for the pieces of cut rows, the kind of cut): a slot for
         either end of every slice, or, where that is too much, for each piece.  Calls are ordered
         (StreamOrder), so those of one size share it."""
-        length, cut = (int(table.numel()) - 2) * n_dense_cols, 1
-        if length * dtype.itemsize > _SUMS_ROOM and (
-                items in self._pieces or not torch.cuda.is_current_stream_capturing()):
-            if items not in self._pieces:  # the count is waited for, which a capture may not do
-                self._pieces[items] = _slices.pieces(self.rowptr, table)
-            table, n = self._pieces[items]
+        length, cut = (table.numel() - 2) * n_dense_cols, 1
+        if length > _SUMS_ROOM // 8 and length * dtype.itemsize > _SUMS_ROOM and (
+                ("pieces", items) in self._shared
+                or not torch.cuda.is_current_stream_capturing()):  # the count is waited for
+            counted = self._shared.get(("pieces", items))
+            if counted is None:
+                counted = self._shared["pieces", items] = _slices.pieces(self.rowptr, table)
+            table, n = counted
             if n == 0:
                 return table, None, 0
             length, cut = n * n_dense_cols, _abi.FSP_CUT_PIECES
-        sums = self._sums.get((length, dtype))
+        sums = self._shared.get(("sums", length, dtype))
         if sums is None:
-            sums = self._sums[length, dtype] = torch.empty(length, dtype=dtype,
-                                                           device=table.device)
+            sums = torch.empty(length, dtype=dtype, device=table.device)
+            self._shared["sums", length, dtype] = sums
         return table, sums, cut
 
     def plan(self, lanes, row_bytes=0, n_cols=0):
@@ -444,9 +444,9 @@ class _SpmmKernelCsr:
                                     self.nnz * row_bytes, False)
         p = self._plans.get((lanes, by_column))
         if p is None:
-            p = self._row_order.get(lanes)
+            p = self._shared.get(("row order", lanes))
             if p is None:
-                p = self._row_order[lanes] = build_row_block_plan_device(
+                p = self._shared["row order", lanes] = build_row_block_plan_device(
                     self.rowptr, cap, ngrp, threshold, chunk,
                     window_rows=SPMM_PLAN_WINDOW_BLOCKS * ngrp)
             if by_column:
@@ -487,13 +487,13 @@ def _bind_sliced(kc, B, acc_f64, lanes, vec):
     if not by_column:
         items, keep = _spmm_slice_shape(lanes, positions)
     table, order = kc.slices(items, keep, n_cols, by_column)
-    if kc.max_row_nnz is None and (int(table.numel()) - 2) * n_dense_cols > _SUMS_UNSEEN:
+    if kc.max_row_nnz is None and (table.numel() - 2) * n_dense_cols > _SUMS_UNSEEN:
         kc.max_row_nnz = int((kc.rowptr[1:] - kc.rowptr[:-1]).max())
     sums, cut = None, 0
     if kc.max_row_nnz is None or kc.max_row_nnz > keep:
         table, sums, cut = kc.piece_slots((items, keep), table, n_dense_cols,
                                           torch.float64 if acc_f64 else B.dtype)
-    kc._names[n_dense_cols] = "spmm_slices_kernel"
+    kc._shared["name", n_dense_cols] = "spmm_slices_kernel"
     kc._keep.extend((table, order, sums))
     return _abi.bind(
         "spmm_sliced", _abi.dtype_code(B.dtype), 1 if acc_f64 else 0, kc.data.data_ptr(),
@@ -513,7 +513,7 @@ def _bind_row_blocks(kc, B, acc_f64, lanes, vec):
     # launch_spmm's rule (csrc/spmm.hip)
     ragged = (vec == 1 and lanes >= 32 and n_dense_cols * B.element_size() >= 16
               and (not acc_f64 or B.dtype == torch.float64))
-    kc._names[n_dense_cols] = "spmm_ragged_kernel" if ragged else "spmm_rowblock_kernel"
+    kc._shared["name", n_dense_cols] = "spmm_ragged_kernel" if ragged else "spmm_rowblock_kernel"
     kc._keep.extend((partials, plan.desc, groups, group_base, split_rows))
     return _abi.bind(
         "spmm_csr", _abi.dtype_code(B.dtype), 1 if acc_f64 else 0, p(kc.data), p(kc.cols),
