@@ -171,11 +171,24 @@ __global__ __launch_bounds__(kThreads) void csr_check_kernel(
         }
       }
     }
-    a = block_reduce<true>(dec, s_w);
     b = block_reduce<false>(~longest, s_w);
-    if constexpr (COUNT) {
-      uneven = block_reduce<true>(uneven, s_w);
-      cut = block_reduce<true>(cut, s_w);
+    if constexpr (COUNT) {  // the three sums behind one barrier
+      __shared__ int64_t s_sum[3][kWaves];
+      const int64_t d = wave_add_i64(dec), u = wave_add_i64(uneven), c = wave_add_i64(cut);
+      if ((tid & (kWave - 1)) == 0) {
+        s_sum[0][tid / kWave] = d;
+        s_sum[1][tid / kWave] = u;
+        s_sum[2][tid / kWave] = c;
+      }
+      __syncthreads();
+      a = uneven = cut = 0;
+      for (int w = 0; w < kWaves; ++w) {
+        a += s_sum[0][w];
+        uneven += s_sum[1][w];
+        cut += s_sum[2][w];
+      }
+    } else {
+      a = block_reduce<true>(dec, s_w);
     }
   }
   constexpr int kWords = COUNT ? kRowWords : kCsrWords;
