@@ -171,6 +171,7 @@ __global__ __launch_bounds__(kThreads) void csr_check_kernel(
         }
       }
     }
+    if constexpr (!COUNT) a = block_reduce<true>(dec, s_w);
     b = block_reduce<false>(~longest, s_w);
     if constexpr (COUNT) {  // the three sums behind one barrier
       __shared__ int64_t s_sum[3][kWaves];
@@ -187,8 +188,6 @@ __global__ __launch_bounds__(kThreads) void csr_check_kernel(
         uneven += s_sum[1][w];
         cut += s_sum[2][w];
       }
-    } else {
-      a = block_reduce<true>(dec, s_w);
     }
   }
   constexpr int kWords = COUNT ? kRowWords : kCsrWords;
