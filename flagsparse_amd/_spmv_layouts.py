@@ -260,7 +260,7 @@ class SliceLayout:
         self._keep = (scratch, self.data, self.cols, self.rowptr)
         self._sums_at = 16 * (n + 1)  # in scratch, behind the table
         self._table_built = int(not one_shot)
-        self._args = _abi.Calls()
+        self._args = {} if one_shot else _abi.Calls()
         self._order = StreamOrder(self.data.device)
 
     def kernel_name(self):
@@ -1443,7 +1443,9 @@ def build_layout(data, cols, rowptr, n_cols, one_shot=False, max_row_nnz=None, r
     knows it and asks for no row map; row_classes: what the check counted by row_class_bounds."""
     mode = FORCE
     nnz = int(data.numel())
-    few = _abi.lib().fsp_spmv_slices(int(rowptr.numel()) - 1, nnz) <= _slices.MAX_SLICES
+    n_rows = int(rowptr.numel()) - 1
+    few = (n_rows + nnz <= _slices.MAX_SLICES  # (then no need to ask)
+           or _abi.lib().fsp_spmv_slices(n_rows, nnz) <= _slices.MAX_SLICES)
     if mode is None and one_shot and few:  # else the row blocks, of which there are fewer
         return SliceLayout(data, cols, rowptr, max_row_nnz, one_shot=True)
     if mode is None and one_shot:
