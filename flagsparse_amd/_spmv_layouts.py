@@ -1500,9 +1500,9 @@ def row_class_bounds(n_rows, nnz):
 
 def slices_pay(cols, rowptr, n_cols, max_row_nnz, uneven_rows, cut_entries):
     """Whether a prepared matrix runs on slices rather than row blocks, by the rows and entries of
-    its row_class_bounds.  Row blocks are the faster
-    where rows are alike: a block sums its rows with the same lanes each, nothing is searched, and
-    it can run in the order of its band.  They lose where
+    its row_class_bounds.  Row blocks are the faster where rows are alike: a block sums its rows
+    with the same lanes each, nothing is searched, and it can run in the order of its band.  They
+    lose where
     * rows of very different lengths share a block, whose other lanes wait for the longest: power
       laws.  Row blocks / slices on MI355X, us, float32: 40k rows of mean 12 30.2 / 8.5, 300k of 20
       49.8 / 28.0, 900k of 6 60.4 / 35.1, all with over 0.6 such rows to a block; 900k rows of 0 to

@@ -1,5 +1,5 @@
 // CSR SpMV without a plan: the matrix cut into slices of about equal work, for calls that use
-// a matrix once (no prepared object).
+// a matrix once (no prepared object) and for prepared matrices with very uneven rows.
 //
 // Reference behaviour followed (src/flagsparse/sparse_operations/):
 //   spmv_csr.py:94-120    y[row] = sum over the row's entries, float32 summed in float64
@@ -10,9 +10,10 @@
 // table sizes.  Here the number of slices is known from the sizes alone: the rows and entries
 // are laid on one line in which row r takes the positions rowptr[r] + r .. rowptr[r+1] + r (its
 // entries, then its end), and slice k starts at position k * W.  slice_table_kernel finds the
-// row there by binary search.  A boundary inside a row of at most T entries moves to that row's
-// start, so only longer rows are cut; a slice holds at most W + T + 3 rows and entries
-// together, whatever the row lengths, empty rows included.
+// row there by binary search.  (The line is that of merge-based CSR SpMV, Merrill and Garland,
+// SC 2016; here whole rows are kept together where they can be.)  A boundary inside a row of at
+// most T entries moves to that row's start, so only longer rows are cut; a slice holds at most
+// W + T + 3 rows and entries together, whatever the row lengths, empty rows included.
 //
 // spmv_slices_kernel: a workgroup reads its slice's entries with 16-byte loads, leaves the
 // products in LDS and sums its rows (G lanes each, rows much longer than their neighbours a

@@ -303,19 +303,18 @@ int launch_upt(const SliceArgs& a) {
   A* head = COUNTED ? carry : carry + n * a.N;
   const int* pieces = COUNTED ? reinterpret_cast<const int*>(a.table + 2 * (n + 1)) : nullptr;
   hipLaunchKernelGGL((spmm_slices_kernel<T, A, P, VW, UPT, COUNTED>),
-                     dim3((unsigned)n, (unsigned)tiles),
-                     dim3(kBlock), lds, a.st, static_cast<const T*>(a.vals), a.cols,
-                     static_cast<const P*>(a.rowptr), (P)a.nnz, static_cast<const T*>(a.B),
-                     (uint32_t)a.ldb, (int)a.N, static_cast<T*>(a.C), a.ldc, a.table, a.order, (int)n, cap,
-                     rows_cap, a.lg, carry, head, pieces, a.xcd_remap);
+                     dim3((unsigned)n, (unsigned)tiles), dim3(kBlock), lds, a.st,
+                     static_cast<const T*>(a.vals), a.cols, static_cast<const P*>(a.rowptr),
+                     (P)a.nnz, static_cast<const T*>(a.B), (uint32_t)a.ldb, (int)a.N,
+                     static_cast<T*>(a.C), a.ldc, a.table, a.order, (int)n, cap, rows_cap, a.lg,
+                     carry, head, pieces, a.xcd_remap);
   int rc = check_hip(hipGetLastError(), "spmm_slices_kernel launch");
   if (rc || !a.cut_rows) return rc;
   int cw = 1;
   while (cw < a.N && cw < kBlock) cw <<= 1;
-  hipLaunchKernelGGL((spmm_slice_fixup_kernel<T, A, P, COUNTED>),
-                     dim3((unsigned)n), dim3(kBlock), 0, a.st,
-                     static_cast<const P*>(a.rowptr), a.table, a.items, carry, head, pieces, (int)a.N,
-                     cw, static_cast<T*>(a.C), a.ldc);
+  hipLaunchKernelGGL((spmm_slice_fixup_kernel<T, A, P, COUNTED>), dim3((unsigned)n),
+                     dim3(kBlock), 0, a.st, static_cast<const P*>(a.rowptr), a.table, a.items,
+                     carry, head, pieces, (int)a.N, cw, static_cast<T*>(a.C), a.ldc);
   return check_hip(hipGetLastError(), "spmm_slice_fixup_kernel launch");
 }
 
