@@ -404,16 +404,9 @@ class _SpmmKernelCsr:
             return True
         if not _SPMM_ROW_SPLIT_THRESHOLD < self.max_row_nnz <= _SPMM_SUMS_KEPT:
             return False
-        return not self.few_long() or (lanes >= 32 and self.nnz <= 16 * self.n_rows)
-
-    def few_long(self):
-        """Whether some widths of this matrix run on row blocks and some on slices."""
-        return (self.long_entries is not None and 10 * self.long_entries < self.nnz
-                and _SPMM_ROW_SPLIT_THRESHOLD < self.max_row_nnz <= _SPMM_SUMS_KEPT)
-
-    def planned(self):
-        """The lanes of the plans that are there."""
-        return [key[1] for key in self._shared if key[0] == "row order"]
+        if self.long_entries is None or 10 * self.long_entries >= self.nnz:
+            return True
+        return lanes >= 32 and self.nnz <= 16 * self.n_rows
 
     def slices(self, items, keep, n_cols, by_column):
         """The slices' boundaries and launch order (built on the current stream, once)."""
@@ -535,24 +528,6 @@ def _bind_row_blocks(kc, B, acc_f64, lanes, vec):
         int(groups.shape[0]), 0 if plan.by_column else XCD_REMAP)
 
 
-def _bind_at_hand(kc, B, acc_f64, blocks, lane_shape, slice_lanes):
-    """The call for a graph's capture, where neither slices nor a plan can be built: with what an
-    earlier width left, which for a matrix of few_long may be the other of the two, or a plan of
-    other lanes (the columns are tiled by them).  Not kept for later calls."""
-    bound, (lanes, vec) = None, lane_shape
-    if blocks and lanes in kc.planned():
-        bound = _bind_row_blocks(kc, B, acc_f64, lanes, vec)
-    if bound is None:
-        try:
-            bound = _bind_sliced(kc, B, acc_f64, *slice_lanes)
-        except RuntimeError:  # no slices
-            for lanes in kc.planned()[:1]:
-                bound = _bind_row_blocks(kc, B, acc_f64, lanes, vec)
-            if bound is None:
-                raise
-    return bound
-
-
 def _run_spmm(kc, B, C, acc_f64, tile_cols=None):
     """C[n_rows, N] = A @ B (B, C contiguous row-major) on slices or row blocks (kc.sliced).
     Without an explicit tile (the reference's block_n), a B over SPMM_B_TILE_BYTES is tiled by
@@ -572,14 +547,12 @@ def _run_spmm(kc, B, C, acc_f64, tile_cols=None):
         lanes, vec = _spmm_lane_shape(n_dense_cols, B.dtype, B, C, tile_cols)
         kept = not kc.one_shot and (kc.max_row_nnz or 0) > _SPMM_SUMS_KEPT
         # the row-block kernel's loads need aligned vectors
-        blocks = not (kc.sliced(lanes) or (vec < slice_vec and not kept))
-        if kc.few_long() and torch.cuda.is_current_stream_capturing():
-            bound = _bind_at_hand(kc, B, acc_f64, blocks, (lanes, vec), (slice_lanes, slice_vec))
-        else:
-            bound = _bind_row_blocks(kc, B, acc_f64, lanes, vec) if blocks else None
-            if bound is None:
-                bound = _bind_sliced(kc, B, acc_f64, slice_lanes, slice_vec)
-            kc._args[key] = bound
+        bound = None
+        if not (kc.sliced(lanes) or (vec < slice_vec and not kept)):
+            bound = _bind_row_blocks(kc, B, acc_f64, lanes, vec)
+        if bound is None:
+            bound = _bind_sliced(kc, B, acc_f64, slice_lanes, slice_vec)
+        kc._args[key] = bound
     _abi.run(bound, b, c, stream)
     return C
 

@@ -405,16 +405,6 @@ def test_more_row_blocks_than_a_launch_holds(dev, monkeypatch):
     assert oracle.rel_l2(C, oracle.spmm_csr(ip, cols, vals, B)) <= 1e-5
 
 
-def _few_long(dev, dtype, base, rows):
-    lengths = torch.full((5000,), base, dtype=torch.int64)
-    lengths[torch.arange(len(rows)) * 7 + 2500] = torch.tensor(rows)
-    ip = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
-    cols = synthetic.randint(3, 1, int(ip[-1]), 4000, "cpu")
-    vals = synthetic.uniform_values(3, 2, cols.numel(), dtype, "cpu")
-    return vals, cols, ip, fs.prepare_spmm_csr_opt(vals.to(dev), cols.to(dev), ip.to(dev),
-                                                   (5000, 4000))
-
-
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 @pytest.mark.parametrize("base,rows,N,blocks", [
     (32, [3000], 16, True), (32, [3000], 256, True), (12, [200, 700], 8, True),
@@ -422,54 +412,14 @@ def _few_long(dev, dtype, base, rows):
     (5, [300], 8, True), (5, [300], 256, False),  # short rows on 64 lanes
     (32, [3000] * 30, 16, False)])      # long rows that matter
 def test_few_long_rows_keep_row_blocks(dev, base, rows, N, blocks, dtype):
-    vals, cols, ip, p = _few_long(dev, dtype, base, rows)
+    lengths = torch.full((5000,), base, dtype=torch.int64)
+    lengths[torch.arange(len(rows)) * 7 + 2500] = torch.tensor(rows)
+    ip = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
+    cols = synthetic.randint(3, 1, int(ip[-1]), 4000, "cpu")
+    vals = synthetic.uniform_values(3, 2, cols.numel(), dtype, "cpu")
     B = synthetic.dense_uniform(4000, N, dtype, seed=3, device="cpu")
+    p = fs.prepare_spmm_csr_opt(vals.to(dev), cols.to(dev), ip.to(dev), (5000, 4000))
     C = fs.flagsparse_spmm_csr_opt(B=B.to(dev), prepared=p)
     assert p._kernel_csr().kernel_name(N) == ("spmm_rowblock_kernel" if blocks
                                               else "spmm_slices_kernel")
     assert oracle.rel_l2(C, oracle.spmm_csr(ip, cols, vals, B)) <= oracle.REL_L2_BOUND[str(dtype)[6:]]
-
-
-@pytest.mark.parametrize("base,first,width", [
-    (32, 16, 64),   # row blocks, of other lanes
-    (32, 64, 16),
-    (32, 15, 16),   # row blocks preferred, slices there
-    (32, 16, 15),   # and the other way round
-    (32, 16, 3),
-    (5, 8, 256),
-    (5, 256, 8)])
-def test_few_long_rows_in_a_capture(dev, base, first, width):
-    # a width first used in a capture runs on what the width before it left
-    vals, cols, ip, p = _few_long(dev, torch.float32, base, [300])
-    B1, B = (synthetic.dense_uniform(4000, n, torch.float32, seed=n, device="cpu")
-             for n in (first, width))
-    fs.flagsparse_spmm_csr_opt(B=B1.to(dev), prepared=p)
-    Bd = B.to(dev)
-    C = torch.zeros(5000, width, device=dev)
-    torch.cuda.synchronize()
-    g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g):
-        fs.flagsparse_spmm_csr_opt(B=Bd, prepared=p, out=C)
-    ref = oracle.spmm_csr(ip, cols, vals, B)
-    for _ in range(3):
-        C.fill_(7)
-        g.replay()
-        torch.cuda.synchronize()
-        assert oracle.rel_l2(C, ref) <= 1e-5
-        assert oracle.rel_l2(fs.flagsparse_spmm_csr_opt(B=Bd, prepared=p), ref) <= 1e-5
-        torch.cuda.synchronize()
-    kc = p._kernel_csr()
-    assert kc.kernel_name(width) == ("spmm_slices_kernel" if width in (15, 256)
-                                     else "spmm_rowblock_kernel")
-
-
-def test_few_long_rows_in_a_capture_of_the_first_call(dev):
-    vals, cols, ip, p = _few_long(dev, torch.float32, 32, [300])
-    Bd = torch.ones(4000, 16, device=dev)
-    torch.cuda.synchronize()
-    with pytest.raises(RuntimeError, match="once before"):
-        with torch.cuda.graph(torch.cuda.CUDAGraph()):
-            fs.flagsparse_spmm_csr_opt(B=Bd, prepared=p)
-    torch.cuda.synchronize()
-    assert oracle.rel_l2(fs.flagsparse_spmm_csr_opt(B=Bd, prepared=p),
-                         oracle.spmm_csr(ip, cols, vals, Bd.cpu())) <= 1e-5
