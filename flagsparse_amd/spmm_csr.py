@@ -143,10 +143,9 @@ def _spmm_opt_reference_error(candidate, reference, value_dtype):
 # ------------------------------------------------------------------------------------------
 
 
-def _check_spmm_csr_matrix(data, indices, indptr, shape, ptr_bits, count_long=False):
+def _check_spmm_csr_matrix(data, indices, indptr, shape, ptr_bits):
     """The checks of spmm_csr.py:197-255 (same order and exceptions): (data, int32 columns, row
-    pointers of ``ptr_bits``, n_rows, n_cols, longest row, and with ``count_long`` the entries in
-    rows that a row block cuts into parts, else None)."""
+    pointers of ``ptr_bits``, n_rows, n_cols, longest row)."""
     if len(shape) != 2:
         raise ValueError("shape must be a 2-tuple: (n_rows, n_cols)")
     if data.ndim != 1 or indices.ndim != 1 or indptr.ndim != 1:
@@ -174,9 +173,8 @@ def _check_spmm_csr_matrix(data, indices, indptr, shape, ptr_bits, count_long=Fa
     nnz = data.numel()
     data, indices, indptr = data.contiguous(), indices.contiguous(), indptr.contiguous()
     # one pass over the index arrays, one host synchronisation
-    stats, kernel_indices, kernel_ptr = csr_check(
-        indices, indptr, ptr_bits, (0, 0, _SPMM_ROW_SPLIT_THRESHOLD) if count_long else ())
-    first, last, decreases, max_row_nnz, min_col, max_col = stats[:6]
+    (first, last, decreases, max_row_nnz, min_col, max_col), kernel_indices, kernel_ptr = \
+        csr_check(indices, indptr, ptr_bits)
     if first != 0:
         raise ValueError("indptr[0] must be 0")
     if last != nnz:
@@ -189,15 +187,23 @@ def _check_spmm_csr_matrix(data, indices, indptr, shape, ptr_bits, count_long=Fa
         if max_col > _INDEX_LIMIT_INT32:
             raise ValueError(
                 "column indices exceed the int32 range supported by the Triton kernel")
-    return (data, kernel_indices, kernel_ptr, n_rows, n_cols, int(max_row_nnz),
-            stats[7] if count_long else None)
+    return data, kernel_indices, kernel_ptr, n_rows, n_cols, int(max_row_nnz)
+
+
+def _prepare_spmm_csr_matrix(data, indices, indptr, shape):
+    """spmm_csr.py:197-255 (same checks, order and exceptions), row pointers as int64."""
+    data, kernel_indices, kernel_indptr, n_rows, n_cols, max_row_nnz = \
+        _check_spmm_csr_matrix(data, indices, indptr, shape, 64)
+    row_lengths = (kernel_indptr[1:] - kernel_indptr[:-1] if n_rows > 0
+                   else kernel_indptr.new_empty((0,)))
+    return data, kernel_indices, kernel_indptr, n_rows, n_cols, row_lengths, max_row_nnz
 
 
 def _prepare_spmm_csr_inputs(data, indices, indptr, B, shape):
     """spmm_csr.py:258-281, row pointers at the width the kernels read."""
     if B.ndim != 2:
         raise ValueError("B must be a 2D dense tensor")
-    data, kernel_indices, kernel_indptr, n_rows, n_cols, max_row_nnz, _ = \
+    data, kernel_indices, kernel_indptr, n_rows, n_cols, max_row_nnz = \
         _check_spmm_csr_matrix(data, indices, indptr, shape,
                                32 if data.numel() <= _common.ROWPTR32_MAX_NNZ else 64)
     if B.shape[0] != n_cols:
@@ -346,17 +352,14 @@ def _parts_by_column(desc, cols, n_cols, rowptr, chunk):
 class _SpmmKernelCsr:
     """Kernel-facing CSR arrays (aligned, int32 offsets when they fit), their row-block plans per
     G and their slices.  max_row_nnz: the longest row, where known; one_shot: the object serves
-    one call, so nothing is planned; long_entries: those in rows of more than
-    _SPMM_ROW_SPLIT_THRESHOLD entries, where counted."""
+    one call, so nothing is planned."""
 
     __slots__ = ("data", "cols", "rowptr", "rowptr_bits", "nnz", "n_rows", "_plans", "_args",
-                 "_keep", "_order", "max_row_nnz", "one_shot", "_tables", "_shared",
-                 "long_entries")
+                 "_keep", "_order", "max_row_nnz", "one_shot", "_tables", "_shared")
 
-    def __init__(self, data, cols, indptr, max_row_nnz=None, one_shot=False, long_entries=None):
+    def __init__(self, data, cols, indptr, max_row_nnz=None, one_shot=False):
         self.max_row_nnz = max_row_nnz
         self.one_shot = one_shot
-        self.long_entries = long_entries
         self.data = _aligned(data)
         self.cols = _aligned(cols)
         self.nnz = int(data.numel())
@@ -388,25 +391,19 @@ class _SpmmKernelCsr:
                 "plans": plans,
                 "slices": {k[0]: int(t[0].numel()) // 2 - 1 for k, t in self._tables.items()}}
 
-    def sliced(self, lanes=1):
-        """Whether products run on slices whatever their N (of ``lanes`` lanes on row blocks).  Row
-        blocks are kept where they are the faster: prepared, every row one group's work but for a
-        tenth of the entries (and, in _run_spmm, N, B and C whole vectors).  Measured on MI355X, row
-        blocks / slices: fp32 N=16, 100k rows of 0 to 32 entries 18.4 / 20.8 us; N=33, 3M entries
-        80.6 / 53.0; a power law, N=128 457 / 316, N=47 326 / 214; 50k rows of 200, N=16 90 / 57.
-        With few long rows, fp32: 300k rows of 32 and one of 3000, N=16 136 / 155, N=64 105 / 150
-        (columns near the diagonal); 1M of 0 to 24 and one of 200, N=8 49 / 55; 300k of 0 to 60 and
-        300 of 400, N=16 53 / 81.  Of those, short rows on 32 lanes and more are left to the slices:
-        1M rows of 5, 100 of 300, fp64 N=64 404 / 335, fp32 N=128 433 / 442.  A matrix used once has
-        no plan to use.  A prepared one with rows of more than _SPMM_SUMS_KEPT entries keeps the row
-        blocks' order of additions (see there)."""
+    def sliced(self):
+        """Whether products run on slices whatever their N.  Row blocks are kept where they are
+        the faster: prepared, every row one group's work (and, in _run_spmm, N, B and C whole
+        vectors).  Measured on MI355X, row blocks / slices: fp32 N=16, 100k rows of 0 to 32
+        entries 18.4 / 20.8 us; N=33, 3M entries 80.6 / 53.0; a power law, N=128 457 / 316, N=47
+        326 / 214.  Short rows with a few of more than 128 entries are the faster on row blocks too
+        (300k rows of 0 to 60 and 300 of 400, fp32 N=16 53 / 81), but sums are more exact on slices
+        (there 1.2e-7 / 6.7e-8 of the result).  A matrix used once has no plan to use.  A prepared
+        one with rows of more than _SPMM_SUMS_KEPT entries keeps the row blocks' order of additions
+        (see there)."""
         if self.one_shot or self.max_row_nnz is None:
             return True
-        if not _SPMM_ROW_SPLIT_THRESHOLD < self.max_row_nnz <= _SPMM_SUMS_KEPT:
-            return False
-        if self.long_entries is None or 10 * self.long_entries >= self.nnz:
-            return True
-        return lanes >= 32 and self.nnz <= 16 * self.n_rows
+        return _SPMM_ROW_SPLIT_THRESHOLD < self.max_row_nnz <= _SPMM_SUMS_KEPT
 
     def slices(self, items, keep, n_cols, by_column):
         """The slices' boundaries and launch order (built on the current stream, once)."""
@@ -548,7 +545,7 @@ def _run_spmm(kc, B, C, acc_f64, tile_cols=None):
         kept = not kc.one_shot and (kc.max_row_nnz or 0) > _SPMM_SUMS_KEPT
         # the row-block kernel's loads need aligned vectors
         bound = None
-        if not (kc.sliced(lanes) or (vec < slice_vec and not kept)):
+        if not (kc.sliced() or (vec < slice_vec and not kept)):
             bound = _bind_row_blocks(kc, B, acc_f64, lanes, vec)
         if bound is None:
             bound = _bind_sliced(kc, B, acc_f64, slice_lanes, slice_vec)
@@ -598,7 +595,6 @@ class PreparedCsrSpmmOpt:
         "long_row_fallback_only",
         "_ref_meta",
         "_kernel",
-        "_long_entries",
     )
 
     def __init__(self, data, kernel_indices, kernel_indptr, shape, n_rows, n_cols, row_lengths,
@@ -615,12 +611,11 @@ class PreparedCsrSpmmOpt:
         self.long_row_fallback_only = False
         self._ref_meta = None
         self._kernel = None
-        self._long_entries = None
 
     def _kernel_csr(self, one_shot=False):
         if self._kernel is None:
             self._kernel = _SpmmKernelCsr(self.data, self.kernel_indices, self.kernel_indptr,
-                                          self.max_row_nnz, one_shot, self._long_entries)
+                                          self.max_row_nnz, one_shot)
         return self._kernel
 
     def _reference_metadata(self):
@@ -702,13 +697,10 @@ def prepare_spmm_csr_opt(data, indices, indptr, shape):
 
 def _prepare_spmm_csr_opt(data, indices, indptr, shape, one_shot):
     """prepare_spmm_csr_opt; one_shot: for a single call, so nothing is planned."""
-    data, kernel_indices, kernel_indptr, n_rows, n_cols, max_row_nnz, long_entries = \
-        _check_spmm_csr_matrix(data, indices, indptr, shape, 64, count_long=not one_shot)
-    row_lengths = (kernel_indptr[1:] - kernel_indptr[:-1] if n_rows > 0
-                   else kernel_indptr.new_empty((0,)))
+    (data, kernel_indices, kernel_indptr, n_rows, n_cols, row_lengths,
+     max_row_nnz) = _prepare_spmm_csr_matrix(data, indices, indptr, shape)
     prepared = PreparedCsrSpmmOpt(data, kernel_indices, kernel_indptr, shape, n_rows, n_cols,
                                   row_lengths, max_row_nnz)
-    prepared._long_entries = long_entries
     if prepared.supports_opt and n_rows > 0:
         prepared._kernel_csr(one_shot)
     return prepared

@@ -325,9 +325,10 @@ def test_room_at_size(dev):
     ptr = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
     cols = torch.arange(int(ptr[-1]), dtype=torch.int32) % 1000
     data = torch.ones(cols.numel())
-    C, kc = _run(data, cols, ptr, torch.ones(1000, 256), (n, 1000), dev, False)
+    p = fs.prepare_spmm_csr_opt(data.to(dev), cols.to(dev), ptr.to(dev), (n, 1000))
+    C = fs.flagsparse_spmm_csr_opt(B=torch.ones(1000, 256, device=dev), prepared=p)
     assert torch.equal(C, lengths.float().to(dev)[:, None].expand_as(C))
-    (sums,) = _shared(kc, "sums")
+    (sums,) = _shared(p._kernel_csr(), "sums")
     assert 2 * 256 <= sums.numel() <= 5 * 256
 
 
@@ -403,23 +404,3 @@ def test_more_row_blocks_than_a_launch_holds(dev, monkeypatch):
     C = fs.flagsparse_spmm_csr_opt(B=B.to(dev), prepared=p)
     assert p._kernel_csr()._tables
     assert oracle.rel_l2(C, oracle.spmm_csr(ip, cols, vals, B)) <= 1e-5
-
-
-@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
-@pytest.mark.parametrize("base,rows,N,blocks", [
-    (32, [3000], 16, True), (32, [3000], 256, True), (12, [200, 700], 8, True),
-    (32, [3000], 15, False),            # no whole vectors
-    (5, [300], 8, True), (5, [300], 256, False),  # short rows on 64 lanes
-    (32, [3000] * 30, 16, False)])      # long rows that matter
-def test_few_long_rows_keep_row_blocks(dev, base, rows, N, blocks, dtype):
-    lengths = torch.full((5000,), base, dtype=torch.int64)
-    lengths[torch.arange(len(rows)) * 7 + 2500] = torch.tensor(rows)
-    ip = torch.cat([torch.zeros(1, dtype=torch.int64), lengths.cumsum(0)])
-    cols = synthetic.randint(3, 1, int(ip[-1]), 4000, "cpu")
-    vals = synthetic.uniform_values(3, 2, cols.numel(), dtype, "cpu")
-    B = synthetic.dense_uniform(4000, N, dtype, seed=3, device="cpu")
-    p = fs.prepare_spmm_csr_opt(vals.to(dev), cols.to(dev), ip.to(dev), (5000, 4000))
-    C = fs.flagsparse_spmm_csr_opt(B=B.to(dev), prepared=p)
-    assert p._kernel_csr().kernel_name(N) == ("spmm_rowblock_kernel" if blocks
-                                              else "spmm_slices_kernel")
-    assert oracle.rel_l2(C, oracle.spmm_csr(ip, cols, vals, B)) <= oracle.REL_L2_BOUND[str(dtype)[6:]]
