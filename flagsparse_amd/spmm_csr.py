@@ -420,7 +420,7 @@ class _SpmmKernelCsr:
         either end of every slice, or, where that is too much, for each piece.  Calls are ordered
         (StreamOrder), so those of one size share it."""
         length, cut = (table.numel() - 2) * n_dense_cols, 1
-        if length > _SUMS_ROOM // 8 and length * dtype.itemsize > _SUMS_ROOM and (
+        if length * dtype.itemsize > _SUMS_ROOM and (
                 ("pieces", items) in self._shared
                 or not torch.cuda.is_current_stream_capturing()):  # the count is waited for
             counted = self._shared.get(("pieces", items))
@@ -490,13 +490,18 @@ def _bind_sliced(kc, B, acc_f64, lanes, vec):
     if not by_column:
         items, keep = _spmm_slice_shape(lanes, positions)
     table, order = kc.slices(items, keep, n_cols, by_column)
-    if kc.max_row_nnz is None and (table.numel() - 2) * n_dense_cols > _SUMS_UNSEEN:
+    length = (table.numel() - 2) * n_dense_cols
+    if kc.max_row_nnz is None and length > _SUMS_UNSEEN:
         kc.max_row_nnz = int((kc.rowptr[1:] - kc.rowptr[:-1]).max())
     sums, cut = None, 0
     if kc.max_row_nnz is None or kc.max_row_nnz > keep:
-        table, sums, cut = kc.piece_slots((items, keep), table, n_dense_cols,
-                                          torch.float64 if acc_f64 else B.dtype)
-    kc._shared["name", n_dense_cols] = "spmm_slices_kernel"
+        dtype = torch.float64 if acc_f64 else B.dtype
+        if kc.one_shot and 8 * length <= _SUMS_ROOM:  # (piece_slots' first answer)
+            sums, cut = torch.empty(length, dtype=dtype, device=table.device), 1
+        else:
+            table, sums, cut = kc.piece_slots((items, keep), table, n_dense_cols, dtype)
+    if not kc.one_shot:
+        kc._shared["name", n_dense_cols] = "spmm_slices_kernel"
     kc._keep.extend((table, order, sums))
     return _abi.bind(
         "spmm_sliced", _abi.dtype_code(B.dtype), 1 if acc_f64 else 0, kc.data.data_ptr(),
